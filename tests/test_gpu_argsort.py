@@ -182,6 +182,27 @@ def test_take_matches_oracle():
     np.testing.assert_array_equal(got.view(np.uint64)[gv], vals[::-1].view(np.uint64)[gv])
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 1023, 1024, 1025, 70001])
+def test_take_null_counts(n):
+    """The null count and bitmap at the edges of a wave's rows and of a workgroup's (256 rows x 4): nulls in
+    the values, in the indices, in both, and a result without any."""
+    rng = np.random.default_rng(n)
+    vals = rng.integers(-100, 100, 501).astype(np.int16)
+    valid = rng.random(501) > 0.3
+    idx = rng.integers(0, 501, n).astype(np.int32)
+    ivalid = rng.random(n) > 0.5
+    for va, iva in ((valid, None), (None, ivalid), (valid, ivalid), (None, None)):
+        r = am.MetalArray.from_numpy(vals, va).take(am.MetalArray.from_numpy(idx, iva))
+        want, wv = O.take(vals, idx, va, iva)
+        got, gv = r.to_numpy()
+        gv = np.ones(n, bool) if gv is None else gv
+        assert r.null_count == n - int(wv.sum())
+        np.testing.assert_array_equal(gv, wv)
+        np.testing.assert_array_equal(got[wv], want[wv])
+    empty = am.MetalArray.from_numpy(np.zeros(0, np.int64))
+    assert empty.take(am.MetalArray.from_numpy(idx, np.zeros(n, bool))).null_count == n
+
+
 def test_take_out_of_range():
     a = am.MetalArray.from_numpy(np.arange(10, dtype=np.int64))
     with pytest.raises(am.ArrowMetalError, match=r"take: index out of range \(array length 10\)"):
