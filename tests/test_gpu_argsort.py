@@ -162,6 +162,27 @@ def test_batch_matches_unbatched():
     np.testing.assert_array_equal(r2.to_numpy()[0], O.argsort(vals, None, True))
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 4097, 16383, 16384, 16385, 40001])
+def test_small_inputs_of_every_width(n):
+    """Up to 16,384 rows the argsort ranks by counting (one launch), above it takes the passes: the edges
+    of a workgroup's 64 rows and of the padding, for every key width, with many ties, the largest and the
+    smallest key (a value whose mapped key is all ones beside NaN and null rows), nulls at both ends."""
+    rng = np.random.default_rng(n)
+    valid = rng.random(n) >= 0.3
+    for dt in (np.int64, np.uint64, np.int32, np.uint32, np.int16, np.uint8, np.float64, np.float32):
+        if np.issubdtype(dt, np.integer):
+            lo, hi = np.iinfo(dt).min, np.iinfo(dt).max
+            vals = np.where(rng.random(n) < 0.5, rng.choice(np.array([lo, 0, hi], dtype=dt), n),
+                            rng.integers(lo, hi, n, dtype=dt, endpoint=True))
+        else:
+            vals = rng.choice(np.array([np.nan, -np.nan, np.inf, -np.inf, -0.0, 0.0, 1.5], dtype=dt), n)
+        vals = vals.astype(dt)
+        for desc, place, order in ((0, 0, 0), (1, 1, 0), (1, 0, 1), (0, 1, 2)):
+            check(vals, valid, desc, place, order, str(dt))
+        check(vals, None, 0, 0, 0, str(dt))
+        check(vals, np.zeros(n, bool), 1, 0, 0, str(dt))
+
+
 # ---------------------------------------------------------------- take
 
 
