@@ -311,6 +311,32 @@ def test_dense_group_by_out_of_range_and_nulls():
         assert_agg(gb2.sum(mv), O.group_by_dense(keys2, K, vals, 0, kv, vv), f"dense sum {it}")
 
 
+@pytest.mark.parametrize("K,n", [(1, 5000), (63, 5000), (64, 70000), (65, 70000), (9217, 100), (65535, 200000),
+                                 (65536, 200000), (65537, 200000), (65537, 3000)])
+def test_result_columns_at_word_and_launch_edges(K, n):
+    """Result columns are written 64 groups (one bitmap word) at a time by the kernel that combines the
+    partial tables, and in a launch of their own above 65,536 groups: null groups, counts and the shared
+    table of min and max, sum and mean at those edges, on the private, cached and partitioned paths."""
+    rng = np.random.default_rng(K + n)
+    keys = rng.integers(0, K, n).astype(np.int32)
+    keys[keys % 5 == 2] = 0                       # every fifth group is empty
+    vals = rng.integers(-10**6, 10**6, n).astype(np.int32)
+    vv = rng.random(n) > 0.3
+    gb = am.MetalArray.from_numpy(keys).group_by(K)
+    mv = am.MetalArray.from_numpy(vals, vv)
+    for agg, name in ((0, "sum"), (1, "count"), (2, "min"), (3, "max"), (4, "mean"), (5, "count_values")):
+        got = gb.count() if agg == 1 else getattr(gb, name)(mv)
+        want = O.group_by_dense(keys, K, vals if agg != 1 else None, agg, None, vv)
+        assert got.null_count == K - int(want[1].sum())
+        assert_agg(got, want, f"dense {name} K={K}")
+    f = rng.standard_normal(n)
+    g = am.group_by([am.MetalArray.from_numpy(keys)])
+    ids, D, _ = O.group_keys([keys])
+    mf = am.MetalArray.from_numpy(f, vv)
+    for op, name in ((0, "sum"), (3, "mean"), (4, "min"), (5, "max"), (2, "count")):
+        assert_agg(getattr(g, name)(mf), O.group_agg(ids, D, f, op, vv), f"float {name} K={K}")
+
+
 @pytest.mark.parametrize("dtype", [np.int64, np.int32, np.float64])
 def test_min_max_struct(dtype):
     """op 6 hash_min_max: a struct<min, max> whose fields equal ops 4 and 5 bit for bit."""
