@@ -12,17 +12,17 @@
 //
 // How it runs here (this build's own design; CDNA4 has native 64-bit global and LDS atomics, so none
 // of the reference's 32-bit carry work-arounds are needed):
-//   gb_build     one read of the key column into an open-addressing table of 16-byte slots
-//                (64-bit key, lowest row) with linear probing and a 64-bit CAS insert; every row
-//                records its slot. The key 0x8000000000000000 is the empty marker and has a slot of
+//   gb_build     one read of the key column into an open-addressing table of 64-bit keys with linear
+//                probing and a 64-bit CAS insert; every row records its slot. The key 0x8000000000000000 is the empty marker and has a slot of
 //                its own past the end of the table.
 //   gb_compact   the occupied slots, in any order
 //   (argsort)    the distinct keys' order keys, sorted by the radix argsort of sort.hip
-//   gb_relabel   slot -> ascending group id, and the representative rows
+//   gb_relabel   slot -> ascending group id
 //   gb_ids       each row's slot -> its group id, in place
 //   gb_agg<P>    one pass over (ids, values) for a family of aggregates: a private LDS table per
 //                workgroup when the groups fit, otherwise an LDS cache of the groups a workgroup sees
-//                (claimed by CAS) in front of global 64-bit atomics; flushed once per workgroup.
+//                (claimed by CAS) in front of global 64-bit atomics; flushed once per workgroup. The
+//                representative (lowest) rows are such a pass too, the minimum of each group's rows.
 #include "am_internal.hpp"
 #include "fsum.hpp"
 
@@ -146,16 +146,13 @@ __device__ __forceinline__ unsigned long long order_key(unsigned long long gk, i
   return gk;
 }
 
-// The hash table is two arrays of cap + 1 entries: the keys (EMPTY when free; entry cap holds the
-// EMPTY key itself) and, for builds that track them, the lowest row of each key.
+// The hash table: cap + 1 keys (EMPTY when free; entry cap holds the EMPTY key itself).
 struct Table {
   unsigned long long* key;
-  uint32_t* first;   // null when not tracked
 };
 
 struct BuildStatus {
   uint32_t overflow;
-  uint32_t null_first;
   uint32_t distinct;
   uint32_t special_used;   // the EMPTY key has been seen: slot C holds it
   unsigned long long nulls;
@@ -167,22 +164,14 @@ __global__ void gb_table_init(Table table, size_t slots, BuildStatus* st) {
   size_t stride = size_t(gridDim.x) * blockDim.x;
   for (; i < slots; i += stride) {
     table.key[i] = EMPTY;
-    if (table.first) table.first[i] = 0xFFFFFFFFu;
   }
   if (st && blockIdx.x == 0 && threadIdx.x == 0) {
     st->overflow = 0;
-    st->null_first = 0xFFFFFFFFu;
     st->distinct = 0;
     st->special_used = 0;
     for (int x = 0; x < NXCD; x++) st->xspecial[x] = 0;
     st->nulls = 0;
   }
-}
-
-// A slot's lowest row only decreases, so a plain (possibly stale) read is a safe filter: a stale
-// value is never below the true one, and the atomic settles every row that could lower it.
-__device__ __forceinline__ void lower_first(uint32_t* p, uint32_t row) {
-  if (row < *p) atomicMin(p, row);
 }
 
 // A probe's read of a slot key, through this XCD's L2. A stale EMPTY only sends the row to the CAS,
@@ -335,7 +324,7 @@ struct ScanAcc {
   uint32_t nf = 0xFFFFFFFFu;
 };
 
-template <int TYPE, bool HAS_VALID>
+template <int TYPE, bool HAS_VALID, bool REGS>
 __device__ __forceinline__ void scan_rows(int64_t voff, uint32_t n, uint64_t row0, uint32_t gsize, const ScanRows& x,
                                           uint32_t* r_lds, ScanAcc& acc) {
   constexpr bool RANGE = TYPE >= T_I8 && TYPE <= T_U64;
@@ -359,11 +348,13 @@ __device__ __forceinline__ void scan_rows(int64_t voff, uint32_t n, uint64_t row
         acc.nf = null_row ? min(acc.nf, uint32_t(i)) : acc.nf;
       }
     }
+    if (!REGS) continue;
     const uint32_t h = hll_hash(gk);
     idx[r] = h >> (32 - HLL_BITS);
     const uint32_t w = h << HLL_BITS;
     rank[r] = !ok ? 0u : w ? uint32_t(__clz(int(w))) + 1u : uint32_t(32 - HLL_BITS + 1);
   }
+  if (!REGS) return;
   // The step's register reads are issued together; a register is raised only when the row's rank is
   // larger (a null row or a row past the end has rank 0).
   uint32_t cur[SCAN_ROWS];
@@ -374,20 +365,22 @@ __device__ __forceinline__ void scan_rows(int64_t voff, uint32_t n, uint64_t row
     if (rank[r] > cur[r]) atomicMax(&r_lds[idx[r]], rank[r]);
 }
 
-template <int W, int TYPE, bool HAS_VALID>
+template <int W, int TYPE, bool HAS_VALID, bool REGS>
 __global__ __launch_bounds__(scan_threads<HAS_VALID>()) void gb_key_scan(const void* vals, const uint8_t* valid, int64_t voff, uint32_t n,
                                                    uint32_t* regs, RangeStat* st) {
   constexpr bool RANGE = TYPE >= T_I8 && TYPE <= T_U64;
-  __shared__ uint32_t r[HLL_M];   // regs: HLL_M bytes per workgroup; st: one per workgroup
+  // regs: HLL_M bytes per workgroup (REGS); st: one per workgroup.
+  __shared__ uint32_t r[REGS ? HLL_M : 4];
   constexpr uint32_t SCAN_WAVES = scan_threads<HAS_VALID>() / 64;
   __shared__ unsigned long long s_lo[SCAN_WAVES], s_hi[SCAN_WAVES], s_nz[SCAN_WAVES];
   __shared__ uint32_t s_nf[SCAN_WAVES];
-  for (uint32_t j = threadIdx.x; j < HLL_M; j += blockDim.x) r[j] = 0u;
+  if (REGS)
+    for (uint32_t j = threadIdx.x; j < HLL_M; j += blockDim.x) r[j] = 0u;
   __syncthreads();
   const uint32_t gsize = gridDim.x * blockDim.x;
   ScanAcc acc;
   scan_steps<W, HAS_VALID>(vals, valid, voff, n, [&](uint64_t row0, const ScanRows& x) {
-    scan_rows<TYPE, HAS_VALID>(voff, n, row0, gsize, x, r, acc);
+    scan_rows<TYPE, HAS_VALID, REGS>(voff, n, row0, gsize, x, r, acc);
   });
   if (RANGE) {
     for (int off = 32; off > 0; off >>= 1) {
@@ -415,6 +408,7 @@ __global__ __launch_bounds__(scan_threads<HAS_VALID>()) void gb_key_scan(const v
     }
     st[blockIdx.x] = RangeStat{acc.lo, acc.hi, acc.nz, acc.nf, 0u};
   }
+  if (!REGS) return;
   for (uint32_t j = threadIdx.x; j < HLL_M / 4; j += blockDim.x)
     regs[size_t(blockIdx.x) * (HLL_M / 4) + j] = r[4 * j] | r[4 * j + 1] << 8 | r[4 * j + 2] << 16 | r[4 * j + 3] << 24;
 }
@@ -431,10 +425,16 @@ void key_scan(int type, hipStream_t s, const void* vals, const uint8_t* valid, i
   const dim3 grid{key_scan_blocks(valid != nullptr, n)}, block{valid ? scan_threads<true>() : scan_threads<false>()};
   with_key_type(type, [&](auto tc) {
     constexpr int TT = decltype(tc)::value;
-    if (valid)
-      hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, true>), grid, block, 0, s, vals, valid, voff, n, regs, st);
-    else
-      hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, false>), grid, block, 0, s, vals, valid, voff, n, regs, st);
+    constexpr bool RANGE = TT != T_F32 && TT != T_F64;   // only integer columns are scanned without registers
+    if (regs) {
+      if (valid) hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, true, true>), grid, block, 0, s, vals, valid, voff, n, regs, st);
+      else hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, false, true>), grid, block, 0, s, vals, valid, voff, n, regs, st);
+    } else if constexpr (RANGE) {
+      if (valid) hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, true, false>), grid, block, 0, s, vals, valid, voff, n, regs, st);
+      else hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, false, false>), grid, block, 0, s, vals, valid, voff, n, regs, st);
+    } else {
+      fail("internal: a span scan of a float column");
+    }
   });
 }
 
@@ -444,6 +444,22 @@ struct FoldCtl {
   unsigned int ticket, pad;
   unsigned long long nulls, redo;
 };
+
+// Waits for an atomic by its result, so that it has been carried out (at the memory side, where every
+// XCD's atomics meet) before anything that follows. A device-scope fence would instead write back the
+// XCD's whole L2: 12 us for the 625 workgroups of a result over 40,000 groups.
+template <typename T>
+__device__ __forceinline__ void atomic_done(T result) {
+  asm volatile("" ::"v"(result) : "memory");
+}
+
+// True in the last workgroup of the grid to ask (one thread each); the counter is 0 again after it.
+__device__ __forceinline__ bool take_ticket(FoldCtl* c) {
+  const unsigned int last = gridDim.x - 1u;
+  const bool mine = atomicInc(&c->ticket, last) == last;
+  asm volatile("" ::: "memory");
+  return mine;
+}
 
 __global__ void gb_clear_ctl(FoldCtl* c) { *c = FoldCtl{0, 0, 0, 0}; }
 
@@ -536,11 +552,9 @@ __global__ __launch_bounds__(1024) void gb_key_estimate(const uint32_t* regs, co
     }
     out->r = r;
   }
-  __hip_atomic_store(&parts[blockIdx.x].sum, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(&parts[blockIdx.x].zeros, zeros, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __threadfence();
-  if (atomicInc(&ctl->ticket, EST_BLOCKS - 1u) != EST_BLOCKS - 1u) return;   // wraps to 0
-  __threadfence();
+  atomic_done(atomicExch(&parts[blockIdx.x].sum, sum));
+  atomic_done(atomicExch(&parts[blockIdx.x].zeros, zeros));
+  if (!take_ticket(ctl)) return;
   sum = 0.f;
   zeros = 0;
   for (uint32_t b = 0; b < EST_BLOCKS; b++) {   // in workgroup order: the same sum whichever is last
@@ -555,8 +569,7 @@ __global__ __launch_bounds__(1024) void gb_key_estimate(const uint32_t* regs, co
 
 // Inserts every row's key; writes the slot of each row (NULL_SLOT for a null key). Each thread keeps
 // BUILD_ROWS rows in flight: their keys are loaded, hashed and their first slots read together, so a
-// wave waits on one memory latency per BUILD_ROWS rows rather than per row. TRACK_FIRST also keeps
-// every slot's lowest row (the representative rows of float and multi-column keys).
+// wave waits on one memory latency per BUILD_ROWS rows rather than per row.
 //
 // Each workgroup keeps the slots of the keys it has seen in an LDS cache (BUILD_CACHE entries, direct
 // mapped by high hash bits, each written once: the key by CAS, then its slot). A row whose key is
@@ -614,7 +627,6 @@ __device__ __forceinline__ void build_load(const void* vals, const uint8_t* vali
 // What a thread of gb_build keeps across its steps.
 struct BuildState {
   unsigned long long* tkey;
-  uint32_t* tfirst;
   uint32_t* special_flag;
   uint32_t tbase, special, cap_mask, budget;
   unsigned long long* ckey;
@@ -627,11 +639,10 @@ struct BuildState {
 // next step's rows are loaded (into `nxt`, at `nbase`), so that those loads are in flight while this
 // step waits for its slots, and waiting for the slots never waits for them (memory operations
 // complete in issue order).
-template <bool TRACK_FIRST, int W, int KT, bool NV>
+template <int W, int KT, bool NV>
 __device__ __forceinline__ void build_step(const void* vals, int type, const uint8_t* valid, int64_t voff, uint32_t n,
                                            uint64_t base, uint64_t nbase, uint32_t gsize, uint32_t tid,
-                                           const BuildRows& cur, BuildRows& nxt, uint32_t* slot_of, BuildStatus* st,
-                                           BuildState& b) {
+                                           const BuildRows& cur, BuildRows& nxt, uint32_t* slot_of, BuildState& b) {
 #pragma unroll
   for (int r = 0; r < BUILD_ROWS; r++) asm volatile("" ::"v"(cur.k[r]), "v"(cur.vb[r]));   // every loaded register taken here
   unsigned long long k[BUILD_ROWS], cv[BUILD_ROWS];
@@ -679,7 +690,6 @@ __device__ __forceinline__ void build_step(const void* vals, int type, const uin
     if (cat[r] == 1) {
       slot = NULL_SLOT;
       b.nulls++;
-      if (TRACK_FIRST) lower_first(&st->null_first, i);
     } else if (cat[r] == 2) {
       slot = b.special;
       if (!*b.special_flag) atomicExch(b.special_flag, 1u);
@@ -693,7 +703,6 @@ __device__ __forceinline__ void build_step(const void* vals, int type, const uin
       continue;
     }
     __builtin_nontemporal_store(slot == NULL_SLOT ? NULL_SLOT : b.tbase + slot, slot_of + i);
-    if (TRACK_FIRST && slot != NULL_SLOT) lower_first(&b.tfirst[slot], i);
   }
   while (slow) {
     const int r = __builtin_ctz(slow);
@@ -706,11 +715,10 @@ __device__ __forceinline__ void build_step(const void* vals, int type, const uin
     if (slot == NULL_SLOT) b.overflow = true;
     else cache_slot(b.ckey, b.cslot, cache_entry(hh), kk, slot);
     __builtin_nontemporal_store(slot == NULL_SLOT ? NULL_SLOT : b.tbase + slot, slot_of + i);
-    if (TRACK_FIRST && slot != NULL_SLOT) lower_first(&b.tfirst[slot], i);
   }
 }
 
-template <bool TRACK_FIRST, int W, int KT, bool NV>
+template <int W, int KT, bool NV>
 __global__ __launch_bounds__(BUILD_THREADS) void gb_build(const void* vals, int type, const uint8_t* valid, int64_t voff,
                                                 uint32_t n, Table table, uint32_t cap_mask, uint32_t budget,
                                                 uint32_t* slot_of, BuildStatus* st, int private_tables) {
@@ -723,7 +731,6 @@ __global__ __launch_bounds__(BUILD_THREADS) void gb_build(const void* vals, int 
   BuildState b;
   b.tbase = tbl * (cap_mask + 2u);
   b.tkey = table.key + b.tbase;
-  b.tfirst = TRACK_FIRST ? table.first + b.tbase : nullptr;
   b.special_flag = private_tables ? &st->xspecial[tbl] : &st->special_used;
   b.special = cap_mask + 1u;
   b.cap_mask = cap_mask;
@@ -747,10 +754,9 @@ __global__ __launch_bounds__(BUILD_THREADS) void gb_build(const void* vals, int 
     build_load<W, NV>(vals, valid, voff, n, 0, gsize, tid, xa);
     for (int t = 0; t < steps; t += 2) {
       const uint64_t base = uint64_t(t) * stride;
-      build_step<TRACK_FIRST, W, KT, NV>(vals, type, valid, voff, n, base, base + stride, gsize, tid, xa, xb, slot_of, st, b);
+      build_step<W, KT, NV>(vals, type, valid, voff, n, base, base + stride, gsize, tid, xa, xb, slot_of, b);
       if (t + 1 >= steps) break;
-      build_step<TRACK_FIRST, W, KT, NV>(vals, type, valid, voff, n, base + stride, base + 2 * stride, gsize, tid, xb, xa,
-                                 slot_of, st, b);
+      build_step<W, KT, NV>(vals, type, valid, voff, n, base + stride, base + 2 * stride, gsize, tid, xb, xa, slot_of, b);
     }
   }
   if (b.overflow) atomicOr(&st->overflow, 1u);
@@ -760,10 +766,8 @@ __global__ __launch_bounds__(BUILD_THREADS) void gb_build(const void* vals, int 
 }
 
 // Folds the eight XCD-private tables into one table of cap + 1 entries: every occupied private slot
-// inserts its key (a few per distinct key, not per row) and records where it went in xmap; lowest
-// rows merge by minimum.
-__global__ __launch_bounds__(256) void gb_merge_tables(const unsigned long long* xkeys, const uint32_t* xfirst,
-                                                       uint32_t cap, BuildStatus* st, Table g, uint32_t* xmap) {
+// inserts its key (a few per distinct key, not per row) and records where it went in xmap.
+__global__ __launch_bounds__(256) void gb_merge_tables(const unsigned long long* xkeys, uint32_t cap, BuildStatus* st, Table g, uint32_t* xmap) {
   const uint32_t per = cap + 1u;
   const uint32_t total = uint32_t(NXCD) * per;
   bool overflow = false;
@@ -784,7 +788,6 @@ __global__ __launch_bounds__(256) void gb_merge_tables(const unsigned long long*
       }
     }
     xmap[xs] = gs;
-    if (xfirst && gs != NULL_SLOT) lower_first(&g.first[gs], xfirst[xs]);
   }
   if (overflow) atomicOr(&st->overflow, 1u);
 }
@@ -852,16 +855,9 @@ __global__ __launch_bounds__(256) void gb_compact(const unsigned long long* tkey
   }
 }
 
-__global__ void gb_relabel(const uint32_t* perm, const uint32_t* slots, uint32_t D, const uint32_t* tfirst,
-                           uint32_t* gid_of_slot, uint32_t* rep, const BuildStatus* st, int has_null, int track) {
-  uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < D) {
-    uint32_t s = slots[perm[r]];
-    gid_of_slot[s] = r;
-    if (track) rep[r] = tfirst[s];
-  } else if (r == D && has_null && track) {
-    rep[D] = st->null_first;
-  }
+__global__ void gb_relabel(const uint32_t* perm, const uint32_t* slots, uint32_t D, uint32_t* gid_of_slot) {
+  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r < D) gid_of_slot[slots[perm[r]]] = r;
 }
 
 #ifndef AM_IDS_CACHE_BITS
@@ -1082,6 +1078,22 @@ struct CountP {
   static constexpr bool NEEDS_ROW = false;  // its contribution depends on the row number
   __device__ static bool contrib(const AggArgs&, int64_t, long long, unsigned long long, unsigned long long (&c)[1]) {
     c[0] = 1;
+    return true;
+  }
+};
+
+// The lowest row of each group (its representative row): no value, null or not.
+struct FirstRowP {
+  static constexpr int W = 1;
+  static constexpr bool SKIP_NULL = false;
+  __host__ __device__ static constexpr int op(int) { return W_MIN; }
+  static constexpr bool USES_VALUE = false;
+  static constexpr int FIXED_VW = 0;
+  static constexpr bool AUX = false;
+  static constexpr bool PART = true;
+  static constexpr bool NEEDS_ROW = true;
+  __device__ static bool contrib(const AggArgs&, int64_t row, long long, unsigned long long, unsigned long long (&c)[1]) {
+    c[0] = (unsigned long long)row;
     return true;
   }
 };
@@ -2175,13 +2187,12 @@ struct FoldOut {
   FoldCtl* ctl;
 };
 
-// One thread per workgroup: adds its null count; the last workgroup of the grid reports and clears.
+// One thread per workgroup: adds its null count; the last workgroup of the grid reports and clears. The
+// groups to sum again were counted by atomics whose results their lanes have stored, so those are done.
 __device__ __forceinline__ void fold_report(const FoldOut& fo, uint32_t nulls) {
   if (!fo.host) return;
-  if (nulls) atomicAdd(&fo.ctl->nulls, (unsigned long long)nulls);
-  __threadfence();
-  if (atomicInc(&fo.ctl->ticket, gridDim.x - 1u) == gridDim.x - 1u) {   // wraps to 0
-    __threadfence();
+  if (nulls) atomic_done(atomicAdd(&fo.ctl->nulls, (unsigned long long)nulls));
+  if (take_ticket(fo.ctl)) {
     *fo.host = atomicExch(&fo.ctl->nulls, 0ull);
     if (fo.redo) *fo.redo = atomicExch(&fo.ctl->redo, 0ull);
   }
@@ -2200,6 +2211,14 @@ struct FinNone {
 // word 1 of a sum table.
 constexpr int KIND_COUNT = 3;
 constexpr int KIND_SUM_COUNT = 6;
+struct FinFirst {
+  uint32_t* rep;
+  __device__ bool operator()(long long k, const unsigned long long (&t)[1], const FoldOut&) const {
+    rep[k] = uint32_t(t[0]);
+    return true;
+  }
+};
+
 struct FinSimple {
   int kind, vtype;
   void* out;
@@ -2481,7 +2500,7 @@ bool run_agg_part(const AggArgs& a, hipStream_t s, const char* name, unsigned lo
         if constexpr (P::NEEDS_ROW) launch(gb_part_reduce<P, 8, true>);
         else launch(gb_part_reduce<P, 8, false>);
       } else {
-        launch(gb_part_reduce<P, 0, false>);
+        launch(gb_part_reduce<P, 0, P::NEEDS_ROW>);
       }
       AM_HIP(hipGetLastError());
     }
@@ -2682,6 +2701,13 @@ __global__ __launch_bounds__(256) void fs_redo_settle(const uint32_t* redo, long
 
 // ================================================================ host: key mapping
 
+// One integer column's place in a composite key: its digit is (composite / div) % span, the column's
+// order key less kmin, or span - 1 for a null when the column has nulls.
+struct ColSpan {
+  unsigned long long kmin, span, div;
+  int has_null;
+};
+
 struct GroupBy {
   std::vector<Array*> columns;
   int64_t n = 0;
@@ -2689,10 +2715,12 @@ struct GroupBy {
   DevBuf ids;     // int32 [n]
   DevBuf rep;     // uint32 [K], the lowest row of each group (when tracked)
   bool has_rep = false;
-  // An integer single-column mapping keeps its sorted distinct keys instead of representative rows.
+  // A mapping of integer columns keeps its sorted distinct keys instead of representative rows: the order
+  // keys themselves, or, for several columns, the composite keys (ColSpan). perm null: already sorted.
   DevBuf okeys, perm;
   uint32_t D = 0;
   bool has_null = false;
+  std::vector<ColSpan> spans;
   std::vector<Array*> key_results;
   // A min and a max of one column share a pass; a sum and a mean of one float64 column share theirs;
   // an integer sum also yields the column's count of non-null values. Keyed by the column's unique
@@ -2734,7 +2762,7 @@ struct Mapped {
   int64_t K = 0;
   uint32_t D = 0;
   bool has_null = false;
-  DevBuf ids, rep, okeys, perm;
+  DevBuf ids, okeys, perm;
 };
 
 // ---------------------------------------------------------------- the range path
@@ -2752,12 +2780,12 @@ bool range_path_enabled() {
 // rows are tracked), a scan of the occupancy turns each present key into its rank, which is its id
 // in ascending key order, and one pass writes every row's id (the null group, last, is D).
 
-// occ[k - kmin] = 1 for every present key; first[k - kmin] = its lowest row when tracked. Both only
-// ever move one way, so a read that already shows the value skips the write. A step's reads are
-// issued together (a null row reads entry 0, which exists, and writes nothing).
-template <int W, int TYPE, bool HAS_VALID, bool TRACK>
+// occ[k - kmin] = 1 for every present key (spans above RANGE_BITS_MAX). A mark that is already there is
+// not written again. A step's reads are issued together (a null row reads entry 0, which exists, and
+// writes nothing).
+template <int W, int TYPE, bool HAS_VALID>
 __global__ __launch_bounds__(256) void gb_range_occ(const void* vals, const uint8_t* valid, int64_t voff, uint32_t n,
-                                                    unsigned long long kmin, uint32_t* occ, uint32_t* first) {
+                                                    unsigned long long kmin, uint32_t* occ) {
   const uint32_t gsize = gridDim.x * blockDim.x;
   scan_steps<W, HAS_VALID>(vals, valid, voff, n, [&](uint64_t row0, const ScanRows& x) {
     scan_take<HAS_VALID>(x);
@@ -2770,32 +2798,26 @@ __global__ __launch_bounds__(256) void gb_range_occ(const void* vals, const uint
       ok[r] = i < n && (HAS_VALID ? vbit(voff, ii, x.vb[r]) != 0u : true);
       xs[r] = ok[r] ? uint32_t(order_key(key_of_raw(x.raw[r], TYPE), TYPE) - kmin) : 0u;
     }
-    uint32_t cur[SCAN_ROWS], low[SCAN_ROWS];
+    uint32_t cur[SCAN_ROWS];
 #pragma unroll
-    for (int r = 0; r < SCAN_ROWS; r++) {
-      cur[r] = occ[xs[r]];
-      if (TRACK) low[r] = first[xs[r]];
-    }
-    // Plain accesses: a stale 0 costs one more store of the same 1; a stale row is larger than the
-    // current lowest one, so it never skips a needed atomicMin.
+    for (int r = 0; r < SCAN_ROWS; r++) cur[r] = occ[xs[r]];
 #pragma unroll
-    for (int r = 0; r < SCAN_ROWS; r++) {
+    for (int r = 0; r < SCAN_ROWS; r++)   // a stale 0 costs one more store of the same 1
       if (ok[r] && cur[r] == 0u) occ[xs[r]] = 1u;
-      const uint32_t i = uint32_t(row0 + uint64_t(r) * gsize);
-      if (TRACK && ok[r] && i < low[r]) atomicMin(&first[xs[r]], i);
-    }
   });
 }
 
-// The occupancy of a span of at most RANGE_BITS_MAX keys without representative rows: each workgroup
-// marks its rows' keys in a bitmap of the span in LDS, then ORs its words into the global bitmap (a word
-// already holding the bits is only read). gb_range_unpack turns the bitmap into occ[].
+// The occupancy of a span of at most RANGE_BITS_MAX keys: each workgroup marks its rows' keys in a bitmap
+// of the span in LDS and writes it out; gb_range_fold combines the workgroups' bitmaps. (ORing every
+// workgroup's words into one global bitmap is an atomic per word and workgroup while the bits are still
+// missing: 62 us for 3M int32 rows over 50,000 keys with nulls, 20 us in both kernels so.)
 constexpr uint32_t RANGE_BITS_MAX = 1u << 19;   // 64 KiB of LDS
+constexpr uint32_t OCC_THREADS = 512;
 
 template <int W, int TYPE, bool HAS_VALID>
-__global__ __launch_bounds__(256) void gb_range_occ_bits(const void* vals, const uint8_t* valid, int64_t voff,
-                                                         uint32_t n, unsigned long long kmin, uint32_t words,
-                                                         uint32_t* bits) {
+__global__ __launch_bounds__(OCC_THREADS) void gb_range_occ_bits(const void* vals, const uint8_t* valid, int64_t voff,
+                                                                 uint32_t n, unsigned long long kmin, uint32_t words,
+                                                                 uint32_t* part) {
   extern __shared__ uint32_t s_bits[];
   for (uint32_t j = threadIdx.x; j < words; j += blockDim.x) s_bits[j] = 0u;
   __syncthreads();
@@ -2820,15 +2842,80 @@ __global__ __launch_bounds__(256) void gb_range_occ_bits(const void* vals, const
       if ((cur[r] & bit[r]) != bit[r]) atomicOr(&s_bits[wd[r]], bit[r]);
   });
   __syncthreads();
-  for (uint32_t j = threadIdx.x; j < words; j += blockDim.x) {
-    const uint32_t v = s_bits[j];
-    if (v && (load_global(&bits[j]) & v) != v) atomicOr(&bits[j], v);
-  }
+  uint32_t* mine = part + size_t(blockIdx.x) * words;
+  for (uint32_t j = threadIdx.x; j < words; j += blockDim.x) mine[j] = s_bits[j];
 }
 
-__global__ void gb_range_unpack(const uint32_t* bits, uint32_t span, uint32_t* occ) {
-  const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x < span) occ[x] = (bits[x >> 5] >> (x & 31u)) & 1u;
+// A word of the combined occupancy: 32 keys' bits, and the number of keys present before them (within
+// the word's tile until gb_range_emit, over the whole span after it).
+struct RangeWord {
+  uint32_t bits, before;
+};
+constexpr uint32_t RANGE_FOLD = 64;   // words per workgroup of the fold: a tile of 2048 keys
+constexpr uint32_t RANGE_TILES_MAX = RANGE_BITS_MAX / 32 / RANGE_FOLD;
+static_assert(RANGE_TILES_MAX <= 1024, "the last workgroup scans the tiles with a thread each");
+
+// Combines the workgroups' bitmaps, 64 words per workgroup (wave w takes every 16th bitmap), counts each
+// word's predecessors in its tile, and, in the last workgroup done, turns the tiles' counts into their
+// bases and reports the number of distinct keys.
+__global__ __launch_bounds__(1024) void gb_range_fold(const uint32_t* part, uint32_t parts, uint32_t words, RangeWord* rw,
+                                                      uint32_t* tile_base, FoldCtl* ctl, unsigned long long* distinct) {
+  __shared__ uint32_t s_or[16][RANGE_FOLD];
+  __shared__ uint32_t s_last, s_tmp[16];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t j = blockIdx.x * RANGE_FOLD + lane, jj = min(j, words - 1u);
+  uint32_t v = 0;
+  constexpr uint32_t U = 8;
+  for (uint32_t c = wave; c < parts; c += 16 * U) {
+    uint32_t x[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) x[u] = part[size_t(min(c + 16 * u, parts - 1u)) * words + jj];
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) v |= x[u];   // a bitmap read twice changes nothing
+  }
+  s_or[wave][lane] = v;
+  __syncthreads();
+  if (wave == 0) {
+    v = 0;
+    for (int k = 0; k < 16; k++) v |= s_or[k][lane];
+    if (j >= words) v = 0;
+    const uint32_t c = uint32_t(__popc(v));
+    uint32_t incl = c;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t y = __shfl_up(incl, d, 64);
+      if (lane >= uint32_t(d)) incl += y;
+    }
+    if (j < words) rw[j] = RangeWord{v, incl - c};
+    if (lane == 63) {
+      atomic_done(atomicExch(&tile_base[blockIdx.x], incl));
+      s_last = take_ticket(ctl) ? 1u : 0u;
+    }
+  }
+  __syncthreads();
+  if (!s_last) return;   // uniform
+  const uint32_t t = threadIdx.x, tiles = gridDim.x;
+  const uint32_t c = t < tiles ? __hip_atomic_load(&tile_base[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+  uint32_t total;
+  const uint32_t before = block_scan_1024(c, s_tmp, total);
+  if (t < tiles) tile_base[t] = before;
+  if (t == 0) *distinct = total;
+}
+
+// Each present key's order key at its rank, and each word's count over the whole span.
+__global__ __launch_bounds__(256) void gb_range_emit(RangeWord* rw, uint32_t span, const uint32_t* tile_base,
+                                                     unsigned long long kmin, unsigned long long* okeys) {
+  const uint32_t x = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t w = x >> 5, bit = x & 31u;
+  RangeWord v{0, 0};
+  if (x < span) {
+    v = rw[w];
+    v.before += tile_base[w / RANGE_FOLD];
+  }
+  __syncthreads();   // the workgroup's words are its own, each read before it is written
+  if (x >= span) return;
+  if (bit == 0u) rw[w].before = v.before;
+  if ((v.bits >> bit) & 1u) okeys[v.before + uint32_t(__popc(v.bits & ((1u << bit) - 1u)))] = kmin + x;
 }
 
 constexpr uint32_t RANGE_TILE = 4096;   // occupancy entries per workgroup of the scan (16 per thread)
@@ -2872,11 +2959,9 @@ __global__ __launch_bounds__(1024) void gb_range_scan_tiles(uint32_t* tile_sum, 
   if (threadIdx.x == 0) *distinct = carry;
 }
 
-// Each present key's rank (its id) in place of its occupancy mark, the ascending order keys, and the
-// lowest row of each group when tracked.
+// Each present key's rank (its id) in place of its occupancy mark, and the ascending order keys.
 __global__ __launch_bounds__(256) void gb_range_rank(uint32_t* occ, uint32_t span, const uint32_t* tile_base,
-                                                     unsigned long long kmin, unsigned long long* okeys,
-                                                     const uint32_t* first, uint32_t* rep) {
+                                                     unsigned long long kmin, unsigned long long* okeys) {
   __shared__ uint32_t s[4];
   const uint32_t t0 = blockIdx.x * RANGE_TILE;
   uint32_t run = tile_base[blockIdx.x];
@@ -2896,16 +2981,18 @@ __global__ __launch_bounds__(256) void gb_range_rank(uint32_t* occ, uint32_t spa
       const uint32_t r = run + before + uint32_t(__popcll(bal & ((1ull << lane) - 1ull)));
       occ[x] = r;
       okeys[r] = kmin + x;
-      if (rep) rep[r] = first[x];
     }
     run += total;
     __syncthreads();
   }
 }
 
-// Every row's id: the rank of its key's occupancy entry, or null_gid for a null row. With DENSE every
-// key of the span is present, so a key's rank is its offset in the span and nothing is looked up.
-template <int W, int TYPE, bool HAS_VALID, bool DENSE>
+// Every row's id: the rank of its key's occupancy entry (RANK_TABLE) or of its bit in the combined bitmap
+// (RANK_WORDS: 8 bytes per 32 keys, so the lookups of a small span stay in L1), or null_gid for a null
+// row. RANK_DENSE: every key of the span is present, so a key's rank is its offset in the span and nothing
+// is looked up.
+enum RankMode : int { RANK_TABLE = 0, RANK_WORDS = 1, RANK_DENSE = 2 };
+template <int W, int TYPE, bool HAS_VALID, int MODE>
 __global__ __launch_bounds__(256) void gb_range_ids(const void* vals, const uint8_t* valid, int64_t voff, uint32_t n,
                                                     unsigned long long kmin, const uint32_t* rank, uint32_t null_gid,
                                                     uint32_t* ids) {
@@ -2922,8 +3009,17 @@ __global__ __launch_bounds__(256) void gb_range_ids(const void* vals, const uint
       xs[r] = ok[r] ? uint32_t(order_key(key_of_raw(x.raw[r], TYPE), TYPE) - kmin) : 0u;
     }
     uint32_t g[SCAN_ROWS];
+    if constexpr (MODE == RANK_WORDS) {
+      RangeWord v[SCAN_ROWS];
 #pragma unroll
-    for (int r = 0; r < SCAN_ROWS; r++) g[r] = DENSE ? xs[r] : rank[xs[r]];
+      for (int r = 0; r < SCAN_ROWS; r++) v[r] = reinterpret_cast<const RangeWord*>(rank)[xs[r] >> 5];
+#pragma unroll
+      for (int r = 0; r < SCAN_ROWS; r++)
+        g[r] = v[r].before + uint32_t(__popc(v[r].bits & ((1u << (xs[r] & 31u)) - 1u)));
+    } else {
+#pragma unroll
+      for (int r = 0; r < SCAN_ROWS; r++) g[r] = MODE == RANK_DENSE ? xs[r] : rank[xs[r]];
+    }
 #pragma unroll
     for (int r = 0; r < SCAN_ROWS; r++) {
       const uint64_t i = row0 + uint64_t(r) * gsize;
@@ -2938,99 +3034,260 @@ __global__ void gb_fill_u32(uint32_t* p, size_t n, uint32_t v) {
   for (; i < n; i += stride) p[i] = v;
 }
 
-__global__ void gb_put_u32(uint32_t* p, uint32_t v) { *p = v; }
+// rep[ids[i]] = min over i; rep starts at all ones. A stale read is never below the current value, so it
+// never skips a row that could lower it. The rows of the wave's first lane's group (a hot one, if any is)
+// ask once, for their lowest row.
+__global__ void gb_first_atomic(const uint32_t* ids, uint32_t n, uint32_t* rep) {
+  for (uint64_t i0 = uint64_t(blockIdx.x) * blockDim.x; i0 < n; i0 += uint64_t(gridDim.x) * blockDim.x) {
+    const uint64_t i = i0 + threadIdx.x;
+    const bool in = i < n;
+    const uint32_t g = in ? ids[i] : 0xFFFFFFFFu;
+    const uint32_t lead = __builtin_amdgcn_readfirstlane(g);
+    const unsigned long long same = __ballot(g == lead);
+    const bool ask = in && (g != lead || int(threadIdx.x & 63) == __builtin_ctzll(same));
+    if (ask && uint32_t(i) < load_global(rep + g)) atomicMin(&rep[g], uint32_t(i));
+  }
+}
+
+// ---------------------------------------------------------------- composite keys of integer columns
+constexpr int COMPOSITE_MAX = 8;
+constexpr int COMP_ROWS = 8;
+
+struct CompositeCol {
+  const void* vals;
+  const uint8_t* valid;
+  int64_t voff;
+  int type;
+  ColSpan span;
+};
+struct CompositeArgs {
+  CompositeCol col[COMPOSITE_MAX];
+  int count;
+};
+
+// One workgroup: the column's statistics from the scan's workgroups, into pinned host memory.
+__global__ __launch_bounds__(512) void gb_span_fold(const RangeStat* st, uint32_t blocks, RangeStat* out) {
+  __shared__ RangeStat s_st[8];
+  RangeStat r{~0ull, 0ull, 0ull, 0xFFFFFFFFu, 0u};
+  for (uint32_t b = threadIdx.x; b < blocks; b += 512) {
+    const RangeStat x = st[b];
+    r.kmin = min(r.kmin, x.kmin);
+    r.kmax = max(r.kmax, x.kmax);
+    r.nulls += x.nulls;
+    r.null_first = min(r.null_first, x.null_first);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    r.kmin = min(r.kmin, (unsigned long long)__shfl_xor(r.kmin, off, 64));
+    r.kmax = max(r.kmax, (unsigned long long)__shfl_xor(r.kmax, off, 64));
+    r.nulls += __shfl_xor(r.nulls, off, 64);
+    r.null_first = min(r.null_first, uint32_t(__shfl_xor(int(r.null_first), off, 64)));
+  }
+  if ((threadIdx.x & 63) == 0) s_st[threadIdx.x >> 6] = r;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 8; w++) {
+      r.kmin = min(r.kmin, s_st[w].kmin);
+      r.kmax = max(r.kmax, s_st[w].kmax);
+      r.nulls += s_st[w].nulls;
+      r.null_first = min(r.null_first, s_st[w].null_first);
+    }
+    *out = r;
+  }
+}
+
+// Each row's composite key. A thread's COMP_ROWS rows of one column are loaded together (the switch on the
+// width is outside the loads), column after column.
+template <typename C>
+__global__ __launch_bounds__(256) void gb_composite(CompositeArgs a, uint32_t n, C* out) {
+  const uint32_t gsize = gridDim.x * blockDim.x;
+  for (uint64_t base = blockIdx.x * blockDim.x + threadIdx.x; base < n; base += uint64_t(gsize) * COMP_ROWS) {
+    C code[COMP_ROWS];
+#pragma unroll
+    for (int r = 0; r < COMP_ROWS; r++) code[r] = 0;
+    for (int c = 0; c < a.count; c++) {
+      const CompositeCol& k = a.col[c];
+      unsigned long long raw[COMP_ROWS];
+      uint32_t vb[COMP_ROWS];
+      int64_t ii[COMP_ROWS];
+#pragma unroll
+      for (int r = 0; r < COMP_ROWS; r++) {   // rows past the end read the last row
+        ii[r] = int64_t(std::min<uint64_t>(base + uint64_t(r) * gsize, uint64_t(n) - 1u));
+        vb[r] = ld_vbyte(k.valid, k.voff, ii[r]);
+      }
+      switch (type_width(k.type)) {   // uniform
+        case 8:
+#pragma unroll
+          for (int r = 0; r < COMP_ROWS; r++) raw[r] = ld_raw<8>(k.vals, ii[r]);
+          break;
+        case 4:
+#pragma unroll
+          for (int r = 0; r < COMP_ROWS; r++) raw[r] = ld_raw<4>(k.vals, ii[r]);
+          break;
+        case 2:
+#pragma unroll
+          for (int r = 0; r < COMP_ROWS; r++) raw[r] = ld_raw<2>(k.vals, ii[r]);
+          break;
+        default:
+#pragma unroll
+          for (int r = 0; r < COMP_ROWS; r++) raw[r] = ld_raw<1>(k.vals, ii[r]);
+          break;
+      }
+#pragma unroll
+      for (int r = 0; r < COMP_ROWS; r++) {
+        const bool ok = vbit(k.voff, ii[r], vb[r]) != 0u;
+        const C digit = ok ? C(order_key(key_of_raw(raw[r], k.type), k.type) - k.span.kmin) : C(k.span.span - 1ull);
+        code[r] = code[r] * C(k.span.span) + digit;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < COMP_ROWS; r++) {
+      const uint64_t i = base + uint64_t(r) * gsize;
+      if (i < n) out[i] = code[r];
+    }
+  }
+}
+
+// One column's group keys from the sorted composites (perm null: in order already), with its bitmap and
+// null count.
+__global__ __launch_bounds__(256) void gb_decode_keys(const unsigned long long* okeys, const uint32_t* perm, uint32_t D,
+                                                      int type, ColSpan sp, void* out, FoldOut fo) {
+  __shared__ uint32_t s_nulls[4];
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t nulls = 0;
+  for (uint32_t base = blockIdx.x * 256u + threadIdx.x - lane; base < D; base += gridDim.x * 256u) {
+    const uint32_t r = base + lane;
+    bool valid = false;
+    if (r < D) {
+      const unsigned long long code = okeys[perm ? perm[r] : r];
+      const unsigned long long digit = (code / sp.div) % sp.span;
+      valid = !(sp.has_null && digit == sp.span - 1ull);
+      unsigned long long v = valid ? sp.kmin + digit : 0ull;
+      if (valid && type_is_signed(type)) v ^= 0x8000000000000000ull;
+      switch (type_width(type)) {
+        case 1: static_cast<uint8_t*>(out)[r] = uint8_t(v); break;
+        case 2: static_cast<uint16_t*>(out)[r] = uint16_t(v); break;
+        case 4: static_cast<uint32_t*>(out)[r] = uint32_t(v); break;
+        default: static_cast<unsigned long long*>(out)[r] = v; break;
+      }
+    }
+    const unsigned long long bal = __ballot(valid);
+    if (lane == 0 && fo.bits) fo.bits[base >> 6] = bal;
+    nulls += min(64u, D - base) - uint32_t(__popcll(bal));
+  }
+  if (lane == 0) s_nulls[threadIdx.x >> 6] = nulls;
+  __syncthreads();
+  if (threadIdx.x == 0) fold_report(fo, s_nulls[0] + s_nulls[1] + s_nulls[2] + s_nulls[3]);
+}
+
+// Calls f(TYPE) for an integer key type (the range path maps no others).
+template <class F>
+void with_int_type(int type, F&& f) {
+  with_key_type(type, [&](auto tc) {
+    if constexpr (decltype(tc)::value != T_F32 && decltype(tc)::value != T_F64) f(tc);
+  });
+}
+
+// The largest span the range path takes for n rows.
+unsigned long long range_limit(int64_t n) {
+  return std::min<unsigned long long>(1ull << 24, std::max<unsigned long long>(1ull << 16, 4ull * uint64_t(n)));
+}
 
 // The range path's mapping from the keys' statistics, or false when their span is too wide for it.
-bool map_range(const void* vals, int type, const uint8_t* valid, int64_t voff, int64_t n, bool track,
-               const RangeStat& host, Mapped& out) {
+bool map_range(const void* vals, int type, const uint8_t* valid, int64_t voff, int64_t n, const RangeStat& host,
+               Mapped& out) {
   hipStream_t s = stream();
   const uint32_t un = uint32_t(n);
-  const unsigned long long limit = std::min<unsigned long long>(1ull << 24, std::max<unsigned long long>(1ull << 16, 4ull * uint64_t(n)));
-  {
-    const bool any = host.kmin <= host.kmax;
-    const unsigned long long span64 = any ? host.kmax - host.kmin + 1ull : 0ull;
-    if (any && (span64 == 0ull || span64 > limit)) return false;   // span64 == 0: the full 2^64 range
-  }
   const bool any = host.kmin <= host.kmax;
   const unsigned long long span64 = any ? host.kmax - host.kmin + 1ull : 0ull;
+  if (any && (span64 == 0ull || span64 > range_limit(n))) return false;   // span64 == 0: the full 2^64 range
   const int grid = grid_for((n + SCAN_ROWS - 1) / SCAN_ROWS, 8);
   const uint32_t span = uint32_t(std::max<unsigned long long>(span64, 1ull));
-  DevBuf occ = device_alloc(size_t(span) * 4);
-  DevBuf first;
-  if (track) first = device_alloc(size_t(span) * 4);
-  hipLaunchKernelGGL(gb_fill_u32, dim3(grid_for(span, 4)), dim3(256), 0, s, static_cast<uint32_t*>(occ->ptr), size_t(span), 0u);
-  if (track)
-    hipLaunchKernelGGL(gb_fill_u32, dim3(grid_for(span, 4)), dim3(256), 0, s, static_cast<uint32_t*>(first->ptr),
-                       size_t(span), 0xFFFFFFFFu);
-  AM_HIP(hipGetLastError());
-  auto* o = static_cast<uint32_t*>(occ->ptr);
-  auto* f = track ? static_cast<uint32_t*>(first->ptr) : nullptr;
-  if (any) {
-    ProfScope ps("gb_range_occ");
-    with_key_type(type, [&](auto tc) {
-      constexpr int TT = decltype(tc)::value;
-      if constexpr (TT != T_F32 && TT != T_F64) {
-        constexpr int WW = width_of(TT);
-        if (!track && span <= RANGE_BITS_MAX) {
-          const uint32_t words = (span + 31u) / 32u;
-          DevBuf bits = device_alloc(size_t(words) * 4);
-          auto* b = static_cast<uint32_t*>(bits->ptr);
-          hipLaunchKernelGGL(gb_fill_u32, dim3(grid_for(words, 4)), dim3(256), 0, s, b, size_t(words), 0u);
-          const dim3 bg(grid_for((n + SCAN_ROWS - 1) / SCAN_ROWS, AM_OCC_BLOCKS_PER_CU));
-          const size_t lds = size_t(words) * 4;
-          if (valid) hipLaunchKernelGGL((gb_range_occ_bits<WW, TT, true>), bg, dim3(256), lds, s, vals, valid, voff, un, host.kmin, words, b);
-          else hipLaunchKernelGGL((gb_range_occ_bits<WW, TT, false>), bg, dim3(256), lds, s, vals, valid, voff, un, host.kmin, words, b);
-          hipLaunchKernelGGL(gb_range_unpack, dim3((span + 255) / 256), dim3(256), 0, s, static_cast<const uint32_t*>(b), span, o);
-        } else if (valid) {
-          if (track) hipLaunchKernelGGL((gb_range_occ<WW, TT, true, true>), dim3(grid), dim3(256), 0, s, vals, valid, voff, un, host.kmin, o, f);
-          else hipLaunchKernelGGL((gb_range_occ<WW, TT, true, false>), dim3(grid), dim3(256), 0, s, vals, valid, voff, un, host.kmin, o, f);
-        } else {
-          if (track) hipLaunchKernelGGL((gb_range_occ<WW, TT, false, true>), dim3(grid), dim3(256), 0, s, vals, valid, voff, un, host.kmin, o, f);
-          else hipLaunchKernelGGL((gb_range_occ<WW, TT, false, false>), dim3(grid), dim3(256), 0, s, vals, valid, voff, un, host.kmin, o, f);
-        }
-      }
-    });
-    AM_HIP(hipGetLastError());
-  }
-  const uint32_t tiles = (span + RANGE_TILE - 1) / RANGE_TILE;
-  DevBuf tsum = device_alloc(size_t(tiles) * 4 + 4);
-  auto* ts = static_cast<uint32_t*>(tsum->ptr);
   out.okeys = device_alloc(size_t(span) * 8);
-  out.rep = device_alloc(size_t(span + 1) * 4);
-  {
-    ProfScope ps("gb_range_scan");
-    hipLaunchKernelGGL(gb_range_count, dim3(tiles), dim3(256), 0, s, o, span, ts);
-    hipLaunchKernelGGL(gb_range_scan_tiles, dim3(1), dim3(1024), 0, s, ts, tiles, ts + tiles);
-    hipLaunchKernelGGL(gb_range_rank, dim3(tiles), dim3(256), 0, s, o, span, ts, host.kmin,
-                       static_cast<unsigned long long*>(out.okeys->ptr), f,
-                       track ? static_cast<uint32_t*>(out.rep->ptr) : nullptr);
-    AM_HIP(hipGetLastError());
+  auto* okeys = static_cast<unsigned long long*>(out.okeys->ptr);
+  DevBuf look;   // what gb_range_ids looks ranks up in
+  int mode = RANK_TABLE;
+  uint32_t D = 0;
+  if (span <= RANGE_BITS_MAX) {   // (with only nulls, one key that is not there)
+    mode = RANK_WORDS;
+    const uint32_t words = (span + 31u) / 32u;
+    const uint32_t parts = uint32_t(std::max<int64_t>(1, std::min<int64_t>((n + OCC_THREADS * SCAN_ROWS - 1) / (OCC_THREADS * SCAN_ROWS),
+                                                                           device().cu_count)));
+    DevBuf part = device_alloc(size_t(parts) * words * 4);
+    auto* pb = static_cast<uint32_t*>(part->ptr);
+    {
+      ProfScope ps("gb_range_occ");
+      const size_t lds = size_t(words) * 4;
+      with_int_type(type, [&](auto tc) {
+        constexpr int TT = decltype(tc)::value, WW = width_of(TT);
+        if (valid) hipLaunchKernelGGL((gb_range_occ_bits<WW, TT, true>), dim3(parts), dim3(OCC_THREADS), lds, s, vals, valid, voff, un, host.kmin, words, pb);
+        else hipLaunchKernelGGL((gb_range_occ_bits<WW, TT, false>), dim3(parts), dim3(OCC_THREADS), lds, s, vals, valid, voff, un, host.kmin, words, pb);
+      });
+      AM_HIP(hipGetLastError());
+    }
+    const uint32_t tiles = (words + RANGE_FOLD - 1) / RANGE_FOLD;
+    look = device_alloc(size_t(words) * sizeof(RangeWord));
+    DevBuf tb = device_alloc(size_t(tiles) * 4);
+    auto* rw = static_cast<RangeWord*>(look->ptr);
+    auto* tbp = static_cast<uint32_t*>(tb->ptr);
+    std::shared_ptr<void> slot = pinned_slot();
+    auto* distinct = static_cast<unsigned long long*>(slot.get());
+    {
+      ProfScope ps("gb_range_scan");
+      hipLaunchKernelGGL(gb_range_fold, dim3(tiles), dim3(1024), 0, s, static_cast<const uint32_t*>(pb), parts, words, rw, tbp,
+                         fold_ctl(), distinct);
+      hipLaunchKernelGGL(gb_range_emit, dim3((span + 255u) / 256u), dim3(256), 0, s, rw, span,
+                         static_cast<const uint32_t*>(tbp), host.kmin, okeys);
+      AM_HIP(hipGetLastError());
+    }
+    AM_HIP(hipStreamSynchronize(s));
+    D = uint32_t(*distinct);
+  } else {
+    look = device_alloc(size_t(span) * 4);
+    auto* o = static_cast<uint32_t*>(look->ptr);
+    hipLaunchKernelGGL(gb_fill_u32, dim3(grid_for(span, 4)), dim3(256), 0, s, o, size_t(span), 0u);
+    {
+      ProfScope ps("gb_range_occ");
+      with_int_type(type, [&](auto tc) {
+        constexpr int TT = decltype(tc)::value, WW = width_of(TT);
+        if (valid) hipLaunchKernelGGL((gb_range_occ<WW, TT, true>), dim3(grid), dim3(256), 0, s, vals, valid, voff, un, host.kmin, o);
+        else hipLaunchKernelGGL((gb_range_occ<WW, TT, false>), dim3(grid), dim3(256), 0, s, vals, valid, voff, un, host.kmin, o);
+      });
+      AM_HIP(hipGetLastError());
+    }
+    const uint32_t tiles = (span + RANGE_TILE - 1) / RANGE_TILE;
+    DevBuf tsum = device_alloc(size_t(tiles) * 4 + 4);
+    auto* ts = static_cast<uint32_t*>(tsum->ptr);
+    {
+      ProfScope ps("gb_range_scan");
+      hipLaunchKernelGGL(gb_range_count, dim3(tiles), dim3(256), 0, s, o, span, ts);
+      hipLaunchKernelGGL(gb_range_scan_tiles, dim3(1), dim3(1024), 0, s, ts, tiles, ts + tiles);
+      hipLaunchKernelGGL(gb_range_rank, dim3(tiles), dim3(256), 0, s, o, span, ts, host.kmin, okeys);
+      AM_HIP(hipGetLastError());
+    }
+    D = read_back(ts + tiles);
   }
-  const uint32_t D = read_back(ts + tiles);
-  out.D = any ? D : 0u;
+  if (D == span) mode = RANK_DENSE;
+  out.D = D;
   out.has_null = host.nulls > 0;
   out.K = int64_t(out.D) + (out.has_null ? 1 : 0);
-  if (track && out.has_null)
-    hipLaunchKernelGGL(gb_put_u32, dim3(1), dim3(1), 0, s, static_cast<uint32_t*>(out.rep->ptr) + out.D, host.null_first);
   out.ids = device_alloc(size_t(std::max<int64_t>(n, 1)) * 4);
   {
     ProfScope ps("gb_ids");
     auto* ids = static_cast<uint32_t*>(out.ids->ptr);
-    with_key_type(type, [&](auto tc) {
-      constexpr int TT = decltype(tc)::value;
-      if constexpr (TT != T_F32 && TT != T_F64) {
-        constexpr int WW = width_of(TT);
-        const bool dense = out.D == span;
-#define AM_RANGE_IDS(HV, DN) hipLaunchKernelGGL((gb_range_ids<WW, TT, HV, DN>), dim3(grid), dim3(256), 0, s, vals, valid, voff, un, host.kmin, o, out.D, ids)
-        if (valid) {
-          if (dense) AM_RANGE_IDS(true, true);
-          else AM_RANGE_IDS(true, false);
-        } else {
-          if (dense) AM_RANGE_IDS(false, true);
-          else AM_RANGE_IDS(false, false);
-        }
-#undef AM_RANGE_IDS
+    auto* o = static_cast<const uint32_t*>(look->ptr);
+    with_int_type(type, [&](auto tc) {
+      constexpr int TT = decltype(tc)::value, WW = width_of(TT);
+#define AM_RANGE_IDS(HV, MD) hipLaunchKernelGGL((gb_range_ids<WW, TT, HV, MD>), dim3(grid), dim3(256), 0, s, vals, valid, voff, un, host.kmin, o, out.D, ids)
+      if (valid) {
+        if (mode == RANK_DENSE) AM_RANGE_IDS(true, RANK_DENSE);
+        else if (mode == RANK_WORDS) AM_RANGE_IDS(true, RANK_WORDS);
+        else AM_RANGE_IDS(true, RANK_TABLE);
+      } else {
+        if (mode == RANK_DENSE) AM_RANGE_IDS(false, RANK_DENSE);
+        else if (mode == RANK_WORDS) AM_RANGE_IDS(false, RANK_WORDS);
+        else AM_RANGE_IDS(false, RANK_TABLE);
       }
+#undef AM_RANGE_IDS
     });
     AM_HIP(hipGetLastError());
   }
@@ -3039,25 +3296,25 @@ bool map_range(const void* vals, int type, const uint8_t* valid, int64_t voff, i
 
 // gb_build for the key column's element width: 64-bit integer keys without a validity bitmap (the
 // common case) take an instantiation with the key mapping and the validity fixed.
-template <bool TRACK>
 void launch_build(int w, int grid, hipStream_t s, const void* vals, int type, const uint8_t* valid, int64_t voff,
                   uint32_t n, Table T, uint32_t mask, uint32_t budget, uint32_t* slot_of, BuildStatus* st, bool priv) {
   const int p = priv ? 1 : 0;
   if (!valid && (type == T_I64 || type == T_U64)) {
-    hipLaunchKernelGGL((gb_build<TRACK, 8, T_U64, true>), dim3(grid), dim3(BUILD_THREADS), 0, s, vals, type, valid, voff, n, T, mask, budget, slot_of, st, p);
+    hipLaunchKernelGGL((gb_build<8, T_U64, true>), dim3(grid), dim3(BUILD_THREADS), 0, s, vals, type, valid, voff, n, T, mask, budget, slot_of, st, p);
     return;
   }
   switch (w) {
-    case 8: hipLaunchKernelGGL((gb_build<TRACK, 8, -1, false>), dim3(grid), dim3(BUILD_THREADS), 0, s, vals, type, valid, voff, n, T, mask, budget, slot_of, st, p); break;
-    case 4: hipLaunchKernelGGL((gb_build<TRACK, 4, -1, false>), dim3(grid), dim3(BUILD_THREADS), 0, s, vals, type, valid, voff, n, T, mask, budget, slot_of, st, p); break;
-    case 2: hipLaunchKernelGGL((gb_build<TRACK, 2, -1, false>), dim3(grid), dim3(BUILD_THREADS), 0, s, vals, type, valid, voff, n, T, mask, budget, slot_of, st, p); break;
-    default: hipLaunchKernelGGL((gb_build<TRACK, 1, -1, false>), dim3(grid), dim3(BUILD_THREADS), 0, s, vals, type, valid, voff, n, T, mask, budget, slot_of, st, p); break;
+    case 8: hipLaunchKernelGGL((gb_build<8, -1, false>), dim3(grid), dim3(BUILD_THREADS), 0, s, vals, type, valid, voff, n, T, mask, budget, slot_of, st, p); break;
+    case 4: hipLaunchKernelGGL((gb_build<4, -1, false>), dim3(grid), dim3(BUILD_THREADS), 0, s, vals, type, valid, voff, n, T, mask, budget, slot_of, st, p); break;
+    case 2: hipLaunchKernelGGL((gb_build<2, -1, false>), dim3(grid), dim3(BUILD_THREADS), 0, s, vals, type, valid, voff, n, T, mask, budget, slot_of, st, p); break;
+    default: hipLaunchKernelGGL((gb_build<1, -1, false>), dim3(grid), dim3(BUILD_THREADS), 0, s, vals, type, valid, voff, n, T, mask, budget, slot_of, st, p); break;
   }
 }
 
-// Maps one key column (values, type, validity) to dense ascending ids; with `track` it also finds
-// the lowest row of every group.
-Mapped map_column(const void* vals, int type, const uint8_t* valid, int64_t voff, int64_t n, bool track) {
+// Maps one key column (values, type, validity) to dense ascending ids. `known`: the column's span, when
+// its values are already known to lie in one (a composite key).
+Mapped map_column(const void* vals, int type, const uint8_t* valid, int64_t voff, int64_t n,
+                  const RangeStat* known = nullptr) {
   hipStream_t s = stream();
   uint32_t un = uint32_t(n);
   Mapped out;
@@ -3071,6 +3328,7 @@ Mapped map_column(const void* vals, int type, const uint8_t* valid, int64_t voff
   uint64_t full = 1024;
   while (full < want) full <<= 1;
   uint64_t cap = 1024;
+  if (known && range_path_enabled() && map_range(vals, type, valid, voff, n, *known, out)) return out;
   if (n >= (int64_t(1) << 16)) {
     const bool range = type_is_int(type) && range_path_enabled();
     const uint32_t scan_blocks = key_scan_blocks(valid != nullptr, un);
@@ -3090,7 +3348,7 @@ Mapped map_column(const void* vals, int type, const uint8_t* valid, int64_t voff
     }
     AM_HIP(hipStreamSynchronize(s));
     const KeyStat stat = *ks;
-    if (range && map_range(vals, type, valid, voff, n, track, stat.r, out)) return out;
+    if (range && !known && map_range(vals, type, valid, voff, n, stat.r, out)) return out;
     const unsigned long long d = stat.est;
 #ifndef AM_CAP_HALVES
 #define AM_CAP_HALVES 10   // table slots per distinct key, in halves
@@ -3105,7 +3363,7 @@ Mapped map_column(const void* vals, int type, const uint8_t* valid, int64_t voff
   DevBuf stb = device_alloc(sizeof(BuildStatus));
   auto* st = static_cast<BuildStatus*>(stb->ptr);
   BuildStatus host{};
-  DevBuf tkeys, tfirst, gkeys, gfirst, xmap, slots;
+  DevBuf tkeys, gkeys, xmap, slots;
   Table T{};          // the table the rows were inserted into (eight private copies, or one)
   Table G{};          // the merged table of distinct keys
   bool priv = false;
@@ -3118,36 +3376,27 @@ Mapped map_column(const void* vals, int type, const uint8_t* valid, int64_t voff
     priv = cap <= (1u << 20);
     const size_t ntab = priv ? NXCD : 1;
     tkeys = device_alloc(ntab * size_t(cap + 1) * 8);
-    if (track) tfirst = device_alloc(ntab * size_t(cap + 1) * 4);
     T.key = static_cast<unsigned long long*>(tkeys->ptr);
-    T.first = track ? static_cast<uint32_t*>(tfirst->ptr) : nullptr;
     hipLaunchKernelGGL(gb_table_init, dim3(grid_for(int64_t(ntab * (cap + 1)), 4)), dim3(256), 0, s, T,
                        ntab * size_t(cap + 1), st);
     AM_HIP(hipGetLastError());
     {
       ProfScope ps("gb_build");
       uint32_t budget = last_try ? uint32_t(cap) : 128u;
-      if (track)
-        launch_build<true>(type_width(type), build_grid, s, vals, type, valid, voff, un, T, uint32_t(cap - 1), budget,
-                           static_cast<uint32_t*>(out.ids->ptr), st, priv);
-      else
-        launch_build<false>(type_width(type), build_grid, s, vals, type, valid, voff, un, T, uint32_t(cap - 1), budget,
-                            static_cast<uint32_t*>(out.ids->ptr), st, priv);
+      launch_build(type_width(type), build_grid, s, vals, type, valid, voff, un, T, uint32_t(cap - 1), budget,
+                   static_cast<uint32_t*>(out.ids->ptr), st, priv);
       AM_HIP(hipGetLastError());
     }
     G = T;
     if (priv) {
       gkeys = device_alloc(size_t(cap + 1) * 8);
-      if (track) gfirst = device_alloc(size_t(cap + 1) * 4);
       xmap = device_alloc(size_t(NXCD) * size_t(cap + 1) * 4);
       G.key = static_cast<unsigned long long*>(gkeys->ptr);
-      G.first = track ? static_cast<uint32_t*>(gfirst->ptr) : nullptr;
       hipLaunchKernelGGL(gb_table_init, dim3(grid_for(int64_t(cap + 1), 4)), dim3(256), 0, s, G, size_t(cap + 1),
                          static_cast<BuildStatus*>(nullptr));
       ProfScope ps("gb_merge");
       hipLaunchKernelGGL(gb_merge_tables, dim3(grid_for(int64_t(NXCD) * (cap + 1), 4)), dim3(256), 0, s,
-                         static_cast<const unsigned long long*>(T.key), static_cast<const uint32_t*>(T.first),
-                         uint32_t(cap), st, G, static_cast<uint32_t*>(xmap->ptr));
+                         static_cast<const unsigned long long*>(T.key), uint32_t(cap), st, G, static_cast<uint32_t*>(xmap->ptr));
       AM_HIP(hipGetLastError());
     }
     // Compact the occupied slots before the status is read: a build that ran out of probes left at
@@ -3174,13 +3423,11 @@ Mapped map_column(const void* vals, int type, const uint8_t* valid, int64_t voff
   if (out.D > 0)
     argsort_device(out.okeys->ptr, T_U64, nullptr, 0, out.D, false, 0, 1, static_cast<uint32_t*>(out.perm->ptr), s);
   DevBuf gid_of_slot = device_alloc(size_t(cap + 1) * 4);
-  out.rep = device_alloc(size_t(std::max<int64_t>(out.K, 1)) * 4);
   {
     ProfScope ps("gb_relabel");
     hipLaunchKernelGGL(gb_relabel, dim3(uint32_t((out.D + 1 + 255) / 256)), dim3(256), 0, s,
-                       static_cast<const uint32_t*>(out.perm->ptr), static_cast<const uint32_t*>(slots->ptr), out.D, G.first,
-                       static_cast<uint32_t*>(gid_of_slot->ptr), static_cast<uint32_t*>(out.rep->ptr), st,
-                       out.has_null ? 1 : 0, track ? 1 : 0);
+                       static_cast<const uint32_t*>(out.perm->ptr), static_cast<const uint32_t*>(slots->ptr), out.D,
+                       static_cast<uint32_t*>(gid_of_slot->ptr));
     AM_HIP(hipGetLastError());
   }
   // Rows hold private-table slots: map those through the merged table first.
@@ -3201,6 +3448,124 @@ Mapped map_column(const void* vals, int type, const uint8_t* valid, int64_t voff
     AM_HIP(hipGetLastError());
   }
   return out;
+}
+
+// A result column under construction: its array, its validity bitmap and the pinned words its null count
+// lands in. `finish` waits for the stream and settles the null count.
+struct Result {
+  Array* out;
+  std::shared_ptr<void> slot;
+  FoldOut fo{};
+  Result(const std::string& fmt, int type, long long K, bool nullable) : out(new_array(fmt, type, K)) {
+    try {
+      out->values = device_alloc(size_t(std::max<long long>(K, 1)) * std::max(type_width(type), 1));
+      out->null_count = 0;
+      if (nullable && K > 0) report(K);
+    } catch (...) {
+      release_array(out);
+      throw;
+    }
+  }
+  void report(long long K) {
+    out->validity = device_alloc(size_t((K + 63) / 64) * 8);
+    slot = pinned_slot();
+    fo = FoldOut{static_cast<unsigned long long*>(out->validity->ptr), static_cast<unsigned long long*>(slot.get()), nullptr,
+                 fold_ctl()};
+  }
+  Result(const Result&) = delete;
+  ~Result() { if (out) release_array(out); }
+  void* values() { return out->values->ptr; }
+  Array* finish() {
+    if (slot) {
+      AM_HIP(hipStreamSynchronize(stream()));   // the null count decides whether there is a bitmap, also inside a batch
+      out->null_count = int64_t(*static_cast<unsigned long long*>(slot.get()));
+      if (out->null_count == 0) out->validity.reset();
+    }
+    sync();
+    Array* r = out;
+    out = nullptr;
+    return r;
+  }
+};
+
+// The lowest row of each of the K groups of `ids`.
+DevBuf first_rows(const DevBuf& ids, int64_t n, int64_t K) {
+  hipStream_t s = stream();
+  DevBuf rep = device_alloc(size_t(std::max<int64_t>(K, 1)) * 4);
+  auto* r = static_cast<uint32_t*>(rep->ptr);
+  if (K > int64_t(PART_MAX_NB) * PART_G) {
+    // More groups than the partitioned passes take: few rows share a group on average.
+    hipLaunchKernelGGL(gb_fill_u32, dim3(grid_for(K, 4)), dim3(256), 0, s, r, size_t(K), 0xFFFFFFFFu);
+    hipLaunchKernelGGL(gb_first_atomic, dim3(grid_for(n)), dim3(256), 0, s, static_cast<const uint32_t*>(ids->ptr), uint32_t(n), r);
+    AM_HIP(hipGetLastError());
+    return rep;
+  }
+  AggArgs a{};
+  a.ids = IdSource{ids->ptr, T_I32, nullptr, 0};
+  a.n = n;
+  a.K = std::max<int64_t>(K, 1);
+  run_agg<FirstRowP>(a, s, "gb_first", FinFirst{r});
+  return rep;
+}
+
+// Maps several integer columns as one composite key: each column's order key less its minimum is a digit
+// in a mixed radix of the columns' spans (a null is the digit above them), so the composite is injective
+// and ascending in the columns, and one mapping replaces one per column and one per fold. The group keys
+// are decoded from the sorted composites. (Int32 x int16 keys with nulls, 3M rows, 40,000 groups, sum, mean,
+// min, max and count: 2.17 ms -> 0.35 ms, of which 1.6 ms were the atomics that found each group's lowest
+// row, one per row on a hot group's word.) False when the spans' product does not fit 62 bits (or more
+// than COMPOSITE_MAX columns): the columns then fold pairwise over their ids.
+bool map_composite(Array* const* columns, int64_t count, int64_t n, std::vector<ColSpan>& out_spans, Mapped& out) {
+  if (count > COMPOSITE_MAX) return false;
+  hipStream_t s = stream();
+  const uint32_t un = uint32_t(n);
+  std::shared_ptr<void> slot = pinned_slot();
+  auto* st = static_cast<RangeStat*>(slot.get());
+  static_assert(COMPOSITE_MAX * sizeof(RangeStat) <= PINNED_SLOT, "one pinned slot");
+  {
+    ProfScope ps("gb_span_scan");
+    for (int64_t c = 0; c < count; c++) {
+      const Array* a = columns[c];
+      const uint8_t* valid = a->has_nulls() ? a->valid_bits() : nullptr;
+      const uint32_t blocks = key_scan_blocks(valid != nullptr, un);
+      DevBuf parts = device_alloc(blocks * sizeof(RangeStat));
+      key_scan(a->type, s, a->data(), valid, a->offset, un, nullptr, static_cast<RangeStat*>(parts->ptr));
+      hipLaunchKernelGGL(gb_span_fold, dim3(1), dim3(512), 0, s, static_cast<const RangeStat*>(parts->ptr), blocks, st + c);
+      AM_HIP(hipGetLastError());
+    }
+  }
+  AM_HIP(hipStreamSynchronize(s));
+  CompositeArgs ca{};
+  std::vector<ColSpan> spans;
+  unsigned __int128 total = 1;
+  for (int64_t c = 0; c < count; c++) {
+    const RangeStat r = st[c];
+    const bool any = r.kmin <= r.kmax;
+    const unsigned __int128 span = (any ? (unsigned __int128)(r.kmax - r.kmin) + 1 : 0) + (r.nulls > 0 ? 1 : 0);
+    total *= span;
+    if (total > (unsigned __int128)1 << 62) return false;
+    spans.push_back(ColSpan{any ? r.kmin : 0ull, (unsigned long long)span, 1ull, r.nulls > 0 ? 1 : 0});
+  }
+  for (int64_t c = count - 1; c > 0; c--) spans[size_t(c - 1)].div = spans[size_t(c)].div * spans[size_t(c)].span;
+  for (int64_t c = 0; c < count; c++) {
+    const Array* a = columns[c];
+    ca.col[c] = CompositeCol{a->data(), a->has_nulls() ? a->valid_bits() : nullptr, a->offset, a->type, spans[size_t(c)]};
+  }
+  ca.count = int(count);
+  const unsigned long long top = (unsigned long long)total;   // composites are below it
+  const bool narrow = top <= (1ull << 32);
+  DevBuf comp = device_alloc(size_t(n) * (narrow ? 4 : 8));
+  {
+    ProfScope ps("gb_composite");
+    const int grid = grid_for((n + COMP_ROWS - 1) / COMP_ROWS, 8);
+    if (narrow) hipLaunchKernelGGL(gb_composite<uint32_t>, dim3(grid), dim3(256), 0, s, ca, un, static_cast<uint32_t*>(comp->ptr));
+    else hipLaunchKernelGGL(gb_composite<unsigned long long>, dim3(grid), dim3(256), 0, s, ca, un, static_cast<unsigned long long*>(comp->ptr));
+    AM_HIP(hipGetLastError());
+  }
+  const RangeStat known{0ull, top - 1ull, 0ull, 0u, 0u};
+  out = map_column(comp->ptr, narrow ? T_U32 : T_U64, nullptr, 0, n, &known);
+  out_spans = std::move(spans);
+  return true;
 }
 
 GroupBy* group_by_keys_impl(Array* const* columns, int64_t count, bool need_rep) {
@@ -3230,46 +3595,52 @@ GroupBy* group_by_keys_impl(Array* const* columns, int64_t count, bool need_rep)
       return g;
     }
     hipStream_t s = stream();
-    const Array* a0 = columns[0];
-    // Representative rows are needed for float keys (-0.0 and 0.0, NaN payloads share a group but
-    // not their bits) and for several columns; integer keys are answered from the sorted keys.
-    bool int_single = count == 1 && type_is_int(a0->type) && !need_rep;
-    Mapped m0 = map_column(a0->data(), a0->type, a0->has_nulls() ? a0->valid_bits() : nullptr, a0->offset, n,
-                           count == 1 && !int_single);
-    int64_t K = m0.K;
-    g->ids = m0.ids;
-    if (int_single) {
-      g->okeys = m0.okeys;
-      g->perm = m0.perm;
-      g->D = m0.D;
-      g->has_null = m0.has_null;
-    } else if (count == 1) {
-      g->rep = m0.rep;
-      g->has_rep = true;
-      g->has_null = m0.has_null;
-    }
-    // Further columns fold pairwise: ids a (K groups) and b (K2) become the key a * K2 + b, which is
-    // injective and ascending in (a, b), and that key is mapped again (GroupByKeys.swift:103-112).
-    for (int64_t c = 1; c < count; c++) {
-      const Array* ac = columns[c];
-      Mapped mc = map_column(ac->data(), ac->type, ac->has_nulls() ? ac->valid_bits() : nullptr, ac->offset, n, false);
-      int64_t K2 = mc.K;
-      if (K2 > 0 && K > INT64_MAX / K2)
-        fail_invalid("multi-column group-by overflowed the 64-bit composite key (" + std::to_string(K) + " x " +
-             std::to_string(K2) + " distinct)");
-      DevBuf comp = device_alloc(size_t(n) * 8);
-      hipLaunchKernelGGL(gb_combine, dim3(grid_for(n)), dim3(256), 0, s, static_cast<const int32_t*>(g->ids->ptr),
-                         static_cast<const int32_t*>(mc.ids->ptr), uint32_t(n), (long long)K2,
-                         static_cast<long long*>(comp->ptr));
-      AM_HIP(hipGetLastError());
-      bool last = c == count - 1;
-      Mapped mm = map_column(comp->ptr, T_I64, nullptr, 0, n, last);
-      K = mm.K;
-      g->ids = mm.ids;
-      if (last) {
-        g->rep = mm.rep;
-        g->has_rep = true;
+    bool ints = true;
+    for (int64_t c = 0; c < count; c++) ints = ints && type_is_int(columns[c]->type);
+    int64_t K = 0;
+    auto mapped = [&](const Array* a) {
+      return map_column(a->data(), a->type, a->has_nulls() ? a->valid_bits() : nullptr, a->offset, n);
+    };
+    Mapped m;
+    bool keys_kept = ints;   // the keys come from the sorted distinct keys
+    if (count == 1) {
+      m = mapped(columns[0]);
+      K = m.K;
+    } else if (ints && map_composite(columns, count, n, g->spans, m)) {
+      K = m.K;
+    } else {
+      // Columns fold pairwise: ids a (K groups) and b (K2) become the key a * K2 + b, which is injective
+      // and ascending in (a, b), and that key is mapped again (GroupByKeys.swift:103-112).
+      keys_kept = false;
+      m = mapped(columns[0]);
+      K = m.K;
+      for (int64_t c = 1; c < count; c++) {
+        Mapped mc = mapped(columns[c]);
+        const int64_t K2 = mc.K;
+        if (K2 > 0 && K > INT64_MAX / K2)
+          fail_invalid("multi-column group-by overflowed the 64-bit composite key (" + std::to_string(K) + " x " +
+               std::to_string(K2) + " distinct)");
+        DevBuf comp = device_alloc(size_t(n) * 8);
+        hipLaunchKernelGGL(gb_combine, dim3(grid_for(n)), dim3(256), 0, s, static_cast<const int32_t*>(m.ids->ptr),
+                           static_cast<const int32_t*>(mc.ids->ptr), uint32_t(n), (long long)K2,
+                           static_cast<long long*>(comp->ptr));
+        AM_HIP(hipGetLastError());
+        m = map_column(comp->ptr, T_I64, nullptr, 0, n);
+        K = m.K;
       }
+    }
+    g->ids = m.ids;
+    g->has_null = m.has_null;
+    if (keys_kept) {
+      g->okeys = m.okeys;
+      g->perm = m.perm;
+      g->D = m.D;
+    }
+    // Representative rows are needed for float keys (-0.0 and 0.0, NaN payloads share a group but not
+    // their bits) and by callers that ask for them; integer keys are answered from the sorted keys.
+    if (!keys_kept || need_rep) {
+      g->rep = first_rows(m.ids, n, K);
+      g->has_rep = true;
     }
     if (K > int64_t(INT32_MAX)) fail("group-by: more than 2^31 groups");
     g->K = K;
@@ -3310,7 +3681,16 @@ Array* group_by_keys_result(GroupBy* g, int64_t i) {
   if (!g->key_results[size_t(i)]) {
     const Array* col = g->columns[size_t(i)];
     Array* keys = nullptr;
-    if (!g->has_rep) {
+    if (!g->spans.empty()) {
+      const ColSpan& sp = g->spans[size_t(i)];
+      Result r(col->format, col->type, g->K, sp.has_null != 0);
+      const int blocks = int(std::max<int64_t>(1, std::min<int64_t>((g->K + 255) / 256, 1024)));
+      hipLaunchKernelGGL(gb_decode_keys, dim3(blocks), dim3(256), 0, stream(),
+                         static_cast<const unsigned long long*>(g->okeys->ptr),
+                         g->perm ? static_cast<const uint32_t*>(g->perm->ptr) : nullptr, g->D, col->type, sp, r.values(), r.fo);
+      AM_HIP(hipGetLastError());
+      keys = r.finish();
+    } else if (!g->has_rep) {
       // Integer keys: the sorted distinct keys themselves, the null group (last) null.
       hipStream_t s = stream();
       keys = new_array(col->format, col->type, g->K);
@@ -3353,44 +3733,6 @@ void group_by_release(GroupBy* g) { delete g; }
 // ================================================================ host: aggregates
 
 namespace {
-
-// A result column under construction: its array, its validity bitmap and the pinned words its null count
-// lands in. `finish` waits for the stream and settles the null count.
-struct Result {
-  Array* out;
-  std::shared_ptr<void> slot;
-  FoldOut fo{};
-  Result(const std::string& fmt, int type, long long K, bool nullable) : out(new_array(fmt, type, K)) {
-    try {
-      out->values = device_alloc(size_t(std::max<long long>(K, 1)) * std::max(type_width(type), 1));
-      out->null_count = 0;
-      if (nullable && K > 0) report(K);
-    } catch (...) {
-      release_array(out);
-      throw;
-    }
-  }
-  void report(long long K) {
-    out->validity = device_alloc(size_t((K + 63) / 64) * 8);
-    slot = pinned_slot();
-    fo = FoldOut{static_cast<unsigned long long*>(out->validity->ptr), static_cast<unsigned long long*>(slot.get()), nullptr,
-                 fold_ctl()};
-  }
-  Result(const Result&) = delete;
-  ~Result() { if (out) release_array(out); }
-  void* values() { return out->values->ptr; }
-  Array* finish() {
-    if (slot) {
-      AM_HIP(hipStreamSynchronize(stream()));   // the null count decides whether there is a bitmap, also inside a batch
-      out->null_count = int64_t(*static_cast<unsigned long long*>(slot.get()));
-      if (out->null_count == 0) out->validity.reset();
-    }
-    sync();
-    Array* r = out;
-    out = nullptr;
-    return r;
-  }
-};
 
 // A count, sum, mean, minimum or maximum (FinSimple kinds) of a finished table of K groups.
 template <int W>

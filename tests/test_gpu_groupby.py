@@ -183,6 +183,68 @@ def test_multi_column_and_unique():
     np.testing.assert_array_equal(got, O.unique_rows([a, b], [av, None]))
 
 
+@pytest.mark.parametrize("case", ["narrow", "two_to_32", "past_32", "full_range", "past_62", "all_null", "one_row",
+                                  "nine_columns", "offset", "with_float", "hot_key"])
+@pytest.mark.parametrize("n", [7001, 200003])
+def test_integer_columns_as_composite_keys(case, n):
+    """Several integer columns group by one composite key where the product of their spans allows it (32-bit
+    composites up to 2^32, 64-bit ones up to 2^62), and fold pairwise otherwise: ids, keys and their
+    validity against the oracle, and the representative rows through unique_rows."""
+    rng = np.random.default_rng(n)
+    pick = lambda lo, hi, dt: rng.integers(lo, hi, n, dtype=np.int64, endpoint=True).astype(dt)
+    valid = [rng.random(n) > 0.1, None, rng.random(n) > 0.2]
+    off = 0
+    if case == "narrow":
+        cols = [pick(-5, 40, np.int32), pick(0, 255, np.uint8), pick(-300, 300, np.int16)]
+    elif case in ("two_to_32", "past_32"):   # spans 2^20 and 2^12, or 2^12 + 1
+        cols = [pick(-2**19, 2**19 - 1, np.int64), pick(0, 4095 + (case == "past_32"), np.uint32)]
+        cols[0][:2], cols[1][:2], valid = [-2**19, 2**19 - 1], [0, 4095 + (case == "past_32")], [None, None]
+    elif case == "full_range":               # one column's span alone is 2^64
+        cols = [rng.choice(np.array([-2**63, 2**63 - 1, 0, 5]), n), pick(0, 3, np.int8), pick(0, 3, np.uint64)]
+    elif case == "past_62":
+        cols = [rng.choice(np.array([0, 2**40]), n), rng.choice(np.array([0, 2**30]), n), pick(0, 1, np.int16)]
+    elif case == "all_null":
+        cols, valid = [pick(0, 9, np.int64), pick(0, 9, np.int32)], [np.zeros(n, bool), rng.random(n) > 0.5]
+    elif case == "one_row":
+        n, cols, valid = 1, [np.array([7], np.int16), np.array([-9], np.int64)], [None, None]
+    elif case == "nine_columns":
+        cols, valid = [pick(0, 1, np.int8) for _ in range(9)], [None] * 9
+    elif case == "with_float":
+        cols = [pick(0, 9, np.int32), rng.choice(np.array([0.0, -0.0, np.nan, 2.5]), n), pick(0, 2, np.uint16)]
+    elif case == "hot_key":                  # most rows in one group, whose lowest row is late
+        cols = [np.where(np.arange(n) < 100, pick(1, 50, np.int64), 0), np.zeros(n, np.int16)]
+        valid = [None, None]
+    else:
+        cols, off = [pick(-5, 40, np.int32), pick(0, 255, np.uint8), pick(0, 1, np.int64)], 13
+    valid = valid[:len(cols)]
+    arrays = [am.MetalArray.from_numpy(c, v) for c, v in zip(cols, valid)]
+    if off:
+        arrays = [a.slice(off, n - off) for a in arrays]
+        cols, valid = [c[off:] for c in cols], [None if v is None else v[off:] for v in valid]
+    ids, K, rep = O.group_keys(cols, valid)
+    g = am.group_by(arrays)
+    assert g.group_count == K
+    np.testing.assert_array_equal(g.ids().to_numpy()[0], ids)
+    for got, col, v in zip(g.key_arrays(), cols, valid):
+        want_valid = np.ones(K, bool) if v is None else v[rep]
+        assert got.null_count == K - int(want_valid.sum())
+        vals, gv = got.to_numpy()
+        gv = np.ones(K, bool) if gv is None else gv
+        np.testing.assert_array_equal(gv, want_valid)
+        np.testing.assert_array_equal(vals[gv].view(np.uint8), col[rep][gv].view(np.uint8))
+    np.testing.assert_array_equal(am.unique_rows(arrays).to_numpy()[0], O.unique_rows(cols, valid))
+
+
+def test_lowest_rows_of_more_groups_than_the_partitioned_passes_take():
+    """Above 2^21 groups the lowest rows come from one pass of atomics."""
+    n = (1 << 21) + 200_000
+    rng = np.random.default_rng(1)
+    keys = rng.permutation(n).astype(np.float64)
+    keys[rng.integers(0, n, 50_000)] = 3.0        # one hot key
+    got = am.unique_rows([am.MetalArray.from_numpy(keys)]).to_numpy()[0]
+    np.testing.assert_array_equal(got, O.unique_rows([keys], [None]))
+
+
 def test_exact_float_sum_edges():
     groups = vectors()["group_sum_edges"]["groups"]
     keys, vals = [], []
