@@ -2354,6 +2354,110 @@ __global__ __launch_bounds__(256) void gb_final(const unsigned long long* table,
   if (threadIdx.x == 0) fold_report(fo, s_nulls[0] + s_nulls[1] + s_nulls[2] + s_nulls[3]);
 }
 
+// Rows up to which one workgroup does a whole aggregate, or a whole key mapping (gb_small_map): its row
+// loop takes about as long as a second kernel's launch.
+constexpr uint32_t SMALL_ROWS = 32768;
+
+// A whole aggregate over at most SMALL_ROWS rows whose table fits in LDS: rows, table and result column in
+// one launch of one workgroup. Each thread has eight rows in flight per step.
+template <class P, int IDW, int VW, class F>
+__global__ __launch_bounds__(1024) void gb_agg_small(AggArgs a, unsigned long long* table, F fin, FoldOut fo) {
+  extern __shared__ unsigned long long lds[];
+  __shared__ uint32_t s_nulls;
+  constexpr int R = 8;
+  const uint32_t K = uint32_t(a.K), n = uint32_t(a.n);
+  for (uint32_t j = threadIdx.x; j < K * P::W; j += 1024) lds[j] = identity(P::op(int(j % P::W)));
+  if (threadIdx.x == 0) s_nulls = 0u;
+  __syncthreads();
+  for (uint32_t base = threadIdx.x; base - threadIdx.x < n; base += 1024 * R) {
+    unsigned long long idr[R], vr[R];
+    uint32_t ib[R], vb[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {   // rows past the end read the last row
+      const int64_t ii = int64_t(min(base + uint32_t(r) * 1024u, n - 1u));
+      idr[r] = ld_raw<IDW>(a.ids.ids, ii);
+      ib[r] = ld_vbyte(a.ids.valid, a.ids.voff, ii);
+      vr[r] = 0;
+      if constexpr (VW != 0) vr[r] = ld_raw<VW>(a.v.vals, ii);
+      vb[r] = P::SKIP_NULL ? ld_vbyte(a.v.valid, a.v.voff, ii) : 0xFFu;
+    }
+    long long gs[R];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      gs[r] = part_gid<P, IDW>(a, int64_t(base) + r * 1024, int64_t(n), idr[r], ib[r], vb[r]);
+    if constexpr (P::AUX) {
+      typename P::AuxT ax[R];
+#pragma unroll
+      for (int r = 0; r < R; r++) ax[r] = P::aux_load(a, gs[r] >= 0 ? gs[r] : 0);
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        unsigned long long c[P::W];
+        if (gs[r] >= 0 && P::contrib(a, int64_t(base) + r * 1024, gs[r], val_in(a.v, vr[r]), ax[r], c))
+          apply<P>(as_lds(&lds[size_t(gs[r]) * P::W]), c);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        unsigned long long c[P::W];
+        if (gs[r] >= 0 && P::contrib(a, int64_t(base) + r * 1024, gs[r], val_in(a.v, vr[r]), c))
+          apply<P>(as_lds(&lds[size_t(gs[r]) * P::W]), c);
+      }
+    }
+  }
+  __syncthreads();
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t nulls = 0;
+  for (uint32_t base = threadIdx.x - lane; base < K; base += 1024) {
+    const uint32_t k = base + lane;
+    bool valid = false;
+    if (k < K) {
+      unsigned long long t[P::W];
+#pragma unroll
+      for (int w = 0; w < P::W; w++) {
+        t[w] = lds[size_t(k) * P::W + w];
+        if (table) table[size_t(k) * P::W + w] = t[w];
+      }
+      valid = fin((long long)k, t, fo);
+    }
+    const unsigned long long bal = __ballot(valid);
+    if (lane == 0 && fo.bits) fo.bits[base >> 6] = bal;
+    nulls += min(64u, K - base) - uint32_t(__popcll(bal));
+  }
+  if (lane == 0 && nulls) atomicAdd(&s_nulls, nulls);
+  __syncthreads();
+  if (threadIdx.x == 0 && fo.host) {
+    *fo.host = s_nulls;
+    if (fo.redo) *fo.redo = atomicExch(&fo.ctl->redo, 0ull);
+  }
+}
+
+template <class P, int IDW, int VW, class F>
+void launch_agg_small_t(const AggArgs& a, hipStream_t s, unsigned long long* table, const F& fin, const FoldOut& fo) {
+  const size_t lds = size_t(a.K) * P::W * 8;
+  if (lds > 32768)
+    AM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gb_agg_small<P, IDW, VW, F>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+  hipLaunchKernelGGL((gb_agg_small<P, IDW, VW, F>), dim3(1), dim3(1024), lds, s, a, table, fin, fo);
+  AM_HIP(hipGetLastError());
+}
+
+template <class P, class F>
+void launch_agg_small(const AggArgs& a, hipStream_t s, unsigned long long* table, const F& fin, const FoldOut& fo) {
+  auto width = [&](auto idw) {
+    constexpr int IDW = decltype(idw)::value;
+    if constexpr (!P::USES_VALUE) launch_agg_small_t<P, IDW, 0>(a, s, table, fin, fo);
+    else if constexpr (P::FIXED_VW != 0) launch_agg_small_t<P, IDW, P::FIXED_VW>(a, s, table, fin, fo);
+    else switch (type_width(a.v.type)) {
+      case 8: launch_agg_small_t<P, IDW, 8>(a, s, table, fin, fo); break;
+      case 4: launch_agg_small_t<P, IDW, 4>(a, s, table, fin, fo); break;
+      case 2: launch_agg_small_t<P, IDW, 2>(a, s, table, fin, fo); break;
+      default: launch_agg_small_t<P, IDW, 1>(a, s, table, fin, fo); break;
+    }
+  };
+  if (a.ids.type == T_I64) width(std::integral_constant<int, 8>{});
+  else width(std::integral_constant<int, 4>{});
+}
+
 // Groups up to which gb_fold also writes the result column: with more, its last-workgroup tickets (one
 // per 64 groups, on one address) would take longer than gb_final's own launch.
 constexpr long long FOLD_FINISH_MAX = 65536;
@@ -2521,6 +2625,11 @@ DevBuf run_agg(const AggArgs& a, hipStream_t s, const char* name, const F& fin =
   auto* o = static_cast<unsigned long long*>(out->ptr);
   const bool fits = a.K <= (long long)agg_dense_cap<P>();
   if (!fits && run_agg_part<P>(a, s, name, o, fin, fo, cache, col, keep_rows)) return out;
+  if (fits && a.n > 0 && a.n <= int64_t(SMALL_ROWS)) {
+    ProfScope ps(name);
+    launch_agg_small<P>(a, s, o, fin, fo);
+    return out;
+  }
   if (fits && a.n > 0) {
     const int blocks = agg_blocks(a.n);
     DevBuf part = device_alloc(size_t(blocks) * size_t(K) * P::W * 8);
@@ -2758,6 +2867,14 @@ void gb_use(const GroupBy* g) {
 
 namespace {
 
+// Marks where the handle's mapping ends on stream s.
+void gb_record(GroupBy* g, hipStream_t s) {
+  if (in_batch()) return;
+  AM_HIP(hipEventCreateWithFlags(&g->ready, hipEventDisableTiming));
+  AM_HIP(hipEventRecord(g->ready, s));
+  g->owner = s;
+}
+
 struct Mapped {
   int64_t K = 0;
   uint32_t D = 0;
@@ -2774,6 +2891,12 @@ bool range_path_enabled() {
   return !(e && e[0] == '0');
 }
 //
+// ARROWMETAL_GROUPBY_SMALL=0 turns the one-launch mapping of small inputs off (tests compare the two).
+bool small_path_enabled() {
+  const char* e = getenv("ARROWMETAL_GROUPBY_SMALL");
+  return !(e && e[0] == '0');
+}
+
 // Integer keys whose values span a small range (GroupByKeys.swift:268-337: span <= 2^24 and
 // <= max(2^16, 4n)) are mapped without hashing: one pass finds the smallest and largest order key, one
 // marks every present key in an occupancy array over the span (and its lowest row when representative
@@ -3177,6 +3300,378 @@ __global__ __launch_bounds__(256) void gb_decode_keys(const unsigned long long* 
   if (lane == 0) s_nulls[threadIdx.x >> 6] = nulls;
   __syncthreads();
   if (threadIdx.x == 0) fold_report(fo, s_nulls[0] + s_nulls[1] + s_nulls[2] + s_nulls[3]);
+}
+
+// ---------------------------------------------------------------- small inputs: the mapping in one launch
+//
+// Up to SMALL_ROWS rows with at most SMALL_KEYS distinct keys, one workgroup maps the key columns alone: a
+// hash table in LDS, ids and representative rows written, the counts in pinned host memory. The general
+// mapping takes nine launches and a read-back in the middle. Up to SMALL_RANKED distinct keys the workgroup
+// also ranks them, by counting; more are ranked by gb_small_rank, many workgroups, and the ids written by
+// gb_small_ids (one workgroup's LDS reads bound the counting: 1,000 keys take it 45 us). The whole call over
+// 20,000 rows: 300 keys 80 -> 48 us, 4,000 keys 73 us; 1,000 rows 21 us; two columns of 20,000 rows 79 us.
+// One CU reads and probes about 1,000 rows per us, so beyond SMALL_ROWS the general mapping is as fast.
+constexpr uint32_t SMALL_KEYS = 4096;
+constexpr uint32_t SMALL_RANKED = 256;
+constexpr uint32_t SMALL_SLOTS = 8192;   // hash slots; then the slot of the key that looks like an empty slot
+constexpr uint32_t SMALL_NULL = SMALL_SLOTS + 1u;   // a null row's "slot" (one key column)
+
+struct SmallStat {
+  uint32_t ok, distinct, has_null, ranked;
+};
+
+// What the one-launch mapping writes besides the ids (null where a caller asks for no such thing).
+struct SmallOut {
+  uint32_t* ids;    // the rows' ids, or their slots when the keys are not ranked yet
+  uint32_t* rep;    // representative rows of the groups, in group order
+  uint32_t* uniq;   // the kept rows in ascending order (then nothing is ranked)
+  unsigned long long* dkey;   // unranked keys, with their slots and lowest rows
+  uint32_t *dslot, *drow, *gid;   // gid[SMALL_SLOTS + 2]: each slot's id, once ranked
+};
+
+// A key's home slot.
+__device__ __forceinline__ uint32_t small_slot(unsigned long long k) {
+  uint32_t x = uint32_t(k) * 0x9E3779B1u ^ uint32_t(k >> 32) * 0x85EBCA77u;
+  x ^= x >> 15;
+  return (x * 0x2C1B3C6Du) >> (32 - 13);
+}
+
+struct SmallLds {
+  union {
+    unsigned long long key[SMALL_SLOTS + 2];
+    uint32_t gid[SMALL_SLOTS + 2];   // once the keys have been collected
+  };
+  uint32_t first[SMALL_SLOTS + 2];   // a slot's lowest row; all ones: free
+  unsigned long long dkey[SMALL_RANKED];   // the distinct keys, and their slots
+  uint32_t dslot[SMALL_RANKED];
+  uint32_t mark[SMALL_ROWS / 32];        // unique rows: a bit per kept row
+  unsigned long long lo[16], hi[16];
+  uint32_t nz[16], tmp[16];
+  ColSpan span[COMPOSITE_MAX];
+  uint32_t distinct, failed, cursor;
+};
+
+// Key words of R rows of one column (order keys; rows ii[r]) and whether each is null.
+template <int R>
+__device__ __forceinline__ void small_load(const CompositeCol& k, const uint32_t (&ii)[R], unsigned long long (&key)[R],
+                                           bool (&null)[R]) {
+  unsigned long long raw[R];
+  uint32_t vb[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) vb[r] = ld_vbyte(k.valid, k.voff, int64_t(ii[r]));
+  switch (type_width(k.type)) {   // uniform
+    case 8:
+#pragma unroll
+      for (int r = 0; r < R; r++) raw[r] = ld_raw<8>(k.vals, int64_t(ii[r]));
+      break;
+    case 4:
+#pragma unroll
+      for (int r = 0; r < R; r++) raw[r] = ld_raw<4>(k.vals, int64_t(ii[r]));
+      break;
+    case 2:
+#pragma unroll
+      for (int r = 0; r < R; r++) raw[r] = ld_raw<2>(k.vals, int64_t(ii[r]));
+      break;
+    default:
+#pragma unroll
+      for (int r = 0; r < R; r++) raw[r] = ld_raw<1>(k.vals, int64_t(ii[r]));
+      break;
+  }
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    null[r] = vbit(k.voff, int64_t(ii[r]), vb[r]) == 0u;
+    key[r] = order_key(key_of_raw(raw[r], k.type), k.type);
+  }
+}
+
+__global__ __launch_bounds__(1024) void gb_small_map(CompositeArgs a, uint32_t n, SmallOut o, SmallStat* st) {
+  extern __shared__ __align__(16) unsigned char small_lds[];
+  SmallLds& L = *reinterpret_cast<SmallLds*>(small_lds);
+  constexpr int R = 8;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  if (tid == 0) L.distinct = L.failed = L.cursor = 0u;
+  // Several columns: their spans, and their places in the composite key.
+  if (a.count > 1) {
+    for (int c = 0; c < a.count; c++) {
+      unsigned long long lo = ~0ull, hi = 0ull;
+      uint32_t nz = 0;
+      for (uint32_t base = tid; base - tid < n; base += 1024 * R) {
+        uint32_t ii[R];
+        unsigned long long key[R];
+        bool null[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) ii[r] = min(base + uint32_t(r) * 1024u, n - 1u);   // a row read twice changes nothing
+        small_load<R>(a.col[c], ii, key, null);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          nz |= null[r] ? 1u : 0u;
+          lo = !null[r] && key[r] < lo ? key[r] : lo;
+          hi = !null[r] && key[r] > hi ? key[r] : hi;
+        }
+      }
+      for (int off = 32; off > 0; off >>= 1) {
+        lo = min(lo, (unsigned long long)__shfl_xor(lo, off, 64));
+        hi = max(hi, (unsigned long long)__shfl_xor(hi, off, 64));
+        nz |= __shfl_xor(nz, off, 64);
+      }
+      if (lane == 0) {
+        L.lo[wave] = lo;
+        L.hi[wave] = hi;
+        L.nz[wave] = nz;
+      }
+      __syncthreads();
+      if (tid == 0) {
+        for (int w = 1; w < 16; w++) {
+          lo = min(lo, L.lo[w]);
+          hi = max(hi, L.hi[w]);
+          nz |= L.nz[w];
+        }
+        const bool any = lo <= hi;
+        const unsigned long long width = any ? hi - lo : 0ull;   // the span less one
+        if (width >= (1ull << 62)) L.failed = 1u;
+        L.span[c] = ColSpan{any ? lo : 0ull, (any ? width + 1ull : 0ull) + (nz ? 1ull : 0ull), 1ull, nz ? 1 : 0};
+      }
+      __syncthreads();
+    }
+    if (tid == 0) {
+      unsigned long long total = 1;
+      for (int c = 0; c < a.count && !L.failed; c++) {
+        if (__umul64hi(total, L.span[c].span) != 0ull || total * L.span[c].span > (1ull << 62)) L.failed = 1u;
+        total *= L.span[c].span;
+      }
+    }
+  }
+  for (uint32_t j = tid; j < SMALL_SLOTS + 2; j += 1024) {
+    L.key[j] = EMPTY;
+    L.first[j] = 0xFFFFFFFFu;
+  }
+  if (o.uniq)
+    for (uint32_t j = tid; j < SMALL_ROWS / 32; j += 1024) L.mark[j] = 0u;
+  __syncthreads();
+  volatile uint32_t* failed = &L.failed;
+  for (uint32_t base = tid; base - tid < n; base += 1024 * R) {
+    if (*failed) break;
+    uint32_t ii[R], slot[R], low[R];
+    unsigned long long key[R];
+    bool null[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) ii[r] = min(base + uint32_t(r) * 1024u, n - 1u);
+    if (a.count == 1) {
+      small_load<R>(a.col[0], ii, key, null);
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; r++) key[r] = 0ull;
+      for (int c = 0; c < a.count; c++) {
+        unsigned long long kc[R];
+        small_load<R>(a.col[c], ii, kc, null);
+        const ColSpan sp = L.span[c];
+#pragma unroll
+        for (int r = 0; r < R; r++) key[r] = key[r] * sp.span + (null[r] ? sp.span - 1ull : kc[r] - sp.kmin);
+      }
+#pragma unroll
+      for (int r = 0; r < R; r++) null[r] = false;
+    }
+    // Every row's home slot and its lowest row are read together; a row whose key is there (most rows of a
+    // repeated key) is done, the others probe on one at a time.
+    unsigned long long cur[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      slot[r] = null[r] ? SMALL_NULL : key[r] == EMPTY ? SMALL_SLOTS : small_slot(key[r]);
+      cur[r] = L.key[slot[r]];
+      low[r] = L.first[slot[r]];
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      if (base + uint32_t(r) * 1024u >= n) continue;
+      if (!null[r] && cur[r] != key[r]) {
+        uint32_t h = slot[r];
+        unsigned long long c = cur[r];
+        while (true) {
+          if (c == EMPTY) {
+            c = atomicCAS(&L.key[h], EMPTY, key[r]);
+            if (c == EMPTY) {
+              if (atomicAdd(&L.distinct, 1u) >= SMALL_KEYS - 1u) *failed = 1u;   // one is left for the key EMPTY
+              c = key[r];
+            }
+          }
+          if (c == key[r]) break;
+          if (*failed) break;   // the table cannot fill up: past SMALL_KEYS keys no row is placed
+          h = (h + 1u) & (SMALL_SLOTS - 1u);
+          c = L.key[h];
+        }
+        slot[r] = h;
+        low[r] = L.first[h];
+      }
+      if (ii[r] < low[r]) atomicMin(&L.first[slot[r]], ii[r]);   // a stale read is never too low
+    }
+    if (o.ids) {
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        if (base + uint32_t(r) * 1024u < n) o.ids[ii[r]] = slot[r];
+    }
+  }
+  __syncthreads();
+  const bool bad = *failed != 0u;
+  const bool has_null = L.first[SMALL_NULL] != 0xFFFFFFFFu;
+  __syncthreads();
+  if (bad) {
+    if (tid == 0) *st = SmallStat{0u, 0u, 0u, 0u};
+    return;
+  }
+  if (o.uniq) {   // the lowest rows, in row order
+    for (uint32_t j = tid; j < SMALL_SLOTS + 2u; j += 1024) {
+      const uint32_t row = L.first[j];
+      if (row != 0xFFFFFFFFu) atomicOr(&L.mark[row >> 5], 1u << (row & 31u));
+    }
+    __syncthreads();
+    static_assert(SMALL_ROWS / 32 == 1024, "a word of marks per thread");
+    uint32_t bits = L.mark[tid], total;
+    uint32_t at = block_scan_1024(uint32_t(__popc(bits)), L.tmp, total);
+    while (bits) {
+      const uint32_t b = uint32_t(__ffs(int(bits))) - 1u;
+      bits &= bits - 1u;
+      o.uniq[at++] = tid * 32u + b;
+    }
+    if (tid == 0) *st = SmallStat{1u, total, 0u, 1u};
+    return;
+  }
+  // The distinct keys, in any order: in LDS when they are ranked here, otherwise out.
+  const bool special = L.first[SMALL_SLOTS] != 0xFFFFFFFFu;
+  const uint32_t D = L.distinct + (special ? 1u : 0u);
+  const bool ranked = D <= SMALL_RANKED;
+  for (uint32_t j = tid; j < SMALL_SLOTS + 1u; j += 1024) {
+    if (L.first[j] != 0xFFFFFFFFu) {
+      const uint32_t at = atomicAdd(&L.cursor, 1u);
+      if (ranked) {
+        L.dkey[at] = L.key[j];   // the slot past the table holds EMPTY, which is its key
+        L.dslot[at] = j;
+      } else {
+        o.dkey[at] = L.key[j];
+        o.dslot[at] = j;
+        o.drow[at] = L.first[j];
+      }
+    }
+  }
+  if (tid == 0) {
+    if (has_null) o.rep[D] = L.first[SMALL_NULL];
+    *st = SmallStat{1u, D, has_null ? 1u : 0u, ranked ? 1u : 0u};
+  }
+  if (!ranked) return;
+  __syncthreads();
+  // Places by counting, 1024 / SMALL_RANKED threads on each key.
+  constexpr uint32_t PARTS = 1024 / SMALL_RANKED;
+  const uint32_t i = tid / PARTS, part = tid % PARTS;
+  uint32_t before = 0;
+  if (i < D) {
+    const unsigned long long mine = L.dkey[i];
+    for (uint32_t j = part; j < D; j += PARTS) before += L.dkey[j] < mine ? 1u : 0u;
+  }
+#pragma unroll
+  for (int off = 1; off < int(PARTS); off <<= 1) before += __shfl_xor(before, off, 64);
+  __syncthreads();   // the slots' keys become their ids
+  if (i < D && part == 0u) {
+    L.gid[L.dslot[i]] = before;
+    o.rep[before] = L.first[L.dslot[i]];
+  }
+  if (tid == 0) L.gid[SMALL_NULL] = D;
+  __syncthreads();
+  for (uint32_t base = tid; base - tid < n; base += 1024 * R) {   // each row's slot was written by this thread
+    uint32_t h[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) h[r] = o.ids[min(base + uint32_t(r) * 1024u, n - 1u)];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const uint32_t row = base + uint32_t(r) * 1024u;
+      if (row < n) o.ids[row] = L.gid[h[r]];
+    }
+  }
+}
+
+// The places of the D unranked keys, 64 per workgroup: every workgroup holds all keys in LDS, and each of
+// its 16 waves counts a sixteenth of them, four keys per lane, as the argsort of small inputs does.
+__global__ __launch_bounds__(1024) void gb_small_rank(const unsigned long long* dkey, const uint32_t* dslot,
+                                                      const uint32_t* drow, uint32_t D, uint32_t* gid, uint32_t* rep) {
+  __shared__ unsigned long long s_key[SMALL_KEYS];
+  __shared__ uint32_t s_cnt[16][64];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+  const uint32_t padded = (D + 255u) / 256u * 256u;
+  for (uint32_t j = tid; j < padded; j += 1024) s_key[j] = j < D ? dkey[j] : ~0ull;   // padding is below no key
+  __syncthreads();
+  const uint32_t r0 = blockIdx.x * 64u, rl = lane & 15u, part = lane >> 4;
+  unsigned long long mine[4];
+  uint32_t cnt[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (uint32_t q = 0; q < 4; q++) mine[q] = s_key[r0 + rl + 16u * q];
+  const uint32_t share = padded / 16u, j0 = w * share;
+  for (uint32_t j = j0 + 4u * part; j < j0 + share; j += 16) {
+#pragma unroll
+    for (uint32_t u = 0; u < 4; u++) {
+      const unsigned long long k = s_key[j + u];
+#pragma unroll
+      for (uint32_t q = 0; q < 4; q++) cnt[q] += k < mine[q] ? 1u : 0u;
+    }
+  }
+#pragma unroll
+  for (uint32_t q = 0; q < 4; q++) {
+    cnt[q] += __shfl_xor(cnt[q], 16, 64);
+    cnt[q] += __shfl_xor(cnt[q], 32, 64);
+    if (part == q) s_cnt[w][16u * q + rl] = cnt[q];
+  }
+  __syncthreads();
+  const uint32_t i = r0 + lane;
+  if (w != 0) return;
+  if (i == 0) gid[SMALL_NULL] = D;
+  if (i >= D) return;
+  uint32_t place = 0;
+  for (uint32_t v = 0; v < 16; v++) place += s_cnt[v][lane];
+  gid[dslot[i]] = place;
+  rep[place] = drow[i];
+}
+
+__global__ void gb_small_ids(uint32_t* ids, uint32_t n, const uint32_t* gid) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) ids[i] = gid[ids[i]];
+}
+
+// Whether the one-launch mapping takes these columns, and the mapping: false when it does not (too many
+// rows, distinct keys or columns, float columns among several, spans whose product is above 2^62).
+bool small_map(Array* const* columns, int64_t count, int64_t n, SmallOut o, SmallStat& out) {
+  if (n < 1 || n > int64_t(SMALL_ROWS) || count > COMPOSITE_MAX || !small_path_enabled()) return false;
+  CompositeArgs a{};
+  a.count = int(count);
+  for (int64_t c = 0; c < count; c++) {
+    const Array* k = columns[c];
+    if (count > 1 && !type_is_int(k->type)) return false;
+    a.col[c] = CompositeCol{k->data(), k->has_nulls() ? k->valid_bits() : nullptr, k->offset, k->type, ColSpan{}};
+  }
+  hipStream_t s = stream();
+  std::shared_ptr<void> slot = pinned_slot();
+  auto* st = static_cast<SmallStat*>(slot.get());
+  DevBuf work;
+  if (!o.uniq) {
+    work = device_alloc(SMALL_KEYS * 16 + (SMALL_SLOTS + 2) * 4);
+    o.dkey = static_cast<unsigned long long*>(work->ptr);
+    o.dslot = reinterpret_cast<uint32_t*>(o.dkey + SMALL_KEYS);
+    o.drow = o.dslot + SMALL_KEYS;
+    o.gid = o.drow + SMALL_KEYS;
+  }
+  AM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gb_small_map), hipFuncAttributeMaxDynamicSharedMemorySize,
+                             int(sizeof(SmallLds))));
+  {
+    ProfScope ps("gb_small_map");
+    hipLaunchKernelGGL(gb_small_map, dim3(1), dim3(1024), sizeof(SmallLds), s, a, uint32_t(n), o, st);
+    AM_HIP(hipGetLastError());
+  }
+  AM_HIP(hipStreamSynchronize(s));
+  out = *st;
+  if (out.ok && !out.ranked) {
+    ProfScope ps("gb_small_rank");
+    hipLaunchKernelGGL(gb_small_rank, dim3((out.distinct + 63u) / 64u), dim3(1024), 0, s, o.dkey, o.dslot, o.drow, out.distinct,
+                       o.gid, o.rep);
+    hipLaunchKernelGGL(gb_small_ids, dim3((uint32_t(n) + 255u) / 256u), dim3(256), 0, s, o.ids, uint32_t(n), o.gid);
+    AM_HIP(hipGetLastError());
+  }
+  return out.ok != 0u;
 }
 
 // Calls f(TYPE) for an integer key type (the range path maps no others).
@@ -3595,6 +4090,22 @@ GroupBy* group_by_keys_impl(Array* const* columns, int64_t count, bool need_rep)
       return g;
     }
     hipStream_t s = stream();
+    if (n <= int64_t(SMALL_ROWS)) {
+      g->ids = device_alloc(size_t(n) * 4);
+      g->rep = device_alloc(size_t(SMALL_KEYS + 1) * 4);
+      SmallStat st;
+      SmallOut so{};
+      so.ids = static_cast<uint32_t*>(g->ids->ptr);
+      so.rep = static_cast<uint32_t*>(g->rep->ptr);
+      if (small_map(columns, count, n, so, st)) {
+        g->D = st.distinct;
+        g->has_null = st.has_null != 0u;
+        g->K = int64_t(g->D) + (g->has_null ? 1 : 0);
+        g->has_rep = true;
+        if (!st.ranked) gb_record(g, s);   // otherwise complete already: nothing to order other streams after
+        return g;
+      }
+    }
     bool ints = true;
     for (int64_t c = 0; c < count; c++) ints = ints && type_is_int(columns[c]->type);
     int64_t K = 0;
@@ -3646,11 +4157,7 @@ GroupBy* group_by_keys_impl(Array* const* columns, int64_t count, bool need_rep)
     g->K = K;
     // No wait here: the ids are only read by later calls, which are ordered after the mapping (the
     // same stream, or `ready`), so the caller's next call is prepared while the last kernels run.
-    if (!in_batch()) {
-      AM_HIP(hipEventCreateWithFlags(&g->ready, hipEventDisableTiming));
-      AM_HIP(hipEventRecord(g->ready, s));
-      g->owner = s;
-    }
+    gb_record(g, s);
   } catch (...) {
     delete g;
     throw;
@@ -4096,6 +4603,20 @@ Array* unique_rows(Array* const* columns, int64_t count) {
     check_length(columns[0]->length);
     // The representative rows come from the row numbers 0 .. n-1 (GroupByKeys.swift:126-149, 436-438).
     check_index_rows(columns[0]->length, "row indices");
+  }
+  if (count >= 1 && columns[0]->length >= 1 && columns[0]->length <= int64_t(SMALL_ROWS)) {
+    bool same = true;
+    for (int64_t c = 0; c < count; c++) same = same && columns[c]->length == columns[0]->length && type_is_primitive(columns[c]->type);
+    DevBuf rows = device_alloc(size_t(SMALL_KEYS + 1) * 4);
+    SmallStat st;
+    SmallOut so{};
+    so.uniq = static_cast<uint32_t*>(rows->ptr);
+    if (same && small_map(columns, count, columns[0]->length, so, st)) {
+      Array* out = new_array("I", T_U32, int64_t(st.distinct));
+      out->values = rows;
+      out->null_count = 0;
+      return out;
+    }
   }
   GroupBy* g = group_by_keys_impl(columns, count, true);
   Array* out = nullptr;

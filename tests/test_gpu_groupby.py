@@ -235,6 +235,58 @@ def test_integer_columns_as_composite_keys(case, n):
     np.testing.assert_array_equal(am.unique_rows(arrays).to_numpy()[0], O.unique_rows(cols, valid))
 
 
+@pytest.mark.parametrize("case", ["int64", "nulls", "extremes", "float64", "float32", "int8", "two", "three_nulls", "wide_pair",
+                                  "all_null", "offset"])
+@pytest.mark.parametrize("n,span", [(1, 1), (63, 5), (1024, 1024), (1025, 700), (8193, 3000), (20011, 4094), (20011, 4097),
+                                    (32768, 300), (32769, 300)])
+def test_small_inputs_in_one_launch(case, n, span, monkeypatch):
+    """Up to 32,768 rows and 4,096 distinct keys the mapping is one launch: ids, keys, aggregates and unique
+    rows against the oracle at the edges of its rows, its key sort (1,024) and its key limit, where it
+    gives up, and the same with it switched off."""
+    rng = np.random.default_rng(n * 7 + span)
+    k = rng.permutation(np.resize(np.arange(span), n))
+    valid = [None]
+    off = 0
+    if case == "int64": cols = [k.astype(np.int64) * 0x9E3779B97F4A7C1 - 2**62]
+    elif case == "nulls": cols, valid = [k.astype(np.uint32)], [rng.random(n) > 0.3]
+    elif case == "extremes": cols = [np.array([-2**63, 2**63 - 1, 0, -1, 1], np.int64)[k % 5]]
+    elif case == "float64": cols = [np.array([np.nan, -0.0, 0.0, np.inf, -np.inf, 2.5, -np.nan, 1e-310])[k % 8]]
+    elif case == "float32": cols, valid = [(k - span / 2).astype(np.float32)], [rng.random(n) > 0.1]
+    elif case == "int8": cols = [k.astype(np.int8)]
+    elif case == "two": cols, valid = [(k // 7).astype(np.int32), (k % 7).astype(np.uint16)], [None, None]
+    elif case == "three_nulls":
+        cols = [(k // 50).astype(np.int64) - 40, (k % 50).astype(np.int8), np.zeros(n, np.uint64)]
+        valid = [rng.random(n) > 0.1, rng.random(n) > 0.1, None]
+    elif case == "wide_pair": cols, valid = [np.where(k % 2, 2**62, -2**62), k.astype(np.int64)], [None, None]
+    elif case == "all_null": cols, valid = [k.astype(np.int32)], [np.zeros(n, bool)]
+    else: cols, valid, off = [k.astype(np.int64)], [rng.random(n) > 0.5], min(5, n - 1)
+    arrays = [am.MetalArray.from_numpy(c, v) for c, v in zip(cols, valid)]
+    if off:
+        arrays = [a.slice(off, n - off) for a in arrays]
+        cols, valid = [c[off:] for c in cols], [None if v is None else v[off:] for v in valid]
+    m = n - off
+    ids, K, rep = O.group_keys(cols, valid)
+    vals = rng.integers(-10**9, 10**9, m)
+    f = rng.standard_normal(m) * 10.0 ** rng.integers(-200, 200, m)
+    vv = rng.random(m) > 0.2
+    for small in ("1", "0") if n < 3000 else ("1",):
+        monkeypatch.setenv("ARROWMETAL_GROUPBY_SMALL", small)
+        g = am.group_by(arrays)
+        assert g.group_count == K
+        np.testing.assert_array_equal(g.ids().to_numpy()[0], ids)
+        for got, col, v in zip(g.key_arrays(), cols, valid):
+            gvals, gv = got.to_numpy()
+            want_valid = np.ones(K, bool) if v is None else v[rep]
+            np.testing.assert_array_equal(np.ones(K, bool) if gv is None else gv, want_valid)
+            np.testing.assert_array_equal(gvals[want_valid].view(np.uint8), col[rep][want_valid].view(np.uint8))
+        for values, ops in ((vals, (0, 1, 2, 3, 4, 5)), (f, (4, 5, 0, 3))):
+            mv = am.MetalArray.from_numpy(values, vv)
+            for op in ops:
+                got = g.count_all() if op == 1 else getattr(g, ("sum", "", "count", "mean", "min", "max")[op])(mv)
+                assert_agg(got, O.group_agg(ids, K, values, op, vv), f"{case} op {op}")
+        np.testing.assert_array_equal(am.unique_rows(arrays).to_numpy()[0], O.unique_rows(cols, valid))
+
+
 def test_lowest_rows_of_more_groups_than_the_partitioned_passes_take():
     """Above 2^21 groups the lowest rows come from one pass of atomics."""
     n = (1 << 21) + 200_000
