@@ -551,7 +551,7 @@ __device__ __forceinline__ void local_lsd(const K* keys_in, const uint32_t* rows
     pos[j] = base_e + uint32_t(j) * 64u;
     keys[j] = keys_in[off + min(pos[j], size - 1u)];
   }
-  if ((low_mask >> 7) & 1u) {
+  if (sizeof(K) == 8 && ((low_mask >> 7) & 1u)) {
     local_split<K, LI>(keys, pos, base_e, size, 7, wc, tile_total, bin_start, tmp, s_keys, s_pos);
     __syncthreads();
     if (!__syncthreads_or(tile_total[threadIdx.x] > run_max ? 1 : 0)) {
@@ -563,7 +563,7 @@ __device__ __forceinline__ void local_lsd(const K* keys_in, const uint32_t* rows
         src[j] = off;
         if (e < size) {
           const K key = s_keys[e];
-          const uint32_t dd = uint32_t(key >> 56);
+          const uint32_t dd = uint32_t((unsigned long long)key >> 56);
           const uint32_t lo = bin_start[dd], hi = lo + tile_total[dd];
           uint32_t below = 0;
 #pragma unroll 4
@@ -939,7 +939,9 @@ inline MsdWork msd_work(uint32_t m, int items, DevBuf (*alloc)(size_t), uint32_t
 // w.large[0] with its count, the bucket sort's list started, the counters and w.mc set).
 // - Read-back form (blind = false; `mask` = the active digits, known on the host): only active
 //   digits get a level, each launch is sized from 64 bytes of counters read back after each level,
-//   and the bucket sort's keys per thread come from the largest bucket. Returns false, with no row
+//   and the bucket sort's keys per thread come from the largest bucket. A caller that knows the lists it
+//   built (large: entries of w.large[0]; biggest_local and local_entries: the bucket sort's) passes their
+//   counts, so that a sort without a large bucket launches no level and reads nothing back. Returns false, with no row
 //   written that a rerun does not write again, when the bucket sort's list ran out of room.
 // - Blind form (blind = true, e.g. inside a graph capture): every digit below `top` gets a level,
 //   sized for the worst case, the kernels read what to do from the device, and the bucket sort takes
@@ -948,7 +950,8 @@ inline MsdWork msd_work(uint32_t m, int items, DevBuf (*alloc)(size_t), uint32_t
 template <typename K, int ITEMS>
 bool msd_levels(const MsdWork& w, uint32_t m, int top, uint32_t mask, bool blind, uint32_t local_max,
                 unsigned long long* status, K* k0, uint32_t* r0, K* k1, uint32_t* r1, uint32_t* out_idx,
-                hipStream_t s, bool keys = false) {
+                hipStream_t s, bool keys = false, const uint32_t* large = nullptr, const uint32_t* biggest_local = nullptr,
+                const uint32_t* local_entries = nullptr) {
   constexpr int P = int(sizeof(K));
   constexpr uint32_t TILE = BLOCK * ITEMS;
   const uint32_t cus = uint32_t(device().cu_count);
@@ -962,7 +965,7 @@ bool msd_levels(const MsdWork& w, uint32_t m, int top, uint32_t mask, bool blind
     return d;
   };
   // Large buckets and their rows (bounds of the grids): at most RADIX top-digit buckets first.
-  uint32_t bound = blind ? w.large_cap : uint32_t(RADIX), rows = m;
+  uint32_t bound = blind ? w.large_cap : large ? *large : uint32_t(RADIX), rows = m;
   int cur = 0;
   bool read = false;
   for (int d = next_digit(top); d >= 0 && bound > 0; d = next_digit(d)) {
@@ -1010,7 +1013,11 @@ bool msd_levels(const MsdWork& w, uint32_t m, int top, uint32_t mask, bool blind
   int li = 8, li_lsd = 8;
   uint32_t grid = cus * 8u, group_grid = cus * 4u;
   if (!blind) {
-    if (!read) {   // no level ran (no active digit below the top one)
+    if (!read && large) {   // no level ran, and the caller knows the lists
+      std::memset(hp, 0, LC_READ * 4);
+      hp[LC_MAXLOCAL] = *biggest_local;
+      hp[LC_LOCAL] = *local_entries;
+    } else if (!read) {
       AM_HIP(hipMemcpyAsync(hp, w.lc, LC_READ * 4, hipMemcpyDeviceToHost, s));
       AM_HIP(hipStreamSynchronize(s));
     }

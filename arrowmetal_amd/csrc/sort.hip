@@ -9,9 +9,9 @@
 //   sort_init      clears the per-call control block (a fill kernel, no hipMemset, so that the
 //                  sequence can be captured in a graph)
 //   sort_upsweep   one read of the column: maps every key, counts values / NaN / nulls, and builds
-//                  the digit histograms of ALL passes at once plus the OR / AND of the keys
-//   sort_plan      one workgroup: active-pass mask, block bases of the three buckets, and the
-//                  exclusive digit prefix of every pass
+//                  the digit histograms of all (varying) digits at once plus the OR / AND of the keys
+//                  The last workgroup done makes the plan: active-pass mask, block bases of the three
+//                  buckets, and the exclusive digit prefix of every pass
 //   sort_first     the first active pass reads the raw column again, maps keys on the fly, and
 //                  scatters values by digit while NaN and null rows go straight to their final slots
 //   sort_mid       one launch per further active digit; the last active pass writes only the row
@@ -32,17 +32,15 @@ namespace am {
 namespace {
 
 struct SortCtl {
-  uint32_t hist[8][RADIX];          // digit histograms of the value keys, one per pass
-  uint32_t m, q, z, pad0;           // value rows, NaN rows (separate block), null rows
-  unsigned long long key_or, key_and;
+  uint32_t m;                       // value rows
   // Bumped by every workgroup of a pass, so on cache lines of their own: a line that also holds
   // words the same workgroups read slows the pass down.
   alignas(128) uint32_t tile_counter[16];   // [0] first pass, [1 + p] pass p, [11] units
   alignas(128) uint32_t digit_base[8][RADIX];   // exclusive digit prefix inside the value block, per pass
+  uint32_t bin_total[NBINS_FIRST], first_base[NBINS_FIRST];   // the hybrid sort's analysis
   uint32_t active_mask, first_active, last_active, pad1;
   uint32_t value_base, nan_base, null_base, pad2;
-  // Per-XCD partials of the upsweep (updated by workgroup-scope atomics in each XCD's own L2), folded
-  // into the fields above by sort_plan.
+  // Per-XCD partials of the upsweep, folded into the fields above by sort_plan.
   uint32_t xhist[NXCD][8][RADIX];
   uint32_t xm[NXCD], xq[NXCD], xz[NXCD], pad3[NXCD];
   unsigned long long xor_[NXCD], xand[NXCD];
@@ -50,14 +48,18 @@ struct SortCtl {
 
 // ---------------------------------------------------------------- kernels
 
-__global__ void sort_init(SortCtl* ctl) {
-  uint32_t* w = reinterpret_cast<uint32_t*>(ctl);
-  const int words = int(sizeof(SortCtl) / 4);
-  for (int i = threadIdx.x; i < words; i += blockDim.x) w[i] = 0u;
-  __syncthreads();
-  if (threadIdx.x == 0) ctl->key_and = ~0ull;
-  if (threadIdx.x < NXCD) ctl->xand[threadIdx.x] = ~0ull;
+// A cleared control block (by one workgroup).
+__device__ __forceinline__ void clear_ctl(SortCtl* ctl) {
+  for (uint32_t i = threadIdx.x; i < uint32_t(NXCD * 8 * RADIX); i += blockDim.x) (&ctl->xhist[0][0][0])[i] = 0u;
+  if (threadIdx.x < NXCD) {
+    ctl->xm[threadIdx.x] = ctl->xq[threadIdx.x] = ctl->xz[threadIdx.x] = 0u;
+    ctl->xor_[threadIdx.x] = 0ull;
+    ctl->xand[threadIdx.x] = ~0ull;
+  }
+  if (threadIdx.x < 16) ctl->tile_counter[threadIdx.x] = 0u;
 }
+
+__global__ void sort_init(SortCtl* ctl) { clear_ctl(ctl); }
 
 // Copies the plan (active mask, first and last active pass, value rows) to pinned host memory.
 __global__ void sort_read_plan(const SortCtl* ctl, uint32_t* out) {
@@ -68,42 +70,57 @@ __global__ void sort_read_plan(const SortCtl* ctl, uint32_t* out) {
 }
 
 
-// Rows per unit of the top-digit partition (a power of two): the upsweep counts the top digit, NaN
-// and null rows per unit when given unit_hist ([NBINS_FIRST][nunits], bin-major), so that the
-// partition knows every unit's destinations before it starts.
-// Units are 2^unit_shift rows: 16K for 4M rows and more, 4K (one tile of the partition) below, so
-// that a 1M-row input still has ~250 units to spread over the CUs.
-constexpr uint32_t UNIT_SHIFT_LARGE = 14, UNIT_SHIFT_SMALL = 12;
-constexpr uint32_t UNITS_PER_BLOCK = 8;   // most units one upsweep workgroup counts
+// Waits for an atomic by its result: it has been carried out at the memory side, where every XCD's
+// atomics meet. (A device-scope fence would write back the XCD's whole L2 instead.)
+template <typename T>
+__device__ __forceinline__ void atomic_done(T result) {
+  asm volatile("" ::"v"(result) : "memory");
+}
 
-template <typename K, int W>
-__global__ __launch_bounds__(BLOCK) void sort_upsweep(const void* vals, const uint8_t* valid, int64_t voff,
-                                                      uint32_t n, int type, int forder, int desc,
-                                                      uint32_t rows_per_block, SortCtl* ctl, uint32_t* unit_hist,
-                                                      uint32_t nunits, uint32_t unit_shift, int all_digits) {
-  constexpr int P = int(sizeof(K));
-  __shared__ uint32_t h[P][RADIX];
-  __shared__ uint32_t hu[UNITS_PER_BLOCK][NBINS_FIRST];
-  __shared__ uint32_t cnt[3];
-  __shared__ unsigned long long s_or, s_and;
-  const bool units = unit_hist != nullptr;   // uniform
-  for (int i = threadIdx.x; i < P * RADIX; i += BLOCK) (&h[0][0])[i] = 0u;
-  if (units)
-    for (int i = threadIdx.x; i < int(UNITS_PER_BLOCK * NBINS_FIRST); i += BLOCK) (&hu[0][0])[i] = 0u;
-  if (threadIdx.x < 3) cnt[threadIdx.x] = 0u;
-  if (threadIdx.x == 0) { s_or = 0ull; s_and = ~0ull; }
-  __syncthreads();
-  uint32_t begin = blockIdx.x * rows_per_block;
-  uint32_t end = min(n, begin + rows_per_block);
-  K o = 0, a = K(~K(0));
-  uint32_t cm = 0, cq = 0, cz = 0;
-  // UP_ITEMS rows per thread per step, loaded before any is counted; two steps' rows take turns, so that
-  // the next step's loads are in flight while this step is counted, and every loaded register is taken
-  // at the top of a step (a load the compiler moved into one of the classification's branches would be
-  // waited for there alone). The step count is the same for every thread of the block.
-  constexpr int UP_ITEMS = 8;
-  constexpr uint32_t UP_STEP = BLOCK * UP_ITEMS;
+// True in the last workgroup of the grid to ask (one thread each); the counter is 0 again after it.
+__device__ __forceinline__ bool last_block(uint32_t* ticket) {
+  const bool mine = atomicInc(ticket, gridDim.x - 1u) == gridDim.x - 1u;
+  asm volatile("" ::: "memory");
+  return mine;
+}
+
+// One LDS count of bin b (b < 2^31; lanes that count nothing pass b = ~0u). The lanes of the wave on the
+// first counting lane's bin take one atomic together: a digit that is the same on most rows (the high
+// digits of small integers, a skewed column) would otherwise serialize its 64 lanes on one address.
+__device__ __forceinline__ void count_bin(uint32_t* h, uint32_t b) {
+  const uint32_t lead = __builtin_amdgcn_readfirstlane(b);
+  const unsigned long long m = __ballot(b == lead);
+  if (b == lead) {
+    if (lead != ~0u && int(threadIdx.x & 63u) == __builtin_ctzll(m)) atomicAdd(&h[lead], uint32_t(__popcll(m)));
+  } else if (b != ~0u) {
+    atomicAdd(&h[b], 1u);
+  }
+}
+
+// The same with a check for a digit that is one on the whole wave only: cheaper, for the LSD passes' analysis
+// of every digit (10M uniform float32 keys: 32 us less than with count_bin).
+__device__ __forceinline__ void count_digit(uint32_t* h, uint32_t b) {
+  const uint32_t lead = __builtin_amdgcn_readfirstlane(b);
+  if (__all(b == lead)) {   // uniform
+    if (lead != ~0u && (threadIdx.x & 63u) == 0u) atomicAdd(&h[lead], 64u);
+  } else if (b != ~0u) {
+    atomicAdd(&h[b], 1u);
+  }
+}
+
+// Runs count(base, raw, vb) over the rows [begin, end) of a workgroup, UP_ITEMS rows per thread per step,
+// loaded before any is counted; two steps' rows take turns, so that the next step's loads are in flight
+// while this step is counted, and every loaded register is taken at the top of a step (a load the compiler
+// moved into one of the classification's branches would be waited for there alone). The step count is the
+// same for every thread of the block.
+constexpr int UP_ITEMS = 8;
+constexpr uint32_t UP_STEP = BLOCK * UP_ITEMS;
+
+template <int W, class F>
+__device__ __forceinline__ void up_steps(const void* vals, const uint8_t* valid, int64_t voff, uint32_t begin,
+                                         uint32_t end, F&& count) {
   const int steps = end > begin ? int((end - begin + UP_STEP - 1) / UP_STEP) : 0;
+  if (steps == 0) return;
   uint64_t raw_a[UP_ITEMS], raw_b[UP_ITEMS];
   uint32_t vb_a[UP_ITEMS], vb_b[UP_ITEMS];
   auto load_step = [&](uint64_t base, uint64_t (&raw)[UP_ITEMS], uint32_t (&vb)[UP_ITEMS]) {
@@ -118,156 +135,208 @@ __global__ __launch_bounds__(BLOCK) void sort_upsweep(const void* vals, const ui
   auto count_step = [&](uint64_t base, const uint64_t (&raw)[UP_ITEMS], const uint32_t (&vb)[UP_ITEMS]) {
 #pragma unroll
     for (int u = 0; u < UP_ITEMS; u++) asm volatile("" ::"v"(raw[u]), "v"(vb[u]));
-    K kk[UP_ITEMS];
-    int cc[UP_ITEMS];
-#pragma unroll
-    for (int u = 0; u < UP_ITEMS; u++) {
-      const uint64_t i = base + uint64_t(u) * BLOCK + threadIdx.x;
-      const uint32_t ic = uint32_t(std::min<uint64_t>(i, uint64_t(end) - 1u));
-      const uint32_t bit = valid ? uint32_t((voff + int64_t(ic)) & 7) : 0u;
-      kk[u] = 0;
-      cc[u] = i < end ? classify_raw<K>(raw[u], (vb[u] >> bit) & 1u, type, forder, desc, kk[u]) : 3;
-    }
-#pragma unroll
-    for (int u = 0; u < UP_ITEMS; u++) {
-      const uint32_t ui = uint32_t(base + uint64_t(u) * BLOCK + threadIdx.x - begin) >> unit_shift;
-      if (cc[u] == 0) {
-        K k = kk[u];
-        cm++;
-        o |= k;
-        a &= k;
-        // all_digits == 0 (the hybrid sort's analysis): only the top digit's histogram, per unit (the
-        // levels count the lower digits per bucket; the LSD passes, if they run instead, analyse again).
-        if (all_digits) {
-#pragma unroll
-          for (int p = 0; p < P - 1; p++) atomicAdd(&h[p][uint32_t(k >> (8 * p)) & 0xFFu], 1u);
-        }
-        const uint32_t top = uint32_t(k >> (8 * (P - 1))) & 0xFFu;
-        atomicAdd(units ? &hu[ui & (UNITS_PER_BLOCK - 1)][top] : &h[P - 1][top], 1u);
-      } else if (cc[u] == 1) {
-        cq++;
-        if (units) atomicAdd(&hu[ui & (UNITS_PER_BLOCK - 1)][BIN_NAN], 1u);
-      } else if (cc[u] == 2) {
-        cz++;
-        if (units) atomicAdd(&hu[ui & (UNITS_PER_BLOCK - 1)][BIN_NULL], 1u);
-      }
-    }
+    count(base, raw, vb);
   };
-  if (steps > 0) {
-    load_step(begin, raw_a, vb_a);
-    for (int t = 0; t < steps; t += 2) {
-      const uint64_t base = uint64_t(begin) + uint64_t(t) * UP_STEP;
-      load_step(base + UP_STEP, raw_b, vb_b);
-      count_step(base, raw_a, vb_a);
-      if (t + 1 >= steps) break;
-      load_step(base + 2 * UP_STEP, raw_a, vb_a);
-      count_step(base + UP_STEP, raw_b, vb_b);
-    }
-  }
-  // Wave reductions of the counters and the OR / AND, then one LDS atomic per wave.
-  unsigned long long o64 = o, a64 = a;
-  if (sizeof(K) == 4) a64 |= 0xFFFFFFFF00000000ull;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    cm += __shfl_down(cm, off, 64);
-    cq += __shfl_down(cq, off, 64);
-    cz += __shfl_down(cz, off, 64);
-    o64 |= __shfl_down(o64, off, 64);
-    a64 &= __shfl_down(a64, off, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    atomicAdd(&cnt[0], cm);
-    atomicAdd(&cnt[1], cq);
-    atomicAdd(&cnt[2], cz);
-    atomicOr(&s_or, o64);
-    atomicAnd(&s_and, a64);
-  }
-  __syncthreads();
-  if (units) {
-    // The block's top-digit histogram is the sum of its units'; every unit's counts go out bin-major.
-    const uint32_t u0 = begin >> unit_shift;
-    const uint32_t nu = (end - begin + (1u << unit_shift) - 1u) >> unit_shift;
-    for (uint32_t b = threadIdx.x; b < uint32_t(NBINS_FIRST); b += BLOCK) {
-      uint32_t sum = 0;
-      for (uint32_t ui = 0; ui < nu; ui++) {
-        sum += hu[ui][b];
-        unit_hist[size_t(b) * nunits + u0 + ui] = hu[ui][b];
-      }
-      if (b < uint32_t(RADIX)) h[P - 1][b] = sum;
-    }
-    __syncthreads();
-  }
-  const uint32_t x = xcd_id();
-  uint32_t* xh = &ctl->xhist[x][0][0];
-  for (int i = threadIdx.x; i < P * RADIX; i += BLOCK) {
-    uint32_t v = (&h[0][0])[i];
-    if (v) __hip_atomic_fetch_add(xh + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  }
-  if (threadIdx.x == 0) {
-    if (cnt[0]) {
-      __hip_atomic_fetch_add(&ctl->xm[x], cnt[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      __hip_atomic_fetch_or(&ctl->xor_[x], s_or, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      __hip_atomic_fetch_and(&ctl->xand[x], s_and, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    if (cnt[1]) __hip_atomic_fetch_add(&ctl->xq[x], cnt[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (cnt[2]) __hip_atomic_fetch_add(&ctl->xz[x], cnt[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  load_step(begin, raw_a, vb_a);
+  for (int t = 0; t < steps; t += 2) {
+    const uint64_t base = uint64_t(begin) + uint64_t(t) * UP_STEP;
+    load_step(base + UP_STEP, raw_b, vb_b);
+    count_step(base, raw_a, vb_a);
+    if (t + 1 >= steps) break;
+    load_step(base + 2 * UP_STEP, raw_a, vb_a);
+    count_step(base + UP_STEP, raw_b, vb_b);
   }
 }
 
-template <int P>
-__global__ __launch_bounds__(BLOCK) void sort_plan(SortCtl* ctl, int nulls_first) {
-  __shared__ uint32_t tmp[WAVES];
-  // Fold the per-XCD partials of the upsweep.
-  for (int p = 0; p < P; p++) {
-    uint32_t v = 0;
+// What the rows of a workgroup have in common: OR / AND of the value keys, and how many rows are values,
+// NaN and null.
+struct UpStat {
+  unsigned long long key_or, key_and;
+  uint32_t m, q, z, pad;
+};
+
+// The classes and keys of one step's rows (3: past the end), counted into this thread's statistics.
+template <typename K>
+__device__ __forceinline__ void up_classify(uint64_t base, uint32_t end, const uint64_t (&raw)[UP_ITEMS],
+                                            const uint32_t (&vb)[UP_ITEMS], bool has_valid, int64_t voff, int type,
+                                            int forder, int desc, K (&kk)[UP_ITEMS], int (&cc)[UP_ITEMS], UpStat& st) {
 #pragma unroll
-    for (int x = 0; x < NXCD; x++) v += ctl->xhist[x][p][threadIdx.x];
-    ctl->hist[p][threadIdx.x] = v;
-  }
-  if (threadIdx.x == 0) {
-    uint32_t m = 0, q = 0, z = 0;
-    unsigned long long o = 0ull, a = ~0ull;
-    for (int x = 0; x < NXCD; x++) {
-      m += ctl->xm[x];
-      q += ctl->xq[x];
-      z += ctl->xz[x];
-      o |= ctl->xor_[x];
-      a &= ctl->xand[x];
+  for (int u = 0; u < UP_ITEMS; u++) {
+    const uint64_t i = base + uint64_t(u) * BLOCK + threadIdx.x;
+    const uint32_t ic = uint32_t(std::min<uint64_t>(i, uint64_t(end) - 1u));
+    const uint32_t bit = has_valid ? uint32_t((voff + int64_t(ic)) & 7) : 0u;
+    kk[u] = 0;
+    cc[u] = i < end ? classify_raw<K>(raw[u], (vb[u] >> bit) & 1u, type, forder, desc, kk[u]) : 3;
+    st.m += cc[u] == 0 ? 1u : 0u;
+    st.q += cc[u] == 1 ? 1u : 0u;
+    st.z += cc[u] == 2 ? 1u : 0u;
+    if (cc[u] == 0) {
+      st.key_or |= (unsigned long long)kk[u];
+      st.key_and &= (unsigned long long)kk[u] | (sizeof(K) == 4 ? 0xFFFFFFFF00000000ull : 0ull);
     }
-    ctl->m = m;
-    ctl->q = q;
-    ctl->z = z;
-    ctl->key_or = o;
-    ctl->key_and = a;
   }
+}
+
+// The workgroup's statistics in thread 0 (s: WAVES entries of LDS).
+__device__ __forceinline__ void up_reduce(UpStat& st, UpStat* s) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    st.m += __shfl_down(st.m, off, 64);
+    st.q += __shfl_down(st.q, off, 64);
+    st.z += __shfl_down(st.z, off, 64);
+    st.key_or |= __shfl_down(st.key_or, off, 64);
+    st.key_and &= __shfl_down(st.key_and, off, 64);
+  }
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = st;
   __syncthreads();
   if (threadIdx.x == 0) {
-    unsigned long long diff = ctl->key_or ^ ctl->key_and;
+    for (int w = 1; w < WAVES; w++) {
+      st.m += s[w].m;
+      st.q += s[w].q;
+      st.z += s[w].z;
+      st.key_or |= s[w].key_or;
+      st.key_and &= s[w].key_and;
+    }
+  }
+}
+
+// The LSD passes' plan, by the analysis' last workgroup: the XCDs' partial counts folded, the active digits,
+// the bases of the three blocks, and the exclusive digit prefix of every active pass.
+template <int P>
+__device__ __forceinline__ void sort_plan(SortCtl* ctl, int nulls_first, uint32_t digits) {
+  __shared__ uint32_t tmp[WAVES];
+  auto fold = [](const uint32_t* p, size_t stride) {
+    uint32_t v = 0;
+#pragma unroll
+    for (int x = 0; x < NXCD; x++) v += __hip_atomic_load(p + x * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return v;
+  };
+  uint32_t v[P];
+#pragma unroll
+  for (int p = 0; p < P; p++) v[p] = fold(&ctl->xhist[0][p][threadIdx.x], 8 * RADIX);   // every load first
+#pragma unroll
+  for (int p = 0; p < P; p++) {
+    if (!((digits >> p) & 1u)) continue;   // uniform
+    uint32_t total;
+    ctl->digit_base[p][threadIdx.x] = block_excl_scan(v[p], tmp, total);
+  }
+  if (threadIdx.x == 0) {
+    const uint32_t m = fold(ctl->xm, 1), q = fold(ctl->xq, 1), z = fold(ctl->xz, 1);
+    unsigned long long o = 0ull, a = ~0ull;
+    for (int x = 0; x < NXCD; x++) {
+      o |= __hip_atomic_load(&ctl->xor_[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      a &= __hip_atomic_load(&ctl->xand[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const unsigned long long diff = o ^ a;
     uint32_t mask = 0;
     for (int p = 0; p < P; p++)
       if ((diff >> (8 * p)) & 0xFFull) mask |= 1u << p;
     // No varying digit (a single value, or one repeated key): one pass over digit 0 is then a
     // stable compaction of the value rows, which is exactly the answer.
-    if (mask == 0 || ctl->m <= 1u) mask = 1;
+    if (mask == 0 || m <= 1u) mask = 1;
+    ctl->m = m;
     ctl->active_mask = mask;
     ctl->first_active = uint32_t(__builtin_ctz(mask));
     ctl->last_active = 31u - uint32_t(__builtin_clz(mask));
-    uint32_t m = ctl->m, q = ctl->q, z = ctl->z;
-    if (nulls_first) {
-      ctl->null_base = 0;
-      ctl->nan_base = z;
-      ctl->value_base = z + q;
-    } else {
-      ctl->value_base = 0;
-      ctl->nan_base = m;
-      ctl->null_base = m + q;
+    ctl->null_base = nulls_first ? 0u : m + q;
+    ctl->nan_base = nulls_first ? z : m;
+    ctl->value_base = nulls_first ? z + q : 0u;
+  }
+}
+
+// The LSD passes' analysis: the histograms of the digits in `digits` (a bit per digit; a digit known not to
+// vary needs none), the row counts and the OR / AND; the last workgroup done makes the plan.
+template <typename K, int W>
+__global__ __launch_bounds__(BLOCK) void sort_upsweep(const void* vals, const uint8_t* valid, int64_t voff,
+                                                      uint32_t n, int type, int forder, int desc,
+                                                      uint32_t rows_per_block, SortCtl* ctl, uint32_t digits,
+                                                      int nulls_first, uint32_t* ticket) {
+  constexpr int P = int(sizeof(K));
+  __shared__ uint32_t h[P][RADIX];
+  __shared__ UpStat s_st[WAVES];
+  __shared__ uint32_t s_last;
+  for (int i = threadIdx.x; i < P * RADIX; i += BLOCK) (&h[0][0])[i] = 0u;
+  __syncthreads();
+  const uint32_t begin = blockIdx.x * rows_per_block;
+  const uint32_t end = min(n, begin + rows_per_block);
+  UpStat st{0ull, ~0ull, 0u, 0u, 0u, 0u};
+  up_steps<W>(vals, valid, voff, begin, end, [&](uint64_t base, const uint64_t (&raw)[UP_ITEMS], const uint32_t (&vb)[UP_ITEMS]) {
+    K kk[UP_ITEMS];
+    int cc[UP_ITEMS];
+    up_classify<K>(base, end, raw, vb, valid != nullptr, voff, type, forder, desc, kk, cc, st);
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+      if (!((digits >> p) & 1u)) continue;   // uniform
+#pragma unroll
+      for (int u = 0; u < UP_ITEMS; u++) count_digit(h[p], cc[u] == 0 ? uint32_t(kk[u] >> (8 * p)) & 0xFFu : ~0u);
     }
+  });
+  up_reduce(st, s_st);
+  __syncthreads();
+  const uint32_t x = xcd_id();
+  uint32_t* xh = &ctl->xhist[x][0][0];
+  uint32_t done = 0;
+  for (int i = threadIdx.x; i < P * RADIX; i += BLOCK) {
+    const uint32_t v = (&h[0][0])[i];
+    if (v) done |= atomicAdd(xh + i, v);
   }
-  for (int p = 0; p < P; p++) {
-    uint32_t total;
-    uint32_t v = ctl->hist[p][threadIdx.x];
-    ctl->digit_base[p][threadIdx.x] = block_excl_scan(v, tmp, total);
+  atomic_done(done);
+  if (threadIdx.x == 0) {
+    if (st.m) {
+      atomic_done(atomicAdd(&ctl->xm[x], st.m));
+      atomic_done(atomicOr(&ctl->xor_[x], st.key_or));
+      atomic_done(atomicAnd(&ctl->xand[x], st.key_and));
+    }
+    if (st.q) atomic_done(atomicAdd(&ctl->xq[x], st.q));
+    if (st.z) atomic_done(atomicAdd(&ctl->xz[x], st.z));
   }
+  __syncthreads();   // every thread's counts are in memory
+  if (threadIdx.x == 0) s_last = last_block(ticket) ? 1u : 0u;
+  __syncthreads();
+  if (s_last) sort_plan<P>(ctl, nulls_first, digits);   // uniform
+}
+
+// ---------------------------------------------------------------- the hybrid sort's analysis
+//
+// Rows per unit of the top-digit partition (a power of two): the analysis counts the top digit, NaN and
+// null rows of every unit, so that the partition knows every unit's destinations before it starts.
+// Units are 2^unit_shift rows: 16K for 4M rows and more, 4K (one tile of the partition) below, so that a
+// 1M-row input still has ~250 units to spread over the CUs.
+constexpr uint32_t UNIT_SHIFT_LARGE = 14, UNIT_SHIFT_SMALL = 12;
+constexpr uint32_t UNITS_PER_BLOCK = 8;   // most units one workgroup counts
+
+// Every unit's counts, bin-major (unit_hist[b][unit]), and every workgroup's statistics.
+template <typename K, int W>
+__global__ __launch_bounds__(BLOCK) void msd_upsweep(const void* vals, const uint8_t* valid, int64_t voff, uint32_t n,
+                                                     int type, int forder, int desc, uint32_t rows_per_block,
+                                                     UpStat* stats, uint32_t* unit_hist, uint32_t nunits,
+                                                     uint32_t unit_shift) {
+  constexpr int P = int(sizeof(K));
+  __shared__ uint32_t hu[UNITS_PER_BLOCK * NBINS_FIRST];
+  __shared__ UpStat s_st[WAVES];
+  const uint32_t begin = blockIdx.x * rows_per_block;
+  const uint32_t end = min(n, begin + rows_per_block);
+  const uint32_t nu = (end - begin + (1u << unit_shift) - 1u) >> unit_shift;
+  for (uint32_t i = threadIdx.x; i < nu * NBINS_FIRST; i += BLOCK) hu[i] = 0u;
+  __syncthreads();
+  UpStat st{0ull, ~0ull, 0u, 0u, 0u, 0u};
+  up_steps<W>(vals, valid, voff, begin, end, [&](uint64_t base, const uint64_t (&raw)[UP_ITEMS], const uint32_t (&vb)[UP_ITEMS]) {
+    K kk[UP_ITEMS];
+    int cc[UP_ITEMS];
+    up_classify<K>(base, end, raw, vb, valid != nullptr, voff, type, forder, desc, kk, cc, st);
+#pragma unroll
+    for (int u = 0; u < UP_ITEMS; u++) {
+      const uint32_t ui = uint32_t(base + uint64_t(u) * BLOCK + threadIdx.x - begin) >> unit_shift;
+      const uint32_t bin = cc[u] == 0 ? uint32_t(kk[u] >> (8 * (P - 1))) & 0xFFu : cc[u] == 1 ? uint32_t(BIN_NAN) : uint32_t(BIN_NULL);
+      count_bin(hu, cc[u] < 3 ? ui * NBINS_FIRST + bin : ~0u);
+    }
+  });
+  up_reduce(st, s_st);
+  if (threadIdx.x == 0) stats[blockIdx.x] = st;
+  __syncthreads();
+  const uint32_t u0 = begin >> unit_shift;
+  for (uint32_t b = threadIdx.x; b < uint32_t(NBINS_FIRST); b += BLOCK)
+    for (uint32_t ui = 0; ui < nu; ui++) unit_hist[size_t(b) * nunits + u0 + ui] = hu[ui * NBINS_FIRST + b];
 }
 
 template <typename K, int W, int ITEMS>
@@ -575,27 +644,104 @@ void run_rank(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
 
 // ---------------------------------------------------------------- top-digit partition by units
 //
-// The hybrid sort's first pass, without look-back: the upsweep counted every unit's top digits, NaN
-// and null rows, so one workgroup per bin scans those counts into every unit's destinations
-// (msd_unit_scan), and persistent workgroups then partition whole units, tile after tile, keeping a
-// running destination per bin in LDS (msd_part). Units are taken from a counter, in any order.
+// The hybrid sort's first pass, without look-back: the analysis counted every unit's top digits, NaN and
+// null rows, so one workgroup per bin scans those counts into every unit's destinations and the last of
+// them makes the plan (msd_unit_scan), and persistent workgroups then partition whole units, tile after
+// tile, keeping a running destination per bin in LDS (msd_part). Units are taken from a counter, in any
+// order. The plan tells the host which digits vary, and whether any bucket needs a level at all: a sort whose
+// buckets all fit the bucket sort is five launches and one read-back (it was twelve and two: 17,000 int64
+// keys 105 -> 62 us, 300,000 108 -> 71 us; with the 32-bit keys' hybrid sort, full-range int32: 300,000 keys
+// 115 -> 65 us, 1M 165 -> 80, 10M 472 -> 298, 40M 1604 -> 914).
 
-// unit_base[b][u] = the first destination of bin b's rows of unit u: inside the value block for
-// digits (positions in the partitioned key array), absolute output slots for NaN and null rows.
+// What the host reads of the analysis, in pinned memory.
+struct MsdPlan {
+  uint32_t mask;             // active digits
+  uint32_t m;                // value rows
+  uint32_t large, biggest;   // top-digit buckets that need a level, the largest of the others (not of equal keys)
+  uint32_t local, top;       // entries of the bucket sort's list; the largest top-digit bucket
+};
+
+// Workgroup b: the exclusive scan of bin b's unit counts in place, and its total. The last workgroup done
+// makes the plan: the active digits, where each bin's rows start (first_base), the level kernels' control
+// words, and the top-digit buckets, into the first large-bucket list or the bucket sort's list.
 template <int P>
-__global__ __launch_bounds__(BLOCK) void msd_unit_scan(const SortCtl* ctl, const uint32_t* unit_hist,
-                                                       uint32_t nunits, uint32_t* unit_base) {
+__global__ __launch_bounds__(BLOCK) void msd_unit_scan(SortCtl* ctl, uint32_t* unit_hist, uint32_t nunits,
+                                                       const UpStat* stats, uint32_t blocks, int nulls_first,
+                                                       MsdCtl* mc, uint32_t epoch, Bucket* large, Bucket* local,
+                                                       uint32_t local_cap, uint32_t* lc, unsigned long long* key_out,
+                                                       unsigned long long key_xor, uint32_t* bucket_base, uint32_t* ticket,
+                                                       MsdPlan* plan) {
   __shared__ uint32_t tmp[WAVES];
+  __shared__ uint32_t s_last, s_mask, s_first[NBINS_FIRST];
+  __shared__ UpStat s_st[WAVES];
   const uint32_t b = blockIdx.x;
-  uint32_t carry = b < uint32_t(RADIX) ? ctl->digit_base[P - 1][b] : (b == uint32_t(BIN_NAN) ? ctl->nan_base
-                                                                                                 : ctl->null_base);
+  uint32_t* h = unit_hist + size_t(b) * nunits;
+  uint32_t carry = 0;
   for (uint32_t u0 = 0; u0 < nunits; u0 += BLOCK) {
     const uint32_t u = u0 + threadIdx.x;
-    const uint32_t v = u < nunits ? unit_hist[size_t(b) * nunits + u] : 0u;
+    const uint32_t v = u < nunits ? h[u] : 0u;
     uint32_t total;
     const uint32_t ex = block_excl_scan(v, tmp, total);
-    if (u < nunits) unit_base[size_t(b) * nunits + u] = carry + ex;
+    if (u < nunits) h[u] = carry + ex;
     carry += total;
+  }
+  if (threadIdx.x == 0) {
+    atomic_done(atomicExch(&ctl->bin_total[b], carry));
+    s_last = last_block(ticket) ? 1u : 0u;
+  }
+  __syncthreads();
+  if (!s_last) return;   // uniform
+  UpStat st{0ull, ~0ull, 0u, 0u, 0u, 0u};
+  for (uint32_t k = threadIdx.x; k < blocks; k += BLOCK) {
+    const UpStat x = stats[k];
+    st.m += x.m;
+    st.q += x.q;
+    st.z += x.z;
+    st.key_or |= x.key_or;
+    st.key_and &= x.key_and;
+  }
+  up_reduce(st, s_st);
+  uint32_t total;
+  const uint32_t size = __hip_atomic_load(&ctl->bin_total[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint32_t start = block_excl_scan(size, tmp, total);
+  if (threadIdx.x < LC_WORDS) lc[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) {
+    const unsigned long long diff = st.m ? st.key_or ^ st.key_and : 0ull;
+    uint32_t mask = 0;
+    for (int p = 0; p < P; p++)
+      if ((diff >> (8 * p)) & 0xFFull) mask |= 1u << p;
+    s_mask = mask;
+    const uint32_t value_base = nulls_first ? st.z + st.q : 0u;
+    s_first[BIN_NAN] = nulls_first ? st.z : st.m;
+    s_first[BIN_NULL] = nulls_first ? 0u : st.m + st.q;
+    *mc = {mask, value_base, epoch, 0u, key_out, key_xor};
+    plan->mask = mask;
+    plan->m = st.m;
+  }
+  clear_ctl(ctl);   // the partition's unit counter, and the rest in case the LSD passes run
+  s_first[threadIdx.x] = start;
+  if (bucket_base) bucket_base[threadIdx.x] = start;
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < uint32_t(NBINS_FIRST); k += BLOCK) ctl->first_base[k] = s_first[k];
+  const uint32_t low = s_mask & ((1u << (P - 1)) - 1u);
+  const bool is_large = size > LOCAL_MAX && low != 0u, is_local = size != 0u && !is_large;
+  const Bucket bk{start, size, 0u, uint32_t(P - 1)};
+  uint32_t n_large, n_local;
+  const uint32_t at_large = block_excl_scan(is_large ? 1u : 0u, tmp, n_large);
+  const uint32_t at_local = block_excl_scan(is_local ? 1u : 0u, tmp, n_local);
+  const uint32_t biggest = block_incl_max(is_local && low != 0u ? size : 0u, tmp);
+  const uint32_t top = block_incl_max(size, tmp);
+  if (is_large) large[at_large] = bk;
+  if (is_local && at_local < local_cap) local[at_local] = bk;
+  if (threadIdx.x == BLOCK - 1) {
+    lc[LC_LIST] = n_large;
+    lc[LC_LOCAL] = n_local;
+    lc[LC_MAXLOCAL] = biggest;
+    lc[LC_OVERFLOW] = n_local > local_cap ? 1u : 0u;
+    plan->large = n_large;
+    plan->biggest = biggest;
+    plan->local = n_local;
+    plan->top = top;
   }
 }
 
@@ -605,7 +751,7 @@ __global__ __launch_bounds__(BLOCK) void msd_unit_scan(const SortCtl* ctl, const
 template <typename K, int W, int ITEMS, bool POS_ROWS = false>
 __global__ __launch_bounds__(BLOCK, 3) void msd_part(const void* vals, const uint8_t* valid, int64_t voff,
                                                      uint32_t n, int type, int forder, int desc, SortCtl* ctl,
-                                                     const uint32_t* unit_base, uint32_t nunits,
+                                                     const uint32_t* unit_off, uint32_t nunits,
                                                      uint32_t unit_shift, K* out_keys, uint32_t* out_rows,
                                                      uint32_t* out_idx, uint32_t* pos_of_row = nullptr) {
   constexpr int P = int(sizeof(K));
@@ -628,7 +774,7 @@ __global__ __launch_bounds__(BLOCK, 3) void msd_part(const void* vals, const uin
     __syncthreads();
     const uint32_t unit = s_unit;
     if (unit >= nunits) return;   // uniform: every workgroup ends here once the units run out
-    for (int b = threadIdx.x; b < NBINS_FIRST; b += BLOCK) running[b] = unit_base[size_t(b) * nunits + unit];
+    for (int b = threadIdx.x; b < NBINS_FIRST; b += BLOCK) running[b] = ctl->first_base[b] + unit_off[size_t(b) * nunits + unit];
     const uint32_t begin = unit << unit_shift;
     const uint32_t end = min(n, begin + (1u << unit_shift));
     for (uint32_t t0 = begin; t0 < end; t0 += TILE) {
@@ -686,9 +832,9 @@ __global__ __launch_bounds__(BLOCK, 3) void msd_part(const void* vals, const uin
   }
 }
 
-// ---------------------------------------------------------------- hybrid MSD sort (64-bit keys)
+// ---------------------------------------------------------------- hybrid MSD sort (64- and 32-bit keys)
 //
-// For large inputs of 64-bit keys whose top digit varies: the first pass partitions the value rows
+// For large inputs of 64- and 32-bit keys whose top digit varies: the first pass partitions the value rows
 // stably by the top digit (msd_part, above). Then, level by level down the active digits, every
 // bucket still larger than LOCAL_MAX rows is partitioned stably by the next digit (onesweep tiles
 // whose look-back stops at their bucket's first tile), into the other key / row buffer at the same
@@ -701,74 +847,42 @@ __global__ __launch_bounds__(BLOCK, 3) void msd_part(const void* vals, const uin
 #ifndef AM_MSD_FITEMS
 #define AM_MSD_FITEMS 16   // keys per thread of the top-digit partition
 #endif
-// One workgroup: the level kernels' MsdCtl; the top-digit buckets msd_part made, into the first
-// large-bucket list or the bucket sort's list; the counters cleared. `low` = the active digits below
-// the top one.
-template <int P>
-__global__ __launch_bounds__(BLOCK) void msd_init_lists(const SortCtl* ctl, MsdCtl* mc, uint32_t epoch,
-                                                        Bucket* large, Bucket* local, uint32_t local_cap,
-                                                        uint32_t* lc, unsigned long long* key_out,
-                                                        unsigned long long key_xor) {
-  if (threadIdx.x < LC_WORDS) lc[threadIdx.x] = 0u;
-  if (threadIdx.x == 0) *mc = {ctl->active_mask, ctl->value_base, epoch, 0u, key_out, key_xor};
-  __syncthreads();
-  const uint32_t b = threadIdx.x;
-  const uint32_t size = ctl->hist[P - 1][b];
-  if (size == 0u) return;
-  const Bucket bk{ctl->digit_base[P - 1][b], size, 0u, uint32_t(P - 1)};
-  const uint32_t low = ctl->active_mask & ((1u << (P - 1)) - 1u);
-  if (size > LOCAL_MAX && low != 0u) large[atomicAdd(&lc[LC_LIST], 1u)] = bk;
-  else push_local(local, local_cap, lc, bk, low == 0u);
-}
-
 // ---------------------------------------------------------------- host side
 
-// The hybrid sort of 64-bit keys (the analysed plan says the top digit varies; `mask` = the active
-// digits). Returns false, with nothing written to out_idx that the LSD passes do not write again, when
-// the bucket sort's list runs out of room.
-template <typename K, int W, int FITEMS, int ITEMS>
-bool run_hybrid(const void* vals, int type, const uint8_t* valid, int64_t voff, uint32_t n, int dsc, int forder,
-                SortCtl* ctl, unsigned long long* status, uint32_t epoch, uint32_t m, uint32_t mask, K* k0,
-                uint32_t* r0, K* k1, uint32_t* r1, uint32_t* out_idx, const uint32_t* unit_hist, uint32_t* unit_base,
-                uint32_t nunits, uint32_t unit_shift, hipStream_t s, uint32_t* pos_of_row,
-                unsigned long long* key_out, unsigned long long key_xor) {
-  constexpr int P = int(sizeof(K));
-  const MsdWork w = msd_work(m, ITEMS, device_alloc);
-  {
-    ProfScope ps("sort_msd_unit_scan");
-    hipLaunchKernelGGL(msd_unit_scan<P>, dim3(NBINS_FIRST), dim3(BLOCK), 0, s, ctl, unit_hist, nunits, unit_base);
+// The counter that the last workgroup of an analysis finds itself by: one per thread, zero between kernels.
+uint32_t* scan_ticket(hipStream_t s) {
+  thread_local DevBuf buf;
+  if (!buf) {
+    void* p = nullptr;
+    AM_HIP(hipMalloc(&p, 128));
+    buf = device_wrap(p, 128, [](void* q) { (void)hipFree(q); });
+    hipLaunchKernelGGL(fill_u64, dim3(1), dim3(64), 0, s, static_cast<unsigned long long*>(p), size_t(16), 0ull);
     AM_HIP(hipGetLastError());
   }
-  {
-    ProfScope ps("sort_msd_first");
-    const uint32_t workers = std::min(nunits, uint32_t(device().cu_count) * 3u);
-    if (pos_of_row)
-      hipLaunchKernelGGL((msd_part<K, W, FITEMS, true>), dim3(workers), dim3(BLOCK), 0, s, vals, valid, voff, n, type,
-                         forder, dsc, ctl, unit_base, nunits, unit_shift, k0, r0, out_idx, pos_of_row);
-    else
-      hipLaunchKernelGGL((msd_part<K, W, FITEMS>), dim3(workers), dim3(BLOCK), 0, s, vals, valid, voff, n, type, forder,
-                         dsc, ctl, unit_base, nunits, unit_shift, k0, r0, out_idx, nullptr);
-    AM_HIP(hipGetLastError());
-  }
-  {
-    ProfScope ps("sort_msd_lists");
-    hipLaunchKernelGGL(msd_init_lists<P>, dim3(1), dim3(BLOCK), 0, s, ctl, w.mc, epoch, w.large[0], w.local,
-                       w.local_cap, w.lc, key_out, key_xor);
-    AM_HIP(hipGetLastError());
-  }
-  return msd_levels<K, ITEMS>(w, m, P - 1, mask, false, LOCAL_MAX, status, k0, r0, k1, r1, out_idx, s,
-                              key_out != nullptr);
+  retain(buf);
+  return static_cast<uint32_t*>(buf->ptr);
 }
 
 // With pos_of_row (the ORDER BY of whole tables): only the hybrid sort runs, with positions for rows
 // (msd_part's POS_ROWS form); when it cannot (too few rows, a constant top digit, a full bucket list)
 // the call returns false and out_idx holds nothing to use. *value_rows receives m. With key_out (an
 // integer key) the bucket sorts also write the value block of the sorted key column there.
-#ifndef AM_HYBRID_MIN_LOG
-#define AM_HYBRID_MIN_LOG 16
-#endif
-// Rows from which a 64-bit key takes the hybrid sort (and the plan is read back).
-constexpr uint32_t HYBRID_MIN = 1u << AM_HYBRID_MIN_LOG;
+// Rows from which the LSD passes' plan is read back.
+constexpr uint32_t PLAN_READ_MIN = 1u << 16;
+// Rows from which a key type's columns are analysed for the hybrid sort. Integers spread over the top digit's
+// values, so from the counting sort's limit (64-bit) and from where the LSD passes read their plan back too
+// (32-bit; int32 values below 5,000, which the LSD passes then take, would lose 10 us before). The top digit
+// of floats holds their sign and exponent: a few buckets hold most rows and take a level or two, which pays
+// from 2^16 rows for eight digits (40,000 rows: 123 us LSD, 148 hybrid; 100,000: 134 against 118) and from
+// 2^24 for four.
+uint32_t hybrid_min(int type) {
+  switch (type) {
+    case T_I64: case T_U64: return RANK_MAX + 1u;
+    case T_F64: case T_I32: case T_U32: return 1u << 16;
+    case T_F32: return 1u << 24;
+    default: return ~0u;   // narrower keys: at most two digits vary
+  }
+}
 
 template <typename K, int W, int ITEMS>
 bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, uint32_t n, bool desc,
@@ -776,7 +890,8 @@ bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
               uint32_t* value_rows = nullptr, uint32_t* bucket_base = nullptr, unsigned long long* key_out = nullptr,
               unsigned long long key_xor = 0) {
   constexpr int P = int(sizeof(K));
-  if (pos_of_row && !(P == 8 && n >= HYBRID_MIN && !capturing(s))) return false;
+  const bool hybrid_ok = n >= hybrid_min(type) && !capturing(s);
+  if (pos_of_row && !hybrid_ok) return false;
   constexpr int TILE = BLOCK * ITEMS;
   // The first pass keeps at most 16 keys per thread: its raw-column loads and 258-bin classification
   // need more registers, and 16 keeps it at three workgroups per CU.
@@ -795,82 +910,101 @@ bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
   DevBuf k0 = device_alloc(size_t(n) * sizeof(K)), k1 = device_alloc(size_t(n) * sizeof(K));
   DevBuf r0 = device_alloc(size_t(n) * 4), r1 = device_alloc(size_t(n) * 4);
   const int dsc = desc ? 1 : 0;
-  {
-    ProfScope ps("sort_init");
-    hipLaunchKernelGGL(sort_init, dim3(1), dim3(BLOCK), 0, s, ctl);
-    AM_HIP(hipGetLastError());
-  }
-  // Large 64-bit inputs may take the hybrid sort: the upsweep then also counts its units.
-  const bool hybrid_ok = P == 8 && n >= HYBRID_MIN && !capturing(s);
-  const uint32_t unit_shift = n >= (1u << 22) ? UNIT_SHIFT_LARGE : UNIT_SHIFT_SMALL;
-  const uint32_t unit_rows = 1u << unit_shift;
-  const uint32_t nunits = hybrid_ok ? (n + unit_rows - 1) / unit_rows : 0u;
-  DevBuf units_buf;
-  uint32_t* unit_hist = nullptr;
-  if (hybrid_ok) {
-    units_buf = device_alloc(size_t(nunits) * NBINS_FIRST * 4 * 2);
-    unit_hist = static_cast<uint32_t*>(units_buf->ptr);
-  }
-  // The upsweep and the plan. With units (the hybrid sort's analysis) the upsweep counts only the top
-  // digit; if the LSD passes run after all, the analysis is redone with every digit.
-  auto analyse_column = [&](bool units) {
-    uint32_t max_blocks = uint32_t(device().cu_count) * 4u;
-    uint32_t blocks = std::max(1u, std::min(max_blocks, (n + 8191u) / 8192u));
-    // Block ranges are whole units when units are counted, at most UNITS_PER_BLOCK of them.
-    const uint32_t align = units ? unit_rows : 2048u;
-    uint32_t rpb = ((n + blocks - 1) / blocks + align - 1) / align * align;
-    if (units) rpb = std::min(rpb, UNITS_PER_BLOCK * unit_rows);
-    blocks = (n + rpb - 1) / rpb;
-    {
-      ProfScope ps("sort_upsweep");
-      hipLaunchKernelGGL((sort_upsweep<K, W>), dim3(blocks), dim3(BLOCK), 0, s, vals, valid, voff, n, type, forder,
-                         dsc, rpb, ctl, units ? unit_hist : nullptr, nunits, unit_shift, units ? 0 : 1);
-      AM_HIP(hipGetLastError());
-    }
-    ProfScope ps("sort_plan");
-    hipLaunchKernelGGL(sort_plan<P>, dim3(1), dim3(BLOCK), 0, s, ctl, placement == 1 ? 1 : 0);
-    AM_HIP(hipGetLastError());
-  };
-  analyse_column(hybrid_ok);
-  if (bucket_base) {   // where each top-digit bucket starts in the value block (the partition's layout)
-    AM_HIP(hipMemcpyAsync(bucket_base, &ctl->digit_base[P - 1][0], RADIX * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
-  }
-  // Large inputs read the plan back once (one sync, as the reference's analysis readback does), so
-  // that only active passes are launched, over the value rows only.
-  struct Plan { uint32_t mask, first, last, m; } plan{0xFFu, 0, uint32_t(P - 1), n};
-  const bool analyse = n >= HYBRID_MIN && !capturing(s);
-  if (analyse) {
-    Plan* hp = reinterpret_cast<Plan*>(host_plan_words());
-    hipLaunchKernelGGL(sort_read_plan, dim3(1), dim3(1), 0, s, ctl, reinterpret_cast<uint32_t*>(hp));
-    AM_HIP(hipGetLastError());
-    AM_HIP(hipStreamSynchronize(s));
-    plan = *hp;
-  }
   K* kp0 = static_cast<K*>(k0->ptr);
   K* kp1 = static_cast<K*>(k1->ptr);
   uint32_t* rp0 = static_cast<uint32_t*>(r0->ptr);
   uint32_t* rp1 = static_cast<uint32_t*>(r1->ptr);
-  if constexpr (P == 8) {
-    // The hybrid sort when the top digit varies; the LSD passes below run instead if its bucket list
-    // runs out of room.
-    if (value_rows) *value_rows = plan.m;
-    if (hybrid_ok && analyse && ((plan.mask >> (P - 1)) & 1u) &&
-        run_hybrid<K, W, AM_MSD_FITEMS, ITEMS>(
-            vals, type, valid, voff, n, dsc, forder, ctl, status, epoch, plan.m, plan.mask, kp0, rp0, kp1, rp1,
-            out_idx, unit_hist, unit_hist + size_t(nunits) * NBINS_FIRST, nunits, unit_shift, s, pos_of_row,
-            key_out, key_xor))
-      return true;
-  }
-  if (pos_of_row) return false;
+  // Large inputs of 32- and 64-bit keys may take the hybrid sort: its analysis is read back once.
+  uint32_t digits = (1u << P) - 1u;
+  bool planned = false, tried = false;   // analysed; partitioned (the control block is used up)
+  MsdPlan plan{};
   if (hybrid_ok) {
-    // The LSD passes need every digit's histogram: the analysis again, from a cleared control block
-    // (the plan read back above stays the same).
+    const uint32_t unit_shift = n >= (1u << 22) ? UNIT_SHIFT_LARGE : UNIT_SHIFT_SMALL;
+    const uint32_t unit_rows = 1u << unit_shift;
+    const uint32_t nunits = (n + unit_rows - 1) / unit_rows;
+    // Workgroups of whole units, at most UNITS_PER_BLOCK: one each until every CU has four.
+    const uint32_t per = std::min(UNITS_PER_BLOCK, std::max(1u, (nunits + uint32_t(device().cu_count) * 4u - 1u) / (uint32_t(device().cu_count) * 4u)));
+    const uint32_t rpb = per * unit_rows, blocks = (n + rpb - 1) / rpb;
+    DevBuf units_buf = device_alloc(size_t(nunits) * NBINS_FIRST * 4 + size_t(blocks) * sizeof(UpStat) + 16);
+    UpStat* stats = static_cast<UpStat*>(units_buf->ptr);
+    uint32_t* unit_hist = reinterpret_cast<uint32_t*>(stats + blocks);
+    const MsdWork w = msd_work(n, ITEMS, device_alloc);
+    MsdPlan* hp = reinterpret_cast<MsdPlan*>(host_plan_words());
     {
-      ProfScope ps("sort_init");
-      hipLaunchKernelGGL(sort_init, dim3(1), dim3(BLOCK), 0, s, ctl);
+      ProfScope ps("sort_upsweep");
+      hipLaunchKernelGGL((msd_upsweep<K, W>), dim3(blocks), dim3(BLOCK), 0, s, vals, valid, voff, n, type, forder, dsc, rpb,
+                         stats, unit_hist, nunits, unit_shift);
       AM_HIP(hipGetLastError());
     }
-    analyse_column(false);
+    {
+      ProfScope ps("sort_msd_unit_scan");
+      hipLaunchKernelGGL(msd_unit_scan<P>, dim3(NBINS_FIRST), dim3(BLOCK), 0, s, ctl, unit_hist, nunits,
+                         static_cast<const UpStat*>(stats), blocks, placement == 1 ? 1 : 0, w.mc, epoch, w.large[0], w.local,
+                         w.local_cap, w.lc, key_out, key_xor, bucket_base, scan_ticket(s), hp);
+      AM_HIP(hipGetLastError());
+    }
+    AM_HIP(hipStreamSynchronize(s));
+    plan = *hp;
+    planned = true;
+    digits = plan.mask ? plan.mask : 1u;
+    if (value_rows) *value_rows = plan.m;
+    // 32-bit keys: the LSD passes are only four, so the hybrid sort must come out with about one level (every
+    // top-digit bucket at most 2^18 rows, which a second digit brings to bucket-sort size), or save whole
+    // passes over a large column. 10M float32 values over 10,000 distinct: LSD 481 us, hybrid 660; 40M
+    // uniform float32: 1.71 against 1.33 ms; 3M full-range int32: 237 against 167 us.
+    const bool take = ((plan.mask >> (P - 1)) & 1u) && (P == 8 || plan.top <= (1u << 18) || n >= (1u << 24));
+    if (pos_of_row && !take) return false;
+    if (take) {
+      tried = true;
+      {
+        ProfScope ps("sort_msd_first");
+        const uint32_t workers = std::min(nunits, uint32_t(device().cu_count) * 3u);
+        if (pos_of_row)
+          hipLaunchKernelGGL((msd_part<K, W, AM_MSD_FITEMS, true>), dim3(workers), dim3(BLOCK), 0, s, vals, valid, voff, n,
+                             type, forder, dsc, ctl, unit_hist, nunits, unit_shift, kp0, rp0, out_idx, pos_of_row);
+        else
+          hipLaunchKernelGGL((msd_part<K, W, AM_MSD_FITEMS>), dim3(workers), dim3(BLOCK), 0, s, vals, valid, voff, n, type,
+                             forder, dsc, ctl, unit_hist, nunits, unit_shift, kp0, rp0, out_idx, nullptr);
+        AM_HIP(hipGetLastError());
+      }
+      if (msd_levels<K, ITEMS>(w, plan.m, P - 1, plan.mask, false, LOCAL_MAX, status, kp0, rp0, kp1, rp1, out_idx, s,
+                               key_out != nullptr, &plan.large, &plan.biggest, &plan.local))
+        return true;
+      // The bucket sort's list ran out of room: the LSD passes below.
+    }
+  }
+  if (pos_of_row) return false;
+  if (!planned || tried) {
+    ProfScope ps("sort_init");
+    hipLaunchKernelGGL(sort_init, dim3(1), dim3(1024), 0, s, ctl);
+    AM_HIP(hipGetLastError());
+  }
+  {
+    // At most two workgroups per CU: each adds up to 256 counts per digit to shared ones.
+    const uint32_t max_blocks = uint32_t(device().cu_count) * 2u;
+    uint32_t blocks = std::max(1u, std::min(max_blocks, (n + 2u * UP_STEP - 1u) / (2u * UP_STEP)));
+    const uint32_t rpb = ((n + blocks - 1) / blocks + UP_STEP - 1) / UP_STEP * UP_STEP;
+    blocks = (n + rpb - 1) / rpb;
+    {
+      ProfScope ps("sort_upsweep");
+      hipLaunchKernelGGL((sort_upsweep<K, W>), dim3(blocks), dim3(BLOCK), 0, s, vals, valid, voff, n, type, forder, dsc, rpb,
+                         ctl, digits, placement == 1 ? 1 : 0, scan_ticket(s));
+      AM_HIP(hipGetLastError());
+    }
+  }
+  // Large inputs read the plan back once (one sync, as the reference's analysis readback does), so
+  // that only active passes are launched, over the value rows only; the hybrid sort's analysis has it.
+  const bool analyse = planned || (n >= PLAN_READ_MIN && !capturing(s));
+  struct Plan { uint32_t mask, first, last, m; } lsd{0xFFu, 0, uint32_t(P - 1), n};
+  if (planned) {
+    const uint32_t mask = plan.m <= 1u ? 1u : digits;   // as sort_plan has it
+    lsd = Plan{mask, uint32_t(__builtin_ctz(mask)), 31u - uint32_t(__builtin_clz(mask)), plan.m};
+  } else if (analyse) {
+    Plan* hp = reinterpret_cast<Plan*>(host_plan_words());
+    hipLaunchKernelGGL(sort_read_plan, dim3(1), dim3(1), 0, s, ctl, reinterpret_cast<uint32_t*>(hp));
+    AM_HIP(hipGetLastError());
+    AM_HIP(hipStreamSynchronize(s));
+    lsd = *hp;
   }
   {
     ProfScope ps("sort_first");
@@ -881,10 +1015,10 @@ bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
   if (analyse) {
     // The host read the plan back: launch only the active passes, each over the value rows, with
     // the last one's kernel known (no key writes).
-    const uint32_t mtiles = std::max<uint32_t>(1, (plan.m + TILE - 1) / TILE);
+    const uint32_t mtiles = std::max<uint32_t>(1, (lsd.m + TILE - 1) / TILE);
     for (int p = 0; p < P; p++) {
-      if (!((plan.mask >> p) & 1u) || uint32_t(p) == plan.first) continue;
-      if (uint32_t(p) == plan.last) {
+      if (!((lsd.mask >> p) & 1u) || uint32_t(p) == lsd.first) continue;
+      if (uint32_t(p) == lsd.last) {
         ProfScope ps("sort_scatter_last");
         hipLaunchKernelGGL((sort_mid<K, ITEMS, PASS_LAST>), dim3(mtiles), dim3(BLOCK), 0, s, p, ctl, status,
                            epoch + 1u + uint32_t(p), kp0, rp0, kp1, rp1, out_idx);

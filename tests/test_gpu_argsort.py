@@ -183,6 +183,41 @@ def test_small_inputs_of_every_width(n):
         check(vals, np.zeros(n, bool), 1, 0, 0, str(dt))
 
 
+@pytest.mark.parametrize("dtype,n,shape,path", [
+    (np.int32, (1 << 16) - 1, "wide", "lsd"), (np.int32, 1 << 16, "wide", "msd"), (np.uint32, 300_001, "wide", "msd"),
+    (np.int32, 3_000_001, "wide", "msd"), (np.int32, 3_000_001, "small", "lsd"), (np.int32, 2_000_003, "skewed", "lsd"),
+    (np.uint32, 1_500_007, "runs", "msd"), (np.int32, 200_003, "two_digits", "msd"), (np.float32, (1 << 24) + 3, "wide", "msd"),
+    (np.float32, 1_000_003, "wide", "lsd"), (np.int64, 16_385, "wide", "msd"), (np.int64, 20_001, "small", "lsd"),
+    (np.uint64, 40_000, "one_key", "lsd")])
+def test_hybrid_sort_of_each_key_type(dtype, n, shape, path):
+    """Where each key type takes the hybrid sort: 32-bit keys with and without a level, long equal runs (the
+    LSD queue and copies), a top-digit bucket too large for it, a constant top digit (the LSD passes over the
+    digits that vary), nulls at both ends, both directions."""
+    rng = np.random.default_rng(n)
+    dt = np.dtype(dtype)
+    if dt.kind == "f":
+        vals = (rng.random(n) * 2e6 - 1e6).astype(dt)
+        vals[::1001] = np.nan
+        vals[::997] = -0.0
+    else:
+        vals = O.splitmix64(n, n).view(np.uint64).astype(np.uint64)
+        vals = (vals >> np.uint64(64 - 8 * dt.itemsize)).astype(f"u{dt.itemsize}").view(dt) if dt.itemsize == 4 else vals.view(dt)
+        if shape == "small": vals = (vals & dt.type(0xFFF)).astype(dt)
+        elif shape == "one_key": vals = np.full(n, 77, dt)
+        elif shape == "skewed": vals = np.where(rng.random(n) < 0.9, vals & dt.type(0xFFFFF), vals).astype(dt)
+        elif shape == "runs": vals = np.where(rng.random(n) < 0.5, vals[rng.integers(0, 3000, n)], vals).astype(dt)
+        elif shape == "two_digits": vals = (vals & dt.type(0x7F0000FF)).astype(dt)
+    valid = rng.random(n) >= 0.03
+    for va, desc, place in ((valid, 1, 0), (None, 0, 0), (valid, 0, 1)):
+        am.prof_reset()
+        am.prof_enable(True)
+        got = gpu_argsort(vals, va, desc, place, 0)
+        am.prof_enable(False)
+        names = set(am.prof_report())
+        assert ("sort_msd_first" in names) == (path == "msd"), names
+        np.testing.assert_array_equal(got, O.argsort(vals, va, desc, place, 0))
+
+
 # ---------------------------------------------------------------- take
 
 
@@ -251,7 +286,7 @@ def test_order_by_gather_config_shape():
 @pytest.mark.parametrize("width", [8, 4])
 def test_large_tiles_first_pass_and_nulls(order, width):
     """9M rows, NaN and null bins included, against the oracle. 64-bit keys take the hybrid sort;
-    32-bit keys keep the LSD passes, whose scatter passes take 20 keys per thread above 8.4M rows and
+    32-bit float keys keep the LSD passes below 2^24 rows, whose scatter passes take 20 keys per thread above 8.4M rows and
     whose first pass takes 16: both tile shapes and their look-back chains."""
     n = 9_000_001
     print(f"large sort n={n} order={order} width={width}", flush=True)
