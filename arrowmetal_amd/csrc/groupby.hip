@@ -3218,9 +3218,20 @@ __global__ __launch_bounds__(512) void gb_span_fold(const RangeStat* st, uint32_
   }
 }
 
-// Each row's composite key. A thread's COMP_ROWS rows of one column are loaded together (the switch on the
+// Bijections of 32 and 64 bits that spread the keys over all digits (odd multipliers and xor-shifts; the
+// 64-bit one is mix64).
+__device__ __forceinline__ unsigned long long spread_key(unsigned long long k) { return mix64(k); }
+__device__ __forceinline__ uint32_t spread_key(uint32_t k) {
+  k ^= k >> 16;
+  k *= 0x7FEB352Du;
+  k ^= k >> 15;
+  k *= 0x846CA68Bu;
+  return k ^ (k >> 16);
+}
+
+// Each row's composite key, or its image under spread_key (SPREAD). A thread's COMP_ROWS rows of one column are loaded together (the switch on the
 // width is outside the loads), column after column.
-template <typename C>
+template <typename C, bool SPREAD>
 __global__ __launch_bounds__(256) void gb_composite(CompositeArgs a, uint32_t n, C* out) {
   const uint32_t gsize = gridDim.x * blockDim.x;
   for (uint64_t base = blockIdx.x * blockDim.x + threadIdx.x; base < n; base += uint64_t(gsize) * COMP_ROWS) {
@@ -3265,7 +3276,7 @@ __global__ __launch_bounds__(256) void gb_composite(CompositeArgs a, uint32_t n,
 #pragma unroll
     for (int r = 0; r < COMP_ROWS; r++) {
       const uint64_t i = base + uint64_t(r) * gsize;
-      if (i < n) out[i] = code[r];
+      if (i < n) out[i] = SPREAD ? spread_key(code[r]) : code[r];
     }
   }
 }
@@ -4010,8 +4021,12 @@ DevBuf first_rows(const DevBuf& ids, int64_t n, int64_t K) {
 // min, max and count: 2.17 ms -> 0.35 ms, of which 1.6 ms were the atomics that found each group's lowest
 // row, one per row on a hot group's word.) False when the spans' product does not fit 62 bits (or more
 // than COMPOSITE_MAX columns): the columns then fold pairwise over their ids.
-bool map_composite(Array* const* columns, int64_t count, int64_t n, std::vector<ColSpan>& out_spans, Mapped& out) {
+// any_span: one column without nulls may span all of its 64 bits (top is then all ones, for the wide form).
+bool plan_composite(Array* const* columns, int64_t count, int64_t n, CompositeArgs& ca, unsigned long long& top,
+                    bool any_span = false) {
   if (count > COMPOSITE_MAX) return false;
+  for (int64_t c = 0; c < count; c++)
+    if (!type_is_int(columns[c]->type)) return false;
   hipStream_t s = stream();
   const uint32_t un = uint32_t(n);
   std::shared_ptr<void> slot = pinned_slot();
@@ -4030,36 +4045,51 @@ bool map_composite(Array* const* columns, int64_t count, int64_t n, std::vector<
     }
   }
   AM_HIP(hipStreamSynchronize(s));
-  CompositeArgs ca{};
-  std::vector<ColSpan> spans;
   unsigned __int128 total = 1;
   for (int64_t c = 0; c < count; c++) {
     const RangeStat r = st[c];
     const bool any = r.kmin <= r.kmax;
     const unsigned __int128 span = (any ? (unsigned __int128)(r.kmax - r.kmin) + 1 : 0) + (r.nulls > 0 ? 1 : 0);
     total *= span;
-    if (total > (unsigned __int128)1 << 62) return false;
-    spans.push_back(ColSpan{any ? r.kmin : 0ull, (unsigned long long)span, 1ull, r.nulls > 0 ? 1 : 0});
-  }
-  for (int64_t c = count - 1; c > 0; c--) spans[size_t(c - 1)].div = spans[size_t(c)].div * spans[size_t(c)].span;
-  for (int64_t c = 0; c < count; c++) {
+    if (total > (unsigned __int128)1 << 62) {
+      if (!(any_span && count == 1 && r.nulls == 0)) return false;
+      total = ~0ull;
+    }
     const Array* a = columns[c];
-    ca.col[c] = CompositeCol{a->data(), a->has_nulls() ? a->valid_bits() : nullptr, a->offset, a->type, spans[size_t(c)]};
+    ca.col[c] = CompositeCol{a->data(), a->has_nulls() ? a->valid_bits() : nullptr, a->offset, a->type,
+                             ColSpan{any ? r.kmin : 0ull, (unsigned long long)span, 1ull, r.nulls > 0 ? 1 : 0}};
   }
+  for (int64_t c = count - 1; c > 0; c--) ca.col[c - 1].span.div = ca.col[c].span.div * ca.col[c].span.span;
   ca.count = int(count);
-  const unsigned long long top = (unsigned long long)total;   // composites are below it
-  const bool narrow = top <= (1ull << 32);
+  top = (unsigned long long)total;   // composites are below it
+  return true;
+}
+
+// Whether composites below `top` are held in 32 bits.
+bool composite_narrow(unsigned long long top) { return top <= (1ull << 32); }
+
+template <bool SPREAD>
+DevBuf write_composite(const CompositeArgs& ca, unsigned long long top, int64_t n) {
+  hipStream_t s = stream();
+  const uint32_t un = uint32_t(n);
+  const bool narrow = composite_narrow(top);
   DevBuf comp = device_alloc(size_t(n) * (narrow ? 4 : 8));
-  {
-    ProfScope ps("gb_composite");
-    const int grid = grid_for((n + COMP_ROWS - 1) / COMP_ROWS, 8);
-    if (narrow) hipLaunchKernelGGL(gb_composite<uint32_t>, dim3(grid), dim3(256), 0, s, ca, un, static_cast<uint32_t*>(comp->ptr));
-    else hipLaunchKernelGGL(gb_composite<unsigned long long>, dim3(grid), dim3(256), 0, s, ca, un, static_cast<unsigned long long*>(comp->ptr));
-    AM_HIP(hipGetLastError());
-  }
+  ProfScope ps("gb_composite");
+  const int grid = grid_for((n + COMP_ROWS - 1) / COMP_ROWS, 8);
+  if (narrow) hipLaunchKernelGGL((gb_composite<uint32_t, SPREAD>), dim3(grid), dim3(256), 0, s, ca, un, static_cast<uint32_t*>(comp->ptr));
+  else hipLaunchKernelGGL((gb_composite<unsigned long long, SPREAD>), dim3(grid), dim3(256), 0, s, ca, un, static_cast<unsigned long long*>(comp->ptr));
+  AM_HIP(hipGetLastError());
+  return comp;
+}
+
+bool map_composite(Array* const* columns, int64_t count, int64_t n, std::vector<ColSpan>& out_spans, Mapped& out) {
+  CompositeArgs ca{};
+  unsigned long long top = 0;
+  if (!plan_composite(columns, count, n, ca, top)) return false;
+  DevBuf comp = write_composite<false>(ca, top, n);
   const RangeStat known{0ull, top - 1ull, 0ull, 0u, 0u};
-  out = map_column(comp->ptr, narrow ? T_U32 : T_U64, nullptr, 0, n, &known);
-  out_spans = std::move(spans);
+  out = map_column(comp->ptr, composite_narrow(top) ? T_U32 : T_U64, nullptr, 0, n, &known);
+  for (int64_t c = 0; c < count; c++) out_spans.push_back(ca.col[c].span);
   return true;
 }
 
@@ -4616,6 +4646,25 @@ Array* unique_rows(Array* const* columns, int64_t count) {
       out->values = rows;
       out->null_count = 0;
       return out;
+    }
+  }
+  // Integer columns whose composite key spans more than a private LDS table's groups: the rows are
+  // partitioned and deduplicated (distinct_rows). Over fewer keys the range path's passes are cheaper.
+  if (count >= 1 && columns[0]->length >= 1) {
+    const int64_t n = columns[0]->length;
+    bool same = true;
+    for (int64_t c = 0; c < count; c++) same = same && columns[c]->length == n;
+    CompositeArgs ca{};
+    unsigned long long top = 0;
+    if (same && plan_composite(columns, count, n, ca, top, true) && top > agg_dense_cap<FirstRowP>()) {
+      DevBuf keys = write_composite<true>(ca, top, n), rows;
+      uint32_t kept = 0;
+      if (distinct_rows(keys->ptr, composite_narrow(top) ? 4 : 8, uint32_t(n), rows, kept)) {
+        Array* out = new_array("I", T_U32, int64_t(kept));
+        out->values = rows;
+        out->null_count = 0;
+        return out;
+      }
     }
   }
   GroupBy* g = group_by_keys_impl(columns, count, true);

@@ -881,6 +881,63 @@ __global__ __launch_bounds__(BLOCK) void hyb_local_lsd(const MsdCtl* mc, const B
 }
 
 
+// Marks the rows whose key an earlier row holds (dup[row] = 1), an entry of the bucket sorts' list per
+// workgroup in turn, in place of sorting them. The rows of an entry with digits left are in input order
+// inside each key, so of the positions with one key the lowest is its first row: a table of positions in
+// LDS (linear probing; twice the rows, a power of two), each slot kept at the lowest of its key. An entry
+// without digits left is runs of equal keys, each in input order. Dynamic LDS: li * BLOCK keys, then twice
+// as many 32-bit slots.
+template <typename K>
+__global__ __launch_bounds__(BLOCK) void hyb_dedupe(const MsdCtl* mc, const Bucket* list, uint32_t local_cap, uint32_t li,
+                                                    const K* keys0, const uint32_t* rows0, const K* keys1,
+                                                    const uint32_t* rows1, uint8_t* dup, const uint32_t* lc) {
+  extern __shared__ __align__(16) unsigned char local_lds[];
+  K* s_key = reinterpret_cast<K*>(local_lds);
+  uint32_t* s_pos = reinterpret_cast<uint32_t*>(s_key + li * BLOCK);
+  if (list_overflow(lc, local_cap)) return;   // uniform
+  const uint32_t nlocal = lc[LC_LOCAL], total = nlocal + lc[LC_GROUPS];
+  for (uint32_t e = blockIdx.x; e < total; e += gridDim.x) {
+    const Bucket bk = list[e < nlocal ? e : local_cap - 1u - (e - nlocal)];
+    const K* keys = bucket_keys(bk, keys0, keys1) + bk.start;
+    const uint32_t* rows = bucket_rows(bk, rows0, rows1) + bk.start;   // never implicit rows here
+    const uint32_t size = bk.size;
+    if ((mc->active_mask & ((1u << (bk.level & LEVEL_BITS)) - 1u)) == 0u) {
+      for (uint32_t p = 1u + threadIdx.x; p < size; p += BLOCK)
+        if (keys[p] == keys[p - 1u]) dup[rows[p]] = 1u;
+      continue;
+    }
+    if (size > li * BLOCK) continue;   // never: li covers every bucket
+    uint32_t slots = 2u * BLOCK;
+    while (slots < 2u * size) slots <<= 1;   // at most 2 * li * BLOCK, a power of two times BLOCK
+    for (uint32_t j = threadIdx.x; j < slots; j += BLOCK) s_pos[j] = 0xFFFFFFFFu;
+    for (uint32_t p = threadIdx.x; p < size; p += BLOCK) s_key[p] = keys[p];
+    __syncthreads();
+    for (uint32_t p = threadIdx.x; p < size; p += BLOCK) {
+      const K k = s_key[p];
+      uint32_t h = (uint32_t(k) * 0x9E3779B1u >> 16) & (slots - 1u);   // the key's low digits vary inside a bucket
+      while (true) {
+        uint32_t q = s_pos[h];
+        if (q == 0xFFFFFFFFu) {
+          q = atomicCAS(&s_pos[h], 0xFFFFFFFFu, p);
+          if (q == 0xFFFFFFFFu) break;
+        }
+        if (s_key[q] == k) {   // a slot's position changes, its key does not
+          if (p < q) {
+            // The higher position is the duplicate: this one displaces it.
+            const uint32_t was = atomicMin(&s_pos[h], p);
+            dup[rows[was < p ? p : was]] = 1u;
+          } else {
+            dup[rows[p]] = 1u;
+          }
+          break;
+        }
+        h = (h + 1u) & (slots - 1u);
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // ---------------------------------------------------------------- host side
 
 // The device buffers of the levels for up to m value rows, with `items` keys per thread in a pass
@@ -941,7 +998,8 @@ inline MsdWork msd_work(uint32_t m, int items, DevBuf (*alloc)(size_t), uint32_t
 //   digits get a level, each launch is sized from 64 bytes of counters read back after each level,
 //   and the bucket sort's keys per thread come from the largest bucket. A caller that knows the lists it
 //   built (large: entries of w.large[0]; biggest_local and local_entries: the bucket sort's) passes their
-//   counts, so that a sort without a large bucket launches no level and reads nothing back. Returns false, with no row
+//   counts, so that a sort without a large bucket launches no level and reads nothing back. With dup, the
+//   rows whose key an earlier row holds are marked there instead of the rows being sorted. Returns false, with no row
 //   written that a rerun does not write again, when the bucket sort's list ran out of room.
 // - Blind form (blind = true, e.g. inside a graph capture): every digit below `top` gets a level,
 //   sized for the worst case, the kernels read what to do from the device, and the bucket sort takes
@@ -951,7 +1009,7 @@ template <typename K, int ITEMS>
 bool msd_levels(const MsdWork& w, uint32_t m, int top, uint32_t mask, bool blind, uint32_t local_max,
                 unsigned long long* status, K* k0, uint32_t* r0, K* k1, uint32_t* r1, uint32_t* out_idx,
                 hipStream_t s, bool keys = false, const uint32_t* large = nullptr, const uint32_t* biggest_local = nullptr,
-                const uint32_t* local_entries = nullptr) {
+                const uint32_t* local_entries = nullptr, uint8_t* dup = nullptr) {
   constexpr int P = int(sizeof(K));
   constexpr uint32_t TILE = BLOCK * ITEMS;
   const uint32_t cus = uint32_t(device().cu_count);
@@ -1027,6 +1085,17 @@ bool msd_levels(const MsdWork& w, uint32_t m, int top, uint32_t mask, bool blind
     li_lsd = hp[LC_GROUPS] != 0u ? std::max(li, int(GROUP_ROWS / BLOCK)) : li;   // a queued group fits
     grid = hp[LC_LOCAL];
     group_grid = std::min(hp[LC_GROUPS], cus * 4u);
+  }
+  if (dup) {   // the rows are deduplicated, not sorted
+    const uint32_t entries = hp[LC_LOCAL] + hp[LC_GROUPS];
+    if (entries == 0u) return true;
+    const int dl = hp[LC_GROUPS] != 0u ? std::max(li, int(GROUP_ROWS / BLOCK)) : li;
+    const size_t bytes = size_t(dl) * BLOCK * (sizeof(K) + 8);
+    ProfScope ps("sort_msd_dedupe");
+    hipLaunchKernelGGL(hyb_dedupe<K>, dim3(std::min(entries, cus * 16u)), dim3(BLOCK), bytes, s, w.mc, w.local, w.local_cap,
+                       uint32_t(dl), k0, r0, k1, r1, dup, w.lc);
+    AM_HIP(hipGetLastError());
+    return true;
   }
   // The LSD kernel takes the buckets the counting sorts queued (its workgroups exit at once when none
   // was).

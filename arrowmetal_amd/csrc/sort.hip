@@ -884,6 +884,42 @@ uint32_t hybrid_min(int type) {
   }
 }
 
+// The analysis of the hybrid sort: units counted and scanned, the plan on its way to host_plan_words().
+struct Units {
+  DevBuf buf;
+  uint32_t* hist;   // [NBINS_FIRST][count], each bin's running offsets
+  uint32_t count, shift;
+};
+
+template <typename K, int W>
+Units msd_analyse(const void* vals, int type, const uint8_t* valid, int64_t voff, uint32_t n, int desc, int placement,
+                  int forder, SortCtl* ctl, const MsdWork& w, uint32_t epoch, unsigned long long* key_out,
+                  unsigned long long key_xor, uint32_t* bucket_base, hipStream_t s) {
+  Units un;
+  un.shift = n >= (1u << 22) ? UNIT_SHIFT_LARGE : UNIT_SHIFT_SMALL;
+  const uint32_t unit_rows = 1u << un.shift, cus = uint32_t(device().cu_count);
+  un.count = (n + unit_rows - 1) / unit_rows;
+  // Workgroups of whole units, at most UNITS_PER_BLOCK: one each until every CU has four.
+  const uint32_t per = std::min(UNITS_PER_BLOCK, std::max(1u, (un.count + cus * 4u - 1u) / (cus * 4u)));
+  const uint32_t rpb = per * unit_rows, blocks = (n + rpb - 1) / rpb;
+  un.buf = device_alloc(size_t(un.count) * NBINS_FIRST * 4 + size_t(blocks) * sizeof(UpStat) + 16);
+  UpStat* stats = static_cast<UpStat*>(un.buf->ptr);
+  un.hist = reinterpret_cast<uint32_t*>(stats + blocks);
+  {
+    ProfScope ps("sort_upsweep");
+    hipLaunchKernelGGL((msd_upsweep<K, W>), dim3(blocks), dim3(BLOCK), 0, s, vals, valid, voff, n, type, forder, desc, rpb,
+                       stats, un.hist, un.count, un.shift);
+    AM_HIP(hipGetLastError());
+  }
+  ProfScope ps("sort_msd_unit_scan");
+  hipLaunchKernelGGL(msd_unit_scan<int(sizeof(K))>, dim3(NBINS_FIRST), dim3(BLOCK), 0, s, ctl, un.hist, un.count,
+                     static_cast<const UpStat*>(stats), blocks, placement == 1 ? 1 : 0, w.mc, epoch, w.large[0], w.local,
+                     w.local_cap, w.lc, key_out, key_xor, bucket_base, scan_ticket(s),
+                     reinterpret_cast<MsdPlan*>(host_plan_words()));
+  AM_HIP(hipGetLastError());
+  return un;
+}
+
 template <typename K, int W, int ITEMS>
 bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, uint32_t n, bool desc,
               int placement, int forder, uint32_t* out_idx, hipStream_t s, uint32_t* pos_of_row = nullptr,
@@ -919,30 +955,12 @@ bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
   bool planned = false, tried = false;   // analysed; partitioned (the control block is used up)
   MsdPlan plan{};
   if (hybrid_ok) {
-    const uint32_t unit_shift = n >= (1u << 22) ? UNIT_SHIFT_LARGE : UNIT_SHIFT_SMALL;
-    const uint32_t unit_rows = 1u << unit_shift;
-    const uint32_t nunits = (n + unit_rows - 1) / unit_rows;
-    // Workgroups of whole units, at most UNITS_PER_BLOCK: one each until every CU has four.
-    const uint32_t per = std::min(UNITS_PER_BLOCK, std::max(1u, (nunits + uint32_t(device().cu_count) * 4u - 1u) / (uint32_t(device().cu_count) * 4u)));
-    const uint32_t rpb = per * unit_rows, blocks = (n + rpb - 1) / rpb;
-    DevBuf units_buf = device_alloc(size_t(nunits) * NBINS_FIRST * 4 + size_t(blocks) * sizeof(UpStat) + 16);
-    UpStat* stats = static_cast<UpStat*>(units_buf->ptr);
-    uint32_t* unit_hist = reinterpret_cast<uint32_t*>(stats + blocks);
     const MsdWork w = msd_work(n, ITEMS, device_alloc);
+    const Units un = msd_analyse<K, W>(vals, type, valid, voff, n, dsc, placement, forder, ctl, w, epoch, key_out, key_xor,
+                                       bucket_base, s);
+    const uint32_t nunits = un.count, unit_shift = un.shift;
+    uint32_t* unit_hist = un.hist;
     MsdPlan* hp = reinterpret_cast<MsdPlan*>(host_plan_words());
-    {
-      ProfScope ps("sort_upsweep");
-      hipLaunchKernelGGL((msd_upsweep<K, W>), dim3(blocks), dim3(BLOCK), 0, s, vals, valid, voff, n, type, forder, dsc, rpb,
-                         stats, unit_hist, nunits, unit_shift);
-      AM_HIP(hipGetLastError());
-    }
-    {
-      ProfScope ps("sort_msd_unit_scan");
-      hipLaunchKernelGGL(msd_unit_scan<P>, dim3(NBINS_FIRST), dim3(BLOCK), 0, s, ctl, unit_hist, nunits,
-                         static_cast<const UpStat*>(stats), blocks, placement == 1 ? 1 : 0, w.mc, epoch, w.large[0], w.local,
-                         w.local_cap, w.lc, key_out, key_xor, bucket_base, scan_ticket(s), hp);
-      AM_HIP(hipGetLastError());
-    }
     AM_HIP(hipStreamSynchronize(s));
     plan = *hp;
     planned = true;
@@ -1050,6 +1068,131 @@ void dispatch_items(int items, const void* vals, int type, const uint8_t* valid,
     case 20: run_sort<K, W, 20>(vals, type, valid, voff, n, desc, placement, forder, out_idx, s); break;
     default: run_sort<K, W, 16>(vals, type, valid, voff, n, desc, placement, forder, out_idx, s); break;
   }
+}
+
+// ---------------------------------------------------------------- keep-first distinct rows
+//
+// The rows of distinct mixed keys (a bijection of the original keys, so that the digits are spread whatever
+// the keys are): partitioned by the hybrid sort's passes until a bucket fits in LDS, deduplicated there
+// (hyb_dedupe marks every row whose key an earlier one holds), and the unmarked rows compacted in row
+// order. No table in global memory is probed (an insert of a new key is an atomic at the memory side), and
+// nothing is sorted beyond the buckets. 10M rows over two int64 columns (9.95M distinct), unique rows and both
+// columns taken: 3.26 ms by the hash mapping, its two sorts and lowest rows, 0.58 ms so; the passes run at 1.5
+// to 3 TB/s, the marks' random bytes at 1.5.
+constexpr uint32_t KEEP_TILE = 4096;   // rows per workgroup of the compaction, 16 consecutive ones per thread
+
+__device__ __forceinline__ uint32_t keep_flags(const uint8_t* dup, uint32_t n, uint32_t row0) {
+  // Sixteen consecutive marks (dup is padded to whole tiles) -> a bit per kept row.
+  const uint4 v = *reinterpret_cast<const uint4*>(dup + row0);
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  uint32_t keep = 0;
+#pragma unroll
+  for (int k = 0; k < 16; k++) keep |= (((w[k >> 2] >> (8 * (k & 3))) & 1u) ^ 1u) << k;
+  const uint32_t left = row0 < n ? min(n - row0, 16u) : 0u;
+  return keep & ((1u << left) - 1u);
+}
+
+// Each tile's kept rows; the last workgroup scans them into bases and reports the total.
+__global__ __launch_bounds__(BLOCK) void keep_count(const uint8_t* dup, uint32_t n, uint32_t* base, uint32_t* ticket,
+                                                    uint32_t* total) {
+  __shared__ uint32_t tmp[WAVES];
+  __shared__ uint32_t s_last;
+  const uint32_t c = uint32_t(__popc(keep_flags(dup, n, blockIdx.x * KEEP_TILE + threadIdx.x * 16u)));
+  uint32_t sum;
+  block_excl_scan(c, tmp, sum);
+  if (threadIdx.x == 0) {
+    atomic_done(atomicExch(&base[blockIdx.x], sum));
+    s_last = last_block(ticket) ? 1u : 0u;
+  }
+  __syncthreads();
+  if (!s_last) return;   // uniform
+  uint32_t carry = 0;
+  for (uint32_t t0 = 0; t0 < gridDim.x; t0 += BLOCK * 4u) {
+    uint32_t v[4], x = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) {
+      const uint32_t t = t0 + threadIdx.x * 4u + k;
+      v[k] = t < gridDim.x ? __hip_atomic_load(&base[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+      x += v[k];
+    }
+    uint32_t step;
+    uint32_t run = carry + block_excl_scan(x, tmp, step);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) {
+      const uint32_t t = t0 + threadIdx.x * 4u + k;
+      if (t < gridDim.x) base[t] = run;
+      run += v[k];
+    }
+    carry += step;
+  }
+  if (threadIdx.x == 0) *total = carry;
+}
+
+__global__ __launch_bounds__(BLOCK) void keep_write(const uint8_t* dup, uint32_t n, const uint32_t* base, uint32_t* out) {
+  __shared__ uint32_t tmp[WAVES];
+  __shared__ uint32_t s_row[KEEP_TILE];
+  const uint32_t row0 = blockIdx.x * KEEP_TILE + threadIdx.x * 16u;
+  uint32_t keep = keep_flags(dup, n, row0), total;
+  uint32_t at = block_excl_scan(uint32_t(__popc(keep)), tmp, total);
+  while (keep) {
+    const uint32_t b = uint32_t(__ffs(int(keep))) - 1u;
+    keep &= keep - 1u;
+    s_row[at++] = row0 + b;
+  }
+  __syncthreads();
+  uint32_t* o = out + base[blockIdx.x];
+  for (uint32_t j = threadIdx.x; j < total; j += BLOCK) o[j] = s_row[j];
+}
+
+template <typename K>
+bool distinct_rows_t(const void* keys, uint32_t n, DevBuf& rows, uint32_t& kept, hipStream_t s) {
+  constexpr int ITEMS = 16, W = int(sizeof(K));
+  constexpr int TYPE = W == 8 ? T_U64 : T_U32;
+  DevBuf ctl_buf = device_alloc(sizeof(SortCtl));
+  SortCtl* ctl = static_cast<SortCtl*>(ctl_buf->ptr);
+  const uint32_t epoch = reserve_status(size_t(n / (BLOCK * ITEMS) + n / 2048u + 4100u) * STATUS_STRIDE, s);
+  unsigned long long* status = static_cast<unsigned long long*>(t_ws.status->ptr);
+  retain(t_ws.status);
+  const MsdWork w = msd_work(n, ITEMS, device_alloc);
+  const Units un = msd_analyse<K, W>(keys, TYPE, nullptr, 0, n, 0, 0, 0, ctl, w, epoch, nullptr, 0, nullptr, s);
+  const uint32_t tiles = (n + KEEP_TILE - 1) / KEEP_TILE;
+  DevBuf dup_buf = device_alloc(size_t(tiles) * KEEP_TILE);
+  auto* dup = static_cast<uint8_t*>(dup_buf->ptr);
+  hipLaunchKernelGGL(fill_u64, dim3(std::min(tiles, 2048u)), dim3(256), 0, s, reinterpret_cast<unsigned long long*>(dup),
+                     size_t(tiles) * KEEP_TILE / 8, 0ull);
+  AM_HIP(hipGetLastError());
+  DevBuf k0 = device_alloc(size_t(n) * W), k1 = device_alloc(size_t(n) * W);
+  DevBuf r0 = device_alloc(size_t(n) * 4), r1 = device_alloc(size_t(n) * 4);
+  K *kp0 = static_cast<K*>(k0->ptr), *kp1 = static_cast<K*>(k1->ptr);
+  auto *rp0 = static_cast<uint32_t*>(r0->ptr), *rp1 = static_cast<uint32_t*>(r1->ptr);
+  AM_HIP(hipStreamSynchronize(s));
+  const MsdPlan plan = *reinterpret_cast<MsdPlan*>(host_plan_words());
+  if (!((plan.mask >> (W - 1)) & 1u)) return false;   // a key or two: any other way is as good
+  {
+    ProfScope ps("sort_msd_first");
+    hipLaunchKernelGGL((msd_part<K, W, AM_MSD_FITEMS>), dim3(std::min(un.count, uint32_t(device().cu_count) * 3u)), dim3(BLOCK),
+                       0, s, keys, static_cast<const uint8_t*>(nullptr), int64_t(0), n, TYPE, 0, 0, ctl, un.hist, un.count,
+                       un.shift, kp0, rp0, static_cast<uint32_t*>(nullptr), nullptr);
+    AM_HIP(hipGetLastError());
+  }
+  if (!msd_levels<K, ITEMS>(w, plan.m, W - 1, plan.mask, false, LOCAL_MAX, status, kp0, rp0, kp1, rp1, nullptr, s, false,
+                            &plan.large, &plan.biggest, &plan.local, dup))
+    return false;
+  rows = device_alloc(size_t(n) * 4);
+  DevBuf base = device_alloc(size_t(tiles) * 4);
+  std::shared_ptr<void> slot = pinned_slot();
+  auto* total = static_cast<uint32_t*>(slot.get());
+  {
+    ProfScope ps("keep_rows");
+    hipLaunchKernelGGL(keep_count, dim3(tiles), dim3(BLOCK), 0, s, static_cast<const uint8_t*>(dup), n,
+                       static_cast<uint32_t*>(base->ptr), scan_ticket(s), total);
+    hipLaunchKernelGGL(keep_write, dim3(tiles), dim3(BLOCK), 0, s, static_cast<const uint8_t*>(dup), n,
+                       static_cast<const uint32_t*>(base->ptr), static_cast<uint32_t*>(rows->ptr));
+    AM_HIP(hipGetLastError());
+  }
+  AM_HIP(hipStreamSynchronize(s));
+  kept = *total;
+  return true;
 }
 
 // ---------------------------------------------------------------- ORDER BY of whole tables
@@ -1277,6 +1420,12 @@ __global__ void ob_key_rest(unsigned long long* out, uint32_t n, uint32_t vbase,
 }
 
 }  // namespace
+
+bool distinct_rows(const void* keys, int width, uint32_t n, DevBuf& rows, uint32_t& kept) {
+  if (capturing(stream())) return false;
+  return width == 8 ? distinct_rows_t<unsigned long long>(keys, n, rows, kept, stream())
+                    : distinct_rows_t<uint32_t>(keys, n, rows, kept, stream());
+}
 
 void argsort_device(const void* vals, int type, const uint8_t* validity, int64_t vbit_off, int64_t n,
                     bool descending, int null_placement, int float_order, uint32_t* out_idx, hipStream_t s) {

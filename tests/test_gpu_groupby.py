@@ -287,6 +287,36 @@ def test_small_inputs_in_one_launch(case, n, span, monkeypatch):
         np.testing.assert_array_equal(am.unique_rows(arrays).to_numpy()[0], O.unique_rows(cols, valid))
 
 
+@pytest.mark.parametrize("case", ["distinct", "few", "hot", "runs", "full_range", "wide_pair", "nulls", "one_key", "narrow"])
+@pytest.mark.parametrize("n", [5001, 32769, 200_003, 1_500_001])
+def test_unique_rows_by_partition(case, n):
+    """Distinct rows by partition and deduplication in LDS: nearly all rows distinct, few, hot keys (buckets
+    of equal keys at every level, copies), 32- and 64-bit composites, a column over its full range, nulls,
+    and one key alone, which the partition leaves to the general path."""
+    rng = np.random.default_rng(n)
+    valid = [None, None]
+    if case == "distinct": cols = [rng.permutation(n).astype(np.int64), rng.integers(0, 1000, n)]
+    elif case == "few": cols = [rng.integers(0, 40_000, n), rng.integers(0, 3, n).astype(np.int8)]
+    elif case == "hot":
+        cols = [np.where(rng.random(n) < 0.7, rng.integers(0, 5, n), rng.integers(0, 10**6, n)), rng.integers(0, 2, n).astype(np.uint16)]
+    elif case == "runs": cols = [np.repeat(rng.permutation(n // 50 + 1), 50)[:n].astype(np.int64) * 999, np.zeros(n, np.int32)]
+    elif case == "full_range": cols = [O.splitmix64(1, n).view(np.int64)[rng.integers(0, n, n)]]
+    elif case == "wide_pair": cols = [rng.integers(-2**40, 2**40, n)[rng.integers(0, n, n)], rng.integers(0, 7, n).astype(np.int16)]
+    elif case == "nulls":
+        cols, valid = [rng.integers(0, 50_000, n), rng.integers(0, 30, n).astype(np.int32)], [rng.random(n) > 0.2, rng.random(n) > 0.1]
+    elif case == "one_key":
+        cols = [np.full(n, 2**61), np.full(n, 3, np.int32)]
+        cols[0][-1] += 2**20
+    else: cols = [rng.integers(0, 2**32, n, dtype=np.uint64).astype(np.uint32)]
+    arrays = [am.MetalArray.from_numpy(c, v) for c, v in zip(cols, valid)]
+    want = O.unique_rows(cols, valid[:len(cols)])
+    for _ in range(2):
+        np.testing.assert_array_equal(am.unique_rows(arrays).to_numpy()[0], want)
+    off = min(11, n - 1)
+    got = am.unique_rows([a.slice(off, n - off) for a in arrays]).to_numpy()[0]
+    np.testing.assert_array_equal(got, O.unique_rows([c[off:] for c in cols], [None if v is None else v[off:] for v in valid[:len(cols)]]))
+
+
 def test_lowest_rows_of_more_groups_than_the_partitioned_passes_take():
     """Above 2^21 groups the lowest rows come from one pass of atomics."""
     n = (1 << 21) + 200_000
