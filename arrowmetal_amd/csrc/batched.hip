@@ -731,6 +731,12 @@ __global__ void bg_widen(const void* keys, int ktype, uint32_t n, unsigned long 
   if (i < n) out[i] = bg_key(keys, i, ktype);
 }
 
+struct PlanStatus {
+  uint32_t lc[LC_READ];
+  uint32_t overflowed, pad;   // batches whose group table ran out of room
+  unsigned long long groups;
+};
+
 struct Batched {
   std::vector<uint32_t> offsets;     // host copy, nseg + 1
   uint32_t nseg = 0, n = 0;
@@ -767,8 +773,43 @@ struct Batched {
     exec = nullptr;
     graph = nullptr;
   }
-  ~Batched() { drop_graph(); }
+  // Levels the MSD sort is recorded with: every digit's, until the tuner has seen how many the batches
+  // need. A run that finds a bucket left over sorts again with every level, and keeps them.
+  int levels = 8;
+  PlanStatus* status_host = nullptr;   // pinned: what a run reports
+  ~Batched() {
+    drop_graph();
+    if (status_host) (void)hipHostFree(status_host);
+  }
 };
+
+namespace {
+
+// The run's report, in pinned host memory: one kernel at the end of the sequence instead of a copy into
+// pageable memory for the sort's counters, the overflow flags and the group count each.
+__global__ __launch_bounds__(256) void seg_status(const uint32_t* lc, const uint32_t* overflow, uint32_t nseg,
+                                                  const unsigned long long* groups, PlanStatus* out) {
+  __shared__ uint32_t s_over[4];
+  if (lc && threadIdx.x < LC_READ) out->lc[threadIdx.x] = lc[threadIdx.x];
+  uint32_t over = 0;
+  if (groups)
+    for (uint32_t i = threadIdx.x; i < nseg; i += 256) over += overflow[i] ? 1u : 0u;
+  for (int off = 32; off > 0; off >>= 1) over += __shfl_xor(over, off, 64);
+  if ((threadIdx.x & 63) == 0) s_over[threadIdx.x >> 6] = over;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    out->overflowed = s_over[0] + s_over[1] + s_over[2] + s_over[3];
+    out->groups = groups ? *groups : 0ull;
+  }
+}
+
+// 16 bytes per thread (both buffers are whole allocations).
+__global__ __launch_bounds__(256) void seg_copy(const uint4* src, uint4* dst, size_t n) {
+  const size_t stride = size_t(gridDim.x) * 256;
+  for (size_t i = size_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += stride) dst[i] = src[i];
+}
+
+}  // namespace
 
 namespace {
 
@@ -830,7 +871,7 @@ void seg_sort_msd(Batched& b, const void* vals, int type, int desc, int forder, 
                      b.msd.local, b.msd.local_cap, b.msd.lc);
   AM_HIP(hipGetLastError());
   msd_levels<K, 16>(b.msd, b.n, P, 0xFFu, true, LOCAL_MAX / 2, static_cast<unsigned long long*>(b.status->ptr), kp0,
-                    rp0, kp1, rp1, static_cast<uint32_t*>(b.out_idx->ptr), s);
+                    rp0, kp1, rp1, static_cast<uint32_t*>(b.out_idx->ptr), s, false, nullptr, nullptr, nullptr, nullptr, b.levels);
 }
 
 template <typename K, int W>
@@ -910,7 +951,7 @@ void group_launch(Batched& b, const void* keys, int ktype, const void* vals, int
 DevBuf persistent(size_t bytes) {
   // Plan buffers live as long as the plan, outside any batch's retention.
   void* p = nullptr;
-  AM_HIP(hipMalloc(&p, std::max<size_t>(bytes, 8)));
+  AM_HIP(hipMalloc(&p, std::max<size_t>((bytes + 255) / 256 * 256, 256)));
   return device_wrap(p, bytes, [](void* q) { (void)hipFree(q); });
 }
 
@@ -1093,6 +1134,7 @@ Batched* batched_create(const int64_t* offsets, int64_t nbatches, int hash_capac
     b->base = persistent(size_t(b->nseg) * 8 * RADIX * 4);
     b->ctl = persistent(sizeof(SegCtl));
     b->epoch = persistent(4);
+    AM_HIP(hipHostMalloc(reinterpret_cast<void**>(&b->status_host), sizeof(PlanStatus), hipHostMallocDefault));
     b->msd = msd_work(b->n, 16, persistent, b->nseg);
     build_tiles(*b, (items == 8 || items == 20) ? items : 16);
     size_t nn = std::max<size_t>(n, 1);
@@ -1145,7 +1187,18 @@ void record(Batched* b, const Array* sort_keys, const Array* group_keys, const A
             hipStream_t s) {
   if (sort_keys) seg_sort(*b, sort_keys->data(), sort_keys->type, desc, forder, s);
   if (group_keys) group_launch(*b, group_keys->data(), group_keys->type, values->data(), values->type, s);
+  hipLaunchKernelGGL(seg_status, dim3(1), dim3(256), 0, s, sort_keys && b->msd_used ? b->msd.lc : nullptr,
+                     static_cast<const uint32_t*>(b->overflow->ptr), b->nseg,
+                     group_keys ? static_cast<const unsigned long long*>(b->goff->ptr) + b->nseg : nullptr, b->status_host);
+  AM_HIP(hipGetLastError());
 }
+
+// Whether the MSD sort of the last sequence ran out of list room, or of levels.
+bool list_full(const Batched* b) {
+  const uint32_t* w = b->status_host->lc;
+  return w[LC_OVERFLOW] || uint64_t(w[LC_LOCAL]) + w[LC_GROUPS] > b->msd.local_cap;
+}
+bool levels_short(const Batched* b) { return b->levels < 8 && b->status_host->lc[LC_LIST + (b->levels & 1)] != 0u; }
 
 }  // namespace
 
@@ -1186,18 +1239,23 @@ void batched_run(Batched* b, const Array* sort_keys, const Array* group_keys, co
     ProfScope pscope("batched_graph");
     AM_HIP(hipGraphLaunch(b->exec, s));
   }
-  if (sort_keys && b->msd_used) {
+  AM_HIP(hipStreamSynchronize(s));
+  const PlanStatus report = *b->status_host;   // the group-by's part holds whatever the sort does below
+  if (sort_keys && b->msd_used && levels_short(b)) {
+    // The tuner's batches needed fewer levels than these: every level from now on, and this sort again.
+    b->levels = 8;
+    b->drop_graph();
+    record(b, sort_keys, nullptr, nullptr, desc, forder, s);
+    AM_HIP(hipStreamSynchronize(s));
+  }
+  if (sort_keys && b->msd_used && list_full(b)) {
     // The MSD sort's bucket list has room for every batch plus m / 32 more buckets; if a run needed
     // more, this plan sorts with the LSD passes from now on, and this run's sort is done again.
-    uint32_t words[LC_READ];
-    AM_HIP(hipMemcpyAsync(words, b->msd.lc, sizeof(words), hipMemcpyDeviceToHost, s));
+    b->use_msd = false;
+    b->msd_overflowed = true;
+    b->drop_graph();
+    seg_sort(*b, sort_keys->data(), sort_keys->type, desc, forder, s);
     AM_HIP(hipStreamSynchronize(s));
-    if (words[LC_OVERFLOW] || uint64_t(words[LC_LOCAL]) + words[LC_GROUPS] > b->msd.local_cap) {
-      b->use_msd = false;
-      b->msd_overflowed = true;
-      b->drop_graph();
-      seg_sort(*b, sort_keys->data(), sort_keys->type, desc, forder, s);
-    }
   }
   b->ran_sort = sort_keys != nullptr;
   b->ran_group = group_keys != nullptr;
@@ -1205,17 +1263,14 @@ void batched_run(Batched* b, const Array* sort_keys, const Array* group_keys, co
   if (group_keys) {
     b->key_format = group_keys->format;
     b->key_type = group_keys->type;
-    std::vector<uint32_t> over(b->nseg);
-    unsigned long long total = 0;
-    AM_HIP(hipMemcpyAsync(over.data(), b->overflow->ptr, size_t(b->nseg) * 4, hipMemcpyDeviceToHost, s));
-    AM_HIP(hipMemcpyAsync(&total, static_cast<unsigned long long*>(b->goff->ptr) + b->nseg, 8,
-                          hipMemcpyDeviceToHost, s));
-    AM_HIP(hipStreamSynchronize(s));
-    b->groups = total;
-    for (uint32_t x : over) b->fallback_batches += x ? 1u : 0u;
-    if (b->fallback_batches) regroup_overflowed(*b, *group_keys, *values, over);
-  } else {
-    AM_HIP(hipStreamSynchronize(s));
+    b->groups = report.groups;
+    b->fallback_batches = report.overflowed;
+    if (report.overflowed) {
+      std::vector<uint32_t> over(b->nseg);
+      AM_HIP(hipMemcpyAsync(over.data(), b->overflow->ptr, size_t(b->nseg) * 4, hipMemcpyDeviceToHost, s));
+      AM_HIP(hipStreamSynchronize(s));
+      regroup_overflowed(*b, *group_keys, *values, over);
+    }
   }
 }
 
@@ -1251,6 +1306,11 @@ void batched_tune(Batched* b, const Array* sort_keys, const Array* group_keys, c
       bool best_msd = false;
       if (type_width(sort_keys->type) == 8 && !b->msd_overflowed) {
         b->use_msd = true;
+        b->levels = 8;
+        record(b, sort_keys, nullptr, nullptr, desc, forder, s);
+        AM_HIP(hipStreamSynchronize(s));
+        // An empty level is five launches that find nothing to do, ~30 us of each run.
+        b->levels = std::min<int>(8, int(b->status_host->lc[LC_LEVELS]));
         best = time_ms(sort_keys, nullptr, nullptr);
         best_msd = true;
       }
@@ -1320,11 +1380,17 @@ Array* batched_result(Batched* b, int which) {
   if (which == 0 && !b->ran_sort) fail("batched: the last run had no sort keys");
   if (which >= 1 && which <= 4 && !b->ran_group) fail("batched: the last run had no group-by");
   hipStream_t s = stream();
+  // Whole 16-byte pieces: plan buffers and pool blocks are both allocated in multiples of 256 bytes at least.
+  auto copy = [&](void* dst, const void* src, size_t bytes) {
+    const size_t pieces = (bytes + 15) / 16;
+    const int blocks = int(std::min<size_t>((pieces + 255) / 256, size_t(device().cu_count) * 16));
+    hipLaunchKernelGGL(seg_copy, dim3(blocks), dim3(256), 0, s, static_cast<const uint4*>(src), static_cast<uint4*>(dst), pieces);
+    AM_HIP(hipGetLastError());
+  };
   auto wrap = [&](const void* src, int64_t len, const char* fmt, int type) {
     Array* a = new_array(fmt, type, len);
     a->values = device_alloc(size_t(std::max<int64_t>(len, 1)) * std::max(type_width(type), 1));
-    if (len > 0)
-      AM_HIP(hipMemcpyAsync(a->values->ptr, src, size_t(len) * type_width(type), hipMemcpyDeviceToDevice, s));
+    if (len > 0) copy(a->values->ptr, src, size_t(len) * type_width(type));
     a->null_count = 0;
     return a;
   };
@@ -1339,7 +1405,7 @@ Array* batched_result(Batched* b, int which) {
       a->values = device_alloc(size_t(std::max<int64_t>(total, 1)) * w);
       a->null_count = 0;
       if (total && w == 8)
-        AM_HIP(hipMemcpyAsync(a->values->ptr, b->okey->ptr, size_t(total) * 8, hipMemcpyDeviceToDevice, s));
+        copy(a->values->ptr, b->okey->ptr, size_t(total) * 8);
       else if (total)
         AM_HIP(hipMemcpy2DAsync(a->values->ptr, w, b->okey->ptr, 8, w, size_t(total), hipMemcpyDeviceToDevice, s));
       break;

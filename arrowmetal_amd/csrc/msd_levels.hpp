@@ -124,6 +124,7 @@ constexpr int LC_OVERFLOW = 6;    // the bucket sort's list ran out of room
 constexpr int LC_QLEN = 7;        // buckets queued for the LSD bucket sort
 constexpr int LC_ROWS = 8;        // rows in the next level's large buckets (bounds its grids)
 constexpr int LC_GROUPS = 9;      // groups of small buckets, at the far end of the bucket sort's list
+constexpr int LC_LEVELS = 10;     // levels that had a large bucket
 constexpr int LC_READ = 16;
 constexpr int LC_NEXT_TILE = 32;  // the next tile of the current level to take (own 128-byte line)
 constexpr int LC_QNEXT = 64;      // the next queued bucket to take (own 128-byte line)
@@ -171,6 +172,7 @@ __global__ __launch_bounds__(BLOCK) void lvl_layout(const Bucket* large, int cur
     lc[LC_NEXT_TILE] = 0u;
     lc[LC_LIST + (cur ^ 1)] = 0u;
     lc[LC_ROWS] = 0u;
+    if (nb != 0u) lc[LC_LEVELS]++;
   }
 }
 
@@ -1003,13 +1005,14 @@ inline MsdWork msd_work(uint32_t m, int items, DevBuf (*alloc)(size_t), uint32_t
 //   written that a rerun does not write again, when the bucket sort's list ran out of room.
 // - Blind form (blind = true, e.g. inside a graph capture): every digit below `top` gets a level,
 //   sized for the worst case, the kernels read what to do from the device, and the bucket sort takes
-//   buckets of at most local_max = LOCAL_MAX / 2 rows. The caller must check LC_OVERFLOW itself.
+//   buckets of at most local_max = LOCAL_MAX / 2 rows. The caller must check LC_OVERFLOW itself, and, when it
+//   asks for fewer levels than digits (max_levels), that the last of them left no large bucket.
 // Look-back epochs: w.mc->epoch + 9 .. + 15.
 template <typename K, int ITEMS>
 bool msd_levels(const MsdWork& w, uint32_t m, int top, uint32_t mask, bool blind, uint32_t local_max,
                 unsigned long long* status, K* k0, uint32_t* r0, K* k1, uint32_t* r1, uint32_t* out_idx,
                 hipStream_t s, bool keys = false, const uint32_t* large = nullptr, const uint32_t* biggest_local = nullptr,
-                const uint32_t* local_entries = nullptr, uint8_t* dup = nullptr) {
+                const uint32_t* local_entries = nullptr, uint8_t* dup = nullptr, int max_levels = int(sizeof(K)) + 1) {
   constexpr int P = int(sizeof(K));
   constexpr uint32_t TILE = BLOCK * ITEMS;
   const uint32_t cus = uint32_t(device().cu_count);
@@ -1026,7 +1029,7 @@ bool msd_levels(const MsdWork& w, uint32_t m, int top, uint32_t mask, bool blind
   uint32_t bound = blind ? w.large_cap : large ? *large : uint32_t(RADIX), rows = m;
   int cur = 0;
   bool read = false;
-  for (int d = next_digit(top); d >= 0 && bound > 0; d = next_digit(d)) {
+  for (int d = next_digit(top), level = 0; d >= 0 && bound > 0 && level < max_levels; d = next_digit(d), level++) {
     {
       ProfScope ps("sort_msd_layout");
       hipLaunchKernelGGL(lvl_layout<ITEMS>, dim3(1), dim3(BLOCK), 0, s, w.large[cur], cur, w.bofs, w.lc);

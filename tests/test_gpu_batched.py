@@ -220,3 +220,32 @@ def test_batched_errors():
         plan.result("indices")
     with pytest.raises(am.ArrowMetalError, match="offsets must not decrease"):
         am.Batched(np.array([0, 10, 5], dtype=np.int64))
+
+
+def test_plan_tuned_on_fewer_levels_than_a_later_run_needs():
+    """The tuner records as many MSD levels as its batches needed; a run whose keys need more (long shared
+    prefixes, equal-prefix runs) finds a bucket left over, sorts again with every level, and keeps them."""
+    rng = np.random.default_rng(77)
+    lens = [300_000, 5, 40_000, 0, 2_000, 70_001]
+    offs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    n = int(offs[-1])
+    easy = O.splitmix64(5, n).view(np.int64)
+    hard = (rng.integers(0, 3, n) << 48) + (rng.integers(0, 2, n) << 24) + rng.integers(0, 60_000, n)
+    gk = rng.integers(0, 50, n)
+    gv = rng.integers(-1000, 1000, n)
+    m = lambda x: am.MetalArray.from_numpy(x)
+    mk, mv, me, mh = m(gk), m(gv), m(easy), m(hard)
+    plan = am.Batched(offs)
+    plan.tune(me, mk, mv)
+    for keys, arr in ((easy, me), (hard, mh), (easy, me), (hard, mh)):
+        plan.run(arr, mk, mv)
+        got = plan.result("indices").to_numpy()[0]
+        goff = plan.result("group_offsets").to_numpy()[0]
+        sums, counts = plan.result("sums").to_numpy()[0], plan.result("counts").to_numpy()[0]
+        for b in range(len(lens)):
+            lo, hi = int(offs[b]), int(offs[b + 1])
+            np.testing.assert_array_equal(got[lo:hi], O.argsort(keys[lo:hi]))
+            u, inv = np.unique(gk[lo:hi], return_inverse=True)
+            assert goff[b + 1] - goff[b] == len(u)
+            np.testing.assert_array_equal(sums[goff[b]:goff[b + 1]], np.bincount(inv, gv[lo:hi], len(u)).astype(np.int64))
+            np.testing.assert_array_equal(counts[goff[b]:goff[b + 1]], np.bincount(inv, minlength=len(u)))
