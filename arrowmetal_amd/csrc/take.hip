@@ -35,11 +35,11 @@ __device__ __forceinline__ uint32_t take_vbyte(const uint8_t* valid, int64_t b) 
 // counter that every wave bumps is one memory-side atomic per 64 rows on one address: it took 150 us of
 // 4M rows' 160.)
 template <typename V, typename I, bool NULLS>
-__global__ __launch_bounds__(256) void take_kernel(const V* __restrict__ vals, const uint8_t* __restrict__ vvalid,
-                                                   int64_t voff, int64_t len, const I* __restrict__ idx,
-                                                   const uint8_t* __restrict__ ivalid, int64_t ioff, int64_t n,
-                                                   V* __restrict__ out, unsigned long long* __restrict__ out_valid,
-                                                   uint32_t* __restrict__ block_nulls, TakeStatus* st) {
+__device__ __forceinline__ void take_rows(const V* __restrict__ vals, const uint8_t* __restrict__ vvalid, int64_t voff,
+                                          int64_t len, const I* __restrict__ idx, const uint8_t* __restrict__ ivalid,
+                                          int64_t ioff, int64_t n, V* __restrict__ out,
+                                          unsigned long long* __restrict__ out_valid,
+                                          uint32_t* __restrict__ block_nulls, TakeStatus* st) {
   __shared__ uint32_t s_nulls[4];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t step = int64_t(gridDim.x) * 256 * TAKE_GROUPS;
@@ -86,6 +86,15 @@ __global__ __launch_bounds__(256) void take_kernel(const V* __restrict__ vals, c
   }
 }
 
+template <typename V, typename I, bool NULLS>
+__global__ __launch_bounds__(256) void take_kernel(const V* __restrict__ vals, const uint8_t* __restrict__ vvalid,
+                                                   int64_t voff, int64_t len, const I* __restrict__ idx,
+                                                   const uint8_t* __restrict__ ivalid, int64_t ioff, int64_t n,
+                                                   V* __restrict__ out, unsigned long long* __restrict__ out_valid,
+                                                   uint32_t* __restrict__ block_nulls, TakeStatus* st) {
+  take_rows<V, I, NULLS>(vals, vvalid, voff, len, idx, ivalid, ioff, n, out, out_valid, block_nulls, st);
+}
+
 // A gather from an empty array: every non-null index is out of range.
 template <typename I>
 __global__ __launch_bounds__(256) void take_empty(const I* idx, const uint8_t* ivalid, int64_t ioff, int64_t n, char* out,
@@ -114,6 +123,263 @@ __global__ __launch_bounds__(1024) void take_nulls(const uint32_t* block_nulls, 
   }
 }
 
+// ---------------------------------------------------------------- large random gathers
+//
+// A gather of random rows from a large column is bound by the 128-byte line it fetches per row, whichever
+// memory that comes from: 50M float64 values took 1006 us, 6.9 GB of lines for 1 GB of data. Such a gather
+// runs in three passes instead:
+//   tk_split   each tile of TK_TILE outputs groups its indices by source slice (a 256th of the column), in
+//              LDS: the grouped indices, each one's place in the tile, and the tile's slice offsets
+//   tk_fetch   slice by slice, every tile's run of indices into it -> the values, in the grouped order. An
+//              XCD's workgroups all work on one slice at a time, so a line comes from its L2, and several
+//              rows of a wave may share one
+//   tk_place   each tile's values to their places, through LDS
+// 50M float64: 113 + 534 + 152 us, 811 us a call (1010 before); 50M float32: 117 + 453 + 88, 656 us (972). The
+// fetch is still bound by L1 filling a line per row: the same loop reads neighbours in 271 us.
+//
+// Which way a call goes is decided on the device from a sample of the indices: runs of neighbours are
+// cheaper read directly, and tk_fetch then is the plain gather: neighbours cost such a call
+// 5 us for the two kernels that return (50M float64 187 and 196, 24M float32 65 and 68).
+constexpr uint32_t TK_TILE = 16384;
+constexpr uint32_t TK_SLICES = 256;
+constexpr uint32_t TK_THREADS = 1024;
+constexpr int TK_PER = int(TK_TILE / TK_THREADS);
+constexpr uint32_t TK_FETCH_TILES = 16;   // tiles per work item of tk_fetch, four per wave
+// Where the passes win over the plain gather, calls of random indices, in us (plain / three passes):
+//   float32, as many rows as the source: 6M 107/115, 8M 145/131, 12M 227/177, 24M 460/335, 50M 972/656
+//   float64:                             6M 125/128, 8M 165/156, 12M 249/231, 24M 487/414, 50M 1010/811
+//   smaller sources, 16M rows:           float32 of 2M 167/200, of 4M 236/209; float64 of 2M 250/253, of 4M 292/261
+//   larger ones:                         float32 16M of 64M 322/273, 8M of 64M 170/173; float64 333/351, 175/224
+// So from 3 * 2^22 rows (below, the gain is near the 5 us that a call of neighbours loses), of a
+// source of at most twice as many rows (a tile's run in a slice is short otherwise) and of 16 MiB (the
+// eight L2s hold a smaller one).
+template <typename V>
+bool take_by_slices(int64_t n, int64_t len) {
+  return n >= int64_t(3) << 22 && n <= int64_t(UINT32_MAX) - TK_TILE && len <= 2 * n && len <= int64_t(UINT32_MAX) &&
+         len * int64_t(sizeof(V)) >= int64_t(1) << 24;
+}
+
+struct TkCtl {
+  uint32_t scattered, pad[31];
+  struct { uint32_t next, pad[31]; } item[NXCD];   // the next work item of each XCD, a line each
+};
+
+// 64 groups of 64 consecutive outputs, evenly spread, four per wave: true, for the whole workgroup, if in most
+// of them at least half of the neighbours lie on different lines and half of the rows 1 MiB or more from
+// the group's first. Every workgroup reads the same sample.
+template <typename I>
+__device__ __forceinline__ bool tk_scattered(const I* idx, int64_t n, int width, uint32_t* s_cnt) {
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x == 0) *s_cnt = 0u;
+  __syncthreads();
+  I j[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) j[k] = idx[(n - 64) / 63 * (int64_t(k) * 16 + (threadIdx.x >> 6)) + lane];
+  uint32_t mine = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const int64_t at = int64_t(uint64_t(j[k]) * uint64_t(width));   // any index, also one out of range
+    const uint64_t line = uint64_t(at) >> 7, prev = __shfl_up(line, 1, 64), first = __shfl(line, 0, 64);
+    const uint64_t far = uint64_t(int64_t(line - first) + 8191);    // within 8191 lines either way: at most 16382
+    const uint32_t moved = uint32_t(__popcll(__ballot(line != prev))), apart = uint32_t(__popcll(__ballot(far > 16382u)));
+    mine += moved >= 32u && apart >= 32u ? 1u : 0u;
+  }
+  if (lane == 0) atomicAdd(s_cnt, mine);
+  __syncthreads();
+  return *s_cnt >= 48u;
+}
+
+// Tile by tile, if the indices are scattered: off[s][tile] = where slice s starts in the tile (off[TK_SLICES][tile]: the tile's rows).
+template <typename I>
+__global__ __launch_bounds__(TK_THREADS) void tk_split(const I* idx, uint32_t n, int64_t len, uint32_t shift,
+                                                       int width, TkCtl* ctl, uint32_t tiles, uint32_t* part_idx,
+                                                       uint16_t* part_pos, uint32_t* off, TakeStatus* st) {
+  __shared__ uint32_t s_cnt[TK_SLICES], s_start[TK_SLICES];
+  __shared__ uint32_t s_idx[TK_TILE];
+  __shared__ uint16_t s_pos[TK_TILE];
+  __shared__ uint32_t s_sample;
+  const bool scattered = tk_scattered(idx, int64_t(n), width, &s_sample);
+  if (blockIdx.x == 0) {   // for the kernels that follow
+    if (threadIdx.x == 0) ctl->scattered = scattered ? 1u : 0u;
+    if (threadIdx.x < uint32_t(NXCD)) ctl->item[threadIdx.x].next = 0u;
+  }
+  if (!scattered) return;   // uniform over the grid
+  for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const uint32_t t0 = tile * TK_TILE, rows = min(TK_TILE, n - t0);
+    if (threadIdx.x < TK_SLICES) s_cnt[threadIdx.x] = 0u;
+    __syncthreads();   // also: the tile before has been written out
+    uint32_t j[TK_PER], rank[TK_PER];
+    bool bad = false;
+#pragma unroll
+    for (int k = 0; k < TK_PER; k++) {   // every load first; rows past the end read the last index
+      const int64_t v = int64_t(idx[t0 + min(uint32_t(k) * TK_THREADS + threadIdx.x, rows - 1u)]);
+      const bool in = v >= 0 && v < len;
+      bad = bad || !in;
+      j[k] = in ? uint32_t(v) : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < TK_PER; k++)
+      rank[k] = uint32_t(k) * TK_THREADS + threadIdx.x < rows ? atomicAdd(&s_cnt[j[k] >> shift], 1u) : 0u;
+    __syncthreads();
+    if (threadIdx.x < 64) {   // the exclusive scan of the counts, PER consecutive ones per lane of the first wave
+      constexpr uint32_t PER = TK_SLICES / 64;
+      uint32_t c[PER], sum = 0;
+#pragma unroll
+      for (uint32_t q = 0; q < PER; q++) {
+        c[q] = s_cnt[PER * threadIdx.x + q];
+        sum += c[q];
+      }
+      uint32_t x = sum;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(x, d, 64);
+        if (int(threadIdx.x) >= d) x += y;
+      }
+      uint32_t run = x - sum;
+#pragma unroll
+      for (uint32_t q = 0; q < PER; q++) {
+        s_start[PER * threadIdx.x + q] = run;
+        run += c[q];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < TK_PER; k++) {
+      const uint32_t r = uint32_t(k) * TK_THREADS + threadIdx.x;
+      if (r < rows) {
+        const uint32_t p = s_start[j[k] >> shift] + rank[k];
+        s_idx[p] = j[k];
+        s_pos[p] = uint16_t(r);
+      }
+    }
+    __syncthreads();
+    for (uint32_t p = threadIdx.x; p < rows; p += TK_THREADS) {
+      part_idx[t0 + p] = s_idx[p];
+      part_pos[t0 + p] = s_pos[p];
+    }
+    if (threadIdx.x <= TK_SLICES)
+      off[size_t(threadIdx.x) * tiles + tile] = threadIdx.x < TK_SLICES ? s_start[threadIdx.x] : rows;
+    if (bad) st->out_of_range = 1u;
+  }
+}
+
+// Slices x, x + 8, x + 16, ... belong to XCD x, in that order; a work item is one slice of TK_FETCH_TILES
+// tiles. A workgroup whose XCD has no item left takes the others'. Without scattered indices: the plain
+// gather.
+template <typename V, typename I>
+__global__ __launch_bounds__(256) void tk_fetch(const V* vals, uint32_t tiles, TkCtl* ctl, const uint32_t* part_idx,
+                                                const uint32_t* off, V* part_val, int64_t len, const I* idx, int64_t n,
+                                                V* out, TakeStatus* st) {
+  __shared__ uint32_t s_item;
+  if (!ctl->scattered) {   // uniform over the grid
+    take_rows<V, I, false>(vals, nullptr, 0, len, idx, nullptr, 0, n, out, nullptr, nullptr, st);
+    return;
+  }
+  const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+  const uint32_t per_slice = (tiles + TK_FETCH_TILES - 1) / TK_FETCH_TILES, items = per_slice * (TK_SLICES / NXCD);
+  const uint32_t home = xcd_id();
+  for (uint32_t h = 0; h < uint32_t(NXCD); h++) {
+    const uint32_t x = (home + h) & uint32_t(NXCD - 1);
+    while (true) {
+      if (threadIdx.x == 0) s_item = atomicAdd(&ctl->item[x].next, 1u);
+      __syncthreads();
+      const uint32_t item = s_item;
+      __syncthreads();
+      if (item >= items) break;   // uniform: this XCD's items are all taken
+      const uint32_t slice = (item / per_slice) * NXCD + x;
+      const uint32_t tile0 = (item % per_slice) * TK_FETCH_TILES + w * 4u;
+      uint32_t begin[4], len[4], most = 0;
+#pragma unroll
+      for (uint32_t u = 0; u < 4; u++) {   // the same for the wave
+        const uint32_t t = min(tile0 + u, tiles - 1u);
+        const uint32_t a = off[size_t(slice) * tiles + t], b = off[size_t(slice + 1u) * tiles + t];
+        begin[u] = t * TK_TILE + a;
+        len[u] = tile0 + u < tiles ? b - a : 0u;
+        most = max(most, len[u]);
+      }
+      for (uint32_t p = lane; p - lane < most; p += 64u) {
+        uint32_t j[4];
+        V v[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) j[u] = p < len[u] ? __builtin_nontemporal_load(part_idx + begin[u] + p) : 0u;
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++)
+          if (p < len[u]) v[u] = vals[j[u]];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++)
+          if (p < len[u]) __builtin_nontemporal_store(v[u], part_val + begin[u] + p);
+      }
+    }
+  }
+}
+
+template <typename V>
+__global__ __launch_bounds__(TK_THREADS) void tk_place(uint32_t n, uint32_t tiles, const TkCtl* ctl, const V* part_val,
+                                                       const uint16_t* part_pos, V* out) {
+  __shared__ V s_val[TK_TILE];
+  if (!ctl->scattered) return;   // uniform over the grid
+  for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const uint32_t t0 = tile * TK_TILE, rows = min(TK_TILE, n - t0);
+    V v[TK_PER];
+    uint32_t p[TK_PER];
+#pragma unroll
+    for (int k = 0; k < TK_PER; k++) {
+      const uint32_t r = t0 + min(uint32_t(k) * TK_THREADS + threadIdx.x, rows - 1u);   // the last row more than once: the same value
+      v[k] = part_val[r];
+      p[k] = part_pos[r];
+    }
+    __syncthreads();   // the tile before has been written out
+#pragma unroll
+    for (int k = 0; k < TK_PER; k++) s_val[p[k]] = v[k];
+    __syncthreads();
+    for (uint32_t r = threadIdx.x; r < rows; r += TK_THREADS) out[t0 + r] = s_val[r];
+  }
+}
+
+// Queues the passes. False, and nothing queued, if their scratch (14 or 10 bytes a row) cannot be had: the
+// plain gather needs none.
+template <typename V, typename I>
+bool launch_take_slices(const Array& a, const Array& ix, Array* out, TakeStatus* st, hipStream_t s) {
+  const uint32_t n = uint32_t(ix.length), tiles = (n + TK_TILE - 1) / TK_TILE, cus = uint32_t(device().cu_count);
+  uint32_t shift = 0;
+  while (((uint64_t(a.length) - 1u) >> shift) >= TK_SLICES) shift++;
+  DevBuf cb, pi, pp, pv, ob;
+  try {
+    cb = device_alloc(sizeof(TkCtl));
+    pi = device_alloc(size_t(n) * 4);
+    pp = device_alloc(size_t(n) * 2);
+    pv = device_alloc(size_t(n) * sizeof(V));
+    ob = device_alloc(size_t(TK_SLICES + 1) * tiles * 4);
+  } catch (const Error&) {
+    return false;
+  }
+  auto* ctl = static_cast<TkCtl*>(cb->ptr);
+  const I* idx = static_cast<const I*>(ix.data());
+  const V* vals = static_cast<const V*>(a.data());
+  V* o = static_cast<V*>(out->values->ptr);
+  auto* part_idx = static_cast<uint32_t*>(pi->ptr);
+  auto* part_pos = static_cast<uint16_t*>(pp->ptr);
+  auto* part_val = static_cast<V*>(pv->ptr);
+  auto* off = static_cast<uint32_t*>(ob->ptr);
+  {
+    ProfScope ps("take_split");
+    hipLaunchKernelGGL(tk_split<I>, dim3(std::min(tiles, cus)), dim3(TK_THREADS), 0, s, idx, n, a.length, shift, int(sizeof(V)),
+                       ctl, tiles, part_idx, part_pos, off, st);
+  }
+  {
+    ProfScope ps("take");
+    hipLaunchKernelGGL((tk_fetch<V, I>), dim3(cus * 8u), dim3(256), 0, s, vals, tiles, ctl, part_idx, off, part_val, a.length,
+                       idx, ix.length, o, st);
+  }
+  {
+    ProfScope ps("take_place");
+    hipLaunchKernelGGL(tk_place<V>, dim3(std::min(tiles, cus * (sizeof(V) == 4 ? 2u : 1u))), dim3(TK_THREADS), 0, s, n, tiles,
+                       ctl, part_val, part_pos, o);
+  }
+  AM_HIP(hipGetLastError());
+  return true;
+}
+
 template <typename V, typename I>
 void launch_take(const Array& a, const Array& ix, Array* out, uint32_t blocks, uint32_t* block_nulls, TakeStatus* st,
                  hipStream_t s) {
@@ -126,12 +392,18 @@ void launch_take(const Array& a, const Array& ix, Array* out, uint32_t blocks, u
   if (a.length == 0)
     hipLaunchKernelGGL((take_empty<I>), dim3(blocks), dim3(256), 0, s, idx, iv, ix.offset, ix.length,
                        reinterpret_cast<char*>(o), int(sizeof(V)), ov, block_nulls, st);
-  else if (ov)
+  else if (ov) {
+    ProfScope ps("take");
     hipLaunchKernelGGL((take_kernel<V, I, true>), dim3(blocks), dim3(256), 0, s, vals, vv, a.offset, a.length, idx, iv,
                        ix.offset, ix.length, o, ov, block_nulls, st);
-  else
+  } else {
+    if constexpr (sizeof(V) >= 4) {   // not in a batch, which would hold the scratch to its end
+      if (!in_batch() && take_by_slices<V>(ix.length, a.length) && launch_take_slices<V, I>(a, ix, out, st, s)) return;
+    }
+    ProfScope ps("take");
     hipLaunchKernelGGL((take_kernel<V, I, false>), dim3(blocks), dim3(256), 0, s, vals, vv, a.offset, a.length, idx, iv,
                        ix.offset, ix.length, o, ov, block_nulls, st);
+  }
   AM_HIP(hipGetLastError());
 }
 
@@ -169,7 +441,6 @@ Array* take(const Array& a, const Array& ix) {
       DevBuf bn;
       if (need_validity) bn = device_alloc(size_t(blocks) * 4);
       uint32_t* block_nulls = bn ? static_cast<uint32_t*>(bn->ptr) : nullptr;
-      ProfScope ps("take");
       switch (w) {
         case 1: launch_take<uint8_t>(a, ix, out, blocks, block_nulls, st, s); break;
         case 2: launch_take<uint16_t>(a, ix, out, blocks, block_nulls, st, s); break;

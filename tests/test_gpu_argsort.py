@@ -259,6 +259,32 @@ def test_take_null_counts(n):
     assert empty.take(am.MetalArray.from_numpy(idx, np.zeros(n, bool))).null_count == n
 
 
+@pytest.mark.parametrize("dtype,itype,n,length", [
+    (np.float32, np.int32, 3 << 22, 1 << 22),                    # whole tiles, the smallest source
+    (np.int32, np.uint32, (3 << 22) + 1, 2 * ((3 << 22) + 1)),   # a tile of one row, the largest source
+    (np.float64, np.int64, (3 << 22) + 16_383, 1 << 21),
+    (np.int64, np.uint32, (3 << 23) + 5, (1 << 25) + 7),
+    (np.float32, np.int64, (3 << 22) - 1, 1 << 23),              # the plain gather on either side of the rule
+    (np.float32, np.int32, 3 << 22, (3 << 23) + 1),
+])
+def test_take_by_slices(dtype, itype, n, length):
+    """Large gathers: random indices by source slice, neighbours and windows directly, a bad index in the last row."""
+    rng = np.random.default_rng(n)
+    vals = np.arange(length, dtype=np.uint32).astype(dtype) if dtype != np.float32 \
+        else np.arange(length, dtype=np.uint32).view(np.float32)   # every bit pattern is one of its own
+    a = am.MetalArray.from_numpy(vals)
+    bits = np.uint32 if vals.itemsize == 4 else np.uint64
+    idx = rng.integers(0, length, n).astype(itype)
+    seq = (np.arange(n, dtype=np.int64) % length).astype(itype)
+    for ix in (idx, seq, np.minimum(seq // 4096 * 4096 + idx % 4096, length - 1).astype(itype)):
+        got, gv = a.take(am.MetalArray.from_numpy(ix)).to_numpy()
+        assert gv is None or gv.all()
+        assert np.array_equal(got.view(bits), vals.view(bits)[ix])
+    idx[-1] = length
+    with pytest.raises(am.ArrowMetalError, match=rf"take: index out of range \(array length {length}\)"):
+        a.take(am.MetalArray.from_numpy(idx))
+
+
 def test_take_out_of_range():
     a = am.MetalArray.from_numpy(np.arange(10, dtype=np.int64))
     with pytest.raises(am.ArrowMetalError, match=r"take: index out of range \(array length 10\)"):
