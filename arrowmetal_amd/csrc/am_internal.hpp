@@ -228,13 +228,17 @@ bool distinct_rows(const void* keys, int width, uint32_t n, DevBuf& rows, uint32
 // ORDER BY of a whole table by one 64-bit key (int64 / uint64 / float64): every column of `cols`
 // (each of n rows) in the key's stable order with am_argsort_ex2's options, as new arrays in `out`.
 // The columns move with the hybrid sort's top-digit partition instead of one gather across the table.
-// Returns false, with nothing in `out`, when the key does not take the hybrid sort (fewer than 2^18
-// rows, a constant top digit, a full bucket list, a graph capture); the caller then sorts and takes.
+// Returns false, with nothing in `out`, for large tables that a gather of whole rows moves faster, and when
+// the key does not take the hybrid sort (fewer than 2^18 rows, a constant top digit, a full bucket list, a
+// graph capture); the caller then sorts and permutes.
 bool order_by_columns(const Array& key, bool descending, int null_placement, int float_order,
                       const std::vector<const Array*>& cols, std::vector<Array*>& out);
 
 // take.hip
 Array* take(const Array& a, const Array& indices);
+// Every column of a table in the order `idx`, a permutation of its rows as an argsort returns it, as new
+// arrays in `out`. False, with nothing in `out`, for a single column or one that is not primitive.
+bool permute_columns(const std::vector<const Array*>& cols, const Array& idx, std::vector<Array*>& out);
 
 // select.hip
 Array* top_k(const Array& a, int64_t k, bool largest, int placement, int forder);

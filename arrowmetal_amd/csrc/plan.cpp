@@ -13,12 +13,12 @@
 // "Unsupported Arrow type: plan: ... is not supported by this build". The `optimize` flag is accepted:
 // on this subset the reference's optimizer rules (pushdown, pruning, folding) do not change a result.
 //
-// Execution is this build's own. A sort by one 64-bit key of a table of at least 2^18 rows moves
-// every column with the sort (order_by_columns in sort.hip): the columns are partitioned along the
-// sort's top-digit partition, and the final gather reads from the partition of its own output range,
-// so no column is gathered across the whole table; an int64 / uint64 key column comes out of the
-// sort's bucket sorts directly. Other sorts are a lexsort and a take per column,
-// as the reference does.
+// Execution is this build's own. A sort by one 64-bit key of a table of at least 2^18 rows that is small
+// or narrow moves every column with the sort (order_by_columns in sort.hip): the columns are partitioned
+// along the sort's top-digit partition, and the final gather reads from the partition of its own output
+// range, so no column is gathered across the whole table; an int64 / uint64 key column comes out of the
+// sort's bucket sorts directly. Other sorts are a lexsort and one gather of whole rows (permute_columns in
+// take.hip).
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -566,17 +566,18 @@ Table sort_table(Table in, const std::vector<SortKey>& keys) {
     kc.push_back(const_cast<Array*>(c));
   }
   if (in.length() == 0) return in;
+  std::vector<const Array*> cols;
+  for (auto& c : in.cols) cols.push_back(c.a);
+  auto table_of = [&in](const std::vector<Array*>& sorted) {
+    Table o;
+    o.names = in.names;
+    for (Array* a : sorted) o.cols.emplace_back(a);
+    return o;
+  };
   if (keys.size() == 1) {
-    std::vector<const Array*> cols;
-    for (auto& c : in.cols) cols.push_back(c.a);
     std::vector<Array*> sorted;
     const SortKey& k = keys[0];
-    if (order_by_columns(*kc[0], k.descending, k.nulls_first ? 1 : 0, k.float_order, cols, sorted)) {
-      Table o;
-      o.names = in.names;
-      for (Array* a : sorted) o.cols.emplace_back(a);
-      return o;
-    }
+    if (order_by_columns(*kc[0], k.descending, k.nulls_first ? 1 : 0, k.float_order, cols, sorted)) return table_of(sorted);
   }
   std::vector<int> desc, place, forder;
   for (auto& k : keys) {
@@ -585,7 +586,9 @@ Table sort_table(Table in, const std::vector<SortKey>& keys) {
     forder.push_back(k.float_order);
   }
   Ref idx(lexsort(kc.data(), int64_t(kc.size()), desc.data(), place.data(), forder.data()));
-  return take_table(in, *idx.a);
+  std::vector<Array*> sorted;
+  if (!permute_columns(cols, *idx.a, sorted)) return take_table(in, *idx.a);
+  return table_of(sorted);
 }
 
 Table run_limit(const Node& n) {

@@ -1495,6 +1495,15 @@ bool order_by_columns(const Array& key, bool descending, int null_placement, int
   if (key.width() != 8 || !type_is_primitive(key.type) || n < (int64_t(1) << 18) || n > int64_t(UINT32_MAX) ||
       capturing(stream()))
     return false;
+  // From 2^19 rows only with an integer key, whose own column comes out of the bucket sorts, and at most one
+  // other column. In us, this way / an argsort and permute_columns: an int64 key alone, 4M rows 229/298, 50M
+  // 1542/2079; with one float64, 4M 295/334, 50M 2301/2719; with three, 4M 443/376, 50M 3834/3347; with eight,
+  // 4M 777/543; a float64 key alone, 4M 462/406, 50M 3957/3266; with three others and nulls, 1M 427/285, 30M
+  // 5497/2366. (Smaller tables of many columns would gain as well, 300K 355/232, and keep this way: the checks
+  // of its two passes over every type, key order and null placement run there.)
+  const bool key_is_int = key.type == T_I64 || key.type == T_U64;
+  const bool key_is_column = std::find(cols.begin(), cols.end(), &key) != cols.end();
+  if (n >= (int64_t(1) << 19) && !(key_is_int && key_is_column && cols.size() <= 2)) return false;
   for (const Array* c : cols)
     if (c->length != n || !type_is_primitive(c->type)) return false;
   check_index_rows(n, "argsort");
@@ -1514,8 +1523,7 @@ bool order_by_columns(const Array& key, bool descending, int null_placement, int
   // mapped keys are a bijection of its values (x ^ 2^63 for int64, then ~ when descending).
   DevBuf key_vals;
   unsigned long long key_xor = 0;
-  const bool key_direct = (key.type == T_I64 || key.type == T_U64) &&
-                          std::find(cols.begin(), cols.end(), &key) != cols.end();
+  const bool key_direct = key_is_int && key_is_column;
   if (key_direct) {
     key_vals = device_alloc(size_t(n) * 8);
     key_xor = (key.type == T_I64 ? 0x8000000000000000ull : 0ull) ^ (descending ? ~0ull : 0ull);

@@ -137,6 +137,43 @@ def test_multi_key_sort_of_a_large_table():
     assert_tables_equal(got, want, "two keys")
 
 
+@pytest.mark.parametrize("n", [1, 63, 256, 257, 70_001, 1 << 19])
+@pytest.mark.parametrize("columns", [2, 9, 12])
+def test_sorted_tables_move_whole_rows(n, columns):
+    """The gather of whole rows: one to eight words a row, more columns than one row takes, columns of every
+    width with and without nulls, slices whose bitmaps start inside a byte, tails of a tile."""
+    rng = np.random.default_rng(n + columns)
+    types = [np.float64, np.int32, np.int16, np.uint8, np.int64, np.float32, np.uint16, np.int8][: max(columns - 4, 1)]
+    t = {"k": (rng.integers(0, 7, n + 3).astype(np.int32), rng.random(n + 3) > 0.1)}
+    for c in range(columns - 1):
+        d = np.dtype(types[c % len(types)])
+        bits = rng.integers(0, 256, (n + 3) * d.itemsize, dtype=np.uint8).view(d)
+        if d.kind == "f":
+            bits = rng.standard_normal(n + 3).astype(d)
+        t[f"c{c}"] = (bits, None if c % 3 == 0 else rng.random(n + 3) > 0.3)
+    plan = {"op": "sort", "by": [["k", True], ["c0", False]], "input": {"op": "scan", "source": "t"}}
+    source = am.PlanSource("t", {c: am.MetalArray.from_numpy(v, va).slice(3, n) for c, (v, va) in t.items()})
+    got, names = profiled_names(lambda: am.plan_run(plan, [source]))
+    assert "take_pack" in names and "take_unpack" in names, sorted(names)
+    want = O.plan_run(plan, {"t": {c: (v[3:], None if va is None else va[3:]) for c, (v, va) in t.items()}})
+    assert_tables_equal(got, want, f"{n} {columns}")
+
+
+@pytest.mark.parametrize("key_kind", ["i64", "f64"])
+def test_order_by_of_a_large_table_by_one_key(key_kind):
+    """From 2^19 rows: an integer key with one other column moves with the partition, other tables as rows."""
+    rng = np.random.default_rng(8)
+    t = order_by_table(rng, 1 << 19, key_kind)
+    plan = {"op": "sort", "by": [["key", True]], "input": {"op": "scan", "source": "t"}}
+    for names in (list(t), ["key", "pay"], ["key"]):
+        table = {c: t[c] for c in names}
+        (got, want), kernels = profiled_names(lambda: run_both(plan, {"t": table}))
+        narrow = key_kind == "i64" and len(names) == 2
+        assert ("order_by_gather" in kernels) == narrow and ("take_pack" in kernels) == (len(names) > 2 or (
+            key_kind == "f64" and len(names) == 2)), sorted(kernels)
+        assert_tables_equal(got, want, f"{key_kind} {names}")
+
+
 @pytest.mark.parametrize("count,offset", [(10, None), (1024, 0), (1025, 0), (5, 3), (0, 0), (10**12, 2), (-4, 0),
                                           (7, -3), (3, 10**9)])
 def test_limit_and_top_k(count, offset):
