@@ -4086,7 +4086,12 @@ bool map_composite(Array* const* columns, int64_t count, int64_t n, std::vector<
   CompositeArgs ca{};
   unsigned long long top = 0;
   if (!plan_composite(columns, count, n, ca, top)) return false;
-  DevBuf comp = write_composite<false>(ca, top, n);
+  DevBuf comp;
+  try {
+    comp = write_composite<false>(ca, top, n);
+  } catch (const Error&) {   // no room for the composite keys: column by column
+    return false;
+  }
   const RangeStat known{0ull, top - 1ull, 0ull, 0u, 0u};
   out = map_column(comp->ptr, composite_narrow(top) ? T_U32 : T_U64, nullptr, 0, n, &known);
   for (int64_t c = 0; c < count; c++) out_spans.push_back(ca.col[c].span);
@@ -4657,9 +4662,15 @@ Array* unique_rows(Array* const* columns, int64_t count) {
     CompositeArgs ca{};
     unsigned long long top = 0;
     if (same && plan_composite(columns, count, n, ca, top, true) && top > agg_dense_cap<FirstRowP>()) {
-      DevBuf keys = write_composite<true>(ca, top, n), rows;
+      DevBuf rows;
       uint32_t kept = 0;
-      if (distinct_rows(keys->ptr, composite_narrow(top) ? 4 : 8, uint32_t(n), rows, kept)) {
+      bool found = false;
+      try {   // up to 37 bytes a row of scratch: without that room the hash path takes the call
+        const DevBuf keys = write_composite<true>(ca, top, n);
+        found = distinct_rows(keys->ptr, composite_narrow(top) ? 4 : 8, uint32_t(n), rows, kept);
+      } catch (const Error&) {
+      }
+      if (found) {
         Array* out = new_array("I", T_U32, int64_t(kept));
         out->values = rows;
         out->null_count = 0;

@@ -62,7 +62,7 @@ size_t footprint_of(int op, int64_t n, int64_t ncols) {
   switch (op) {
     case OP_ARGSORT: return 29 * un + (size_t(16) << 20);   // keys + rows ping-pong, out, status
     case OP_GROUP_SUM_COUNT: return 16 * un + 2 * table;   // ids, aggregate tables, outputs
-    default: return size_t(ncols) * (12 * un + table) + 16 * un;
+    default: return size_t(ncols) * (12 * un + table) + 26 * un;   // also the composite keys' partition: 37 B/row
   }
 }
 
