@@ -19,7 +19,8 @@
 //                  launch only the active passes; smaller ones (and graph captures) launch one kernel
 //                  per digit that exits at once when its digit is inactive
 //
-// Inputs of at most 16,384 rows take none of these: sort_rank sorts them in one launch.
+// Inputs of at most 16,384 rows take none of these: sort_rank sorts them in one launch. Larger ones of 32 or
+// 64 bits take the MSD sort of msd_levels.hpp from the row counts at hybrid_min, below.
 //
 // Each scatter pass is "onesweep": tiles of 256 threads x ITEMS keys take dynamic tile ids, rank
 // their keys inside the tile with wave64 ballots (a 9-bit match per 64-lane row), publish their

@@ -4,7 +4,8 @@
 // KernelSource.swift:209-227): a null index gives a null output, a null source element gives a null,
 // and an index outside [0, length) makes the call fail with "take: index out of range (array length
 // N)" once the kernel has run. Each wave handles 64 consecutive outputs, so the output validity is one
-// 64-bit ballot per wave, written as one word; nulls are counted per workgroup, without atomics.
+// 64-bit ballot per wave, written as one word; nulls are counted per workgroup, without atomics. Large random
+// gathers run in three passes by source slice, and whole tables are gathered as rows (both below).
 #include "am_internal.hpp"
 
 #include <algorithm>

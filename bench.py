@@ -142,8 +142,8 @@ PMC_SUMMARY = os.path.join(ROOT, "profiles", "orderby_groupby_50M_pmc_traffic.tx
 
 # rocprofv3's kernel names (as written in the committed PMC summary) of the library's launch names.
 ROCPROF_NAME = {
-    "take": "take_kernel<u64, u32>",
-    "sort_upsweep": "sort_upsweep<u64, 8>",
+    "take": "tk_fetch<u64, u32>",
+    "sort_upsweep": "msd_upsweep<u64, 8>",
     "sort_msd_first": "msd_part<u64, 8, 16, false>",
     "sort_msd_hist": "lvl_hist<u64>",
     "sort_msd_scatter": "lvl_pass<u64, 20>",
@@ -151,8 +151,8 @@ ROCPROF_NAME = {
     "sort_first": "sort_first<u64, 8, 16>",
     "sort_scatter": "sort_mid<u64, 20, 0>",
     "sort_scatter_last": "sort_mid<u64, 20, 1>",
-    "gb_key_scan": "gb_key_scan<8, 3, false>",
-    "gb_build": "gb_build<false, 8, 7, true>",
+    "gb_key_scan": "gb_key_scan<8, 3, false, true>",
+    "gb_build": "gb_build<8, 7, true>",
     "gb_ids": "gb_ids",
     "gb_part_hist": "gb_part_hist<SumCountP, 4>",
     "gb_part_scatter": "gb_part_scatter<SumCountP, 4, 8, false>",
@@ -197,7 +197,7 @@ def sort_alg_bytes(n: int, m: int):
 
 def orderby_alg_bytes(n: int, m: int):
     d = sort_alg_bytes(n, m)
-    d["take"] = (20 * n, "gather: read u32 index + f64 value, write f64; 20 B/row")
+    d["take"] = (20 * n, "gather's fetch: read grouped u32 index + f64 value, write f64; 20 B/row")
     return d
 
 
