@@ -225,6 +225,10 @@ void argsort_device(const void* vals, int type, const uint8_t* validity, int64_t
 // do not take the partition (a constant top digit, a full bucket list, a graph capture).
 bool distinct_rows(const void* keys, int width, uint32_t n, DevBuf& rows, uint32_t& kept);
 
+// The sorted values of an int32, uint32, int64 or uint64 column of at least the hybrid sort's rows, whose
+// bucket sorts write them; nullptr for any other column (and in a graph capture): argsort and take.
+Array* sorted_ints(const Array& a, bool descending, int null_placement);
+
 // ORDER BY of a whole table by one 64-bit key (int64 / uint64 / float64): every column of `cols`
 // (each of n rows) in the key's stable order with am_argsort_ex2's options, as new arrays in `out`.
 // The columns move with the hybrid sort's top-digit partition instead of one gather across the table.

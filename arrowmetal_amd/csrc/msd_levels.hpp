@@ -72,30 +72,32 @@ struct LvlTile {
 // the value keys), where the value block starts in the output, and the run's look-back epoch.
 struct MsdCtl {
   uint32_t active_mask, value_base, epoch, pad;
-  // The ORDER BY of whole tables by a 64-bit integer key also takes the sorted key column from the
+  // Sorted integer columns and the ORDER BY of whole tables by one take the sorted key column from the
   // bucket sorts: key_out[value_base + i] = the mapped key of output i XOR key_xor (its original
-  // bits). Null when not asked for.
-  unsigned long long* key_out;
+  // bits), of the keys' width. Null when not asked for.
+  void* key_out;
   unsigned long long key_xor;
 };
 
 // The sorted key column's output as one bucket sort sees it (already offset to the value block).
+template <typename K>
 struct KeyOut {
-  unsigned long long* p;
-  unsigned long long x;
+  K* p;
+  K x;
 };
 
-__device__ __forceinline__ KeyOut key_out_of(const MsdCtl* mc) {
-  return KeyOut{mc->key_out ? mc->key_out + mc->value_base : nullptr, mc->key_xor};
+template <typename K>
+__device__ __forceinline__ KeyOut<K> key_out_of(const MsdCtl* mc) {
+  return KeyOut<K>{mc->key_out ? static_cast<K*>(mc->key_out) + mc->value_base : nullptr, K(mc->key_xor)};
 }
 
 // Beside the rows a bucket sort writes (dest[j] != ~0u), their keys, when the key column is asked for:
 // load_keys reads keys_in[src[j]] (src[j] is always a position of the bucket, so every load stays in
 // bounds; issued with the row loads, before any store), write_keys stores them.
 template <typename K, int LI, bool KEYS>
-__device__ __forceinline__ void load_keys(const KeyOut& ko, const K* keys_in, const uint32_t (&src)[LI],
-                                          unsigned long long (&v)[LI]) {
-  if constexpr (KEYS && sizeof(K) == 8) {
+__device__ __forceinline__ void load_keys(const KeyOut<K>& ko, const K* keys_in, const uint32_t (&src)[LI],
+                                          K (&v)[LI]) {
+  if constexpr (KEYS) {
     if (!ko.p) return;   // uniform
 #pragma unroll
     for (int j = 0; j < LI; j++) v[j] = keys_in[src[j]];
@@ -103,8 +105,8 @@ __device__ __forceinline__ void load_keys(const KeyOut& ko, const K* keys_in, co
 }
 
 template <typename K, int LI, bool KEYS>
-__device__ __forceinline__ void write_keys(const KeyOut& ko, const uint32_t (&dest)[LI], const unsigned long long (&v)[LI]) {
-  if constexpr (KEYS && sizeof(K) == 8) {
+__device__ __forceinline__ void write_keys(const KeyOut<K>& ko, const uint32_t (&dest)[LI], const K (&v)[LI]) {
+  if constexpr (KEYS) {
     if (!ko.p) return;   // uniform
 #pragma unroll
     for (int j = 0; j < LI; j++)
@@ -541,7 +543,7 @@ __device__ __forceinline__ void local_split(const K (&keys)[LI], const uint32_t 
 // order inside a run). Otherwise stable LSD passes run over every varying digit.
 template <typename K, int LI, bool KEYS>
 __device__ __forceinline__ void local_lsd(const K* keys_in, const uint32_t* rows_in, uint32_t off, uint32_t size,
-                                          uint32_t low_mask, uint32_t run_max, uint32_t* out_idx, const KeyOut& ko,
+                                          uint32_t low_mask, uint32_t run_max, uint32_t* out_idx, const KeyOut<K>& ko,
                                           uint32_t (*wc)[WC_STRIDE], uint32_t* tile_total, uint32_t* bin_start,
                                           uint32_t* tmp, K* s_keys, uint16_t* s_pos) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -577,7 +579,7 @@ __device__ __forceinline__ void local_lsd(const K* keys_in, const uint32_t* rows
         }
       }
       uint32_t r[LI];
-      unsigned long long kv[LI];
+      K kv[LI];
       load_rows<LI>(rows_in, off, src, r);
       load_keys<K, LI, KEYS>(ko, keys_in, src, kv);
 #pragma unroll
@@ -600,7 +602,7 @@ __device__ __forceinline__ void local_lsd(const K* keys_in, const uint32_t* rows
     __syncthreads();
   }
   uint32_t src[LI], r[LI], dest[LI];
-  unsigned long long kv[LI];
+  K kv[LI];
 #pragma unroll
   for (int j = 0; j < LI; j++) src[j] = off + min(pos[j], size - 1u);
   load_rows<LI>(rows_in, off, src, r);
@@ -623,7 +625,7 @@ __device__ __forceinline__ void local_lsd(const K* keys_in, const uint32_t* rows
 // end).
 template <typename K, int LI, uint32_t SPAN_LOG, bool KEYS>
 __device__ __forceinline__ bool local_group(const K* keys_in, const uint32_t* rows_in, uint32_t off, uint32_t size,
-                                            int top, int sub, uint32_t* out, const KeyOut& ko, uint32_t* tmp, uint32_t* g,
+                                            int top, int sub, uint32_t* out, const KeyOut<K>& ko, uint32_t* tmp, uint32_t* g,
                                             K* s_words, uint16_t* s_bin) {
   static_assert(RADIX == BLOCK, "a thread per digit value");
   constexpr uint32_t per = 1u << SPAN_LOG;   // bins per thread
@@ -687,7 +689,7 @@ __device__ __forceinline__ bool local_group(const K* keys_in, const uint32_t* ro
     }
   }
   uint32_t r[LI];
-  unsigned long long kv[LI];
+  K kv[LI];
   load_rows<LI>(rows_in, off, src, r);   // every row and key load before the first store
   load_keys<K, LI, KEYS>(ko, keys_in, src, kv);
 #pragma unroll
@@ -717,10 +719,10 @@ __device__ __forceinline__ void local_one(const MsdCtl* mc, const Bucket* list, 
   const uint32_t size = bk.size, off = bk.start;
   const uint32_t low_mask = mc->active_mask & ((1u << (bk.level & LEVEL_BITS)) - 1u);
   uint32_t* out = out_idx + mc->value_base;
-  const KeyOut ko = key_out_of(mc);
+  const KeyOut<K> ko = key_out_of<K>(mc);
   if (low_mask == 0u) {   // equal keys: the bucket is in order already
     for (uint32_t p = threadIdx.x; p < size; p += BLOCK) out[off + p] = rows_in ? rows_in[off + p] : p;
-    if constexpr (KEYS && sizeof(K) == 8) {
+    if constexpr (KEYS) {
       if (ko.p)
         for (uint32_t p = threadIdx.x; p < size; p += BLOCK) ko.p[off + p] = keys_in[off + p] ^ ko.x;
     }
@@ -781,7 +783,7 @@ __device__ __forceinline__ void local_one(const MsdCtl* mc, const Bucket* list, 
     }
   }
   uint32_t r[LI];
-  unsigned long long kv[LI];
+  K kv[LI];
   load_rows<LI>(rows_in, off, src, r);   // every row and key load before the first store
   load_keys<K, LI, KEYS>(ko, keys_in, src, kv);
 #pragma unroll
@@ -826,7 +828,7 @@ __global__ __launch_bounds__(BLOCK) void hyb_group(const MsdCtl* mc, const Bucke
   if (list_overflow(lc, local_cap)) return;   // uniform
   const uint32_t ngroups = lc[LC_GROUPS];
   uint32_t* out = out_idx + mc->value_base;
-  const KeyOut ko = key_out_of(mc);
+  const KeyOut<K> ko = key_out_of<K>(mc);
   for (uint32_t g = blockIdx.x; g < ngroups; g += gridDim.x) {
     const uint32_t idx = local_cap - 1u - g;
     const Bucket bk = list[idx];
@@ -877,7 +879,7 @@ __global__ __launch_bounds__(BLOCK) void hyb_local_lsd(const MsdCtl* mc, const B
     const uint32_t low_mask = mc->active_mask & ((1u << (bk.level & LEVEL_BITS)) - 1u);
     if (bk.size <= uint32_t(LI * BLOCK))   // always: the host sizes LI for every queued bucket
       local_lsd<K, LI, KEYS>(bucket_keys(bk, keys0, keys1), bucket_rows(bk, rows0, rows1), bk.start, bk.size, low_mask, SUB_MAX,
-                       out_idx + mc->value_base, key_out_of(mc), wc, tile_total, bin_start, tmp, s_keys, s_pos);
+                       out_idx + mc->value_base, key_out_of<K>(mc), wc, tile_total, bin_start, tmp, s_keys, s_pos);
     __syncthreads();
   }
 }
@@ -1142,12 +1144,8 @@ bool msd_levels(const MsdWork& w, uint32_t m, int top, uint32_t mask, bool blind
       AM_HIP(hipGetLastError());
     }
   };
-  if constexpr (sizeof(K) == 8) {
-    if (keys) bucket_sorts(std::true_type{});
-    else bucket_sorts(std::false_type{});
-  } else {
-    bucket_sorts(std::false_type{});
-  }
+  if (keys) bucket_sorts(std::true_type{});
+  else bucket_sorts(std::false_type{});
   return true;
 }
 

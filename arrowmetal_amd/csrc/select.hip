@@ -355,7 +355,9 @@ Array* top_k(const Array& a, int64_t k, bool largest, int placement, int forder)
   return out;
 }
 
+// Integer columns that take the hybrid sort get their values from it; others are gathered by their argsort.
 Array* sort_values(const Array& a, bool descending, int placement, int forder) {
+  if (Array* sorted = sorted_ints(a, descending, placement)) return sorted;
   Array* idx = argsort(a, descending, placement, forder);
   Array* out = nullptr;
   try {

@@ -47,6 +47,32 @@ def test_sorted_values_keep_bits(n):
     np.testing.assert_array_equal(got, ints[O.argsort(ints, None, True)])
 
 
+@pytest.mark.parametrize("dtype", [np.int64, np.uint64, np.int32, np.uint32])
+@pytest.mark.parametrize("n", [16_385, 65_535, 65_536, 1_000_003, 5_000_011])
+def test_sorted_integers(dtype, n):
+    """Integer columns whose values come out of the bucket sorts: full-range keys, long runs of equal keys, half
+    of the rows on one key, groups of small buckets, and keys that only the LSD passes take."""
+    rng = np.random.default_rng(n)
+    bits = O.splitmix64(n, n + 5).astype(f"u{np.dtype(dtype).itemsize}").view(dtype)
+    table = bits[:3000]
+    runs = table[rng.integers(0, 3000, n + 5)]
+    half = np.where(rng.random(n + 5) < 0.5, bits, dtype(77))
+    small = rng.integers(0, 250, n + 5).astype(dtype)
+    valid = rng.random(n + 5) > 0.02
+    for k, x in enumerate((bits, runs, half, small)):
+        for va in (None, valid):
+            a = am.MetalArray.from_numpy(x, va).slice(5, n)
+            desc, p = (k + (va is None)) % 2 == 0, k % 2
+            got, gv = a.sort(desc, PLACES[p], "ieee").to_numpy()
+            ok = np.ones(n, bool) if va is None else va[5:]
+            want = np.sort(x[5:][ok])[:: -1 if desc else 1]
+            nulls = n - len(want)
+            at = slice(nulls, n) if p == 1 else slice(0, len(want))
+            np.testing.assert_array_equal(got[at], want)
+            assert (np.ones(n, bool) if gv is None else gv)[at].all()
+            assert nulls == 0 or (gv is not None and (~gv).sum() == nulls)
+
+
 @pytest.mark.parametrize("n,ks", [(1, [1, 2]), (1000, [1, 7, 999, 1000, 5000]),
                                   (300_007, [1, 10, 1000, 65_536, 299_000]),
                                   (2_000_003, [1, 100, 100_000])])
