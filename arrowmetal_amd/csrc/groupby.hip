@@ -4557,7 +4557,7 @@ Array* group_by_dense_ex(const Array& keys, int64_t key_count, long long bias, i
 constexpr long long NOALLOC_MAX_KEYS = 65536;
 constexpr size_t NOALLOC_G8_WORDS = size_t(NXCD) * NOALLOC_MAX_KEYS * 2;
 constexpr size_t NOALLOC_TAB_WORDS = size_t(NOALLOC_MAX_KEYS) * 2;
-constexpr size_t NOALLOC_CTL_WORDS = 32;   // a FoldCtl (zero at load, and zero again after every call)
+constexpr size_t NOALLOC_CTL_WORDS = 32;   // a FoldCtl
 static __device__ __align__(256) unsigned long long scratch[NOALLOC_G8_WORDS + NOALLOC_TAB_WORDS + NOALLOC_CTL_WORDS];
 
 namespace {
@@ -4585,8 +4585,12 @@ void noalloc_run(const AggArgs& a, int kind, int vtype, void* out_values, unsign
                  unsigned long long* out_nulls, unsigned long long* ws, hipStream_t s) {
   unsigned long long* g8 = ws;
   unsigned long long* tab = ws + NOALLOC_G8_WORDS;
+  // Cleared here and not only by its last user: calls that overlapped (and raced) may have left it anywhere.
+  auto* ctl = reinterpret_cast<FoldCtl*>(ws + NOALLOC_G8_WORDS + NOALLOC_TAB_WORDS);
+  hipLaunchKernelGGL(gb_clear_ctl, dim3(1), dim3(1), 0, s, ctl);
+  AM_HIP(hipGetLastError());
   run_agg_into<P>(a, s, "gb_noalloc", g8, tab);
-  const FoldOut fo{out_valid, out_nulls, nullptr, reinterpret_cast<FoldCtl*>(ws + NOALLOC_G8_WORDS + NOALLOC_TAB_WORDS)};
+  const FoldOut fo{out_valid, out_nulls, nullptr, ctl};
   launch_final<P::W>(static_cast<const unsigned long long*>(tab), a.K, FinSimple{kind, vtype, out_values}, fo, s);
 }
 }  // namespace

@@ -2,6 +2,7 @@
 calls in a row on one GPU, the second with fewer rows and fewer groups, every aggregate it takes, and
 its refusals. Outputs go into device buffers the caller owns (arrays imported from NumPy)."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -63,6 +64,27 @@ def test_noalloc_matches_group_by_on_two_calls(agg, vdt):
         assert nulls == int((~wvalid).sum())
         np.testing.assert_array_equal(got[wvalid].view(f"u{got.dtype.itemsize}"),
                                       want[wvalid].view(f"u{want.dtype.itemsize}"))
+
+
+def test_noalloc_alone_after_calls_that_overlapped():
+    """Overlapping calls race for the workspace, and their results with it; the next call alone is right again."""
+    rng = np.random.default_rng(5)
+    forms = []
+    for n, K in ((60_001, 65_536), (70_001, 700)):   # grids of 256 and of 3 workgroups write the results
+        keys, kvalid, v, vvalid = make(rng, n, K, np.int32)
+        forms.append((am.MetalArray.from_numpy(keys, kvalid), K, am.MetalArray.from_numpy(v, vvalid)))
+    threads = [threading.Thread(target=lambda f=f: [noalloc(f[0], f[1], 0, f[2], np.int64) for _ in range(25)])
+               for f in forms]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for ka, K, va in forms * 2:
+        want, wvalid = reference(ka, K, 0, va)
+        got, gvalid, nulls = noalloc(ka, K, 0, va, np.int64)
+        np.testing.assert_array_equal(gvalid, wvalid)
+        assert nulls == int((~wvalid).sum())
+        np.testing.assert_array_equal(got[wvalid], want[wvalid])
 
 
 def test_noalloc_refusals():
