@@ -62,6 +62,11 @@ __device__ __forceinline__ void load_rows(const uint32_t* rows, uint32_t start, 
 constexpr uint32_t LEVEL_BITS = 0xFFu;    // Bucket::level: the level ...
 constexpr uint32_t GROUP_FLAG = 0x100u;   // ... and, in the bucket sort's list, a group of small buckets
 constexpr int SPAN_SHIFT = 12;            // ... whose digits share an aligned window of 1 << (level >> 12)
+// A long run of equal keys leaves in pieces of COPY_MAX rows, so that the whole GPU copies it: one workgroup
+// alone copies about 0.7 rows per ns (32M int32 keys, 30% of them on one value: 14.0 ms, 1.05 ms in pieces).
+// Every piece but the first has CONT_FLAG: the row before it is in its buffer and has the same key.
+constexpr uint32_t COPY_MAX = 4096;
+constexpr uint32_t CONT_FLAG = 0x200u;
 struct LvlChunk {
   uint32_t bucket, start, end, pad;
 };
@@ -144,6 +149,35 @@ __device__ __forceinline__ void push_local(Bucket* local, uint32_t local_cap, ui
 __device__ __forceinline__ bool list_overflow(const uint32_t* lc, uint32_t local_cap) {
   return lc[LC_OVERFLOW] != 0u || uint64_t(lc[LC_LOCAL]) + lc[LC_GROUPS] > local_cap;
 }
+
+// The entries a copy of `rows` rows of buffer `buf` leaves as. (Implicit rows count from their batch's start,
+// so such a copy stays whole.)
+__device__ __forceinline__ uint32_t copy_pieces(uint32_t rows, uint32_t buf) {
+  return buf == BUF_IMPLICIT ? 1u : rows / COPY_MAX + (rows % COPY_MAX != 0u ? 1u : 0u);
+}
+
+// The copies of more than one piece that a workgroup has found (in LDS, count 0 at first); the workgroup
+// writes their entries together.
+struct LongCopies {
+  uint32_t count, start[RADIX], rows[RADIX], at[RADIX];
+  __device__ __forceinline__ void add(uint32_t first, uint32_t size, uint32_t entry) {
+    const uint32_t k = atomicAdd(&count, 1u);
+    start[k] = first;
+    rows[k] = size;
+    at[k] = entry;
+  }
+  // After a barrier, by every thread; the entries start at `base` + at[k] of the list.
+  __device__ __forceinline__ void write(Bucket* local, uint32_t local_cap, uint32_t base, uint32_t buf, uint32_t level) const {
+    for (uint32_t k = 0; k < count; k++) {
+      const uint32_t pieces = copy_pieces(rows[k], buf);
+      for (uint32_t p = threadIdx.x; p < pieces; p += BLOCK) {
+        const uint32_t off = p * COPY_MAX, entry = base + at[k] + p;
+        if (entry < local_cap)
+          local[entry] = Bucket{start[k] + off, min(COPY_MAX, rows[k] - off), buf, level | (p != 0u ? CONT_FLAG : 0u)};
+      }
+    }
+  }
+};
 
 // One workgroup: where each large bucket's chunks and tiles start in a level's tables (list `cur`
 // order; bofs[2b], bofs[2b + 1]); the other list's counter, the tile counter and the row count reset.
@@ -281,7 +315,7 @@ __device__ __forceinline__ uint32_t block_incl_max(uint32_t v, uint32_t* tmp) {
 // below d), or to the next level's list. A bucket whose rows all share digit d (every bucket, when
 // digit d is inactive) is carried (carried[b] = 1): it keeps its buffer and the pass skips it.
 // Neighbouring sub-buckets are adjacent in memory and in key order, so several leave as one entry:
-// - a run of sub-buckets of equal keys, as one copy;
+// - a run of sub-buckets of equal keys, as one copy (in pieces of COPY_MAX rows);
 // - sub-buckets of at most small_max rows, as a group: the sub-buckets of the widest aligned window of
 //   digits (1, 2, 4, 8 or GROUP_SPAN values) around each that holds at most group_max rows and only
 //   such sub-buckets, sorted together by the digits from d down (level d + 1).
@@ -295,6 +329,7 @@ __global__ __launch_bounds__(BLOCK) void lvl_plan(const Bucket* large, int cur, 
   __shared__ uint32_t tmp[WAVES];
   __shared__ uint2 s_sub[RADIX];   // (rows, start) of each non-empty sub-bucket of equal keys
   __shared__ uint32_t s_base[3];   // where this bucket's entries go in the three lists
+  __shared__ LongCopies s_long;
   const uint32_t nb = lc[LC_LIST + cur];
   const uint32_t mask = mc->active_mask;
   const bool active = (mask >> d) & 1u;
@@ -304,6 +339,7 @@ __global__ __launch_bounds__(BLOCK) void lvl_plan(const Bucket* large, int cur, 
     const Bucket bk = large[b];
     uint32_t v, base;
     bool carry;
+    if (threadIdx.x == 0) s_long.count = 0u;
     if (active) {
       v = bucket_hist[size_t(b) * RADIX + threadIdx.x];
       uint32_t total;
@@ -370,7 +406,8 @@ __global__ __launch_bounds__(BLOCK) void lvl_plan(const Bucket* large, int cur, 
     // Every entry of this bucket into its list with one counter bump per list.
     const bool single = kind == SUB_SINGLE, to_next = kind == SUB_LARGE;
     uint32_t n_local, n_group, n_next, n_rows;
-    const uint32_t r_local = block_excl_scan((single ? 1u : 0u) + (copy_end ? 1u : 0u), tmp, n_local);
+    const uint32_t pieces = copy_end ? copy_pieces(copy_rows, buf) : 0u;
+    const uint32_t r_local = block_excl_scan((single ? 1u : 0u) + pieces, tmp, n_local);
     const uint32_t r_group = block_excl_scan(group_head ? 1u : 0u, tmp, n_group);
     const uint32_t r_next = block_excl_scan(to_next ? 1u : 0u, tmp, n_next);
     block_excl_scan(to_next ? v : 0u, tmp, n_rows);
@@ -382,13 +419,13 @@ __global__ __launch_bounds__(BLOCK) void lvl_plan(const Bucket* large, int cur, 
       if (n_rows) atomicAdd(&lc[LC_ROWS], n_rows);
     }
     if (threadIdx.x == BLOCK - 1 && biggest) atomicMax(&lc[LC_MAXLOCAL], biggest);
+    const uint32_t r_copy = r_local + (single ? 1u : 0u);
+    if (pieces > 1u) s_long.add(copy_start, copy_rows, r_copy);
     __syncthreads();
-    uint32_t at = s_base[0] + r_local;
-    if (single) {
-      if (at < local_cap) local[at] = Bucket{base, v, buf, uint32_t(d)};
-      at++;
-    }
-    if (copy_end && at < local_cap) local[at] = Bucket{copy_start, copy_rows, buf, 0u};   // level 0: no digit left
+    if (single && s_base[0] + r_local < local_cap) local[s_base[0] + r_local] = Bucket{base, v, buf, uint32_t(d)};
+    if (pieces == 1u && s_base[0] + r_copy < local_cap)
+      local[s_base[0] + r_copy] = Bucket{copy_start, copy_rows, buf, 0u};   // level 0: no digit left
+    s_long.write(local, local_cap, s_base[0], buf, 0u);
     if (group_head) {
       const uint32_t g = s_base[1] + r_group;
       if (g < local_cap)
@@ -707,7 +744,7 @@ __device__ __forceinline__ bool local_group(const K* keys_in, const uint32_t* ro
 // digit in a byte beside it; inside a run, words order as the pairs do, and a row's place there is the
 // number of words below its own. A bucket whose words would not fit 64 bits (top = 7), or with a run
 // longer than SUB_MAX rows, is queued for hyb_local_lsd instead. A bucket of equal keys (no varying
-// digit left), of any size, is copied.
+// digit left) is copied.
 template <typename K, int LI, bool KEYS>
 __device__ __forceinline__ void local_one(const MsdCtl* mc, const Bucket* list, uint32_t idx, const K* keys0,
                                           const uint32_t* rows0, const K* keys1, const uint32_t* rows1,
@@ -889,7 +926,7 @@ __global__ __launch_bounds__(BLOCK) void hyb_local_lsd(const MsdCtl* mc, const B
 // workgroup in turn, in place of sorting them. The rows of an entry with digits left are in input order
 // inside each key, so of the positions with one key the lowest is its first row: a table of positions in
 // LDS (linear probing; twice the rows, a power of two), each slot kept at the lowest of its key. An entry
-// without digits left is runs of equal keys, each in input order. Dynamic LDS: li * BLOCK keys, then twice
+// without digits left is runs of equal keys, each in input order, or a later piece of one. Dynamic LDS: li * BLOCK keys, then twice
 // as many 32-bit slots.
 template <typename K>
 __global__ __launch_bounds__(BLOCK) void hyb_dedupe(const MsdCtl* mc, const Bucket* list, uint32_t local_cap, uint32_t li,
@@ -906,8 +943,9 @@ __global__ __launch_bounds__(BLOCK) void hyb_dedupe(const MsdCtl* mc, const Buck
     const uint32_t* rows = bucket_rows(bk, rows0, rows1) + bk.start;   // never implicit rows here
     const uint32_t size = bk.size;
     if ((mc->active_mask & ((1u << (bk.level & LEVEL_BITS)) - 1u)) == 0u) {
-      for (uint32_t p = 1u + threadIdx.x; p < size; p += BLOCK)
-        if (keys[p] == keys[p - 1u]) dup[rows[p]] = 1u;
+      const K* before = keys - 1;   // before[0] is read by a later piece only, and is a key of its run
+      for (uint32_t p = (bk.level & CONT_FLAG ? 0u : 1u) + threadIdx.x; p < size; p += BLOCK)
+        if (keys[p] == before[p]) dup[rows[p]] = 1u;
       continue;
     }
     if (size > li * BLOCK) continue;   // never: li covers every bucket
@@ -948,8 +986,8 @@ __global__ __launch_bounds__(BLOCK) void hyb_dedupe(const MsdCtl* mc, const Buck
 // (the tile tables are sized for that many or more), and extra_local more entries in the bucket
 // sort's list (a batched plan's batches).
 // Capacities: buckets above LOCAL_MAX / 2 rows at one level (the least local_max used); entries of the
-// bucket sort's list (every entry has a row, and runs of many tiny buckets are what fills it); chunks
-// and tiles of a level.
+// bucket sort's list (every entry has a row, and runs of many tiny buckets are what fills it; a long copy's
+// pieces come on top); chunks and tiles of a level.
 struct MsdWork {
   uint32_t large_cap = 0, local_cap = 0;
   DevBuf lists, tabs, words, wide;
@@ -967,7 +1005,7 @@ inline MsdWork msd_work(uint32_t m, int items, DevBuf (*alloc)(size_t), uint32_t
   MsdWork w;
   const uint32_t tile = uint32_t(BLOCK * items);
   w.large_cap = m / (LOCAL_MAX / 2) + 4096u;
-  w.local_cap = m / 32u + (1u << 17) + extra_local;
+  w.local_cap = m / 32u + (1u << 17) + m / COPY_MAX + extra_local;
   // ARROWMETAL_MSD_LIST_CAP (tests only) caps the bucket-sort list, so that a test can send a sort down
   // the overflow path: the plain argsort falls back to the LSD passes, a batched plan to its segmented
   // LSD passes.

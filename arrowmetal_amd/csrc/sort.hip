@@ -675,6 +675,7 @@ __global__ __launch_bounds__(BLOCK) void msd_unit_scan(SortCtl* ctl, uint32_t* u
   __shared__ uint32_t tmp[WAVES];
   __shared__ uint32_t s_last, s_mask, s_first[NBINS_FIRST];
   __shared__ UpStat s_st[WAVES];
+  __shared__ LongCopies s_long;
   const uint32_t b = blockIdx.x;
   uint32_t* h = unit_hist + size_t(b) * nunits;
   uint32_t carry = 0;
@@ -712,6 +713,7 @@ __global__ __launch_bounds__(BLOCK) void msd_unit_scan(SortCtl* ctl, uint32_t* u
     for (int p = 0; p < P; p++)
       if ((diff >> (8 * p)) & 0xFFull) mask |= 1u << p;
     s_mask = mask;
+    s_long.count = 0u;
     const uint32_t value_base = nulls_first ? st.z + st.q : 0u;
     s_first[BIN_NAN] = nulls_first ? st.z : st.m;
     s_first[BIN_NULL] = nulls_first ? 0u : st.m + st.q;
@@ -727,13 +729,17 @@ __global__ __launch_bounds__(BLOCK) void msd_unit_scan(SortCtl* ctl, uint32_t* u
   const uint32_t low = s_mask & ((1u << (P - 1)) - 1u);
   const bool is_large = size > LOCAL_MAX && low != 0u, is_local = size != 0u && !is_large;
   const Bucket bk{start, size, 0u, uint32_t(P - 1)};
+  const uint32_t pieces = !is_local ? 0u : low == 0u ? copy_pieces(size, 0u) : 1u;   // without a lower digit: copies
   uint32_t n_large, n_local;
   const uint32_t at_large = block_excl_scan(is_large ? 1u : 0u, tmp, n_large);
-  const uint32_t at_local = block_excl_scan(is_local ? 1u : 0u, tmp, n_local);
+  const uint32_t at_local = block_excl_scan(pieces, tmp, n_local);
   const uint32_t biggest = block_incl_max(is_local && low != 0u ? size : 0u, tmp);
   const uint32_t top = block_incl_max(size, tmp);
   if (is_large) large[at_large] = bk;
-  if (is_local && at_local < local_cap) local[at_local] = bk;
+  if (pieces == 1u && at_local < local_cap) local[at_local] = bk;
+  if (pieces > 1u) s_long.add(start, size, at_local);
+  __syncthreads();
+  s_long.write(local, local_cap, 0u, 0u, uint32_t(P - 1));
   if (threadIdx.x == BLOCK - 1) {
     lc[LC_LIST] = n_large;
     lc[LC_LOCAL] = n_local;

@@ -3,6 +3,7 @@ CPU oracle, bit-exact, on the sizes and key shapes of the reference's own suites
 (Tests/ArrowMetalTests/RadixSortScaleTests.swift:28-201, SortOptionsTests.swift, SortTests.swift)."""
 import json
 import os
+import time
 
 import numpy as np
 import pytest
@@ -216,6 +217,59 @@ def test_hybrid_sort_of_each_key_type(dtype, n, shape, path):
         names = set(am.prof_report())
         assert ("sort_msd_first" in names) == (path == "msd"), names
         np.testing.assert_array_equal(got, O.argsort(vals, va, desc, place, 0))
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.uint64])
+@pytest.mark.parametrize("shape", ["runs", "top_digit_only"])
+def test_runs_of_equal_keys_at_the_edges_of_a_copy(dtype, shape):
+    """Runs of equal keys leave the sort as copies of 4,096 rows each: runs of about that many rows and of
+    several times as many, among keys that are all different, and keys that differ in their top digit alone."""
+    rng = np.random.default_rng(3)
+    bits = 8 * np.dtype(dtype).itemsize
+    lens = [4095, 4096, 4097, 8191, 8192, 8193, 50_000, 1, 2]
+    keys = O.splitmix64(11, len(lens)) >> np.uint64(64 - bits)
+    if shape == "top_digit_only":
+        keys = np.arange(1, len(lens) + 1, dtype=np.uint64) << np.uint64(bits - 5)
+        x = np.repeat(keys, lens)
+    else:
+        x = np.concatenate([np.repeat(keys, lens), O.splitmix64(12, 60_000) >> np.uint64(64 - bits)])
+    x = rng.permutation(x).astype(f"u{bits // 8}").view(dtype)
+    valid = rng.random(len(x)) > 0.01
+    for va, desc, place in ((None, False, 0), (valid, True, 1)):
+        a = am.MetalArray.from_numpy(x, va)
+        want = O.argsort(x, va, desc, place, 0)
+        got, names = sort_with_kernels(x, va, desc, place, 0)
+        assert "sort_msd_local" in names, sorted(names)
+        np.testing.assert_array_equal(got, want)
+        ok = np.ones(len(x), bool) if va is None else va
+        vals, gv = a.sort(desc, am.NULL_PLACEMENTS[place]).to_numpy()
+        gv = np.ones(len(x), bool) if gv is None else gv
+        np.testing.assert_array_equal(gv, ok[want])
+        np.testing.assert_array_equal(vals[gv], x[want][gv])
+        np.testing.assert_array_equal(am.unique_rows([a]).to_numpy()[0], O.unique_rows([x], [va]))
+
+
+@pytest.mark.parametrize("call", ["argsort", "sort", "unique"])
+def test_a_hot_value_costs_no_more_than_the_rest(call):
+    """30% of 32M int32 rows on one value: about the time of the column without it (a lone workgroup copying
+    the value's rows would take ten times as long)."""
+    n = 32_000_000
+    rng = np.random.default_rng(1)
+    x = rng.integers(-2**31, 2**31 - 1, n, dtype=np.int32)
+    hot = np.where(rng.random(n) < 0.3, np.int32(12345), x)
+    times = []
+    for col in (x, hot):
+        a = am.MetalArray.from_numpy(col)
+        run = (lambda: am.unique_rows([a])) if call == "unique" else getattr(a, call)
+        run()
+        t = []
+        for _ in range(5):
+            t0 = time.perf_counter()
+            run()
+            t.append(time.perf_counter() - t0)
+        times.append(min(t))
+    print(call, [f"{t * 1e6:.0f} us" for t in times], flush=True)
+    assert times[1] < 3 * times[0]
 
 
 # ---------------------------------------------------------------- take
