@@ -166,6 +166,7 @@ _SIGNATURES = {
                                ctypes.c_int),
     "am_stream_result_release": ([_P], None),
     "am_set_max_row_index": ([ctypes.c_int64], ctypes.c_int64),
+    "am_fail_alloc": ([ctypes.c_int64], ctypes.c_int64),
     "am_prof_enable": ([ctypes.c_int], ctypes.c_int),
     "am_prof_reset": ([], ctypes.c_int),
     "am_prof_report": ([ctypes.c_char_p, ctypes.c_int64], ctypes.c_int64),
@@ -828,6 +829,12 @@ def set_max_row_index(max_row):
     """Test hook (the reference's Dispatch.maxRowIndex): the largest row number index-returning calls
     may produce; None or an out-of-range value restores 2^32 - 1. Returns the previous limit."""
     return lib().am_set_max_row_index(-1 if max_row is None else int(max_row))
+
+
+def fail_alloc(k=0):
+    """Test hook: the k-th allocation of device memory from now on fails once (0: none does). Returns what
+    was left of the previous count: above 0, no allocation has failed."""
+    return lib().am_fail_alloc(int(k))
 
 
 def prof_enable(on=True):

@@ -37,6 +37,10 @@ namespace am {
 struct Error : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
+// Device memory ran out: a caller that has a form with less scratch takes that one.
+struct OutOfMemory : Error {
+  using Error::Error;
+};
 [[noreturn]] void fail(const std::string& msg);
 // The reference's error texts (ArrowMetalError.description, Sources/ArrowMetal/MetalContext.swift:19-31):
 // "Invalid ArrowArray: <msg>", "Unsupported Arrow type: <msg>", "Array length mismatch: <a> vs <b>".
@@ -109,6 +113,11 @@ using DevBuf = std::shared_ptr<DevBlock>;
 // The pool never hands a block back to the driver while the process runs, so steady-state calls
 // allocate nothing from HIP.
 DevBuf device_alloc(size_t bytes);
+// Memory outside the pool, for as long as the calling thread lives (its counters and tables).
+DevBuf device_alloc_thread(size_t bytes);
+// Test hook: the k-th allocation of device memory from now on fails (0: none does). Returns what was left
+// of the previous count.
+int64_t fail_alloc(int64_t k);
 // A view of memory owned elsewhere (zero-copy device import); `release` runs when the view dies.
 DevBuf device_wrap(void* ptr, size_t bytes, std::function<void(void*)> release);
 // Bytes the pool holds (in use + cached), for admission control and tests.

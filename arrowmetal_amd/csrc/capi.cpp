@@ -552,6 +552,7 @@ int am_group_by_noalloc(am_array* keys, int64_t key_count, int agg, am_array* va
 }
 
 int64_t am_set_max_row_index(int64_t max_row) { return am::set_max_row_index(max_row); }
+int64_t am_fail_alloc(int64_t k) { return am::fail_alloc(k); }
 
 int am_prof_enable(int on) {
   am::prof_enable(on != 0);

@@ -467,10 +467,8 @@ __global__ void gb_clear_ctl(FoldCtl* c) { *c = FoldCtl{0, 0, 0, 0}; }
 FoldCtl* fold_ctl() {
   thread_local DevBuf buf;
   if (!buf) {
-    void* p = nullptr;
-    AM_HIP(hipMalloc(&p, sizeof(FoldCtl)));
-    buf = device_wrap(p, sizeof(FoldCtl), [](void* q) { (void)hipFree(q); });
-    hipLaunchKernelGGL(gb_clear_ctl, dim3(1), dim3(1), 0, stream(), static_cast<FoldCtl*>(p));
+    buf = device_alloc_thread(sizeof(FoldCtl));
+    hipLaunchKernelGGL(gb_clear_ctl, dim3(1), dim3(1), 0, stream(), static_cast<FoldCtl*>(buf->ptr));
     AM_HIP(hipGetLastError());
   }
   retain(buf);

@@ -37,7 +37,9 @@ const char* last_error_cstr() { return t_last_error.c_str(); }
 void hip_check(hipError_t e, const char* what) {
   if (e != hipSuccess) {
     (void)hipGetLastError();
-    throw Error(std::string("HIP error ") + hipGetErrorName(e) + " (" + hipGetErrorString(e) + ") in " + what);
+    const std::string msg = std::string("HIP error ") + hipGetErrorName(e) + " (" + hipGetErrorString(e) + ") in " + what;
+    if (e == hipErrorOutOfMemory) throw OutOfMemory(msg);
+    throw Error(msg);
   }
 }
 
@@ -184,7 +186,30 @@ DevBlock::~DevBlock() {
   else pool_free(ptr, bytes, owner);
 }
 
+namespace {
+std::atomic<int64_t> g_fail_alloc{0};   // allocations up to the one that fails; 0: none
+[[noreturn]] void out_of_memory(size_t bytes) {
+  throw OutOfMemory("out of device memory allocating " + std::to_string(bytes) + " bytes");
+}
+void check_fail_alloc(size_t bytes) {
+  if (g_fail_alloc.load(std::memory_order_relaxed) > 0 && g_fail_alloc.fetch_sub(1) == 1) out_of_memory(bytes);
+}
+}  // namespace
+
+int64_t fail_alloc(int64_t k) { return g_fail_alloc.exchange(std::max<int64_t>(k, 0)); }
+
+DevBuf device_alloc_thread(size_t bytes) {
+  check_fail_alloc(bytes);
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    out_of_memory(bytes);
+  }
+  return device_wrap(p, bytes, [](void* q) { (void)hipFree(q); });
+}
+
 DevBuf device_alloc(size_t bytes) {
+  check_fail_alloc(bytes);
   size_t cls = size_class(bytes ? bytes : 1);
   Pool& P = pool();
   hipStream_t s = stream();
@@ -202,7 +227,7 @@ DevBuf device_alloc(size_t bytes) {
       e = hipMalloc(&ptr, cls);
       if (e != hipSuccess) {
         (void)hipGetLastError();
-        fail("out of device memory allocating " + std::to_string(bytes) + " bytes");
+        out_of_memory(bytes);
       }
     }
     std::lock_guard<std::mutex> g(P.mu);

@@ -860,10 +860,8 @@ __global__ __launch_bounds__(BLOCK, 3) void msd_part(const void* vals, const uin
 uint32_t* scan_ticket(hipStream_t s) {
   thread_local DevBuf buf;
   if (!buf) {
-    void* p = nullptr;
-    AM_HIP(hipMalloc(&p, 128));
-    buf = device_wrap(p, 128, [](void* q) { (void)hipFree(q); });
-    hipLaunchKernelGGL(fill_u64, dim3(1), dim3(64), 0, s, static_cast<unsigned long long*>(p), size_t(16), 0ull);
+    buf = device_alloc_thread(128);
+    hipLaunchKernelGGL(fill_u64, dim3(1), dim3(64), 0, s, static_cast<unsigned long long*>(buf->ptr), size_t(16), 0ull);
     AM_HIP(hipGetLastError());
   }
   retain(buf);

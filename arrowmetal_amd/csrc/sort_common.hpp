@@ -377,12 +377,12 @@ uint32_t reserve_status(size_t entries, hipStream_t s) {
     size_t want = std::max(entries, t_ws.entries);
     // Allocated outside the pool's batch retention: the table lives as long as the thread.
     t_ws.status.reset();
-    void* p = nullptr;
-    AM_HIP(hipMalloc(&p, want * 8));
-    t_ws.status = device_wrap(p, want * 8, [](void* q) { (void)hipFree(q); });
+    t_ws.entries = 0;   // no table, should the allocation fail
+    t_ws.status = device_alloc_thread(want * 8);
     t_ws.entries = want;
     int blocks = int(std::min<size_t>((want + 255) / 256, 4096));
-    hipLaunchKernelGGL(fill_u64, dim3(blocks), dim3(256), 0, s, static_cast<unsigned long long*>(p), want, 0ull);
+    hipLaunchKernelGGL(fill_u64, dim3(blocks), dim3(256), 0, s, static_cast<unsigned long long*>(t_ws.status->ptr),
+                       want, 0ull);
     AM_HIP(hipGetLastError());
     t_ws.epoch = 1;
   }

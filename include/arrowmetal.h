@@ -347,6 +347,11 @@ void am_server_release(am_server* s);
  * Process-wide. */
 int64_t am_set_max_row_index(int64_t max_row);
 
+/* Test hook: the k-th allocation of device memory from now on fails once, as if there were none left; 0:
+ * none does. Calls that have a form with less scratch take it, others fail with "out of device memory
+ * ...". Returns what was left of the previous count. Process-wide. */
+int64_t am_fail_alloc(int64_t k);
+
 /* Kernel timing of the library's own launches, measured with HIP events on the stream each kernel
  * is launched on. am_prof_report writes "name count total_ms\n" lines into buf (NUL-terminated) and
  * returns the number of bytes needed. */
