@@ -4087,7 +4087,7 @@ bool map_composite(Array* const* columns, int64_t count, int64_t n, std::vector<
   DevBuf comp;
   try {
     comp = write_composite<false>(ca, top, n);
-  } catch (const Error&) {   // no room for the composite keys: column by column
+  } catch (const OutOfMemory&) {   // no room for the composite keys: column by column
     return false;
   }
   const RangeStat known{0ull, top - 1ull, 0ull, 0u, 0u};
@@ -4670,7 +4670,7 @@ Array* unique_rows(Array* const* columns, int64_t count) {
       try {   // up to 37 bytes a row of scratch: without that room the hash path takes the call
         const DevBuf keys = write_composite<true>(ca, top, n);
         found = distinct_rows(keys->ptr, composite_narrow(top) ? 4 : 8, uint32_t(n), rows, kept);
-      } catch (const Error&) {
+      } catch (const OutOfMemory&) {
       }
       if (found) {
         Array* out = new_array("I", T_U32, int64_t(kept));

@@ -351,7 +351,7 @@ bool launch_take_slices(const Array& a, const Array& ix, Array* out, TakeStatus*
     pp = device_alloc(size_t(n) * 2);
     pv = device_alloc(size_t(n) * sizeof(V));
     ob = device_alloc(size_t(TK_SLICES + 1) * tiles * 4);
-  } catch (const Error&) {
+  } catch (const OutOfMemory&) {
     return false;
   }
   auto* ctl = static_cast<TkCtl*>(cb->ptr);
@@ -613,7 +613,7 @@ bool permute_columns(const std::vector<const Array*>& cols, const Array& idx, st
       DevBuf rows;
       try {
         rows = device_alloc(size_t(n) * p.words * 8u);
-      } catch (const Error&) {   // no room: column by column, which needs none
+      } catch (const OutOfMemory&) {   // no room: column by column, which needs none
         for (Array* a : out) release_array(a);
         out.clear();
         return false;

@@ -50,3 +50,63 @@ def test_a_thread_whose_table_could_not_be_had():
         if not outcomes[-1][0]:
             break
     assert not outcomes[-1][0] and len(outcomes) > 6, outcomes
+
+
+def wide_pair(n):
+    rng = np.random.default_rng(7)
+    return [rng.integers(-2**40, 2**40, n)[rng.integers(0, n, n)], rng.integers(0, 7, n).astype(np.int16)]
+
+
+def unique_two():
+    cols = wide_pair(200_003)
+    want = O.unique_rows(cols, [None, None])
+    arrays = [am.MetalArray.from_numpy(c) for c in cols]
+    return lambda: am.unique_rows(arrays), lambda r: np.testing.assert_array_equal(r.to_numpy()[0], want)
+
+
+def group_two():
+    cols = wide_pair(200_003)
+    ids, K, _ = O.group_keys(cols, [None, None])
+    arrays = [am.MetalArray.from_numpy(c) for c in cols]
+
+    def check(g):
+        assert g.group_count == K
+        np.testing.assert_array_equal(g.ids().to_numpy()[0], ids)
+    return lambda: am.group_by(arrays), check
+
+
+def take_random():
+    n = 3 << 22
+    x = O.splitmix64(3, n)
+    at = np.random.default_rng(3).integers(0, n, n).astype(np.uint32)
+    a, ix = am.MetalArray.from_numpy(x), am.MetalArray.from_numpy(at)
+    return lambda: a.take(ix), lambda r: np.testing.assert_array_equal(r.to_numpy()[0], x[at])
+
+
+def table():
+    n = 100_003
+    rng = np.random.default_rng(9)
+    t = {"k": rng.standard_normal(n), "a": rng.integers(0, 9, n), "b": rng.integers(0, 99, n).astype(np.int16)}
+    at = O.argsort(t["k"], None)
+    src = am.PlanSource("t", {c: am.MetalArray.from_numpy(v) for c, v in t.items()})
+    plan = {"op": "sort", "by": [["k", False]], "input": {"op": "scan", "source": "t"}}
+
+    def check(got):
+        for c, v in t.items():
+            np.testing.assert_array_equal(got[c].to_numpy()[0], v[at])
+    return lambda: am.plan_run(plan, [src]), check
+
+
+# call, and how many of its allocations it can do without (their scratch has a form that needs less).
+@pytest.mark.parametrize("make,spared", [(unique_two, 14), (group_two, 1), (take_random, 5), (table, 1)])
+def test_calls_with_a_form_that_needs_less_scratch(make, spared):
+    call, check = make()
+    check(call())
+    outcomes = []
+    for k in range(1, 200):
+        outcomes.append(failing(call, check, k))
+        check(call())
+        if not outcomes[-1][0]:
+            break
+    assert not outcomes[-1][0], "more allocations than expected"
+    assert sum(done for hit, done in outcomes if hit) >= spared, outcomes
