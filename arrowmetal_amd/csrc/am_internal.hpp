@@ -235,7 +235,8 @@ void argsort_device(const void* vals, int type, const uint8_t* validity, int64_t
 bool distinct_rows(const void* keys, int width, uint32_t n, DevBuf& rows, uint32_t& kept);
 
 // The sorted values of an int32, uint32, int64 or uint64 column of at least the hybrid sort's rows, whose
-// bucket sorts write them; nullptr for any other column (and in a graph capture): argsort and take.
+// bucket sorts write them; nullptr for any other column, in a graph capture and without room for the values
+// beside the sort's scratch: argsort and take.
 Array* sorted_ints(const Array& a, bool descending, int null_placement);
 
 // ORDER BY of a whole table by one 64-bit key (int64 / uint64 / float64): every column of `cols`

@@ -893,8 +893,8 @@ uint32_t hybrid_min(int type) {
 // The analysis of the hybrid sort: units counted and scanned, the plan on its way to host_plan_words().
 struct Units {
   DevBuf buf;
-  uint32_t* hist;   // [NBINS_FIRST][count], each bin's running offsets
-  uint32_t count, shift;
+  uint32_t* hist = nullptr;   // [NBINS_FIRST][count], each bin's running offsets
+  uint32_t count = 0, shift = 0;
 };
 
 template <typename K, int W>
@@ -960,10 +960,19 @@ bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
   uint32_t digits = (1u << P) - 1u;
   bool planned = false, tried = false;   // analysed; partitioned (the control block is used up)
   MsdPlan plan{};
-  if (hybrid_ok) {
-    const MsdWork w = msd_work(n, ITEMS, device_alloc);
-    const Units un = msd_analyse<K, W>(vals, type, valid, voff, n, dsc, placement, forder, ctl, w, epoch, key_out, key_xor,
-                                       bucket_base, s);
+  MsdWork w;
+  Units un;
+  bool hybrid = hybrid_ok;
+  if (hybrid) {
+    try {   // some 3 bytes a row beside the buffers above, without which the LSD passes sort
+      w = msd_work(n, ITEMS, device_alloc);
+      un = msd_analyse<K, W>(vals, type, valid, voff, n, dsc, placement, forder, ctl, w, epoch, key_out, key_xor,
+                             bucket_base, s);
+    } catch (const OutOfMemory&) {
+      hybrid = false;
+    }
+  }
+  if (hybrid) {
     const uint32_t nunits = un.count, unit_shift = un.shift;
     uint32_t* unit_hist = un.hist;
     MsdPlan* hp = reinterpret_cast<MsdPlan*>(host_plan_words());
@@ -1442,7 +1451,10 @@ Array* sorted_ints_t(const Array& a, bool desc, int placement, Array* idx, hipSt
   run_sort<K, W, ITEMS>(a.data(), a.type, a.has_nulls() ? a.valid_bits() : nullptr, a.offset, n, desc, placement, 0,
                         static_cast<uint32_t*>(idx->values->ptr), s, nullptr, &m, nullptr, values->ptr,
                         (unsigned long long)(flip), &written);
-  if (!written) return take(a, *idx);   // the LSD passes sorted the rows only
+  if (!written) {   // the LSD passes sorted the rows only
+    values.reset();
+    return take(a, *idx);
+  }
   Array* out = new_array(a.format, a.type, a.length);
   try {
     out->values = values;
@@ -1552,10 +1564,14 @@ Array* sorted_ints(const Array& a, bool descending, int null_placement) {
     Array* a;
     ~Drop() { release_array(a); }
   } drop{idx};
-  idx->values = device_alloc(size_t(a.length) * 4);
-  idx->null_count = 0;
-  return a.width() == 8 ? sorted_ints_t<unsigned long long>(a, descending, null_placement, idx, stream())
-                        : sorted_ints_t<uint32_t>(a, descending, null_placement, idx, stream());
+  try {
+    idx->values = device_alloc(size_t(a.length) * 4);
+    idx->null_count = 0;
+    return a.width() == 8 ? sorted_ints_t<unsigned long long>(a, descending, null_placement, idx, stream())
+                          : sorted_ints_t<uint32_t>(a, descending, null_placement, idx, stream());
+  } catch (const OutOfMemory&) {   // the values beside the sort's scratch; an argsort and a take hold them apart
+    return nullptr;
+  }
 }
 
 bool order_by_columns(const Array& key, bool descending, int null_placement, int float_order,

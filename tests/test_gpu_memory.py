@@ -97,8 +97,30 @@ def table():
     return lambda: am.plan_run(plan, [src]), check
 
 
+def sorted_values():
+    x = O.splitmix64(3, 100_003).astype(np.uint32).view(np.int32)
+    valid = np.random.default_rng(2).random(len(x)) > 0.1
+    a = am.MetalArray.from_numpy(x, valid)
+    want = x[O.argsort(x, valid)]
+
+    def check(r):
+        got, gv = r.to_numpy()
+        m = int(valid.sum())
+        assert gv[:m].all() and not gv[m:].any()
+        np.testing.assert_array_equal(got[:m], want[:m])
+    return a.sort, check
+
+
+def argsort_i32():
+    x = O.splitmix64(4, 100_003).astype(np.uint32).view(np.int32)
+    a = am.MetalArray.from_numpy(x)
+    want = O.argsort(x, None)
+    return a.argsort, lambda r: np.testing.assert_array_equal(r.to_numpy()[0], want)
+
+
 # call, and how many of its allocations it can do without (their scratch has a form that needs less).
-@pytest.mark.parametrize("make,spared", [(unique_two, 14), (group_two, 1), (take_random, 5), (table, 1)])
+@pytest.mark.parametrize("make,spared", [(sorted_values, 12), (argsort_i32, 5),
+                                         (unique_two, 14), (group_two, 1), (take_random, 5), (table, 1)])
 def test_calls_with_a_form_that_needs_less_scratch(make, spared):
     call, check = make()
     check(call())
