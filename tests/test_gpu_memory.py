@@ -4,6 +4,7 @@ import threading
 
 import numpy as np
 import pytest
+import torch
 
 import arrowmetal_amd as am
 import oracle_py as O
@@ -50,6 +51,17 @@ def test_a_thread_whose_table_could_not_be_had():
         if not outcomes[-1][0]:
             break
     assert not outcomes[-1][0] and len(outcomes) > 6, outcomes
+
+
+def test_unique_rows_hold_the_kept_rows_only():
+    n = 10_000_000
+    rng = np.random.default_rng(4)
+    a = am.MetalArray.from_numpy(rng.integers(-2**62, 2**62, 1000)[rng.integers(0, 1000, n)])
+    held = [am.unique_rows([a])]
+    before = torch.cuda.mem_get_info()[0]
+    held += [am.unique_rows([a]) for _ in range(40)]
+    assert all(len(r) == 1000 for r in held)
+    assert before - torch.cuda.mem_get_info()[0] < 200 << 20
 
 
 def wide_pair(n):
