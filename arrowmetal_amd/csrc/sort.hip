@@ -1195,25 +1195,25 @@ bool distinct_rows_t(const void* keys, uint32_t n, DevBuf& rows, uint32_t& kept,
   if (!msd_levels<K, ITEMS>(w, plan.m, W - 1, plan.mask, false, LOCAL_MAX, status, kp0, rp0, kp1, rp1, nullptr, s, false,
                             &plan.large, &plan.biggest, &plan.local, dup))
     return false;
-  DevBuf base = device_alloc(size_t(tiles) * 4);
+  DevBuf all = device_alloc(size_t(n) * 4), base = device_alloc(size_t(tiles) * 4);
   std::shared_ptr<void> slot = pinned_slot();
   auto* total = static_cast<uint32_t*>(slot.get());
   {
     ProfScope ps("keep_rows");
     hipLaunchKernelGGL(keep_count, dim3(tiles), dim3(BLOCK), 0, s, static_cast<const uint8_t*>(dup), n,
                        static_cast<uint32_t*>(base->ptr), scan_ticket(s), total);
+    hipLaunchKernelGGL(keep_write, dim3(tiles), dim3(BLOCK), 0, s, static_cast<const uint8_t*>(dup), n,
+                       static_cast<const uint32_t*>(base->ptr), static_cast<uint32_t*>(all->ptr));
     AM_HIP(hipGetLastError());
   }
   AM_HIP(hipStreamSynchronize(s));
   kept = *total;
-  rows = device_alloc(size_t(kept) * 4);   // the caller's result holds the kept rows only
-  {
-    ProfScope ps("keep_rows");
-    hipLaunchKernelGGL(keep_write, dim3(tiles), dim3(BLOCK), 0, s, static_cast<const uint8_t*>(dup), n,
-                       static_cast<const uint32_t*>(base->ptr), static_cast<uint32_t*>(rows->ptr));
-    AM_HIP(hipGetLastError());
+  rows = all;
+  if (kept < n / 2) {   // the result outlives the call: in a block of its own size
+    rows = device_alloc(size_t(kept) * 4);
+    AM_HIP(hipMemcpyAsync(rows->ptr, all->ptr, size_t(kept) * 4, hipMemcpyDeviceToDevice, s));
+    sync();
   }
-  sync();
   return true;
 }
 
