@@ -200,8 +200,8 @@ __device__ __forceinline__ uint32_t probe_insert(unsigned long long* tkey, unsig
 // Statistics of a key column, read back once before the column is mapped:
 //  - a HyperLogLog estimate of its distinct keys (2^10 registers: within about 3%), which sizes the hash table at about
 //    5 slots per distinct key rather than two per row, so that the table stays small enough for L2;
-//  - for integer keys, the smallest and largest order key, the nulls and the lowest null row, which
-//    decide whether the range path maps the column.
+//  - for integer keys, the smallest and largest order key and the nulls, which decide whether the range path
+//    maps the column, and how several columns form one composite key.
 constexpr int HLL_BITS = 10;
 constexpr uint32_t HLL_M = 1u << HLL_BITS;
 
@@ -219,17 +219,18 @@ __device__ __forceinline__ uint32_t hll_hash(unsigned long long k) {
 
 struct RangeStat {
   unsigned long long kmin, kmax, nulls;
-  uint32_t null_first, pad;
 };
 
 struct KeyStat {
   RangeStat r;
-  unsigned long long est;
+  unsigned long long est;   // distinct keys, about; 0: not known
 };
 
+// Most key columns read as one composite key.
+constexpr int COMPOSITE_MAX = 8;
+
 // One pass over the keys: each workgroup keeps its own registers in LDS and writes them out as bytes, with
-// the smallest and largest order key, the nulls and the lowest null row of its rows (integer keys);
-// gb_key_estimate folds the workgroups' results. Plain stores: raising shared registers with atomics
+// the smallest and largest order key and the nulls of its rows (integer keys); gb_key_estimate folds the workgroups' results. Plain stores: raising shared registers with atomics
 // costs an atomic per register and workgroup at the memory side, all of them while the registers are
 // still low (4096 registers, 256 workgroups: 45 us for 3M rows that are read in 5).
 //
@@ -245,9 +246,6 @@ template <bool HAS_VALID>
 constexpr uint32_t scan_threads() {
   return HAS_VALID ? 512u : 1024u;
 }
-#ifndef AM_OCC_BLOCKS_PER_CU
-#define AM_OCC_BLOCKS_PER_CU 2
-#endif
 
 struct ScanRows {
   unsigned long long raw[SCAN_ROWS];
@@ -321,10 +319,9 @@ void with_key_type(int type, F&& f) {
 
 struct ScanAcc {
   unsigned long long lo = ~0ull, hi = 0ull, nz = 0ull;
-  uint32_t nf = 0xFFFFFFFFu;
 };
 
-template <int TYPE, bool HAS_VALID, bool REGS>
+template <int TYPE, bool HAS_VALID>
 __device__ __forceinline__ void scan_rows(int64_t voff, uint32_t n, uint64_t row0, uint32_t gsize, const ScanRows& x,
                                           uint32_t* r_lds, ScanAcc& acc) {
   constexpr bool RANGE = TYPE >= T_I8 && TYPE <= T_U64;
@@ -342,19 +339,13 @@ __device__ __forceinline__ void scan_rows(int64_t voff, uint32_t n, uint64_t row
       const unsigned long long k = order_key(gk, TYPE);
       acc.lo = ok && k < acc.lo ? k : acc.lo;
       acc.hi = ok && k > acc.hi ? k : acc.hi;
-      if (HAS_VALID) {
-        const bool null_row = in && !v;
-        acc.nz += null_row ? 1u : 0u;
-        acc.nf = null_row ? min(acc.nf, uint32_t(i)) : acc.nf;
-      }
+      if (HAS_VALID) acc.nz += in && !v ? 1u : 0u;
     }
-    if (!REGS) continue;
     const uint32_t h = hll_hash(gk);
     idx[r] = h >> (32 - HLL_BITS);
     const uint32_t w = h << HLL_BITS;
     rank[r] = !ok ? 0u : w ? uint32_t(__clz(int(w))) + 1u : uint32_t(32 - HLL_BITS + 1);
   }
-  if (!REGS) return;
   // The step's register reads are issued together; a register is raised only when the row's rank is
   // larger (a null row or a row past the end has rank 0).
   uint32_t cur[SCAN_ROWS];
@@ -365,22 +356,20 @@ __device__ __forceinline__ void scan_rows(int64_t voff, uint32_t n, uint64_t row
     if (rank[r] > cur[r]) atomicMax(&r_lds[idx[r]], rank[r]);
 }
 
-template <int W, int TYPE, bool HAS_VALID, bool REGS>
+// regs: HLL_M bytes per workgroup; st: one per workgroup (integer keys).
+template <int W, int TYPE, bool HAS_VALID>
 __global__ __launch_bounds__(scan_threads<HAS_VALID>()) void gb_key_scan(const void* vals, const uint8_t* valid, int64_t voff, uint32_t n,
                                                    uint32_t* regs, RangeStat* st) {
   constexpr bool RANGE = TYPE >= T_I8 && TYPE <= T_U64;
-  // regs: HLL_M bytes per workgroup (REGS); st: one per workgroup.
-  __shared__ uint32_t r[REGS ? HLL_M : 4];
+  __shared__ uint32_t r[HLL_M];
   constexpr uint32_t SCAN_WAVES = scan_threads<HAS_VALID>() / 64;
   __shared__ unsigned long long s_lo[SCAN_WAVES], s_hi[SCAN_WAVES], s_nz[SCAN_WAVES];
-  __shared__ uint32_t s_nf[SCAN_WAVES];
-  if (REGS)
-    for (uint32_t j = threadIdx.x; j < HLL_M; j += blockDim.x) r[j] = 0u;
+  for (uint32_t j = threadIdx.x; j < HLL_M; j += blockDim.x) r[j] = 0u;
   __syncthreads();
   const uint32_t gsize = gridDim.x * blockDim.x;
   ScanAcc acc;
   scan_steps<W, HAS_VALID>(vals, valid, voff, n, [&](uint64_t row0, const ScanRows& x) {
-    scan_rows<TYPE, HAS_VALID, REGS>(voff, n, row0, gsize, x, r, acc);
+    scan_rows<TYPE, HAS_VALID>(voff, n, row0, gsize, x, r, acc);
   });
   if (RANGE) {
     for (int off = 32; off > 0; off >>= 1) {
@@ -388,14 +377,12 @@ __global__ __launch_bounds__(scan_threads<HAS_VALID>()) void gb_key_scan(const v
       acc.lo = l2 < acc.lo ? l2 : acc.lo;
       acc.hi = h2 > acc.hi ? h2 : acc.hi;
       acc.nz += __shfl_xor(acc.nz, off, 64);
-      acc.nf = min(acc.nf, uint32_t(__shfl_xor(int(acc.nf), off, 64)));
     }
     const int wv = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
       s_lo[wv] = acc.lo;
       s_hi[wv] = acc.hi;
       s_nz[wv] = acc.nz;
-      s_nf[wv] = acc.nf;
     }
   }
   __syncthreads();
@@ -404,11 +391,9 @@ __global__ __launch_bounds__(scan_threads<HAS_VALID>()) void gb_key_scan(const v
       acc.lo = s_lo[k] < acc.lo ? s_lo[k] : acc.lo;
       acc.hi = s_hi[k] > acc.hi ? s_hi[k] : acc.hi;
       acc.nz += s_nz[k];
-      acc.nf = min(acc.nf, s_nf[k]);
     }
-    st[blockIdx.x] = RangeStat{acc.lo, acc.hi, acc.nz, acc.nf, 0u};
+    st[blockIdx.x] = RangeStat{acc.lo, acc.hi, acc.nz};
   }
-  if (!REGS) return;
   for (uint32_t j = threadIdx.x; j < HLL_M / 4; j += blockDim.x)
     regs[size_t(blockIdx.x) * (HLL_M / 4) + j] = r[4 * j] | r[4 * j + 1] << 8 | r[4 * j + 2] << 16 | r[4 * j + 3] << 24;
 }
@@ -425,16 +410,8 @@ void key_scan(int type, hipStream_t s, const void* vals, const uint8_t* valid, i
   const dim3 grid{key_scan_blocks(valid != nullptr, n)}, block{valid ? scan_threads<true>() : scan_threads<false>()};
   with_key_type(type, [&](auto tc) {
     constexpr int TT = decltype(tc)::value;
-    constexpr bool RANGE = TT != T_F32 && TT != T_F64;   // only integer columns are scanned without registers
-    if (regs) {
-      if (valid) hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, true, true>), grid, block, 0, s, vals, valid, voff, n, regs, st);
-      else hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, false, true>), grid, block, 0, s, vals, valid, voff, n, regs, st);
-    } else if constexpr (RANGE) {
-      if (valid) hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, true, false>), grid, block, 0, s, vals, valid, voff, n, regs, st);
-      else hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, false, false>), grid, block, 0, s, vals, valid, voff, n, regs, st);
-    } else {
-      fail("internal: a span scan of a float column");
-    }
+    if (valid) hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, true>), grid, block, 0, s, vals, valid, voff, n, regs, st);
+    else hipLaunchKernelGGL((gb_key_scan<width_of(TT), TT, false>), grid, block, 0, s, vals, valid, voff, n, regs, st);
   });
 }
 
@@ -455,7 +432,7 @@ __device__ __forceinline__ void atomic_done(T result) {
 
 // True in the last workgroup of the grid to ask (one thread each); the counter is 0 again after it.
 __device__ __forceinline__ bool take_ticket(FoldCtl* c) {
-  const unsigned int last = gridDim.x - 1u;
+  const unsigned int last = gridDim.x * gridDim.y - 1u;
   const bool mine = atomicInc(&c->ticket, last) == last;
   asm volatile("" ::: "memory");
   return mine;
@@ -475,23 +452,28 @@ FoldCtl* fold_ctl() {
   return static_cast<FoldCtl*>(buf->ptr);
 }
 
-// Folds the key scan's workgroups (registers by maximum), then the HyperLogLog estimate (with the
+// Folds the key scans' workgroups (registers by maximum), then the HyperLogLog estimate (with the
 // linear-counting correction for small counts), written with the range statistics straight into pinned
-// host memory by the last workgroup done. Each of the EST_BLOCKS workgroups folds its own registers: one
-// workgroup alone took 16 us to read the registers of 366.
+// host memory by the last workgroup done; a row of the grid per column. Each of a column's EST_BLOCKS
+// workgroups folds its own registers: one workgroup alone took 16 us to read the registers of 366.
 constexpr uint32_t EST_BLOCKS = 8;
-struct EstPart {
-  float sum;
-  uint32_t zeros;
+using EstPart = unsigned long long;   // a workgroup's sum (float bits) and, above it, its empty registers
+struct EstCols {
+  struct {
+    const uint32_t* regs;
+    const RangeStat* st;   // null: not an integer column
+    uint32_t blocks;
+  } col[COMPOSITE_MAX];
 };
-__global__ __launch_bounds__(1024) void gb_key_estimate(const uint32_t* regs, const RangeStat* st, uint32_t blocks,
-                                                        int range, EstPart* parts, FoldCtl* ctl, KeyStat* out) {
+__global__ __launch_bounds__(1024) void gb_key_estimate(EstCols cols, EstPart* parts, FoldCtl* ctl, KeyStat* out) {
   constexpr uint32_t WORDS = HLL_M / 4 / EST_BLOCKS, PARTS = 1024 / WORDS;   // this workgroup's words, readers of each
   static_assert(WORDS * PARTS == 1024 && WORDS <= 64, "a thread per register word and part");
   __shared__ uint32_t s_reg[PARTS][WORDS];
   __shared__ RangeStat s_st[16];
   const uint32_t word = threadIdx.x % WORDS, part = threadIdx.x / WORDS;
-  const uint32_t* mine = regs + blockIdx.x * WORDS + word;
+  const RangeStat* st = cols.col[blockIdx.y].st;
+  const uint32_t blocks = cols.col[blockIdx.y].blocks;
+  const uint32_t* mine = cols.col[blockIdx.y].regs + blockIdx.x * WORDS + word;
   uint32_t lo = 0, hi = 0;   // registers 0 and 2, 1 and 3 of the word, 16 bits each
   constexpr uint32_t U = 8;
   for (uint32_t b = part; b < blocks; b += PARTS * U) {
@@ -506,21 +488,19 @@ __global__ __launch_bounds__(1024) void gb_key_estimate(const uint32_t* regs, co
     }
   }
   s_reg[part][word] = lo | hi << 8;
-  RangeStat r{~0ull, 0ull, 0ull, 0xFFFFFFFFu, 0u};
-  const bool stats = range && blockIdx.x == 0;
+  RangeStat r{~0ull, 0ull, 0ull};
+  const bool stats = st && blockIdx.x == 0;
   if (stats) {
     for (uint32_t b = threadIdx.x; b < blocks; b += 1024) {
       const RangeStat x = st[b];
       r.kmin = min(r.kmin, x.kmin);
       r.kmax = max(r.kmax, x.kmax);
       r.nulls += x.nulls;
-      r.null_first = min(r.null_first, x.null_first);
     }
     for (int off = 32; off > 0; off >>= 1) {
       r.kmin = min(r.kmin, (unsigned long long)__shfl_xor(r.kmin, off, 64));
       r.kmax = max(r.kmax, (unsigned long long)__shfl_xor(r.kmax, off, 64));
       r.nulls += __shfl_xor(r.nulls, off, 64);
-      r.null_first = min(r.null_first, uint32_t(__shfl_xor(int(r.null_first), off, 64)));
     }
     if ((threadIdx.x & 63) == 0) s_st[threadIdx.x >> 6] = r;
   }
@@ -546,23 +526,29 @@ __global__ __launch_bounds__(1024) void gb_key_estimate(const uint32_t* regs, co
       r.kmin = min(r.kmin, s_st[w].kmin);
       r.kmax = max(r.kmax, s_st[w].kmax);
       r.nulls += s_st[w].nulls;
-      r.null_first = min(r.null_first, s_st[w].null_first);
     }
-    out->r = r;
+    out[blockIdx.y].r = r;
   }
-  atomic_done(atomicExch(&parts[blockIdx.x].sum, sum));
-  atomic_done(atomicExch(&parts[blockIdx.x].zeros, zeros));
+  EstPart* ours = parts + blockIdx.y * EST_BLOCKS;
+  atomic_done(atomicExch(&ours[blockIdx.x], (unsigned long long)zeros << 32 | __float_as_uint(sum)));
   if (!take_ticket(ctl)) return;
-  sum = 0.f;
-  zeros = 0;
-  for (uint32_t b = 0; b < EST_BLOCKS; b++) {   // in workgroup order: the same sum whichever is last
-    sum += __hip_atomic_load(&parts[b].sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    zeros += __hip_atomic_load(&parts[b].zeros, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (uint32_t c = 0; c < gridDim.y; c++) {
+    const EstPart* of = parts + c * EST_BLOCKS;
+    sum = 0.f;
+    zeros = 0;
+    EstPart x[EST_BLOCKS];
+#pragma unroll
+    for (uint32_t b = 0; b < EST_BLOCKS; b++) x[b] = __hip_atomic_load(&of[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (uint32_t b = 0; b < EST_BLOCKS; b++) {   // in workgroup order: the same sum whichever is last
+      sum += __uint_as_float(uint32_t(x[b]));
+      zeros += uint32_t(x[b] >> 32);
+    }
+    const float m = float(HLL_M);
+    float e = (0.7213f / (1.0f + 1.079f / m)) * m * m / sum;
+    if (e <= 2.5f * m && zeros > 0) e = m * logf(m / float(zeros));
+    out[c].est = (unsigned long long)(e + 0.5f);
   }
-  const float m = float(HLL_M);
-  float e = (0.7213f / (1.0f + 1.079f / m)) * m * m / sum;
-  if (e <= 2.5f * m && zeros > 0) e = m * logf(m / float(zeros));
-  out->est = (unsigned long long)(e + 0.5f);
 }
 
 // Inserts every row's key; writes the slot of each row (NULL_SLOT for a null key). Each thread keeps
@@ -3171,7 +3157,6 @@ __global__ void gb_first_atomic(const uint32_t* ids, uint32_t n, uint32_t* rep) 
 }
 
 // ---------------------------------------------------------------- composite keys of integer columns
-constexpr int COMPOSITE_MAX = 8;
 constexpr int COMP_ROWS = 8;
 
 struct CompositeCol {
@@ -3186,34 +3171,8 @@ struct CompositeArgs {
   int count;
 };
 
-// One workgroup: the column's statistics from the scan's workgroups, into pinned host memory.
-__global__ __launch_bounds__(512) void gb_span_fold(const RangeStat* st, uint32_t blocks, RangeStat* out) {
-  __shared__ RangeStat s_st[8];
-  RangeStat r{~0ull, 0ull, 0ull, 0xFFFFFFFFu, 0u};
-  for (uint32_t b = threadIdx.x; b < blocks; b += 512) {
-    const RangeStat x = st[b];
-    r.kmin = min(r.kmin, x.kmin);
-    r.kmax = max(r.kmax, x.kmax);
-    r.nulls += x.nulls;
-    r.null_first = min(r.null_first, x.null_first);
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    r.kmin = min(r.kmin, (unsigned long long)__shfl_xor(r.kmin, off, 64));
-    r.kmax = max(r.kmax, (unsigned long long)__shfl_xor(r.kmax, off, 64));
-    r.nulls += __shfl_xor(r.nulls, off, 64);
-    r.null_first = min(r.null_first, uint32_t(__shfl_xor(int(r.null_first), off, 64)));
-  }
-  if ((threadIdx.x & 63) == 0) s_st[threadIdx.x >> 6] = r;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 8; w++) {
-      r.kmin = min(r.kmin, s_st[w].kmin);
-      r.kmax = max(r.kmax, s_st[w].kmax);
-      r.nulls += s_st[w].nulls;
-      r.null_first = min(r.null_first, s_st[w].null_first);
-    }
-    *out = r;
-  }
+CompositeCol key_col(const Array& a) {
+  return CompositeCol{a.data(), a.has_nulls() ? a.valid_bits() : nullptr, a.offset, a.type, ColSpan{}};
 }
 
 // Bijections of 32 and 64 bits that spread the keys over all digits (odd multipliers and xor-shifts; the
@@ -3651,7 +3610,7 @@ bool small_map(Array* const* columns, int64_t count, int64_t n, SmallOut o, Smal
   for (int64_t c = 0; c < count; c++) {
     const Array* k = columns[c];
     if (count > 1 && !type_is_int(k->type)) return false;
-    a.col[c] = CompositeCol{k->data(), k->has_nulls() ? k->valid_bits() : nullptr, k->offset, k->type, ColSpan{}};
+    a.col[c] = key_col(*k);
   }
   hipStream_t s = stream();
   std::shared_ptr<void> slot = pinned_slot();
@@ -3815,10 +3774,43 @@ void launch_build(int w, int grid, hipStream_t s, const void* vals, int type, co
   }
 }
 
-// Maps one key column (values, type, validity) to dense ascending ids. `known`: the column's span, when
-// its values are already known to lie in one (a composite key).
-Mapped map_column(const void* vals, int type, const uint8_t* valid, int64_t voff, int64_t n,
-                  const RangeStat* known = nullptr) {
+// The statistics of `a.count` key columns: a pass over each, one fold and one wait for all.
+void scan_columns(const CompositeArgs& a, int64_t n, KeyStat* out) {
+  hipStream_t s = stream();
+  const uint32_t un = uint32_t(n);
+  static_assert(COMPOSITE_MAX * sizeof(KeyStat) <= PINNED_SLOT, "one pinned slot");
+  std::shared_ptr<void> landing = pinned_slot();
+  auto* ks = static_cast<KeyStat*>(landing.get());
+  EstCols cols{};
+  size_t blocks = 0;
+  for (int c = 0; c < a.count; c++) blocks += cols.col[c].blocks = key_scan_blocks(a.col[c].valid != nullptr, un);
+  DevBuf regs = device_alloc(blocks * HLL_M);
+  DevBuf rsb = device_alloc(blocks * sizeof(RangeStat) + size_t(a.count) * EST_BLOCKS * sizeof(EstPart));
+  auto* rg = static_cast<uint32_t*>(regs->ptr);
+  auto* rs = static_cast<RangeStat*>(rsb->ptr);
+  ProfScope ps("gb_key_scan");
+  for (int c = 0; c < a.count; c++) {
+    const CompositeCol& k = a.col[c];
+    cols.col[c].regs = rg;
+    cols.col[c].st = type_is_int(k.type) ? rs : nullptr;
+    key_scan(k.type, s, k.vals, k.valid, k.voff, un, rg, rs);
+    rg += size_t(cols.col[c].blocks) * (HLL_M / 4);
+    rs += cols.col[c].blocks;
+  }
+  hipLaunchKernelGGL(gb_key_estimate, dim3(EST_BLOCKS, uint32_t(a.count)), dim3(1024), 0, s, cols, reinterpret_cast<EstPart*>(rs),
+                     fold_ctl(), ks);
+  AM_HIP(hipGetLastError());
+  AM_HIP(hipStreamSynchronize(s));
+  std::copy(ks, ks + a.count, out);
+}
+
+// Maps one key column to dense ascending ids. `known`: what its caller knows of it (its statistics, or the
+// span of a composite key).
+Mapped map_column(const CompositeCol& col, int64_t n, const KeyStat* known = nullptr) {
+  const void* vals = col.vals;
+  const int type = col.type;
+  const uint8_t* valid = col.valid;
+  const int64_t voff = col.voff;
   hipStream_t s = stream();
   uint32_t un = uint32_t(n);
   Mapped out;
@@ -3832,27 +3824,18 @@ Mapped map_column(const void* vals, int type, const uint8_t* valid, int64_t voff
   uint64_t full = 1024;
   while (full < want) full <<= 1;
   uint64_t cap = 1024;
-  if (known && range_path_enabled() && map_range(vals, type, valid, voff, n, *known, out)) return out;
+  KeyStat stat{};
+  if (known) stat = *known;
+  const bool range = type_is_int(type) && range_path_enabled();
+  if (known && range && map_range(vals, type, valid, voff, n, stat.r, out)) return out;
   if (n >= (int64_t(1) << 16)) {
-    const bool range = type_is_int(type) && range_path_enabled();
-    const uint32_t scan_blocks = key_scan_blocks(valid != nullptr, un);
-    DevBuf regs = device_alloc(size_t(scan_blocks) * HLL_M);
-    DevBuf rsb = device_alloc(scan_blocks * sizeof(RangeStat) + EST_BLOCKS * sizeof(EstPart));
-    std::shared_ptr<void> landing = pinned_slot();
-    auto* ks = static_cast<KeyStat*>(landing.get());
-    {
-      ProfScope ps("gb_key_scan");
-      auto* rg = static_cast<uint32_t*>(regs->ptr);
-      auto* rs = static_cast<RangeStat*>(rsb->ptr);
-      key_scan(type, s, vals, valid, voff, un, rg, rs);
-      hipLaunchKernelGGL(gb_key_estimate, dim3(EST_BLOCKS), dim3(1024), 0, s, static_cast<const uint32_t*>(rg),
-                         static_cast<const RangeStat*>(rs), scan_blocks, type_is_int(type) ? 1 : 0,
-                         reinterpret_cast<EstPart*>(rs + scan_blocks), fold_ctl(), ks);
-      AM_HIP(hipGetLastError());
+    if (stat.est == 0) {
+      CompositeArgs one{};
+      one.count = 1;
+      one.col[0] = col;
+      scan_columns(one, n, &stat);
+      if (range && !known && map_range(vals, type, valid, voff, n, stat.r, out)) return out;
     }
-    AM_HIP(hipStreamSynchronize(s));
-    const KeyStat stat = *ks;
-    if (range && !known && map_range(vals, type, valid, voff, n, stat.r, out)) return out;
     const unsigned long long d = stat.est;
 #ifndef AM_CAP_HALVES
 #define AM_CAP_HALVES 10   // table slots per distinct key, in halves
@@ -4020,45 +4003,20 @@ DevBuf first_rows(const DevBuf& ids, int64_t n, int64_t K) {
 // row, one per row on a hot group's word.) False when the spans' product does not fit 62 bits (or more
 // than COMPOSITE_MAX columns): the columns then fold pairwise over their ids.
 // any_span: one column without nulls may span all of its 64 bits (top is then all ones, for the wide form).
-bool plan_composite(Array* const* columns, int64_t count, int64_t n, CompositeArgs& ca, unsigned long long& top,
-                    bool any_span = false) {
-  if (count > COMPOSITE_MAX) return false;
-  for (int64_t c = 0; c < count; c++)
-    if (!type_is_int(columns[c]->type)) return false;
-  hipStream_t s = stream();
-  const uint32_t un = uint32_t(n);
-  std::shared_ptr<void> slot = pinned_slot();
-  auto* st = static_cast<RangeStat*>(slot.get());
-  static_assert(COMPOSITE_MAX * sizeof(RangeStat) <= PINNED_SLOT, "one pinned slot");
-  {
-    ProfScope ps("gb_span_scan");
-    for (int64_t c = 0; c < count; c++) {
-      const Array* a = columns[c];
-      const uint8_t* valid = a->has_nulls() ? a->valid_bits() : nullptr;
-      const uint32_t blocks = key_scan_blocks(valid != nullptr, un);
-      DevBuf parts = device_alloc(blocks * sizeof(RangeStat));
-      key_scan(a->type, s, a->data(), valid, a->offset, un, nullptr, static_cast<RangeStat*>(parts->ptr));
-      hipLaunchKernelGGL(gb_span_fold, dim3(1), dim3(512), 0, s, static_cast<const RangeStat*>(parts->ptr), blocks, st + c);
-      AM_HIP(hipGetLastError());
-    }
-  }
-  AM_HIP(hipStreamSynchronize(s));
+bool plan_composite(CompositeArgs& ca, const KeyStat* stat, unsigned long long& top, bool any_span = false) {
   unsigned __int128 total = 1;
-  for (int64_t c = 0; c < count; c++) {
-    const RangeStat r = st[c];
+  for (int c = 0; c < ca.count; c++) {
+    const RangeStat& r = stat[c].r;
     const bool any = r.kmin <= r.kmax;
     const unsigned __int128 span = (any ? (unsigned __int128)(r.kmax - r.kmin) + 1 : 0) + (r.nulls > 0 ? 1 : 0);
     total *= span;
     if (total > (unsigned __int128)1 << 62) {
-      if (!(any_span && count == 1 && r.nulls == 0)) return false;
+      if (!(any_span && ca.count == 1 && r.nulls == 0)) return false;
       total = ~0ull;
     }
-    const Array* a = columns[c];
-    ca.col[c] = CompositeCol{a->data(), a->has_nulls() ? a->valid_bits() : nullptr, a->offset, a->type,
-                             ColSpan{any ? r.kmin : 0ull, (unsigned long long)span, 1ull, r.nulls > 0 ? 1 : 0}};
+    ca.col[c].span = ColSpan{any ? r.kmin : 0ull, (unsigned long long)span, 1ull, r.nulls > 0 ? 1 : 0};
   }
-  for (int64_t c = count - 1; c > 0; c--) ca.col[c - 1].span.div = ca.col[c].span.div * ca.col[c].span.span;
-  ca.count = int(count);
+  for (int c = ca.count - 1; c > 0; c--) ca.col[c - 1].span.div = ca.col[c].span.div * ca.col[c].span.span;
   top = (unsigned long long)total;   // composites are below it
   return true;
 }
@@ -4080,23 +4038,29 @@ DevBuf write_composite(const CompositeArgs& ca, unsigned long long top, int64_t 
   return comp;
 }
 
-bool map_composite(Array* const* columns, int64_t count, int64_t n, std::vector<ColSpan>& out_spans, Mapped& out) {
-  CompositeArgs ca{};
+bool map_composite(CompositeArgs& ca, const KeyStat* stat, int64_t n, std::vector<ColSpan>& out_spans, Mapped& out) {
   unsigned long long top = 0;
-  if (!plan_composite(columns, count, n, ca, top)) return false;
+  if (!plan_composite(ca, stat, top)) return false;
   DevBuf comp;
   try {
     comp = write_composite<false>(ca, top, n);
   } catch (const OutOfMemory&) {   // no room for the composite keys: column by column
     return false;
   }
-  const RangeStat known{0ull, top - 1ull, 0ull, 0u, 0u};
-  out = map_column(comp->ptr, composite_narrow(top) ? T_U32 : T_U64, nullptr, 0, n, &known);
-  for (int64_t c = 0; c < count; c++) out_spans.push_back(ca.col[c].span);
+  const KeyStat known{RangeStat{0ull, top - 1ull, 0ull}, 0ull};
+  out = map_column(CompositeCol{comp->ptr, nullptr, 0, composite_narrow(top) ? T_U32 : T_U64, ColSpan{}}, n, &known);
+  for (int c = 0; c < ca.count; c++) out_spans.push_back(ca.col[c].span);
   return true;
 }
 
-GroupBy* group_by_keys_impl(Array* const* columns, int64_t count, bool need_rep) {
+// What a caller has found out about the key columns before it asks for their mapping.
+struct KeyScan {
+  bool not_small = false;   // the one-launch mapping has refused them
+  bool scanned = false;     // stat holds every column's statistics
+  KeyStat stat[COMPOSITE_MAX];
+};
+
+GroupBy* group_by_keys_impl(Array* const* columns, int64_t count, bool need_rep, KeyScan ks = {}) {
   if (count < 1) fail_invalid("group-by needs at least one key column");
   int64_t n = columns[0]->length;
   for (int64_t c = 1; c < count; c++)
@@ -4123,7 +4087,7 @@ GroupBy* group_by_keys_impl(Array* const* columns, int64_t count, bool need_rep)
       return g;
     }
     hipStream_t s = stream();
-    if (n <= int64_t(SMALL_ROWS)) {
+    if (n <= int64_t(SMALL_ROWS) && !ks.not_small) {
       g->ids = device_alloc(size_t(n) * 4);
       g->rep = device_alloc(size_t(SMALL_KEYS + 1) * 4);
       SmallStat st;
@@ -4142,24 +4106,29 @@ GroupBy* group_by_keys_impl(Array* const* columns, int64_t count, bool need_rep)
     bool ints = true;
     for (int64_t c = 0; c < count; c++) ints = ints && type_is_int(columns[c]->type);
     int64_t K = 0;
-    auto mapped = [&](const Array* a) {
-      return map_column(a->data(), a->type, a->has_nulls() ? a->valid_bits() : nullptr, a->offset, n);
-    };
+    CompositeArgs ca{};
+    if (ints && count > 1 && count <= COMPOSITE_MAX) {
+      ca.count = int(count);
+      for (int64_t c = 0; c < count; c++) ca.col[c] = key_col(*columns[c]);
+      if (!ks.scanned) scan_columns(ca, n, ks.stat);
+      ks.scanned = true;
+    }
+    auto mapped = [&](int64_t c) { return map_column(key_col(*columns[c]), n, ks.scanned ? &ks.stat[c] : nullptr); };
     Mapped m;
     bool keys_kept = ints;   // the keys come from the sorted distinct keys
     if (count == 1) {
-      m = mapped(columns[0]);
+      m = mapped(0);
       K = m.K;
-    } else if (ints && map_composite(columns, count, n, g->spans, m)) {
+    } else if (ca.count != 0 && map_composite(ca, ks.stat, n, g->spans, m)) {
       K = m.K;
     } else {
       // Columns fold pairwise: ids a (K groups) and b (K2) become the key a * K2 + b, which is injective
       // and ascending in (a, b), and that key is mapped again (GroupByKeys.swift:103-112).
       keys_kept = false;
-      m = mapped(columns[0]);
+      m = mapped(0);
       K = m.K;
       for (int64_t c = 1; c < count; c++) {
-        Mapped mc = mapped(columns[c]);
+        Mapped mc = mapped(c);
         const int64_t K2 = mc.K;
         if (K2 > 0 && K > INT64_MAX / K2)
           fail_invalid("multi-column group-by overflowed the 64-bit composite key (" + std::to_string(K) + " x " +
@@ -4169,7 +4138,7 @@ GroupBy* group_by_keys_impl(Array* const* columns, int64_t count, bool need_rep)
                            static_cast<const int32_t*>(mc.ids->ptr), uint32_t(n), (long long)K2,
                            static_cast<long long*>(comp->ptr));
         AM_HIP(hipGetLastError());
-        m = map_column(comp->ptr, T_I64, nullptr, 0, n);
+        m = map_column(CompositeCol{comp->ptr, nullptr, 0, T_I64, ColSpan{}}, n);
         K = m.K;
       }
     }
@@ -4641,29 +4610,36 @@ Array* unique_rows(Array* const* columns, int64_t count) {
     // The representative rows come from the row numbers 0 .. n-1 (GroupByKeys.swift:126-149, 436-438).
     check_index_rows(columns[0]->length, "row indices");
   }
-  if (count >= 1 && columns[0]->length >= 1 && columns[0]->length <= int64_t(SMALL_ROWS)) {
-    bool same = true;
-    for (int64_t c = 0; c < count; c++) same = same && columns[c]->length == columns[0]->length && type_is_primitive(columns[c]->type);
+  const int64_t n = count >= 1 ? columns[0]->length : 0;
+  bool plain = n >= 1, ints = count <= COMPOSITE_MAX;   // columns of one length, primitive; integers
+  for (int64_t c = 0; c < count; c++) {
+    plain = plain && columns[c]->length == n && type_is_primitive(columns[c]->type);
+    ints = ints && type_is_int(columns[c]->type);
+  }
+  KeyScan ks;
+  if (plain && n <= int64_t(SMALL_ROWS)) {
     DevBuf rows = device_alloc(size_t(SMALL_KEYS + 1) * 4);
     SmallStat st;
     SmallOut so{};
     so.uniq = static_cast<uint32_t*>(rows->ptr);
-    if (same && small_map(columns, count, columns[0]->length, so, st)) {
+    if (small_map(columns, count, n, so, st)) {
       Array* out = new_array("I", T_U32, int64_t(st.distinct));
       out->values = rows;
       out->null_count = 0;
       return out;
     }
+    ks.not_small = true;
   }
   // Integer columns whose composite key spans more than a private LDS table's groups: the rows are
   // partitioned and deduplicated (distinct_rows). Over fewer keys the range path's passes are cheaper.
-  if (count >= 1 && columns[0]->length >= 1) {
-    const int64_t n = columns[0]->length;
-    bool same = true;
-    for (int64_t c = 0; c < count; c++) same = same && columns[c]->length == n;
+  if (plain && ints) {
     CompositeArgs ca{};
+    ca.count = int(count);
+    for (int64_t c = 0; c < count; c++) ca.col[c] = key_col(*columns[c]);
+    scan_columns(ca, n, ks.stat);
+    ks.scanned = true;
     unsigned long long top = 0;
-    if (same && plan_composite(columns, count, n, ca, top, true) && top > agg_dense_cap<FirstRowP>()) {
+    if (plan_composite(ca, ks.stat, top, true) && top > agg_dense_cap<FirstRowP>()) {
       DevBuf rows;
       uint32_t kept = 0;
       bool found = false;
@@ -4680,7 +4656,7 @@ Array* unique_rows(Array* const* columns, int64_t count) {
       }
     }
   }
-  GroupBy* g = group_by_keys_impl(columns, count, true);
+  GroupBy* g = group_by_keys_impl(columns, count, true, ks);
   Array* out = nullptr;
   try {
     // The representative rows sorted ascending: keep-first order (Executor.swift:134-148).

@@ -317,6 +317,37 @@ def test_unique_rows_by_partition(case, n):
     np.testing.assert_array_equal(got, O.unique_rows([c[off:] for c in cols], [None if v is None else v[off:] for v in valid[:len(cols)]]))
 
 
+@pytest.mark.parametrize("case,scans,small", [("wide_pair", 2, 0), ("three_wide", 3, 0), ("narrow_pair", 1, 0),
+                                              ("one_column", 1, 0), ("small_floats", 0, 1), ("small_wide", 1, 1)])
+@pytest.mark.parametrize("call", ["unique", "group"])
+def test_key_columns_are_scanned_once(case, scans, small, call):
+    """Columns whose composite key does not fit, or that another way takes, are not scanned again for it: one
+    scan of all columns and one for every fold of two, and the one-launch mapping asked once."""
+    rng = np.random.default_rng(6)
+    n = 20_011 if case.startswith("small") else 150_001
+    wide = lambda k: rng.integers(-2**62, 2**62, k)[rng.integers(0, k, n)]
+    cols = {"wide_pair": lambda: [wide(300), wide(50)], "three_wide": lambda: [wide(30), wide(20), wide(9)],
+            "narrow_pair": lambda: [rng.integers(0, 30, n), rng.integers(0, 20, n).astype(np.int16)],
+            "one_column": lambda: [wide(40)], "small_floats": lambda: [rng.standard_normal(n)],
+            "small_wide": lambda: [wide(n)]}[case]()
+    if call == "group" and case == "small_wide":
+        scans = 0
+    arrays = [am.MetalArray.from_numpy(c) for c in cols]
+    am.prof_reset()
+    am.prof_enable(True)
+    got = (am.unique_rows if call == "unique" else am.group_by)(arrays)
+    if call == "group":
+        got.count_all()
+    am.prof_enable(False)
+    ran = am.prof_report()
+    am.prof_reset()
+    assert (ran.get("gb_key_scan", (0,))[0], ran.get("gb_small_map", (0,))[0]) == (scans, small), sorted(ran.items())
+    if call == "unique":
+        np.testing.assert_array_equal(got.to_numpy()[0], O.unique_rows(cols, [None] * len(cols)))
+    else:
+        np.testing.assert_array_equal(got.ids().to_numpy()[0], O.group_keys(cols, [None] * len(cols))[0])
+
+
 def test_lowest_rows_of_more_groups_than_the_partitioned_passes_take():
     """Above 2^21 groups the lowest rows come from one pass of atomics."""
     n = (1 << 21) + 200_000
