@@ -4604,6 +4604,30 @@ void group_by_noalloc(const Array& keys, int64_t key_count, int agg, const Array
   AM_HIP(hipStreamSynchronize(s));
 }
 
+// Whether the rows of distinct composite keys (below `top`) are found sooner by distinct_rows than by the
+// mapping and its lowest rows. The partition moves every row through a pass for its top digit and a level or
+// three, whatever the keys; the mapping's time grows with the distinct keys, whose bound is the product of
+// the columns' estimates. In us, mapping / partition, uniform int64 keys; through the range path (a span near
+// the number of keys), and by hash (64-bit keys anywhere):
+//     rows     keys: 1,000    10,000     50,000     200,000    1M         4M         16M
+//     200,000  range 78/113   96/111     158/113    191/114
+//              hash  128/115  198/116    315/116    375/117
+//     4M       range 101/364  126/299    200/296    250/291    430/279    626/273
+//              hash  179/388  241/315    410/313    581/310    711/302    989/304
+//     50M      range 368/2799 389/3149   685/2481   768/2484   1260/2545  2795/2467  4325/2250
+//              hash  564/3269 807/3696   1376/2912  1771/2915  2868/2928  4044/2888  6976/2635
+// So the lines: range path, keys from a twelfth of the rows (and from 16,384, below which its passes are
+// launches); hash, from a 50th, or, while the rows fit in the caches, a 160th. Skewed keys move the lines up
+// (50M Zipf keys, 16M in the support: 2984/3535) but are not told apart here.
+bool distinct_by_partition(const CompositeArgs& ca, const KeyStat* stat, unsigned long long top, int64_t n) {
+  double keys = double(top);
+  double bound = 1.0;
+  for (int c = 0; c < ca.count; c++) bound *= double(std::max<unsigned long long>(stat[c].est, 1)) + ca.col[c].span.has_null;
+  keys = std::min({keys, bound, double(n)});
+  if (top <= range_limit(n) && range_path_enabled()) return keys >= 16384.0 && keys * 12.0 >= double(n);
+  return keys * (n <= (int64_t(1) << 23) ? 160.0 : 50.0) >= double(n);
+}
+
 Array* unique_rows(Array* const* columns, int64_t count) {
   if (count >= 1) {
     check_length(columns[0]->length);
@@ -4630,8 +4654,7 @@ Array* unique_rows(Array* const* columns, int64_t count) {
     }
     ks.not_small = true;
   }
-  // Integer columns whose composite key spans more than a private LDS table's groups: the rows are
-  // partitioned and deduplicated (distinct_rows). Over fewer keys the range path's passes are cheaper.
+  // Integer columns of many distinct keys: the rows are partitioned and deduplicated.
   if (plain && ints) {
     CompositeArgs ca{};
     ca.count = int(count);
@@ -4639,7 +4662,7 @@ Array* unique_rows(Array* const* columns, int64_t count) {
     scan_columns(ca, n, ks.stat);
     ks.scanned = true;
     unsigned long long top = 0;
-    if (plan_composite(ca, ks.stat, top, true) && top > agg_dense_cap<FirstRowP>()) {
+    if (plan_composite(ca, ks.stat, top, true) && distinct_by_partition(ca, ks.stat, top, n)) {
       DevBuf rows;
       uint32_t kept = 0;
       bool found = false;

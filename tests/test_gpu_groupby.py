@@ -317,6 +317,34 @@ def test_unique_rows_by_partition(case, n):
     np.testing.assert_array_equal(got, O.unique_rows([c[off:] for c in cols], [None if v is None else v[off:] for v in valid[:len(cols)]]))
 
 
+@pytest.mark.parametrize("n,keys,form,partition", [
+    (100_003, 16_000, "dense", False), (100_003, 20_000, "dense", True), (1_000_003, 60_000, "dense", False),
+    (1_000_003, 120_000, "dense", True), (1_000_003, 120_000, "pair", True), (1_000_003, 3_000, "pair", False),
+    (1_000_003, 4_000, "wide", False), (1_000_003, 9_000, "wide", True), (9_000_001, 150_000, "wide", False),
+    (9_000_001, 220_000, "wide", True), (9_000_001, 4_000, "zipf", False), (800_003, 800_003, "dense", True),
+    (400_003, 400_003, "nulls", True), (1_200_001, 900_000, "nulls", True)])
+def test_unique_rows_by_the_number_of_keys(n, keys, form, partition):
+    """Both sides of the lines between the mapping and the partition, by the distinct keys for the rows; buckets
+    of up to 4,096 rows in the deduplication (800,003 keys leave some 3,100 a bucket without a level)."""
+    rng = np.random.default_rng(n + keys)
+    r = rng.permutation(n) % keys if keys < n else rng.permutation(n)
+    valid = [None, None]
+    if form == "wide": cols = [rng.integers(-2**62, 2**62, keys)[r]]
+    elif form == "pair": cols = [r // 10, (r % 10).astype(np.int16)]
+    elif form == "zipf": cols = [rng.integers(-2**62, 2**62, keys)[np.minimum((rng.pareto(0.8, n) * 2).astype(np.int64), keys - 1)]]
+    else: cols = [r.astype(np.int64)]
+    if form == "nulls": valid = [rng.random(n) > 0.2]
+    arrays = [am.MetalArray.from_numpy(c, v) for c, v in zip(cols, valid)]
+    am.prof_reset()
+    am.prof_enable(True)
+    got = am.unique_rows(arrays)
+    am.prof_enable(False)
+    names = set(am.prof_report())
+    am.prof_reset()
+    assert ("sort_msd_dedupe" in names) == partition, sorted(names)
+    np.testing.assert_array_equal(got.to_numpy()[0], O.unique_rows(cols, valid[:len(cols)]))
+
+
 @pytest.mark.parametrize("case,scans,small", [("wide_pair", 2, 0), ("three_wide", 3, 0), ("narrow_pair", 1, 0),
                                               ("one_column", 1, 0), ("small_floats", 0, 1), ("small_wide", 1, 1)])
 @pytest.mark.parametrize("call", ["unique", "group"])
