@@ -4616,16 +4616,17 @@ void group_by_noalloc(const Array& keys, int64_t key_count, int agg, const Array
 //              hash  179/388  241/315    410/313    581/310    711/302    989/304
 //     50M      range 368/2799 389/3149   685/2481   768/2484   1260/2545  2795/2467  4325/2250
 //              hash  564/3269 807/3696   1376/2912  1771/2915  2868/2928  4044/2888  6976/2635
-// So the lines: range path, keys from a twelfth of the rows (and from 16,384, below which its passes are
-// launches); hash, from a 50th, or, while the rows fit in the caches, a 160th. Skewed keys move the lines up
-// (50M Zipf keys, 16M in the support: 2984/3535) but are not told apart here.
+// So the lines: range path, keys from a twelfth of the rows (and from 16,384: fewer are mapped in less than the
+// partition's launches take); hash, from a 160th while the rows fit in the caches. Beyond, uniform keys cross at a
+// 50th, Zipf keys, whose hot ones the hash mapping caches and the partition moves level by level, at a tenth
+// (16M rows of 690,000 Zipf keys 899/1289, 50M of 2.3M 2552/3534); they are not told apart, and the line is a 20th.
 bool distinct_by_partition(const CompositeArgs& ca, const KeyStat* stat, unsigned long long top, int64_t n) {
   double keys = double(top);
   double bound = 1.0;
   for (int c = 0; c < ca.count; c++) bound *= double(std::max<unsigned long long>(stat[c].est, 1)) + ca.col[c].span.has_null;
   keys = std::min({keys, bound, double(n)});
   if (top <= range_limit(n) && range_path_enabled()) return keys >= 16384.0 && keys * 12.0 >= double(n);
-  return keys * (n <= (int64_t(1) << 23) ? 160.0 : 50.0) >= double(n);
+  return keys * (n <= (int64_t(1) << 23) ? 160.0 : 20.0) >= double(n);
 }
 
 Array* unique_rows(Array* const* columns, int64_t count) {
