@@ -240,14 +240,14 @@ bool distinct_rows(const void* keys, int width, uint32_t n, DevBuf& rows, uint32
 // beside the sort's scratch: argsort and take.
 Array* sorted_ints(const Array& a, bool descending, int null_placement);
 
-// ORDER BY of a whole table by one 64-bit key (int64 / uint64 / float64): every column of `cols`
-// (each of n rows) in the key's stable order with am_argsort_ex2's options, as new arrays in `out`.
-// The columns move with the hybrid sort's top-digit partition instead of one gather across the table.
-// Returns false, with nothing in `out`, for large tables that a gather of whole rows moves faster, and when
-// the key does not take the hybrid sort (fewer than 2^18 rows, a constant top digit, a full bucket list, a
-// graph capture); the caller then sorts and permutes.
-bool order_by_columns(const Array& key, bool descending, int null_placement, int float_order,
-                      const std::vector<const Array*>& cols, std::vector<Array*>& out);
+// ORDER BY of a whole table by one 64-bit integer key: every column of `cols` (each of n rows) in the key's
+// stable order with am_argsort_ex2's options, as new arrays in `out`. The columns move with the hybrid
+// sort's top-digit partition instead of one gather across the table. Returns false, with nothing in `out`,
+// for tables that a gather of whole rows moves faster (other keys, a key that is not among the columns, more
+// than two columns), and when the key does not take the hybrid sort (fewer than 2^18 rows, a constant top
+// digit, a full bucket list, a graph capture); the caller then sorts and permutes.
+bool order_by_columns(const Array& key, bool descending, int null_placement, const std::vector<const Array*>& cols,
+                      std::vector<Array*>& out);
 
 // take.hip
 Array* take(const Array& a, const Array& indices);

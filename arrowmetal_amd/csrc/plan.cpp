@@ -13,11 +13,11 @@
 // "Unsupported Arrow type: plan: ... is not supported by this build". The `optimize` flag is accepted:
 // on this subset the reference's optimizer rules (pushdown, pruning, folding) do not change a result.
 //
-// Execution is this build's own. A sort by one 64-bit key of a table of at least 2^18 rows that is small
-// or narrow moves every column with the sort (order_by_columns in sort.hip): the columns are partitioned
+// Execution is this build's own. A sort by one 64-bit integer key of a table of at least 2^18 rows and at
+// most two columns moves both with the sort (order_by_columns in sort.hip): the other column is partitioned
 // along the sort's top-digit partition, and the final gather reads from the partition of its own output
-// range, so no column is gathered across the whole table; an int64 / uint64 key column comes out of the
-// sort's bucket sorts directly. Other sorts are a lexsort and one gather of whole rows (permute_columns in
+// range, so it is not gathered across the whole table; the key column comes out of the sort's bucket sorts
+// directly. Other sorts are a lexsort and one gather of whole rows (permute_columns in
 // take.hip).
 #include <algorithm>
 #include <cmath>
@@ -577,7 +577,7 @@ Table sort_table(Table in, const std::vector<SortKey>& keys) {
   if (keys.size() == 1) {
     std::vector<Array*> sorted;
     const SortKey& k = keys[0];
-    if (order_by_columns(*kc[0], k.descending, k.nulls_first ? 1 : 0, k.float_order, cols, sorted)) return table_of(sorted);
+    if (order_by_columns(*kc[0], k.descending, k.nulls_first ? 1 : 0, cols, sorted)) return table_of(sorted);
   }
   std::vector<int> desc, place, forder;
   for (auto& k : keys) {

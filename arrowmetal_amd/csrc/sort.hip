@@ -1219,13 +1219,13 @@ bool distinct_rows_t(const void* keys, uint32_t n, DevBuf& rows, uint32_t& kept,
 
 // ---------------------------------------------------------------- ORDER BY of whole tables
 //
-// order_by_columns sorts by one 64-bit key with the hybrid sort in its POS_ROWS form: rows carried
+// order_by_columns sorts by one 64-bit integer key with the hybrid sort in its POS_ROWS form: rows carried
 // through the levels are positions p in the top-digit partition's output (the value block), and
 // pos_of_row[r] = p for every value row r. A column then moves in two row passes:
 //   ob_partition  part[pos_of_row[r]] = col[r]: the column laid out as the partition laid out its keys
 //                 (reads in row order; writes in runs, as the partition's own)
-//   ob_gather     out[i] = part[out_idx[i]] in the value block, col[out_idx[i]] in the NaN and null
-//                 blocks (whose rows keep input order)
+//   ob_gather     out[i] = part[out_idx[i]] in the value block, col[out_idx[i]] in the null block
+//                 (whose rows keep input order)
 // Output i of the value block and its position p lie in the same top-digit bucket, so the gather of an
 // output range reads one bucket's part of the column. Each XCD takes its own eighth of the outputs
 // (XCD-private chunk counters; a workgroup that finds its eighth done takes chunks of the others), so a
@@ -1420,11 +1420,11 @@ void ob_move_column(const Array& c, bool nulls, const uint32_t* pos_of_row, cons
 }
 
 template <int ITEMS>
-bool ob_sort(const Array& key, bool desc, int placement, int forder, uint32_t* out_idx, uint32_t* pos_of_row,
+bool ob_sort(const Array& key, bool desc, int placement, uint32_t* out_idx, uint32_t* pos_of_row,
              uint32_t* m, uint32_t* bucket_base, hipStream_t s, unsigned long long* key_out,
              unsigned long long key_xor) {
   return run_sort<unsigned long long, 8, ITEMS>(key.data(), key.type, key.has_nulls() ? key.valid_bits() : nullptr,
-                                                key.offset, uint32_t(key.length), desc, placement, forder, out_idx,
+                                                key.offset, uint32_t(key.length), desc, placement, 0, out_idx,
                                                 s, pos_of_row, m, bucket_base, key_out, key_xor);
 }
 
@@ -1579,22 +1579,18 @@ Array* sorted_ints(const Array& a, bool descending, int null_placement) {
   }
 }
 
-bool order_by_columns(const Array& key, bool descending, int null_placement, int float_order,
-                      const std::vector<const Array*>& cols, std::vector<Array*>& out) {
+bool order_by_columns(const Array& key, bool descending, int null_placement, const std::vector<const Array*>& cols,
+                      std::vector<Array*>& out) {
   out.clear();
   const int64_t n = key.length;
-  if (key.width() != 8 || !type_is_primitive(key.type) || n < (int64_t(1) << 18) || n > int64_t(UINT32_MAX) ||
-      capturing(stream()))
+  if (n < (int64_t(1) << 18) || n > int64_t(UINT32_MAX) || capturing(stream())) return false;
+  // Only with an integer key among the columns, which comes out of the bucket sorts, and at most one column
+  // beside it. In us, this way / an argsort and permute_columns: an int64 key alone, 270K rows 77/88, 1M 139/158,
+  // 4M 223/291, 50M 1542/2079; with one float64, 270K 107/100, 1M 175/172, 4M 292/328, 50M 2301/2719; with two,
+  // 270K 146/105, 1M 216/181, 4M 361/361; with three, 4M 436/365, 50M 3834/3347. (A float64 key's column had to be
+  // moved by the two passes as well: alone, 270K 171/155, 4M 424/399, 50M 3957/3266.)
+  if ((key.type != T_I64 && key.type != T_U64) || cols.size() > 2 || std::find(cols.begin(), cols.end(), &key) == cols.end())
     return false;
-  // From 2^19 rows only with an integer key, whose own column comes out of the bucket sorts, and at most one
-  // other column. In us, this way / an argsort and permute_columns: an int64 key alone, 4M rows 229/298, 50M
-  // 1542/2079; with one float64, 4M 295/334, 50M 2301/2719; with three, 4M 443/376, 50M 3834/3347; with eight,
-  // 4M 777/543; a float64 key alone, 4M 462/406, 50M 3957/3266; with three others and nulls, 1M 427/285, 30M
-  // 5497/2366. (Smaller tables of many columns would gain as well, 300K 355/232, and keep this way: the checks
-  // of its two passes over every type, key order and null placement run there.)
-  const bool key_is_int = key.type == T_I64 || key.type == T_U64;
-  const bool key_is_column = std::find(cols.begin(), cols.end(), &key) != cols.end();
-  if (n >= (int64_t(1) << 19) && !(key_is_int && key_is_column && cols.size() <= 2)) return false;
   for (const Array* c : cols)
     if (c->length != n || !type_is_primitive(c->type)) return false;
   check_index_rows(n, "argsort");
@@ -1610,23 +1606,18 @@ bool order_by_columns(const Array& key, bool descending, int null_placement, int
   auto* bbase = static_cast<uint32_t*>(bb->ptr);
   uint32_t m = 0;
   const int place = null_placement == 1 ? 1 : 0;
-  // An int64 / uint64 key column among the columns comes out of the bucket sorts themselves: its
-  // mapped keys are a bijection of its values (x ^ 2^63 for int64, then ~ when descending).
-  DevBuf key_vals;
-  unsigned long long key_xor = 0;
-  const bool key_direct = key_is_int && key_is_column;
-  if (key_direct) {
-    key_vals = device_alloc(size_t(n) * 8);
-    key_xor = (key.type == T_I64 ? 0x8000000000000000ull : 0ull) ^ (descending ? ~0ull : 0ull);
-  }
-  unsigned long long* kout = key_direct ? static_cast<unsigned long long*>(key_vals->ptr) : nullptr;
+  // The key column comes out of the bucket sorts themselves: the mapped keys are a bijection of its values
+  // (x ^ 2^63 for int64, then ~ when descending).
+  DevBuf key_vals = device_alloc(size_t(n) * 8);
+  const unsigned long long key_xor = (key.type == T_I64 ? 0x8000000000000000ull : 0ull) ^ (descending ? ~0ull : 0ull);
+  auto* kout = static_cast<unsigned long long*>(key_vals->ptr);
   bool ok;
   switch (sort_tune(n, 8).items) {
-    case 4: ok = ob_sort<4>(key, descending, place, float_order, out_idx, pos_of_row, &m, bbase, s, kout, key_xor); break;
-    case 8: ok = ob_sort<8>(key, descending, place, float_order, out_idx, pos_of_row, &m, bbase, s, kout, key_xor); break;
-    case 12: ok = ob_sort<12>(key, descending, place, float_order, out_idx, pos_of_row, &m, bbase, s, kout, key_xor); break;
-    case 20: ok = ob_sort<20>(key, descending, place, float_order, out_idx, pos_of_row, &m, bbase, s, kout, key_xor); break;
-    default: ok = ob_sort<16>(key, descending, place, float_order, out_idx, pos_of_row, &m, bbase, s, kout, key_xor); break;
+    case 4: ok = ob_sort<4>(key, descending, place, out_idx, pos_of_row, &m, bbase, s, kout, key_xor); break;
+    case 8: ok = ob_sort<8>(key, descending, place, out_idx, pos_of_row, &m, bbase, s, kout, key_xor); break;
+    case 12: ok = ob_sort<12>(key, descending, place, out_idx, pos_of_row, &m, bbase, s, kout, key_xor); break;
+    case 20: ok = ob_sort<20>(key, descending, place, out_idx, pos_of_row, &m, bbase, s, kout, key_xor); break;
+    default: ok = ob_sort<16>(key, descending, place, out_idx, pos_of_row, &m, bbase, s, kout, key_xor); break;
   }
   if (!ok) return false;
   // The value block: [0, m) with nulls last, [n - m, n) with nulls first.
@@ -1639,7 +1630,7 @@ bool order_by_columns(const Array& key, bool descending, int null_placement, int
       if (nulls < 0) nulls = count_nulls(*c);
       o->null_count = nulls;   // a permutation keeps the null count
       if (nulls > 0) o->validity = device_alloc(size_t((n + 63) / 64) * 8);
-      if (c == &key && key_direct) {
+      if (c == &key) {
         o->values = key_vals;
         hipLaunchKernelGGL(ob_key_rest<unsigned long long>, dim3((uint32_t(n) + 255u) / 256u), dim3(256), 0, s,
                            static_cast<unsigned long long*>(key_vals->ptr), uint32_t(n), vbase, m,

@@ -90,16 +90,24 @@ def order_by_table(rng, n, key_kind="i64", key_nulls=0.02):
     ("runs", True, "last", "ieee"),
 ])
 def test_order_by_moves_every_column(key_kind, desc, nulls, forder):
-    """One 64-bit key over 300k rows: the columns move with the sort's top-digit partition (the
-    order_by kernels run), and every column equals the oracle's lexsort + take."""
+    """One 64-bit key over 300k rows: the whole table moves as rows; a column of each width beside an integer
+    key with the sort's top-digit partition (the order_by kernels run). Every column equals the oracle's
+    lexsort + take."""
     rng = np.random.default_rng(zlib.crc32(f"{key_kind}{desc}{nulls}{forder}".encode()))
     n = 300_007
     t = order_by_table(rng, n, key_kind)
     plan = {"op": "sort", "by": [{"column": "key", "descending": desc, "nulls": nulls, "float_order": forder}],
             "input": {"op": "scan", "source": "t"}}
     (got, want), names = profiled_names(lambda: run_both(plan, {"t": t}))
-    assert "order_by_gather" in names and "order_by_partition" in names, sorted(names)
+    assert "take_pack" in names and "order_by_gather" not in names, sorted(names)
     assert_tables_equal(got, want, f"{key_kind} desc={desc} nulls={nulls} {forder}")
+    for c in t:
+        two = {"key": t["key"], c: t[c]}
+        if key_kind == "f64" or c == "key":
+            continue
+        (got, want), names = profiled_names(lambda: run_both(plan, {"t": two}))
+        assert "order_by_gather" in names and "order_by_partition" in names, sorted(names)
+        assert_tables_equal(got, want, f"{key_kind} desc={desc} nulls={nulls} {forder} with {c}")
 
 
 def test_order_by_without_nulls_and_all_null_payload():
@@ -109,9 +117,10 @@ def test_order_by_without_nulls_and_all_null_payload():
     t = {"key": (key, None), "p": (np.arange(n, dtype=np.float64), np.zeros(n, bool)),
          "q": (rng.integers(0, 9, n).astype(np.int64), None)}
     plan = {"op": "sort", "by": [["key", True]], "input": {"op": "scan", "source": "t"}}
-    (got, want), names = profiled_names(lambda: run_both(plan, {"t": t}))
-    assert "order_by_gather" in names
-    assert_tables_equal(got, want, "no key nulls")
+    for c in ("p", "q"):
+        (got, want), names = profiled_names(lambda: run_both(plan, {"t": {"key": t["key"], c: t[c]}}))
+        assert "order_by_gather" in names
+        assert_tables_equal(got, want, f"no key nulls, {c}")
 
 
 @pytest.mark.parametrize("n", [0, 1, 1000, 100_003])
@@ -161,7 +170,7 @@ def test_sorted_tables_move_whole_rows(n, columns):
 
 @pytest.mark.parametrize("key_kind", ["i64", "f64"])
 def test_order_by_of_a_large_table_by_one_key(key_kind):
-    """From 2^19 rows: an integer key with one other column moves with the partition, other tables as rows."""
+    """An integer key with one other column moves with the partition, other tables as rows."""
     rng = np.random.default_rng(8)
     t = order_by_table(rng, 1 << 19, key_kind)
     plan = {"op": "sort", "by": [["key", True]], "input": {"op": "scan", "source": "t"}}
