@@ -39,7 +39,8 @@ struct SortCtl {
   alignas(128) uint32_t tile_counter[16];   // [0] first pass, [1 + p] pass p, [11] units
   alignas(128) uint32_t digit_base[8][RADIX];   // exclusive digit prefix inside the value block, per pass
   uint32_t bin_total[NBINS_FIRST], first_base[NBINS_FIRST];   // the hybrid sort's analysis
-  uint32_t active_mask, first_active, last_active, pad1;
+  uint32_t active_mask, first_active, last_active;
+  uint32_t lsd;                     // the hybrid sort's analysis has counted for the LSD passes instead
   uint32_t value_base, nan_base, null_base, pad2;
   // Per-XCD partials of the upsweep, folded into the fields above by sort_plan.
   uint32_t xhist[NXCD][8][RADIX];
@@ -201,6 +202,21 @@ __device__ __forceinline__ void up_reduce(UpStat& st, UpStat* s) {
   }
 }
 
+// The digits that the LSD passes sort, and the bases of the three blocks, for m values, q NaN and z null rows.
+__device__ __forceinline__ void set_lsd_plan(SortCtl* ctl, uint32_t varying, uint32_t m, uint32_t q, uint32_t z,
+                                             int nulls_first) {
+  // No varying digit (a single value, or one repeated key): one pass over digit 0 is then a
+  // stable compaction of the value rows, which is exactly the answer.
+  const uint32_t mask = varying == 0u || m <= 1u ? 1u : varying;
+  ctl->m = m;
+  ctl->active_mask = mask;
+  ctl->first_active = uint32_t(__builtin_ctz(mask));
+  ctl->last_active = 31u - uint32_t(__builtin_clz(mask));
+  ctl->null_base = nulls_first ? 0u : m + q;
+  ctl->nan_base = nulls_first ? z : m;
+  ctl->value_base = nulls_first ? z + q : 0u;
+}
+
 // The LSD passes' plan, by the analysis' last workgroup: the XCDs' partial counts folded, the active digits,
 // the bases of the three blocks, and the exclusive digit prefix of every active pass.
 template <int P>
@@ -232,16 +248,7 @@ __device__ __forceinline__ void sort_plan(SortCtl* ctl, int nulls_first, uint32_
     uint32_t mask = 0;
     for (int p = 0; p < P; p++)
       if ((diff >> (8 * p)) & 0xFFull) mask |= 1u << p;
-    // No varying digit (a single value, or one repeated key): one pass over digit 0 is then a
-    // stable compaction of the value rows, which is exactly the answer.
-    if (mask == 0 || m <= 1u) mask = 1;
-    ctl->m = m;
-    ctl->active_mask = mask;
-    ctl->first_active = uint32_t(__builtin_ctz(mask));
-    ctl->last_active = 31u - uint32_t(__builtin_clz(mask));
-    ctl->null_base = nulls_first ? 0u : m + q;
-    ctl->nan_base = nulls_first ? z : m;
-    ctl->value_base = nulls_first ? z + q : 0u;
+    set_lsd_plan(ctl, mask, m, q, z, nulls_first);
   }
 }
 
@@ -306,21 +313,72 @@ __global__ __launch_bounds__(BLOCK) void sort_upsweep(const void* vals, const ui
 constexpr uint32_t UNIT_SHIFT_LARGE = 14, UNIT_SHIFT_SMALL = 12;
 constexpr uint32_t UNITS_PER_BLOCK = 8;   // most units one workgroup counts
 
-// Every unit's counts, bin-major (unit_hist[b][unit]), and every workgroup's statistics.
+// 32-bit keys have four LSD passes only, so the hybrid sort must come out with about one level (every
+// top-digit bucket at most 2^18 rows, which a second digit brings to bucket-sort size), or save whole passes
+// over a large column. 10M float32 values over 10,000 distinct: LSD 481 us, hybrid 660; 40M uniform float32:
+// 1.71 against 1.33 ms; 3M full-range int32: 237 against 167 us.
+constexpr uint32_t MSD32_TOP_MAX = 1u << 18, MSD32_SAVES = 1u << 24;
+
+// Whether the LSD passes sort a 32-bit column, from 16 neighbours (a line) at each of 16 places over its length: one top digit on all of them, or
+// one on so many that its bucket is too large. (Only a guess at the faster way: either sorts any column. A
+// column that is counted for the one and sorted by the other is read once more: 1M int32 values of 0 to 2^20
+// 154 us so, 140 when guessed; full-range ones 125 and 126.) Every workgroup reads the same rows.
+template <typename K, int W>
+__device__ __forceinline__ bool sampled_lsd(const void* vals, const uint8_t* valid, int64_t voff, uint32_t n, int type,
+                                            int forder, int desc, uint32_t* h) {
+  h[threadIdx.x] = 0u;
+  __syncthreads();
+  const uint32_t i = uint32_t(uint64_t(n - 16u) * (threadIdx.x >> 4) / (BLOCK / 16u - 1u)) + (threadIdx.x & 15u);
+  const uint64_t raw = load_raw<W>(vals, i);
+  uint32_t bit;
+  const uint32_t vb = load_valid_byte(valid, voff, i, bit);
+  K key = 0;
+  const int cat = classify_raw<K>(raw, (vb >> bit) & 1u, type, forder, desc, key);
+  count_bin(h, cat == 0 ? uint32_t(key >> (8 * (sizeof(K) - 1))) & 0xFFu : ~0u);
+  __syncthreads();
+  const uint32_t most = n < MSD32_SAVES ? uint32_t(uint64_t(MSD32_TOP_MAX) * BLOCK / n) : uint32_t(BLOCK);
+  const bool over = __syncthreads_or(h[threadIdx.x] > most ? 1 : 0);
+  return __syncthreads_count(h[threadIdx.x] != 0u ? 1 : 0) <= 1 || over;
+}
+
+// Every unit's counts, bin-major (unit_hist[b][unit]), and every workgroup's statistics. With guess (32-bit keys),
+// for a column that the LSD passes will sort: every digit's counts of every workgroup (unit_hist[256 p + b][workgroup]).
 template <typename K, int W>
 __global__ __launch_bounds__(BLOCK) void msd_upsweep(const void* vals, const uint8_t* valid, int64_t voff, uint32_t n,
                                                      int type, int forder, int desc, uint32_t rows_per_block,
                                                      UpStat* stats, uint32_t* unit_hist, uint32_t nunits,
-                                                     uint32_t unit_shift) {
+                                                     uint32_t unit_shift, int guess, SortCtl* ctl) {
   constexpr int P = int(sizeof(K));
   __shared__ uint32_t hu[UNITS_PER_BLOCK * NBINS_FIRST];
   __shared__ UpStat s_st[WAVES];
+  bool lsd = false;
+  if constexpr (P == 4) lsd = guess && sampled_lsd<K, W>(vals, valid, voff, n, type, forder, desc, hu);
+  if (blockIdx.x == 0 && threadIdx.x == 0) ctl->lsd = lsd ? 1u : 0u;
+  __syncthreads();
   const uint32_t begin = blockIdx.x * rows_per_block;
   const uint32_t end = min(n, begin + rows_per_block);
   const uint32_t nu = (end - begin + (1u << unit_shift) - 1u) >> unit_shift;
-  for (uint32_t i = threadIdx.x; i < nu * NBINS_FIRST; i += BLOCK) hu[i] = 0u;
+  for (uint32_t i = threadIdx.x; i < (lsd ? 4u * RADIX : nu * NBINS_FIRST); i += BLOCK) hu[i] = 0u;
   __syncthreads();
   UpStat st{0ull, ~0ull, 0u, 0u, 0u, 0u};
+  if (lsd) {   // uniform over the grid
+    static_assert(UNITS_PER_BLOCK * NBINS_FIRST >= 4 * RADIX, "the digits' counts fit where the units' are");
+    up_steps<W>(vals, valid, voff, begin, end, [&](uint64_t base, const uint64_t (&raw)[UP_ITEMS], const uint32_t (&vb)[UP_ITEMS]) {
+      K kk[UP_ITEMS];
+      int cc[UP_ITEMS];
+      up_classify<K>(base, end, raw, vb, valid != nullptr, voff, type, forder, desc, kk, cc, st);
+#pragma unroll
+      for (uint32_t p = 0; p < 4; p++)
+#pragma unroll
+        for (int u = 0; u < UP_ITEMS; u++)
+          count_digit(hu + p * RADIX, cc[u] == 0 ? uint32_t(kk[u] >> (8 * p)) & 0xFFu : ~0u);
+    });
+    up_reduce(st, s_st);
+    if (threadIdx.x == 0) stats[blockIdx.x] = st;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < 4u * RADIX; i += BLOCK) unit_hist[size_t(i) * gridDim.x + blockIdx.x] = hu[i];
+    return;
+  }
   up_steps<W>(vals, valid, voff, begin, end, [&](uint64_t base, const uint64_t (&raw)[UP_ITEMS], const uint32_t (&vb)[UP_ITEMS]) {
     K kk[UP_ITEMS];
     int cc[UP_ITEMS];
@@ -660,7 +718,80 @@ struct MsdPlan {
   uint32_t m;                // value rows
   uint32_t large, biggest;   // top-digit buckets that need a level, the largest of the others (not of equal keys)
   uint32_t local, top;       // entries of the bucket sort's list; the largest top-digit bucket
+  uint32_t lsd;              // the control block holds the LSD passes' plan instead (of the rest, mask and m are set)
 };
+
+// The statistics of all workgroups of an analysis, in thread 0.
+__device__ __forceinline__ UpStat fold_stats(const UpStat* stats, uint32_t blocks, UpStat* s) {
+  UpStat st{0ull, ~0ull, 0u, 0u, 0u, 0u};
+  for (uint32_t k = threadIdx.x; k < blocks; k += BLOCK) {
+    const UpStat x = stats[k];
+    st.m += x.m;
+    st.q += x.q;
+    st.z += x.z;
+    st.key_or |= x.key_or;
+    st.key_and &= x.key_and;
+  }
+  up_reduce(st, s);
+  return st;
+}
+
+template <int P>
+__device__ __forceinline__ uint32_t varying_digits(const UpStat& st) {
+  const unsigned long long diff = st.m ? st.key_or ^ st.key_and : 0ull;
+  uint32_t mask = 0;
+  for (int p = 0; p < P; p++)
+    if ((diff >> (8 * p)) & 0xFFull) mask |= 1u << p;
+  return mask;
+}
+
+// The LSD passes' plan from the counts of their digits, workgroup b totalling value b of each of the four; the
+// last one done makes the plan.
+__device__ __forceinline__ void lsd_scan(SortCtl* ctl, const uint32_t* counts, const UpStat* stats, uint32_t blocks,
+                                         int nulls_first, uint32_t* ticket, MsdPlan* plan) {
+  __shared__ uint32_t tmp[WAVES], s_sum[WAVES][4];
+  __shared__ UpStat s_st[WAVES];
+  __shared__ uint32_t s_last;
+  const uint32_t b = blockIdx.x;
+  uint32_t sum[4] = {0u, 0u, 0u, 0u};
+  if (b < uint32_t(RADIX))
+    for (uint32_t k = threadIdx.x; k < blocks; k += BLOCK)
+#pragma unroll
+      for (uint32_t p = 0; p < 4; p++) sum[p] += counts[(size_t(p) * RADIX + b) * blocks + k];
+#pragma unroll
+  for (uint32_t p = 0; p < 4; p++) {
+    for (int off = 32; off > 0; off >>= 1) sum[p] += __shfl_xor(sum[p], off, 64);
+    if ((threadIdx.x & 63u) == 0u) s_sum[threadIdx.x >> 6][p] = sum[p];
+  }
+  __syncthreads();
+  if (threadIdx.x < 4u && b < uint32_t(RADIX)) {
+    uint32_t t = 0;
+    for (int w = 0; w < WAVES; w++) t += s_sum[w][threadIdx.x];
+    atomic_done(atomicExch(&ctl->digit_base[threadIdx.x][b], t));
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) s_last = last_block(ticket) ? 1u : 0u;
+  __syncthreads();
+  if (!s_last) return;   // uniform
+  const UpStat st = fold_stats(stats, blocks, s_st);
+  uint32_t v[4];
+#pragma unroll
+  for (uint32_t p = 0; p < 4; p++)   // every load first
+    v[p] = __hip_atomic_load(&ctl->digit_base[p][threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (uint32_t p = 0; p < 4; p++) {
+    uint32_t total;
+    ctl->digit_base[p][threadIdx.x] = block_excl_scan(v[p], tmp, total);
+  }
+  if (threadIdx.x < 16) ctl->tile_counter[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) {
+    const uint32_t varying = varying_digits<4>(st);
+    set_lsd_plan(ctl, varying, st.m, st.q, st.z, nulls_first);
+    plan->mask = varying;
+    plan->m = st.m;
+    plan->lsd = 1u;
+  }
+}
 
 // Workgroup b: the exclusive scan of bin b's unit counts in place, and its total. The last workgroup done
 // makes the plan: the active digits, where each bin's rows start (first_base), the level kernels' control
@@ -676,6 +807,12 @@ __global__ __launch_bounds__(BLOCK) void msd_unit_scan(SortCtl* ctl, uint32_t* u
   __shared__ uint32_t s_last, s_mask, s_first[NBINS_FIRST];
   __shared__ UpStat s_st[WAVES];
   __shared__ LongCopies s_long;
+  if constexpr (P == 4) {
+    if (ctl->lsd) {   // uniform over the grid
+      lsd_scan(ctl, unit_hist, stats, blocks, nulls_first, ticket, plan);
+      return;
+    }
+  }
   const uint32_t b = blockIdx.x;
   uint32_t* h = unit_hist + size_t(b) * nunits;
   uint32_t carry = 0;
@@ -693,25 +830,13 @@ __global__ __launch_bounds__(BLOCK) void msd_unit_scan(SortCtl* ctl, uint32_t* u
   }
   __syncthreads();
   if (!s_last) return;   // uniform
-  UpStat st{0ull, ~0ull, 0u, 0u, 0u, 0u};
-  for (uint32_t k = threadIdx.x; k < blocks; k += BLOCK) {
-    const UpStat x = stats[k];
-    st.m += x.m;
-    st.q += x.q;
-    st.z += x.z;
-    st.key_or |= x.key_or;
-    st.key_and &= x.key_and;
-  }
-  up_reduce(st, s_st);
+  const UpStat st = fold_stats(stats, blocks, s_st);
   uint32_t total;
   const uint32_t size = __hip_atomic_load(&ctl->bin_total[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const uint32_t start = block_excl_scan(size, tmp, total);
   if (threadIdx.x < LC_WORDS) lc[threadIdx.x] = 0u;
   if (threadIdx.x == 0) {
-    const unsigned long long diff = st.m ? st.key_or ^ st.key_and : 0ull;
-    uint32_t mask = 0;
-    for (int p = 0; p < P; p++)
-      if ((diff >> (8 * p)) & 0xFFull) mask |= 1u << p;
+    const uint32_t mask = varying_digits<P>(st);
     s_mask = mask;
     s_long.count = 0u;
     const uint32_t value_base = nulls_first ? st.z + st.q : 0u;
@@ -720,6 +845,7 @@ __global__ __launch_bounds__(BLOCK) void msd_unit_scan(SortCtl* ctl, uint32_t* u
     *mc = {mask, value_base, epoch, 0u, key_out, key_xor};
     plan->mask = mask;
     plan->m = st.m;
+    plan->lsd = 0u;
   }
   clear_ctl(ctl);   // the partition's unit counter, and the rest in case the LSD passes run
   s_first[threadIdx.x] = start;
@@ -900,7 +1026,7 @@ struct Units {
 template <typename K, int W>
 Units msd_analyse(const void* vals, int type, const uint8_t* valid, int64_t voff, uint32_t n, int desc, int placement,
                   int forder, SortCtl* ctl, const MsdWork& w, uint32_t epoch, void* key_out,
-                  unsigned long long key_xor, uint32_t* bucket_base, hipStream_t s) {
+                  unsigned long long key_xor, uint32_t* bucket_base, hipStream_t s, bool guess = false) {
   Units un;
   un.shift = n >= (1u << 22) ? UNIT_SHIFT_LARGE : UNIT_SHIFT_SMALL;
   const uint32_t unit_rows = 1u << un.shift, cus = uint32_t(device().cu_count);
@@ -908,13 +1034,15 @@ Units msd_analyse(const void* vals, int type, const uint8_t* valid, int64_t voff
   // Workgroups of whole units, at most UNITS_PER_BLOCK: one each until every CU has four.
   const uint32_t per = std::min(UNITS_PER_BLOCK, std::max(1u, (un.count + cus * 4u - 1u) / (cus * 4u)));
   const uint32_t rpb = per * unit_rows, blocks = (n + rpb - 1) / rpb;
-  un.buf = device_alloc(size_t(un.count) * NBINS_FIRST * 4 + size_t(blocks) * sizeof(UpStat) + 16);
+  size_t words = size_t(un.count) * NBINS_FIRST;
+  if (guess) words = std::max(words, size_t(blocks) * 4 * RADIX);
+  un.buf = device_alloc(words * 4 + size_t(blocks) * sizeof(UpStat) + 16);
   UpStat* stats = static_cast<UpStat*>(un.buf->ptr);
   un.hist = reinterpret_cast<uint32_t*>(stats + blocks);
   {
     ProfScope ps("sort_upsweep");
     hipLaunchKernelGGL((msd_upsweep<K, W>), dim3(blocks), dim3(BLOCK), 0, s, vals, valid, voff, n, type, forder, desc, rpb,
-                       stats, un.hist, un.count, un.shift);
+                       stats, un.hist, un.count, un.shift, guess ? 1 : 0, ctl);
     AM_HIP(hipGetLastError());
   }
   ProfScope ps("sort_msd_unit_scan");
@@ -967,7 +1095,7 @@ bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
     try {   // some 3 bytes a row beside the buffers above, without which the LSD passes sort
       w = msd_work(n, ITEMS, device_alloc);
       un = msd_analyse<K, W>(vals, type, valid, voff, n, dsc, placement, forder, ctl, w, epoch, key_out, key_xor,
-                             bucket_base, s);
+                             bucket_base, s, P == 4);
     } catch (const OutOfMemory&) {
       hybrid = false;
     }
@@ -981,11 +1109,7 @@ bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
     planned = true;
     digits = plan.mask ? plan.mask : 1u;
     if (value_rows) *value_rows = plan.m;
-    // 32-bit keys: the LSD passes are only four, so the hybrid sort must come out with about one level (every
-    // top-digit bucket at most 2^18 rows, which a second digit brings to bucket-sort size), or save whole
-    // passes over a large column. 10M float32 values over 10,000 distinct: LSD 481 us, hybrid 660; 40M
-    // uniform float32: 1.71 against 1.33 ms; 3M full-range int32: 237 against 167 us.
-    const bool take = ((plan.mask >> (P - 1)) & 1u) && (P == 8 || plan.top <= (1u << 18) || n >= (1u << 24));
+    const bool take = !plan.lsd && ((plan.mask >> (P - 1)) & 1u) && (P == 8 || plan.top <= MSD32_TOP_MAX || n >= MSD32_SAVES);
     if (pos_of_row && !take) return false;
     if (take) {
       tried = true;
@@ -1014,7 +1138,7 @@ bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
     hipLaunchKernelGGL(sort_init, dim3(1), dim3(1024), 0, s, ctl);
     AM_HIP(hipGetLastError());
   }
-  {
+  if (!plan.lsd) {
     // At most two workgroups per CU: each adds up to 256 counts per digit to shared ones.
     const uint32_t max_blocks = uint32_t(device().cu_count) * 2u;
     uint32_t blocks = std::max(1u, std::min(max_blocks, (n + 2u * UP_STEP - 1u) / (2u * UP_STEP)));

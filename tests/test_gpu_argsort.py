@@ -110,6 +110,35 @@ def test_key_shapes(n):
             check(vals, valid, True, place, label=f"nulls {frac}")
 
 
+@pytest.mark.parametrize("n", [1 << 16, 300_001, 2_000_003])
+@pytest.mark.parametrize("case,sweeps", [("small", 1), ("rare", 1), ("sampled_wide", 2), ("all_null", 1), ("one_value", 1),
+                                         ("hot", 1)])
+def test_analysis_of_32_bit_columns(case, sweeps, n):
+    """Columns that the LSD passes sort are counted for them in the first analysis, by a sample of 16 neighbours
+    at 16 places; a sample that misses the wide values, or sees nothing else, still leaves a sorted column."""
+    rng = np.random.default_rng(n)
+    x = rng.integers(-30_000, 30_000, n).astype(np.int32) if case == "hot" else rng.integers(0, 5000, n).astype(np.int32)
+    wide = O.splitmix64(9, n).astype(np.uint32).view(np.int32)
+    valid = rng.random(n) > 0.1
+    places = ((n - 16) * np.arange(16) // 15)[:, None] + np.arange(16)
+    if case == "rare": x[places[:-1, 0] + 50] = wide[:15]
+    elif case == "sampled_wide": x[places.ravel()] = wide[places.ravel()]
+    elif case == "all_null": valid[:] = False
+    elif case == "one_value": x[:] = -77
+    elif case == "hot": x = np.where(rng.random(n) < 0.97, x & 0xFFFF, wide).astype(np.int32)
+    if case == "hot": sweeps = 1 if n > 300_001 else None       # up to 2^18 rows on a digit the hybrid sort takes it
+    if case == "sampled_wide" and n <= 1 << 18: sweeps = None
+    for va, desc, place in ((valid, 1, 0), (None, 0, 1)):
+        am.prof_reset()
+        am.prof_enable(True)
+        got = gpu_argsort(x, va, desc, place, 0)
+        am.prof_enable(False)
+        ran = am.prof_report()
+        if sweeps is not None:
+            assert ran["sort_upsweep"][0] == sweeps and "sort_msd_first" not in ran, sorted(ran.items())
+        np.testing.assert_array_equal(got, O.argsort(x, va, desc, place, 0))
+
+
 @pytest.mark.parametrize("dtype", [np.int32, np.uint32, np.float32, np.int8, np.int16, np.uint8, np.uint16, np.uint64])
 def test_other_key_widths(dtype):
     rng = np.random.default_rng(3)
