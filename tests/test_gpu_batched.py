@@ -237,6 +237,7 @@ def test_plan_tuned_on_fewer_levels_than_a_later_run_needs():
     mk, mv, me, mh = m(gk), m(gv), m(easy), m(hard)
     plan = am.Batched(offs)
     plan.tune(me, mk, mv)
+    assert plan.config["sort_path"] == "msd"
     for keys, arr in ((easy, me), (hard, mh), (easy, me), (hard, mh)):
         plan.run(arr, mk, mv)
         got = plan.result("indices").to_numpy()[0]
@@ -249,3 +250,46 @@ def test_plan_tuned_on_fewer_levels_than_a_later_run_needs():
             assert goff[b + 1] - goff[b] == len(u)
             np.testing.assert_array_equal(sums[goff[b]:goff[b + 1]], np.bincount(inv, gv[lo:hi], len(u)).astype(np.int64))
             np.testing.assert_array_equal(counts[goff[b]:goff[b + 1]], np.bincount(inv, minlength=len(u)))
+
+
+def test_plan_short_of_levels_and_of_list_room_in_one_run(monkeypatch):
+    """Tuned on equal keys (no level, an entry per batch) with room for 64 entries: random keys need levels that
+    were not recorded, and then more entries than there are, and end in the LSD passes."""
+    monkeypatch.setenv("ARROWMETAL_MSD_LIST_CAP", "64")
+    offs = np.concatenate([[0], np.cumsum([300_000, 5, 40_000, 0, 2_000, 70_001])]).astype(np.int64)
+    n = int(offs[-1])
+    rng = np.random.default_rng(1)
+    gk, gv = rng.integers(0, 50, n), rng.integers(-1000, 1000, n)
+    equal, wide = np.full(n, 7, np.int64), O.splitmix64(5, n).view(np.int64)
+    m = lambda x: am.MetalArray.from_numpy(x)
+    mk, mv = m(gk), m(gv)
+    plan = am.Batched(offs)
+    plan.tune(m(equal), mk, mv)
+    assert plan.config["sort_path"] == "msd"
+    paths = []
+    for keys in (equal, wide, wide, equal):
+        plan.run(m(keys), mk, mv)
+        got = plan.result("indices").to_numpy()[0]
+        for b in range(len(offs) - 1):
+            lo, hi = int(offs[b]), int(offs[b + 1])
+            np.testing.assert_array_equal(got[lo:hi], O.argsort(keys[lo:hi]))
+        check_groups(plan, gk, gv, offs, "after the sort")
+        paths.append(plan.config["sort_path"])
+    assert paths == ["msd", "lsd", "lsd", "lsd"]
+
+
+@pytest.mark.parametrize("nbatches", [1023, 8192, 8193, 17_001])
+def test_overflowing_batches_are_counted(nbatches):
+    """The run's report counts the batches whose group table ran out of room, 8,192 flags at a time."""
+    over = sorted({0, nbatches // 2, nbatches - 1, min(8191, nbatches - 2)})
+    lens = np.full(nbatches, 2)
+    lens[over] = 400
+    offs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    gk = np.arange(int(offs[-1]), dtype=np.int64) * 1_000_003
+    gv = np.ones(len(gk), np.int64)
+    plan = am.Batched(offs, hash_capacity=64)
+    plan.run(None, am.MetalArray.from_numpy(gk), am.MetalArray.from_numpy(gv))
+    assert plan.config["regrouped_batches"] == len(over)
+    goff = plan.result("group_offsets").to_numpy()[0]
+    np.testing.assert_array_equal(goff, offs)
+    np.testing.assert_array_equal(plan.result("keys").to_numpy()[0], gk)
