@@ -266,7 +266,7 @@ __global__ __launch_bounds__(BLOCK) void sort_upsweep(const void* vals, const ui
   for (int i = threadIdx.x; i < P * RADIX; i += BLOCK) (&h[0][0])[i] = 0u;
   __syncthreads();
   const uint32_t begin = blockIdx.x * rows_per_block;
-  const uint32_t end = min(n, begin + rows_per_block);
+  const uint32_t end = begin + min(n - begin, rows_per_block);   // (begin + rows_per_block may pass 2^32)
   UpStat st{0ull, ~0ull, 0u, 0u, 0u, 0u};
   up_steps<W>(vals, valid, voff, begin, end, [&](uint64_t base, const uint64_t (&raw)[UP_ITEMS], const uint32_t (&vb)[UP_ITEMS]) {
     K kk[UP_ITEMS];
@@ -312,6 +312,8 @@ __global__ __launch_bounds__(BLOCK) void sort_upsweep(const void* vals, const ui
 // 1M-row input still has ~250 units to spread over the CUs.
 constexpr uint32_t UNIT_SHIFT_LARGE = 14, UNIT_SHIFT_SMALL = 12;
 constexpr uint32_t UNITS_PER_BLOCK = 8;   // most units one workgroup counts
+// Most rows of the hybrid sort: a workgroup's, a unit's and a tile's first row past the end are 32-bit numbers.
+constexpr uint32_t HYBRID_MAX_ROWS = UINT32_MAX - (UNITS_PER_BLOCK << UNIT_SHIFT_LARGE);
 
 // 32-bit keys have four LSD passes only, so the hybrid sort must come out with about one level (every
 // top-digit bucket at most 2^18 rows, which a second digit brings to bucket-sort size), or save whole passes
@@ -1060,7 +1062,7 @@ bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
               uint32_t* value_rows = nullptr, uint32_t* bucket_base = nullptr, void* key_out = nullptr,
               unsigned long long key_xor = 0, bool* keys_written = nullptr) {
   constexpr int P = int(sizeof(K));
-  const bool hybrid_ok = n >= hybrid_min(type) && !capturing(s);
+  const bool hybrid_ok = n >= hybrid_min(type) && n <= HYBRID_MAX_ROWS && !capturing(s);
   if (pos_of_row && !hybrid_ok) return false;
   constexpr int TILE = BLOCK * ITEMS;
   // The first pass keeps at most 16 keys per thread: its raw-column loads and 258-bin classification
@@ -1616,7 +1618,7 @@ Array* sorted_ints_t(const Array& a, bool desc, int placement, Array* idx, hipSt
 }  // namespace
 
 bool distinct_rows(const void* keys, int width, uint32_t n, DevBuf& rows, uint32_t& kept) {
-  if (capturing(stream())) return false;
+  if (n > HYBRID_MAX_ROWS || capturing(stream())) return false;
   return width == 8 ? distinct_rows_t<unsigned long long>(keys, n, rows, kept, stream())
                     : distinct_rows_t<uint32_t>(keys, n, rows, kept, stream());
 }
@@ -1686,7 +1688,7 @@ Array* sorted_ints(const Array& a, bool descending, int null_placement) {
   check_length(a.length);
   check_index_rows(a.length, "argsort");
   if ((a.type != T_I64 && a.type != T_U64 && a.type != T_I32 && a.type != T_U32) || a.length < int64_t(hybrid_min(a.type)) ||
-      capturing(stream()))
+      a.length > int64_t(HYBRID_MAX_ROWS) || capturing(stream()))
     return nullptr;
   Array* idx = new_array("I", T_U32, a.length);
   struct Drop {

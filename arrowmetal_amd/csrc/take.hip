@@ -607,7 +607,7 @@ bool permute_columns(const std::vector<const Array*>& cols, const Array& idx, st
       o->values = device_alloc(size_t(n) * c->width());
       if (o->null_count > 0) o->validity = device_alloc(size_t((n + 63) / 64) * 8);
     }
-    const dim3 grid((uint32_t(n) + 255u) / 256u), block(256);
+    const dim3 grid(uint32_t((n + 255) / 256)), block(256);
     for (size_t k = 0; k < order.size();) {
       const PackCols p = pack_group(cols, out, order, k);
       DevBuf rows;
