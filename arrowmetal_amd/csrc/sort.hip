@@ -1142,10 +1142,10 @@ bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
   }
   if (!plan.lsd) {
     // At most two workgroups per CU: each adds up to 256 counts per digit to shared ones.
-    const uint32_t max_blocks = uint32_t(device().cu_count) * 2u;
-    uint32_t blocks = std::max(1u, std::min(max_blocks, (n + 2u * UP_STEP - 1u) / (2u * UP_STEP)));
-    const uint32_t rpb = ((n + blocks - 1) / blocks + UP_STEP - 1) / UP_STEP * UP_STEP;
-    blocks = (n + rpb - 1) / rpb;
+    const uint64_t rows = n, max_blocks = uint64_t(device().cu_count) * 2u;   // 64 bits: the sums may pass 2^32
+    const uint64_t wanted = std::max<uint64_t>(1, std::min(max_blocks, (rows + 2u * UP_STEP - 1u) / (2u * UP_STEP)));
+    const uint32_t rpb = uint32_t(std::min<uint64_t>(((rows + wanted - 1) / wanted + UP_STEP - 1) / UP_STEP * UP_STEP, UINT32_MAX));
+    const uint32_t blocks = uint32_t((rows + rpb - 1) / rpb);
     {
       ProfScope ps("sort_upsweep");
       hipLaunchKernelGGL((sort_upsweep<K, W>), dim3(blocks), dim3(BLOCK), 0, s, vals, valid, voff, n, type, forder, dsc, rpb,
