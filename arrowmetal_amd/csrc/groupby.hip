@@ -1037,17 +1037,7 @@ struct AggArgs {
   int64_t n;
   long long K;
   const void* aux;               // family-specific (exact float sums: the groups' grid words)
-  const long long* hot;          // HOT_GROUPS ids (-1: none) summed in registers, or null
 };
-
-// Up to this many of a column's most frequent groups (from a sample of its ids) are summed in each
-// lane's registers by the families whose words are all additions (sums and counts), so that the rows
-// of a hot group take no atomic at all: with Zipf(1.1) keys the top group alone is ~13% of the rows,
-// about nine lanes of every wave, whose LDS atomics on one word would otherwise serialize.
-#ifndef AM_HOT_GROUPS
-#define AM_HOT_GROUPS 8
-#endif
-constexpr int HOT_GROUPS = AM_HOT_GROUPS;
 
 // count_all (values ignored) and count (non-null values).
 template <bool VALID_ONLY>
@@ -1302,16 +1292,6 @@ constexpr int AGG_ROWS = AM_AGG_ROWS;   // rows per thread per step, whose loads
 #ifndef AM_AGG_PROBES
 #define AM_AGG_PROBES 8   // LDS cache slots a row probes before its group goes to the XCD's table
 #endif
-#ifndef AM_AGG_HOT
-#define AM_AGG_HOT 0      // sampled hot groups summed in registers (1), or not (0)
-#endif
-
-template <class P>
-__host__ __device__ constexpr bool all_add() {
-  for (int w = 0; w < P::W; w++)
-    if (P::op(w) != W_ADD) return false;
-  return true;
-}
 
 // The rows one thread has in flight: group ids, values and validity bytes exactly as loaded. The bits
 // are taken out only when the rows are used, so that nothing that is loaded is waited on before the
@@ -1347,15 +1327,12 @@ struct AggState {
   unsigned long long* gtab;   // this XCD's table [K][W] (not in mode 2)
   int mode;
   uint32_t cap;
-  long long hot[HOT_GROUPS];
-  unsigned long long hacc[HOT_GROUPS][P::W];
 };
 
 // The updates of one step's rows (loaded by agg_load at `base`).
 template <class P, int IDW, int VW>
 __device__ __forceinline__ void agg_rows(const AggArgs& a, int64_t base, int64_t end, const AggRows<IDW>& cur,
                                          AggState<P>& st) {
-  constexpr bool HOTREG = AM_AGG_HOT && all_add<P>();
   // Every loaded register is taken here, on every path: a load whose register is only read on some
   // paths is still in flight, as far as the compiler knows, when that register is next written, and
   // that write then waits for all memory operations.
@@ -1390,22 +1367,6 @@ __device__ __forceinline__ void agg_rows(const AggArgs& a, int64_t base, int64_t
     for (int r = 0; r < AGG_ROWS; r++) {
       const int64_t i = base + int64_t(r) * blockDim.x + threadIdx.x;
       if (!P::contrib(a, i, gs[r], val_in(a.v, cur.vr[r]), cs[r])) gs[r] = -1;
-    }
-  }
-  if (HOTREG && st.hot[0] >= 0) {   // uniform; the sampler fills hot[] most frequent first
-    // A hot group's contribution goes to this lane's registers (the hot ids are distinct, and an
-    // unused entry's accumulator is never flushed).
-#pragma unroll
-    for (int r = 0; r < AGG_ROWS; r++) {
-      bool any = false;
-#pragma unroll
-      for (int j = 0; j < HOT_GROUPS; j++) {
-        const bool m = gs[r] == st.hot[j];
-#pragma unroll
-        for (int w = 0; w < P::W; w++) st.hacc[j][w] += m ? cs[r][w] : 0ull;
-        any = any || m;
-      }
-      if (any) gs[r] = -1;
     }
   }
   if (st.mode != 1) {
@@ -1465,21 +1426,12 @@ template <class P, int IDW, int VW>
 __global__ __launch_bounds__(AM_AGG_THREADS) void gb_agg(AggArgs a, int mode, uint32_t cap, int64_t rpb,
                                               unsigned long long* gtab8) {
   extern __shared__ unsigned long long lds[];
-  constexpr bool HOTREG = AM_AGG_HOT && all_add<P>();
   AggState<P> st;
   st.lacc = lds;
   st.lkey = reinterpret_cast<unsigned int*>(lds + size_t(cap) * P::W);
   st.gtab = gtab8 + size_t(mode == 2 ? blockIdx.x : xcd_id()) * size_t(a.K) * P::W;
   st.mode = mode;
   st.cap = cap;
-#pragma unroll
-  for (int j = 0; j < HOT_GROUPS; j++) {
-    const long long h = HOTREG && a.hot ? a.hot[j] : -1;   // the same for every lane
-    st.hot[j] = (long long)(((unsigned long long)uint32_t(__builtin_amdgcn_readfirstlane(int(h >> 32))) << 32) |
-                            uint32_t(__builtin_amdgcn_readfirstlane(int(h))));
-#pragma unroll
-    for (int w = 0; w < P::W; w++) st.hacc[j][w] = 0ull;
-  }
   for (uint32_t s = threadIdx.x; s < cap; s += blockDim.x) {
 #pragma unroll
     for (int w = 0; w < P::W; w++) st.lacc[size_t(s) * P::W + w] = identity(P::op(w));
@@ -1503,21 +1455,6 @@ __global__ __launch_bounds__(AM_AGG_THREADS) void gb_agg(AggArgs a, int mode, ui
       agg_rows<P, IDW, VW>(a, base + step, end, rb, st);
     }
   }
-  if constexpr (HOTREG) {
-    // Each wave's sum of its lanes' hot accumulators, added once into this XCD's table.
-#pragma unroll
-    for (int j = 0; j < HOT_GROUPS; j++) {
-      if (st.hot[j] < 0) continue;   // uniform
-#pragma unroll
-      for (int w = 0; w < P::W; w++) {
-        unsigned long long v = st.hacc[j][w];
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-        st.hacc[j][w] = v;
-      }
-      if ((threadIdx.x & 63) == 0) apply<P>(as_global(&st.gtab[size_t(st.hot[j]) * P::W]), st.hacc[j]);
-    }
-  }
   __syncthreads();
   if (mode == 2) {
     for (uint32_t j = threadIdx.x; j < uint32_t(a.K) * P::W; j += blockDim.x) st.gtab[j] = st.lacc[j];
@@ -1528,76 +1465,6 @@ __global__ __launch_bounds__(AM_AGG_THREADS) void gb_agg(AggArgs a, int mode, ui
     if (mode == 0) g = sl < uint32_t(a.K) ? (long long)sl : -1;
     else g = st.lkey[sl] == 0xFFFFFFFFu ? -1 : (long long)st.lkey[sl];
     if (g >= 0) flush_one<P>(as_global(&st.gtab[size_t(g) * P::W]), as_lds(&st.lacc[size_t(sl) * P::W]));
-  }
-}
-
-// The most frequent group ids of a sample of the rows: S rows at even strides counted in an LDS
-// table, then the HOT_GROUPS largest counts of at least S / 64 (about one lane per wave). One
-// workgroup of 1024 threads (four rows each); hot[j] = -1 where there is no such group.
-constexpr uint32_t HOT_SAMPLE = 4096;   // a group of >= 1/64 of the rows shows ~64 times
-constexpr uint32_t HOT_SLOTS = 8192;    // twice the sample: probe chains stay short
-__global__ __launch_bounds__(1024) void gb_hot_sample(IdSource ids, int64_t n, long long K, long long* hot) {
-  __shared__ uint32_t skey[HOT_SLOTS];
-  __shared__ uint32_t scnt[HOT_SLOTS];
-  __shared__ unsigned long long best[32];
-  for (uint32_t i = threadIdx.x; i < HOT_SLOTS; i += blockDim.x) {
-    skey[i] = 0xFFFFFFFFu;
-    scnt[i] = 0u;
-  }
-  __syncthreads();
-  const uint32_t S = uint32_t(std::min<int64_t>(n, HOT_SAMPLE));
-  constexpr int IN_FLIGHT = 4;
-  for (uint32_t b = threadIdx.x; b < S; b += blockDim.x * IN_FLIGHT) {
-    long long g[IN_FLIGHT];
-#pragma unroll
-    for (int k = 0; k < IN_FLIGHT; k++) {
-      const uint32_t t = b + uint32_t(k) * blockDim.x;
-      const int64_t row = t < S ? int64_t(uint64_t(t) * uint64_t(n) / S) : 0;   // n < 2^33, S <= 2^16
-      g[k] = t < S ? load_gid(ids, row, K) : -1;
-    }
-#pragma unroll
-    for (int k = 0; k < IN_FLIGHT; k++) {
-      if (g[k] < 0) continue;
-      uint32_t h = uint32_t(g[k]) * 2654435761u;
-      uint32_t sl = (h ^ (h >> 15)) & (HOT_SLOTS - 1);
-      for (uint32_t probe = 0; probe < 64; probe++) {   // a full table drops the row from the sample
-        uint32_t c = skey[sl];
-        if (c == 0xFFFFFFFFu) {
-          const uint32_t prev = atomicCAS(&skey[sl], 0xFFFFFFFFu, uint32_t(g[k]));
-          c = prev == 0xFFFFFFFFu ? uint32_t(g[k]) : prev;
-        }
-        if (c == uint32_t(g[k])) {
-          atomicAdd(&scnt[sl], 1u);
-          break;
-        }
-        sl = (sl + 1u) & (HOT_SLOTS - 1);
-      }
-    }
-  }
-  __syncthreads();
-  const uint32_t floor = std::max<uint32_t>(S / 64u, 2u);
-  for (int j = 0; j < HOT_GROUPS; j++) {
-    // (count << 32 | ~slot): the largest count, lowest slot on ties.
-    unsigned long long mine = 0ull;
-    for (uint32_t i = threadIdx.x; i < HOT_SLOTS; i += blockDim.x) {
-      const unsigned long long c = (unsigned long long)scnt[i] << 32 | (0xFFFFFFFFull - i);
-      mine = c > mine ? c : mine;
-    }
-    for (int off = 32; off >= 1; off >>= 1) {
-      const unsigned long long o = __shfl_xor(mine, off, 64);
-      mine = o > mine ? o : mine;
-    }
-    if ((threadIdx.x & 63) == 0) best[threadIdx.x >> 6] = mine;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      unsigned long long m = 0ull;
-      for (uint32_t w = 0; w < blockDim.x / 64; w++) m = best[w] > m ? best[w] : m;
-      const uint32_t slot = 0xFFFFFFFFu - uint32_t(m);
-      const uint32_t cnt = uint32_t(m >> 32);
-      hot[j] = cnt >= floor ? (long long)skey[slot] : -1;
-      if (cnt > 0u) scnt[slot] = 0u;
-    }
-    __syncthreads();
   }
 }
 
@@ -2828,7 +2695,6 @@ struct GroupBy {
   bool cnt_all_rows = false;   // column cnt_col had no nulls: its counts are the rows per group
   DevBuf count_all_tab;    // K x 1 rows per group
   PartSet part;            // the partitioned records of the last value column (many groups)
-  DevBuf hot;              // HOT_GROUPS sampled frequent ids (sums and counts in registers)
   // The mapping is left running when am_group_by_keys returns: `ready` is recorded on `owner` after
   // its last kernel. Calls on another thread's stream wait for it, and the handle's release waits
   // before the key columns can be freed.
@@ -4335,22 +4201,6 @@ Array* fs_array(const DevBuf& vals, const DevBuf& bits, int64_t nulls, long long
 }
 
 // The shared op table of am_group_agg_ex and am_group_by over an id source.
-// The sampled hot groups of the ids (gb_hot_sample), once per mapping; none for small inputs.
-const long long* hot_groups(const IdSource& ids, int64_t n, long long K, GroupBy* cache, DevBuf& holder) {
-  if (!AM_AGG_HOT || n < (int64_t(1) << 20)) return nullptr;
-  if (cache && cache->hot) return static_cast<const long long*>(cache->hot->ptr);
-  holder = device_alloc(HOT_GROUPS * sizeof(long long));
-  retain(holder);
-  {
-    ProfScope ps("gb_hot_sample");
-    hipLaunchKernelGGL(gb_hot_sample, dim3(1), dim3(1024), 0, stream(), ids, n, K,
-                       static_cast<long long*>(holder->ptr));
-    AM_HIP(hipGetLastError());
-  }
-  if (cache) cache->hot = holder;
-  return static_cast<const long long*>(holder->ptr);
-}
-
 // A transform of the value column (am_query's (shr c N) / (bit_and c N)).
 struct ValX {
   int op = VX_NONE;
@@ -4359,14 +4209,12 @@ struct ValX {
 
 Array* aggregate(const IdSource& ids, int64_t n, long long K, const Array* v, int op, GroupBy* cache, ValX vx = {}) {
   hipStream_t s = stream();
-  DevBuf hot_holder;
   if (op == 1) {
     // An integer sum of a column without nulls already counted every row of each group (word 1).
     if (cache && !cache->count_all_tab && cache->cnt_tab && cache->cnt_all_rows)
       return column_of_table<2>(cache->cnt_tab, K, KIND_SUM_COUNT, T_I64, "l", T_I64);
     if (cache && cache->count_all_tab) return column_of_table<1>(cache->count_all_tab, K, KIND_COUNT, T_I64, "l", T_I64);
     AggArgs a = make_args(ids, nullptr, n, K);
-    a.hot = hot_groups(ids, n, K, cache, hot_holder);
     Result r("l", T_I64, K, false);
     DevBuf t = run_agg<CountP<false>>(a, s, "gb_count", FinSimple{KIND_COUNT, T_I64, r.values()}, r.fo);
     if (cache) cache->count_all_tab = t;
@@ -4381,7 +4229,6 @@ Array* aggregate(const IdSource& ids, int64_t n, long long K, const Array* v, in
     // A column without nulls has as many non-null values per group as rows.
     if (cache && cache->count_all_tab && !v->has_nulls()) return column_of_table<1>(cache->count_all_tab, K, KIND_COUNT, T_I64, "l", T_I64);
     AggArgs a = make_args(ids, v, n, K);
-    a.hot = hot_groups(ids, n, K, cache, hot_holder);
     Result r("l", T_I64, K, false);
     run_agg<CountP<true>>(a, s, "gb_count", FinSimple{KIND_COUNT, T_I64, r.values()}, r.fo, cache ? &cache->part : nullptr, v->uid);
     return r.finish();
@@ -4414,7 +4261,6 @@ Array* aggregate(const IdSource& ids, int64_t n, long long K, const Array* v, in
     const char* fmt = op == 3 ? "g" : u64 ? "L" : "l";
     const int otype = op == 3 ? T_F64 : u64 ? T_U64 : T_I64;
     if (cache && cache->cnt_col == v->uid && cache->cnt_tab) return column_of_table<2>(cache->cnt_tab, K, kind, v->type, fmt, otype);
-    a.hot = hot_groups(ids, n, K, cache, hot_holder);
     Result r(fmt, otype, K, true);
     DevBuf t = run_agg<SumCountP>(a, s, "gb_sum", FinSimple{kind, v->type, r.values()}, r.fo, cache ? &cache->part : nullptr, v->uid);
     if (cache) { cache->cnt_col = v->uid; cache->cnt_tab = t; cache->cnt_all_rows = !v->has_nulls(); }
