@@ -3041,8 +3041,8 @@ CompositeCol key_col(const Array& a) {
   return CompositeCol{a.data(), a.has_nulls() ? a.valid_bits() : nullptr, a.offset, a.type, ColSpan{}};
 }
 
-// Bijections of 32 and 64 bits that spread the keys over all digits (odd multipliers and xor-shifts; the
-// 64-bit one is mix64).
+// Bijections of 32 and 64 bits that spread the keys over all digits. The 64-bit one is mix64; the 32-bit one is
+// "lowbias32" of C. Wellons' Hash Prospector (2018, public domain): xor-shifts and odd multipliers of low bias.
 __device__ __forceinline__ unsigned long long spread_key(unsigned long long k) { return mix64(k); }
 __device__ __forceinline__ uint32_t spread_key(uint32_t k) {
   k ^= k >> 16;
@@ -3163,7 +3163,8 @@ struct SmallOut {
   uint32_t *dslot, *drow, *gid;   // gid[SMALL_SLOTS + 2]: each slot's id, once ranked
 };
 
-// A key's home slot.
+// A key's home slot: its halves by the first two 32-bit primes of xxHash (Y. Collet; the first is 2^32 over the
+// golden ratio, next odd), folded and multiplied once more (a multiplier of the Hash Prospector).
 __device__ __forceinline__ uint32_t small_slot(unsigned long long k) {
   uint32_t x = uint32_t(k) * 0x9E3779B1u ^ uint32_t(k >> 32) * 0x85EBCA77u;
   x ^= x >> 15;
