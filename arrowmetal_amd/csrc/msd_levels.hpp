@@ -1,4 +1,4 @@
-// The levels of the adaptive MSD radix argsort of 64-bit keys, shared by the plain argsort (sort.hip)
+// The levels of the adaptive MSD radix argsort of 64- and 32-bit keys, shared by the plain argsort (sort.hip)
 // and the batched plan (batched.hip).
 //
 // Rows are in buckets (Bucket: a range of the value block, in one of two key / row buffers, or in the

@@ -562,8 +562,8 @@ __global__ __launch_bounds__(BLOCK) void sort_mid(int pass, SortCtl* ctl, unsign
 // the places of its own 64 rows, each the number of keys before it in the stable order. No workgroup
 // waits for another, and nothing is read back; the work is n^2 compares spread over n / 64 workgroups.
 // The LSD passes need a launch per digit, each bound by its launch and one tile's latency. Measured, the
-// whole call, int64 (int32) keys with nulls: 1,000 rows 81 -> 18 us (63 -> 18), 8,000 rows 107 -> 31
-// (71 -> 30), 16,000 rows 111 -> 47 (75 -> 45). Beyond 16,384 rows the keys no longer fit in LDS and the
+// whole call, int64 (int32) keys with nulls: 1,000 rows 75 -> 18 us (55 -> 18), 8,000 rows 102 -> 30
+// (67 -> 30), 16,000 rows 109 -> 46 (71 -> 44). Beyond 16,384 rows the keys no longer fit in LDS and the
 // compares of every CU grow with n^2: the passes take over.
 constexpr uint32_t RANK_THREADS = 1024;
 constexpr uint32_t RANK_WAVES = RANK_THREADS / 64;

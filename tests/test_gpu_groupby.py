@@ -241,7 +241,7 @@ def test_integer_columns_as_composite_keys(case, n):
                                     (32768, 300), (32769, 300)])
 def test_small_inputs_in_one_launch(case, n, span, monkeypatch):
     """Up to 32,768 rows and 4,096 distinct keys the mapping is one launch: ids, keys, aggregates and unique
-    rows against the oracle at the edges of its rows, its key sort (1,024) and its key limit, where it
+    rows against the oracle at the edges of its rows and its key limit, where it
     gives up, and the same with it switched off."""
     rng = np.random.default_rng(n * 7 + span)
     k = rng.permutation(np.resize(np.arange(span), n))
@@ -285,6 +285,40 @@ def test_small_inputs_in_one_launch(case, n, span, monkeypatch):
                 got = g.count_all() if op == 1 else getattr(g, ("sum", "", "count", "mean", "min", "max")[op])(mv)
                 assert_agg(got, O.group_agg(ids, K, values, op, vv), f"{case} op {op}")
         np.testing.assert_array_equal(am.unique_rows(arrays).to_numpy()[0], O.unique_rows(cols, valid))
+
+
+@pytest.mark.parametrize("distinct,zero,ranks_apart,taken", [
+    (255, True, False, True), (256, False, False, True), (256, True, False, True), (257, False, True, True),
+    (257, True, True, True), (4095, False, True, True), (4095, True, True, True), (4096, True, True, True),
+    (4096, False, False, False), (4097, True, False, False)])
+@pytest.mark.parametrize("nulls", [False, True])
+def test_small_inputs_at_the_edges_of_their_key_counts(distinct, zero, ranks_apart, taken, nulls):
+    """Up to 256 keys the one launch ranks them itself; up to 4,095, and the key 0 beside them (its order key
+    looks like an empty slot), other launches do; beyond, the general mapping takes the input."""
+    rng = np.random.default_rng(distinct)
+    n = 12_345
+    keys = rng.choice(np.arange(1, 1 << 20), distinct, replace=False).astype(np.int64) * 0x9E3779B97F - 2**58
+    if zero:
+        keys[rng.integers(0, distinct)] = 0
+    k = rng.permutation(np.resize(keys, n))
+    valid = rng.random(n) > 0.01 if nulls else None
+    if nulls:
+        valid[np.unique(k, return_index=True)[1]] = True
+    a = am.MetalArray.from_numpy(k, valid)
+    ids, K, rep = O.group_keys([k], [valid])
+    assert K == distinct + nulls
+    am.prof_reset()
+    am.prof_enable(True)
+    g = am.group_by([a])
+    got = g.ids().to_numpy()[0]
+    am.prof_enable(False)
+    names = set(am.prof_report())
+    assert "gb_small_map" in names and ("gb_small_rank" in names) == ranks_apart and ("gb_build" in names) != taken, names
+    np.testing.assert_array_equal(got, ids)
+    gvals, gv = g.key_arrays()[0].to_numpy()
+    np.testing.assert_array_equal(gvals[:distinct], k[rep][:distinct])
+    assert (gv is None) == (not nulls) and (gv is None or (gv[:distinct].all() and not gv[distinct]))
+    np.testing.assert_array_equal(am.unique_rows([a]).to_numpy()[0], O.unique_rows([k], [valid]))
 
 
 @pytest.mark.parametrize("case", ["distinct", "few", "hot", "runs", "full_range", "wide_pair", "nulls", "one_key", "narrow"])
