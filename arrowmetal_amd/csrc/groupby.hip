@@ -3847,8 +3847,10 @@ DevBuf first_rows(const DevBuf& ids, int64_t n, int64_t K) {
   hipStream_t s = stream();
   DevBuf rep = device_alloc(size_t(std::max<int64_t>(K, 1)) * 4);
   auto* r = static_cast<uint32_t*>(rep->ptr);
-  if (K > int64_t(PART_MAX_NB) * PART_G) {
-    // More groups than the partitioned passes take: few rows share a group on average.
+  if (K > int64_t(PART_MAX_NB) * PART_G || (n <= int64_t(SMALL_ROWS) && K > int64_t(agg_dense_cap<FirstRowP>()))) {
+    // More groups than the partitioned passes take: few rows share a group on average. Or few rows: two launches
+    // instead of five (20,000 different float64 keys, the call 302 -> 274 us; from 50,000 rows a hot key's
+    // atomics, one after another, cost more than that: 100,000 rows, half on one key, 333 against 504).
     hipLaunchKernelGGL(gb_fill_u32, dim3(grid_for(K, 4)), dim3(256), 0, s, r, size_t(K), 0xFFFFFFFFu);
     hipLaunchKernelGGL(gb_first_atomic, dim3(grid_for(n)), dim3(256), 0, s, static_cast<const uint32_t*>(ids->ptr), uint32_t(n), r);
     AM_HIP(hipGetLastError());

@@ -420,6 +420,20 @@ def test_lowest_rows_of_more_groups_than_the_partitioned_passes_take():
     np.testing.assert_array_equal(got, O.unique_rows([keys], [None]))
 
 
+@pytest.mark.parametrize("n", [8193, 20_011, 32_768, 32_769])
+@pytest.mark.parametrize("hot", [0.0, 0.4])
+def test_lowest_rows_of_few_rows_in_many_groups(n, hot):
+    """Up to 32,768 rows in more groups than an LDS table holds: atomics, with and without a hot key."""
+    rng = np.random.default_rng(n)
+    keys = np.where(rng.random(n) < hot, 2.5, rng.permutation(n).astype(np.float64))
+    valid = rng.random(n) > 0.01
+    a = am.MetalArray.from_numpy(keys, valid)
+    np.testing.assert_array_equal(am.unique_rows([a]).to_numpy()[0], O.unique_rows([keys], [valid]))
+    ids, K, rep = O.group_keys([keys], [valid])
+    gvals, gv = am.group_by([a]).key_arrays()[0].to_numpy()
+    np.testing.assert_array_equal(gvals[gv], keys[rep][valid[rep]])
+
+
 def test_exact_float_sum_edges():
     groups = vectors()["group_sum_edges"]["groups"]
     keys, vals = [], []
