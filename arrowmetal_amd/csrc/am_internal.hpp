@@ -229,8 +229,8 @@ void argsort_device(const void* vals, int type, const uint8_t* validity, int64_t
                     bool descending, int null_placement, int float_order, uint32_t* out_idx,
                     hipStream_t s);
 
-// The lowest row of every distinct key, ascending, in `rows` (`kept` entries, in a block of
-// at most about twice their size): n mixed keys of
+// The lowest row of every distinct key, ascending, in `rows` (`kept` entries, in a block of at most about
+// eight times their size, or 4 MiB): n mixed keys of
 // `width` bytes (4 or 8), bits spread over all digits. Returns false, with nothing in `rows`, when the keys
 // do not take the partition (a constant top digit, a full bucket list, a graph capture).
 bool distinct_rows(const void* keys, int width, uint32_t n, DevBuf& rows, uint32_t& kept);
