@@ -99,18 +99,35 @@ __device__ __forceinline__ void count_bin(uint32_t* h, uint32_t b) {
   }
 }
 
-// The same with a check for a digit that is one on all counting lanes only: cheaper, for the LSD passes' analysis
-// of every digit (10M uniform float32 keys: 32 us less than with count_bin).
+// The same with a check for a digit that is one on the whole wave only: cheaper, for the LSD passes' analysis
+// of every digit (10M uniform float32 keys: 32 us less than with count_bin). In a column with nulls, one on all
+// lanes that count.
+template <bool NULLS>
 __device__ __forceinline__ void count_digit(uint32_t* h, uint32_t b) {
-  const unsigned long long m = __ballot(b != ~0u);
-  if (m == 0ull) return;   // uniform
-  const int first = __builtin_ctzll(m);
-  const uint32_t lead = __builtin_amdgcn_readlane(b, first);
-  if (__ballot(b == lead) == m) {   // uniform
-    if (int(threadIdx.x & 63u) == first) atomicAdd(&h[lead], uint32_t(__popcll(m)));
-  } else if (b != ~0u) {
-    atomicAdd(&h[b], 1u);
+  if constexpr (!NULLS) {
+    const uint32_t lead = __builtin_amdgcn_readfirstlane(b);
+    if (__all(b == lead)) {   // uniform
+      if (lead != ~0u && (threadIdx.x & 63u) == 0u) atomicAdd(&h[lead], 64u);
+      return;
+    }
+  } else {
+    const unsigned long long m = __ballot(b != ~0u);
+    if (m == 0ull) return;
+    const int first = __builtin_ctzll(m);
+    const uint32_t lead = __builtin_amdgcn_readlane(b, first);
+    if (__ballot(b == lead) == m) {   // uniform
+      if (int(threadIdx.x & 63u) == first) atomicAdd(&h[lead], uint32_t(__popcll(m)));
+      return;
+    }
   }
+  if (b != ~0u) atomicAdd(&h[b], 1u);
+}
+
+// f(std::true_type) for a column with a validity bitmap, f(std::false_type) for one without.
+template <class F>
+__device__ __forceinline__ void with_nulls(const uint8_t* valid, F&& f) {
+  if (valid) f(std::true_type{});
+  else f(std::false_type{});
 }
 
 // Runs count(base, raw, vb) over the rows [begin, end) of a workgroup, UP_ITEMS rows per thread per step,
@@ -271,16 +288,19 @@ __global__ __launch_bounds__(BLOCK) void sort_upsweep(const void* vals, const ui
   const uint32_t begin = blockIdx.x * rows_per_block;
   const uint32_t end = begin + min(n - begin, rows_per_block);   // (begin + rows_per_block may pass 2^32)
   UpStat st{0ull, ~0ull, 0u, 0u, 0u, 0u};
-  up_steps<W>(vals, valid, voff, begin, end, [&](uint64_t base, const uint64_t (&raw)[UP_ITEMS], const uint32_t (&vb)[UP_ITEMS]) {
-    K kk[UP_ITEMS];
-    int cc[UP_ITEMS];
-    up_classify<K>(base, end, raw, vb, valid != nullptr, voff, type, forder, desc, kk, cc, st);
+  with_nulls(valid, [&](auto nulls) {
+    constexpr bool NULLS = decltype(nulls)::value;
+    up_steps<W>(vals, valid, voff, begin, end, [&](uint64_t base, const uint64_t (&raw)[UP_ITEMS], const uint32_t (&vb)[UP_ITEMS]) {
+      K kk[UP_ITEMS];
+      int cc[UP_ITEMS];
+      up_classify<K>(base, end, raw, vb, NULLS, voff, type, forder, desc, kk, cc, st);
 #pragma unroll
-    for (int p = 0; p < P; p++) {
-      if (!((digits >> p) & 1u)) continue;   // uniform
+      for (int p = 0; p < P; p++) {
+        if (!((digits >> p) & 1u)) continue;   // uniform
 #pragma unroll
-      for (int u = 0; u < UP_ITEMS; u++) count_digit(h[p], cc[u] == 0 ? uint32_t(kk[u] >> (8 * p)) & 0xFFu : ~0u);
-    }
+        for (int u = 0; u < UP_ITEMS; u++) count_digit<NULLS>(h[p], cc[u] == 0 ? uint32_t(kk[u] >> (8 * p)) & 0xFFu : ~0u);
+      }
+    });
   });
   up_reduce(st, s_st);
   __syncthreads();
@@ -368,15 +388,18 @@ __global__ __launch_bounds__(BLOCK) void msd_upsweep(const void* vals, const uin
   UpStat st{0ull, ~0ull, 0u, 0u, 0u, 0u};
   if (lsd) {   // uniform over the grid
     static_assert(UNITS_PER_BLOCK * NBINS_FIRST >= 4 * RADIX, "the digits' counts fit where the units' are");
-    up_steps<W>(vals, valid, voff, begin, end, [&](uint64_t base, const uint64_t (&raw)[UP_ITEMS], const uint32_t (&vb)[UP_ITEMS]) {
-      K kk[UP_ITEMS];
-      int cc[UP_ITEMS];
-      up_classify<K>(base, end, raw, vb, valid != nullptr, voff, type, forder, desc, kk, cc, st);
+    with_nulls(valid, [&](auto nulls) {
+      constexpr bool NULLS = decltype(nulls)::value;
+      up_steps<W>(vals, valid, voff, begin, end, [&](uint64_t base, const uint64_t (&raw)[UP_ITEMS], const uint32_t (&vb)[UP_ITEMS]) {
+        K kk[UP_ITEMS];
+        int cc[UP_ITEMS];
+        up_classify<K>(base, end, raw, vb, NULLS, voff, type, forder, desc, kk, cc, st);
 #pragma unroll
-      for (uint32_t p = 0; p < 4; p++)
+        for (uint32_t p = 0; p < 4; p++)
 #pragma unroll
-        for (int u = 0; u < UP_ITEMS; u++)
-          count_digit(hu + p * RADIX, cc[u] == 0 ? uint32_t(kk[u] >> (8 * p)) & 0xFFu : ~0u);
+          for (int u = 0; u < UP_ITEMS; u++)
+            count_digit<NULLS>(hu + p * RADIX, cc[u] == 0 ? uint32_t(kk[u] >> (8 * p)) & 0xFFu : ~0u);
+      });
     });
     up_reduce(st, s_st);
     if (threadIdx.x == 0) stats[blockIdx.x] = st;
@@ -1144,8 +1167,9 @@ bool run_sort(const void* vals, int type, const uint8_t* valid, int64_t voff, ui
     AM_HIP(hipGetLastError());
   }
   if (!plan.lsd) {
-    // At most two workgroups per CU: each adds up to 256 counts per digit to shared ones.
-    const uint64_t rows = n, max_blocks = uint64_t(device().cu_count) * 2u;   // 64 bits: the sums may pass 2^32
+    // Two workgroups per CU, and four from 2^23 rows: each adds up to 256 counts per digit to shared ones, which a
+    // long share of rows repays (int64 below 5,000, 50M rows 1294 -> 1244 us; 1M float32 170 either way).
+    const uint64_t rows = n, max_blocks = uint64_t(device().cu_count) * (n >= (1u << 23) ? 4u : 2u);   // 64 bits: the sums may pass 2^32
     const uint64_t wanted = std::max<uint64_t>(1, std::min(max_blocks, (rows + 2u * UP_STEP - 1u) / (2u * UP_STEP)));
     const uint32_t rpb = uint32_t(std::min<uint64_t>(((rows + wanted - 1) / wanted + UP_STEP - 1) / UP_STEP * UP_STEP, UINT32_MAX));
     const uint32_t blocks = uint32_t((rows + rpb - 1) / rpb);
