@@ -344,26 +344,36 @@ constexpr uint32_t HYBRID_MAX_ROWS = UINT32_MAX - (UNITS_PER_BLOCK << UNIT_SHIFT
 // 1.71 against 1.33 ms; 3M full-range int32: 237 against 167 us.
 constexpr uint32_t MSD32_TOP_MAX = 1u << 18, MSD32_SAVES = 1u << 24;
 
-// Whether the LSD passes sort a 32-bit column, from 16 neighbours (a line) at each of 16 places over its length: one top digit on all of them, or
-// one on so many that its bucket is too large. (Only a guess at the faster way: either sorts any column. A
-// column that is counted for the one and sorted by the other is read once more: 1M int32 values of 0 to 2^20
-// 154 us so, 140 when guessed; full-range ones 125 and 126.) Every workgroup reads the same rows.
+// Whether the LSD passes sort a 32-bit column, from 4 neighbours at each of 16 places over its length, which every
+// wave reads: one top digit on all of them, or one on so many that its bucket is too large. (Only a guess at the
+// faster way: either sorts any column. A column that is counted for the one and sorted by the other is read once
+// more: 1M int32 values of 0 to 2^20 154 us so, 140 when guessed; of 6M full-range
+// ones 261 and 264.)
 template <typename K, int W>
 __device__ __forceinline__ bool sampled_lsd(const void* vals, const uint8_t* valid, int64_t voff, uint32_t n, int type,
-                                            int forder, int desc, uint32_t* h) {
-  h[threadIdx.x] = 0u;
-  __syncthreads();
-  const uint32_t i = uint32_t(uint64_t(n - 16u) * (threadIdx.x >> 4) / (BLOCK / 16u - 1u)) + (threadIdx.x & 15u);
+                                            int forder, int desc) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t i = uint32_t(uint64_t(n - 4u) * (lane >> 2) / 15u) + (lane & 3u);
   const uint64_t raw = load_raw<W>(vals, i);
   uint32_t bit;
   const uint32_t vb = load_valid_byte(valid, voff, i, bit);
   K key = 0;
   const int cat = classify_raw<K>(raw, (vb >> bit) & 1u, type, forder, desc, key);
-  count_bin(h, cat == 0 ? uint32_t(key >> (8 * (sizeof(K) - 1))) & 0xFFu : ~0u);
-  __syncthreads();
-  const uint32_t most = n < MSD32_SAVES ? uint32_t(uint64_t(MSD32_TOP_MAX) * BLOCK / n) : uint32_t(BLOCK);
-  const bool over = __syncthreads_or(h[threadIdx.x] > most ? 1 : 0);
-  return __syncthreads_count(h[threadIdx.x] != 0u ? 1 : 0) <= 1 || over;
+  const uint32_t b = cat == 0 ? uint32_t(key >> (8 * (sizeof(K) - 1))) & 0xFFu : ~0u;
+  const unsigned long long counting = __ballot(b != ~0u);
+  if (counting == 0ull) return true;
+  if (__ballot(b == uint32_t(__builtin_amdgcn_readlane(b, __builtin_ctzll(counting)))) == counting) return true;
+  if (n >= MSD32_SAVES) return false;
+  // The digits of eight lanes: a digit on many rows is one of them. Well over the share that makes a bucket too
+  // large, and over what chance gives one of 256 evenly spread digits.
+  uint32_t most = 0;
+#pragma unroll
+  for (int k = 0; k < 64; k += 8) {
+    const uint32_t d = __builtin_amdgcn_readlane(b, k);
+    if (d != ~0u) most = max(most, uint32_t(__popcll(__ballot(b == d))));
+  }
+  const uint32_t share = uint32_t(uint64_t(MSD32_TOP_MAX) * 64u / n);
+  return most > max(8u, share + share / 2u + 4u);
 }
 
 // Every unit's counts, bin-major (unit_hist[b][unit]), and every workgroup's statistics. With guess (32-bit keys),
@@ -377,9 +387,8 @@ __global__ __launch_bounds__(BLOCK) void msd_upsweep(const void* vals, const uin
   __shared__ uint32_t hu[UNITS_PER_BLOCK * NBINS_FIRST];
   __shared__ UpStat s_st[WAVES];
   bool lsd = false;
-  if constexpr (P == 4) lsd = guess && sampled_lsd<K, W>(vals, valid, voff, n, type, forder, desc, hu);
+  if constexpr (P == 4) lsd = guess && sampled_lsd<K, W>(vals, valid, voff, n, type, forder, desc);
   if (blockIdx.x == 0 && threadIdx.x == 0) ctl->lsd = lsd ? 1u : 0u;
-  __syncthreads();
   const uint32_t begin = blockIdx.x * rows_per_block;
   const uint32_t end = min(n, begin + rows_per_block);
   const uint32_t nu = (end - begin + (1u << unit_shift) - 1u) >> unit_shift;

@@ -110,17 +110,33 @@ def test_key_shapes(n):
             check(vals, valid, True, place, label=f"nulls {frac}")
 
 
+@pytest.mark.parametrize("seed", range(6))
+def test_full_range_columns_are_not_taken_for_skewed(seed):
+    """Below 2^24 rows, where a top digit may hold 1 / 64 of the rows, chance alone fills none of the sample."""
+    x = O.splitmix64(seed + 1, (1 << 24) - 5).astype(np.uint32).view(np.int32)
+    a = am.MetalArray.from_numpy(x)
+    am.prof_reset()
+    am.prof_enable(True)
+    got = a.argsort().to_numpy()[0]
+    am.prof_enable(False)
+    names = set(am.prof_report())
+    am.prof_reset()
+    assert "sort_msd_first" in names, sorted(names)
+    if seed == 0:
+        np.testing.assert_array_equal(got, O.argsort(x, None))
+
+
 @pytest.mark.parametrize("n", [1 << 16, 300_001, 2_000_003])
 @pytest.mark.parametrize("case,sweeps", [("small", 1), ("rare", 1), ("sampled_wide", 2), ("all_null", 1), ("one_value", 1),
                                          ("hot", 1)])
 def test_analysis_of_32_bit_columns(case, sweeps, n):
-    """Columns that the LSD passes sort are counted for them in the first analysis, by a sample of 16 neighbours
+    """Columns that the LSD passes sort are counted for them in the first analysis, by a sample of 4 neighbours
     at 16 places; a sample that misses the wide values, or sees nothing else, still leaves a sorted column."""
     rng = np.random.default_rng(n)
     x = rng.integers(-30_000, 30_000, n).astype(np.int32) if case == "hot" else rng.integers(0, 5000, n).astype(np.int32)
     wide = O.splitmix64(9, n).astype(np.uint32).view(np.int32)
     valid = rng.random(n) > 0.1
-    places = ((n - 16) * np.arange(16) // 15)[:, None] + np.arange(16)
+    places = ((n - 4) * np.arange(16) // 15)[:, None] + np.arange(4)
     if case == "rare": x[places[:-1, 0] + 50] = wide[:15]
     elif case == "sampled_wide": x[places.ravel()] = wide[places.ravel()]
     elif case == "all_null": valid[:] = False
