@@ -138,7 +138,8 @@ __global__ __launch_bounds__(1024) void take_nulls(const uint32_t* block_nulls, 
 // 50M float64: 113 + 534 + 152 us, 811 us a call (1010 before); 50M float32: 117 + 453 + 88, 656 us (972). The
 // fetch is still bound by L1 filling a line per row: the same loop reads neighbours in 271 us.
 //
-// Which way a call goes is decided on the device from a sample of the indices: runs of neighbours are
+// Values and indices without nulls only: the passes carry no validity. Which way a call goes is decided on the
+// device from a sample of the indices: runs of neighbours are
 // cheaper read directly, and tk_fetch then is the plain gather: neighbours cost such a call
 // 5 us for the two kernels that return (50M float64 187 and 196, 24M float32 65 and 68).
 constexpr uint32_t TK_TILE = 16384;
