@@ -230,9 +230,10 @@ struct KeyStat {
 constexpr int COMPOSITE_MAX = 8;
 
 // One pass over the keys: each workgroup keeps its own registers in LDS and writes them out as bytes, with
-// the smallest and largest order key and the nulls of its rows (integer keys); gb_key_estimate folds the workgroups' results. Plain stores: raising shared registers with atomics
-// costs an atomic per register and workgroup at the memory side, all of them while the registers are
-// still low (4096 registers, 256 workgroups: 45 us for 3M rows that are read in 5).
+// the smallest and largest order key and the nulls of its rows (integer keys); gb_key_estimate or
+// gb_span_fold folds the workgroups' results. Plain stores: raising shared registers with atomics costs an
+// atomic per register and workgroup at the memory side, all of them while the registers are still low (4096
+// registers, 256 workgroups: 45 us for 3M rows that are read in 5).
 //
 // The key type is a template argument (no type switch per row) and each thread has two steps of
 // SCAN_ROWS rows in flight: the next step's keys and validity bytes are loaded before this step's are
