@@ -4522,8 +4522,13 @@ void group_by_noalloc(const Array& keys, int64_t key_count, int agg, const Array
 //              hash  179/388  241/315    410/313    581/310    711/302    989/304
 //     50M      range 368/2799 389/3149   685/2481   768/2484   1260/2545  2795/2467  4325/2250
 //              hash  564/3269 807/3696   1376/2912  1771/2915  2868/2928  4044/2888  6976/2635
-// So the lines: range path, keys from a twelfth of the rows (and from 16,384: fewer are mapped in less than the
-// partition's launches take); hash, from a 160th while the rows fit in the caches. Beyond, uniform keys cross at a
+// Range path, near the line (rows: keys mapping/partition):
+//     200,000  15,000 110/106  17,000 146/105  20,000 168/106     600,000  15,000 118/119  17,000 158/119
+//     1M       17,000 158/172  20,000 176/172  80,000 197/173     1.5M     55,000 188/203  80,000 205/201
+//     2.5M     160,000 228/235  240,000 243/233                   4M       320,000 265/297  1M 430/279
+// So the lines: range path, keys from a sixth of the rows past 2^20, at most a twelfth of all rows, and from 16,384
+// (fewer are mapped in less than the partition's launches take, or in as much); hash, from a 160th while the rows
+// fit in the caches. Beyond, uniform keys cross at a
 // 50th, Zipf keys, whose hot ones the hash mapping caches and the partition moves level by level, at a tenth
 // (16M rows of 690,000 Zipf keys 899/1289, 50M of 2.3M 2552/3534); they are not told apart, and the line is a 20th.
 bool distinct_by_partition(const CompositeArgs& ca, const KeyStat* stat, unsigned long long top, int64_t n) {
@@ -4531,7 +4536,8 @@ bool distinct_by_partition(const CompositeArgs& ca, const KeyStat* stat, unsigne
   double bound = 1.0;
   for (int c = 0; c < ca.count; c++) bound *= double(std::max<unsigned long long>(stat[c].est, 1)) + ca.col[c].span.has_null;
   keys = std::min({keys, bound, double(n)});
-  if (top <= range_limit(n) && range_path_enabled()) return keys >= 16384.0 && keys * 12.0 >= double(n);
+  if (top <= range_limit(n) && range_path_enabled())
+    return keys >= std::max(16384.0, std::min((double(n) - double(1 << 20)) / 6.0, double(n) / 12.0));
   return keys * (n <= (int64_t(1) << 23) ? 160.0 : 20.0) >= double(n);
 }
 

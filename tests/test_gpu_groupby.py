@@ -352,8 +352,10 @@ def test_unique_rows_by_partition(case, n):
 
 
 @pytest.mark.parametrize("n,keys,form,partition", [
-    (100_003, 16_000, "dense", False), (100_003, 20_000, "dense", True), (1_000_003, 60_000, "dense", False),
-    (1_000_003, 120_000, "dense", True), (1_000_003, 120_000, "pair", True), (1_000_003, 3_000, "pair", False),
+    (100_003, 16_000, "dense", False), (100_003, 20_000, "dense", True), (1_000_003, 16_000, "dense", False),
+    (1_000_003, 20_000, "dense", True), (1_500_003, 60_000, "dense", False), (1_500_003, 95_000, "dense", True),
+    (3_000_017, 210_000, "dense", False), (3_000_017, 300_000, "dense", True),
+    (1_000_003, 120_000, "pair", True), (1_000_003, 3_000, "pair", False),
     (1_000_003, 4_000, "wide", False), (1_000_003, 9_000, "wide", True), (9_000_001, 400_000, "wide", False),
     (9_000_001, 520_000, "wide", True), (9_000_001, 4_000, "zipf", False), (800_003, 800_003, "dense", True),
     (400_003, 400_003, "nulls", True), (1_200_001, 900_000, "nulls", True)])
