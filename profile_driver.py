@@ -101,12 +101,12 @@ def summarize(fetch_dir: str, write_dir: str, n: int = 50_000_000) -> str:
     lines = [
         "# rocprofv3 PMC: HBM traffic per dispatch, ORDER BY 50M (two calls and through the plan) + group-by 50M",
         "",
-        "commands (from the repo root, R = repo root; each counter in its own run):",
-        "  cd /tmp && timeout -s KILL 240 rocprofv3 --pmc FETCH_SIZE --output-format csv -d $R/gpurun_out/pmc_fetch "
+        "commands (from the repo root, R = repo root, OUT = a scratch folder; each counter in its own run):",
+        "  cd /tmp && timeout -s KILL 240 rocprofv3 --pmc FETCH_SIZE --output-format csv -d $OUT/pmc_fetch "
         "-o run -- python3 $R/profile_driver.py",
-        "  cd /tmp && timeout -s KILL 240 rocprofv3 --pmc WRITE_SIZE --output-format csv -d $R/gpurun_out/pmc_write "
+        "  cd /tmp && timeout -s KILL 240 rocprofv3 --pmc WRITE_SIZE --output-format csv -d $OUT/pmc_write "
         "-o run -- python3 $R/profile_driver.py",
-        "  python3 profile_driver.py --summarize gpurun_out/pmc_fetch gpurun_out/pmc_write",
+        "  python3 profile_driver.py --summarize $OUT/pmc_fetch $OUT/pmc_write",
         "",
         "workload: profile_driver.py (3 ORDER BY steps over 50M int64 keys with 2% nulls, 3 ORDER BY steps of the "
         "same table through am_plan_run, 2 group-by steps over 50M Zipf(1.1) keys from 100k values, then three "
